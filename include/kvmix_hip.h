@@ -393,6 +393,57 @@ typedef struct kvmix_rope_append {
 int kvmix_rope_append(const kvmix_rope_append_t *step, kvmix_stream_t stream);
 
 /*
+ * A projection of a decode step, y[m][n] = sum_k x[m][k] w[n][k] for up to sixteen rows m (one per sequence; fp16
+ * operands, fp32 sums), with what stands around it in a decoder layer in the same launch.  No operator of the
+ * reference: it is the torch modules around LlamaAttention_KVmix's cache code
+ * (models/modeling_llama_KVmix.py:84-112,268-283) and the stock layer around that.
+ *
+ *   x            [m, k] fp16, row stride x_stride
+ *   norm_weight  NULL, or [k] fp16: x is RMS-normalised first (fp32, rounded to fp16 once, as rms_norm does)
+ *   w[0..2]      row-major [rows, k] fp16 matrices, one row stride; which are used depends on the epilogue:
+ *   KVMIX_LINEAR_PLAIN        out [m, rows[0]] fp16
+ *   KVMIX_LINEAR_FLOAT        out [m, rows[0]] fp32 holding the values rounded to fp16
+ *   KVMIX_LINEAR_RESIDUAL     out = residual + fp16(w[0] x), fp16; out may be residual
+ *   KVMIX_LINEAR_SWIGLU       out [m, rows[0]] = fp16(silu(fp16(w[0] x))) * fp16(w[1] x), rows[1] == rows[0]
+ *   KVMIX_LINEAR_ROPE_APPEND  w = query, key, value projections (rows = heads * head_dim, kv_heads * head_dim twice):
+ *                             out = rotated queries [m, rows[0]]; the rotated keys and the values go to slot k_slot /
+ *                             v_slot of the tail windows, exactly as kvmix_rope_append writes them; cos, sin
+ *                             [head_dim] fp16 per sequence, cos_sin_batch_stride elements apart (0: shared)
+ * k a multiple of 128, rows 16-byte aligned, m <= 16 and the x rows small enough to stay in registers, else
+ * KVMIX_ERR_UNSUPPORTED: kvmix_linear_rows_supported tells (every epilogue takes k <= 4096; the plain ones without a
+ * norm k <= 6144, k <= 11264 for m <= 8, k <= 14336 for m <= 4).  Only sizes, strides and the pointers' alignment are
+ * read there.
+ */
+#define KVMIX_LINEAR_PLAIN 0
+#define KVMIX_LINEAR_FLOAT 1
+#define KVMIX_LINEAR_RESIDUAL 2
+#define KVMIX_LINEAR_SWIGLU 3
+#define KVMIX_LINEAR_ROPE_APPEND 4
+typedef struct kvmix_linear_rows {
+    const void *x;
+    int64_t x_stride, m, k;
+    const void *norm_weight;
+    float norm_eps;
+    int epilogue;
+    const void *w[3];
+    int64_t w_stride, rows[3];
+    const void *residual;
+    int64_t residual_stride;
+    void *out;
+    int64_t out_stride;
+    const void *cos, *sin;
+    int64_t cos_sin_batch_stride, head_dim;
+    void *k_tail;
+    int64_t k_tail_batch_stride, k_tail_head_stride, k_tail_token_stride, k_tail_slots, k_slot;
+    const int64_t *k_slot_dev;
+    void *v_tail;
+    int64_t v_tail_batch_stride, v_tail_head_stride, v_tail_token_stride, v_tail_slots, v_slot;
+    const int64_t *v_slot_dev;
+} kvmix_linear_rows_t;
+int kvmix_linear_rows_supported(const kvmix_linear_rows_t *step);
+int kvmix_linear_rows(const kvmix_linear_rows_t *step, kvmix_stream_t stream);
+
+/*
  * Measurement support, no counterpart in the reference and not called by any operator: a kernel
  * that only reads, in the access patterns of the GEMV kernels, to establish what streaming rate
  * the GPU reaches without arithmetic (the ceiling the GEMV figures are compared with), and how

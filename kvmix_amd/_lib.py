@@ -36,6 +36,8 @@ EXPORTS = (
     "kvmix_decode_attention_fused",
     "kvmix_decode_attention_fused_plan",
     "kvmix_rope_append",
+    "kvmix_linear_rows_supported",
+    "kvmix_linear_rows",
     "kvmix_probe_stream_read",
 )
 
@@ -91,6 +93,22 @@ class RopeAppend(ctypes.Structure):
                 ("v_tail", _vp), ("v_tail_batch_stride", _i64), ("v_tail_head_stride", _i64),
                 ("v_tail_token_stride", _i64), ("v_tail_slots", _i64), ("v_slot", _i64), ("v_slot_dev", _vp),
                 ("batch", _i64), ("heads", _i32), ("kv_heads", _i32), ("D", _i64)]
+
+
+class LinearRows(ctypes.Structure):
+    """kvmix_linear_rows_t"""
+    _i64, _i32, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p
+    _fields_ = [("x", _vp), ("x_stride", _i64), ("m", _i64), ("k", _i64), ("norm_weight", _vp), ("norm_eps", ctypes.c_float),
+                ("epilogue", _i32), ("w", _vp * 3), ("w_stride", _i64), ("rows", _i64 * 3), ("residual", _vp),
+                ("residual_stride", _i64), ("out", _vp), ("out_stride", _i64), ("cos", _vp), ("sin", _vp),
+                ("cos_sin_batch_stride", _i64), ("head_dim", _i64),
+                ("k_tail", _vp), ("k_tail_batch_stride", _i64), ("k_tail_head_stride", _i64),
+                ("k_tail_token_stride", _i64), ("k_tail_slots", _i64), ("k_slot", _i64), ("k_slot_dev", _vp),
+                ("v_tail", _vp), ("v_tail_batch_stride", _i64), ("v_tail_head_stride", _i64),
+                ("v_tail_token_stride", _i64), ("v_tail_slots", _i64), ("v_slot", _i64), ("v_slot_dev", _vp)]
+
+
+LINEAR_PLAIN, LINEAR_FLOAT, LINEAR_RESIDUAL, LINEAR_SWIGLU, LINEAR_ROPE_APPEND = range(5)
 
 
 class GemvPlan(ctypes.Structure):
@@ -160,6 +178,10 @@ def load() -> ctypes.CDLL:
     L.kvmix_decode_attention_fused_plan.argtypes = [ctypes.POINTER(DecodeAttn), ctypes.POINTER(AttnPlan)]
     L.kvmix_rope_append.restype = i32
     L.kvmix_rope_append.argtypes = [ctypes.POINTER(RopeAppend), vp]
+    L.kvmix_linear_rows_supported.restype = i32
+    L.kvmix_linear_rows_supported.argtypes = [ctypes.POINTER(LinearRows)]
+    L.kvmix_linear_rows.restype = i32
+    L.kvmix_linear_rows.argtypes = [ctypes.POINTER(LinearRows), vp]
     L.kvmix_probe_stream_read.restype = i32
     L.kvmix_probe_stream_read.argtypes = [vp, i32, i64, i64, i32, i32, i32, i32, i32, vp, vp]
     _lib = L

@@ -4,18 +4,19 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libkvmix_hip.so")
-SOURCES = ["abi.hip", "quant_pack.hip", "dequant_gemv.hip", "decode_attn.hip", "fused_attn.hip", "rope_append.hip", "stream_probe.hip"]
+SOURCES = ["abi.hip", "quant_pack.hip", "dequant_gemv.hip", "decode_attn.hip", "fused_attn.hip", "linear_rows.hip", "rope_append.hip", "stream_probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-fno-fast-math",
     # packed fp32 instructions are kept out of the generated code on purpose
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -23,11 +24,20 @@ HIPCC_FLAGS = [
 
 
 def build(verbose: bool = False) -> str:
+    """Compiles every source (in parallel: one of them takes as long as all the others) and links the library."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    cmd = [hipcc] + HIPCC_FLAGS + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", LIB]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.check_call(cmd)
+    with tempfile.TemporaryDirectory() as tmp:
+        objects = [os.path.join(tmp, s + ".o") for s in SOURCES]
+
+        def compile_one(pair):
+            cmd = [hipcc] + HIPCC_FLAGS + ["-c", os.path.join(CSRC, pair[0]), "-o", pair[1]]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            subprocess.check_call(cmd)
+
+        with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+            list(pool.map(compile_one, zip(SOURCES, objects)))
+        subprocess.check_call([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objects + ["-o", LIB])
     return LIB
 
 

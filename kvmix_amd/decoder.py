@@ -93,6 +93,58 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return x * cos + rot * sin
 
 
+def _few_rows(x: torch.Tensor) -> bool:
+    """One new token of a few fp16 sequences on the GPU: the projections then go through the library's kernels, which
+    stream the weights and take the normalisation before and the elementwise work after along (kvmix_linear_rows)."""
+    return x.is_cuda and x.dtype == torch.float16 and x.shape[1] == 1
+
+
+def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tensor, sin: torch.Tensor, k_tail: torch.Tensor,
+                 v_tail: torch.Tensor, k_slot, v_slot) -> torch.Tensor:
+    """One new token: norm, q/k/v projections, RoPE; keys and values to the given slots of the tail windows, the
+    rotated queries [B,nh,1,D] returned."""
+    from . import _lib, ops
+
+    h, kvh = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
+    if ops.linear_rows_supported(x.shape[0], x.shape[2], h, _lib.LINEAR_ROPE_APPEND, True, cfg.head_dim, kvh):
+        return ops.qkv_rope_append(x, lw["wqkv"], cfg.num_heads, cfg.num_kv_heads, cos, sin, k_tail, v_tail, k_slot, v_slot,
+                                   lw["input_norm"], cfg.rms_norm_eps)
+    qkv = F.linear(rms_norm(x, lw["input_norm"], cfg.rms_norm_eps), lw["wqkv"])
+    return ops.rope_append(qkv, cos, sin, cfg.num_heads, cfg.num_kv_heads, k_tail, v_tail, k_slot, v_slot)
+
+
+def add_projection(x: torch.Tensor, h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x + h @ w.T"""
+    if _few_rows(x):
+        from . import _lib, ops
+
+        if ops.linear_rows_supported(h.shape[0], h.shape[2], w.shape[0], _lib.LINEAR_RESIDUAL):
+            return ops.linear_rows(h, w, residual=x)
+    return x + F.linear(h, w)
+
+
+def add_mlp(x: torch.Tensor, lw: dict, eps: float) -> torch.Tensor:
+    """x + mlp(norm(x))"""
+    w = lw["w_gate_up"]
+    if _few_rows(x):
+        from . import _lib, ops
+
+        if ops.linear_rows_supported(x.shape[0], x.shape[2], w.shape[0] // 2, _lib.LINEAR_SWIGLU, True):
+            return add_projection(x, ops.swiglu_rows(x, w, lw["post_norm"], eps), lw["w_down"])
+    return x + mlp(rms_norm(x, lw["post_norm"], eps), w, lw["w_down"])
+
+
+def head_logits(x: torch.Tensor, weights: dict, eps: float) -> torch.Tensor:
+    """x [B,1,hidden] -> logits [B, vocab], fp32 holding the head's output in the weights' type"""
+    w = weights["lm_head"]
+    if _few_rows(x):
+        from . import _lib, ops
+
+        if ops.linear_rows_supported(x.shape[0], x.shape[2], w.shape[0], _lib.LINEAR_FLOAT, True):
+            return ops.linear_rows(x[:, 0], w, weights["norm"], eps, fp32=True)
+    return F.linear(rms_norm(x[:, 0], weights["norm"], eps), w).to(torch.float32)
+
+
 class Decoder:
     """weights: the dict of init_weights; attention: one callable per layer with the signature
     attention(q [B,nh,Q,D], k [B,nkv,Q,D], v [B,nkv,Q,D], cache, attention_mask=..., need_weights=False) ->
@@ -124,16 +176,17 @@ class Decoder:
 
             flush_ahead(self.caches)
         for li, lw in enumerate(self.w["layers"]):
-            h = rms_norm(x, lw["input_norm"], cfg.rms_norm_eps)
-            q, k, v = project_qkv(cfg, h, lw["wqkv"], cos, sin)
+            if _few_rows(x):
+                k, v = (torch.empty((B, cfg.num_kv_heads, 1, cfg.head_dim), dtype=x.dtype, device=x.device) for _ in range(2))
+                q = qkv_of_token(cfg, x, lw, cos, sin, k, v, 0, 0)
+            else:
+                h = rms_norm(x, lw["input_norm"], cfg.rms_norm_eps)
+                q, k, v = project_qkv(cfg, h, lw["wqkv"], cos, sin)
             out, _, self.caches[li] = self.attention[li](q, k, v, self.caches[li], attention_mask=mask, need_weights=False)
-            out = out.transpose(1, 2).reshape(B, Q, cfg.hidden_size)
-            x = x + F.linear(out, lw["wo"])
-            h = rms_norm(x, lw["post_norm"], cfg.rms_norm_eps)
-            x = x + mlp(h, lw["w_gate_up"], lw["w_down"])
+            x = add_projection(x, out.transpose(1, 2).reshape(B, Q, cfg.hidden_size), lw["wo"])
+            x = add_mlp(x, lw, cfg.rms_norm_eps)
         self.position += Q
-        x = rms_norm(x[:, -1], self.w["norm"], cfg.rms_norm_eps)
-        return F.linear(x, self.w["lm_head"]).to(torch.float32)
+        return head_logits(x[:, -1:], self.w, cfg.rms_norm_eps)
 
     def generate(self, prompt_ids: torch.Tensor, new_tokens: int, on_step: Optional[Callable] = None) -> torch.Tensor:
         """Greedy decoding: returns the new token ids [B, new_tokens].  on_step(step, logits) is
@@ -199,11 +252,9 @@ class GraphDecoder(Decoder):
         cos, sin = emb.cos()[None, None].to(x.dtype), emb.sin()[None, None].to(x.dtype)
         for li, lw in enumerate(self.w["layers"]):
             cache = self.caches[li]
-            h = rms_norm(x, lw["input_norm"], cfg.rms_norm_eps)
             kwin, vwin, _, _ = cache.tail_windows(R)
             (kslot, klive), (vslot, vlive) = self._len[li]
-            # rotary embedding of q and k and the append of k and v to the tail windows: one launch
-            q = ops.rope_append(F.linear(h, lw["wqkv"]), cos, sin, cfg.num_heads, cfg.num_kv_heads, kwin, vwin, kslot, vslot)
+            q = qkv_of_token(cfg, x, lw, cos, sin, kwin, vwin, kslot, vslot)
             kc, _, ks, km, vc, _, vs, vm, _ = cache.as_tuple()
             width = max(cache.k_tokens, cache.v_tokens) + R
             single = ops.prefer_single_pass(B, cfg.num_heads, cfg.num_kv_heads, D, width, cache.k_bits, cache.k_fmt,
@@ -212,16 +263,13 @@ class GraphDecoder(Decoder):
             out, _ = ops.decode_attention(q, (kc, ks, km), (vc, vs, vm), kwin, vwin, cache.Kgroup_size, cache.k_bits,
                                           cache.Vgroup_size, cache.v_bits, cache.k_fmt, cache.v_fmt,
                                           k_tail_len=klive, v_tail_len=vlive, single_pass=single)
-            out = out.transpose(1, 2).reshape(B, 1, cfg.hidden_size)
-            x = x + F.linear(out, lw["wo"])
-            h = rms_norm(x, lw["post_norm"], cfg.rms_norm_eps)
-            x = x + mlp(h, lw["w_gate_up"], lw["w_down"])
+            x = add_projection(x, out.transpose(1, 2).reshape(B, 1, cfg.hidden_size), lw["wo"])
+            x = add_mlp(x, lw, cfg.rms_norm_eps)
         self._pos.add_(1)
         for slot, live in self._counters.values():
             slot.add_(1)
             live.add_(1)
-        x = rms_norm(x[:, -1], self.w["norm"], cfg.rms_norm_eps)
-        return F.linear(x, self.w["lm_head"]).to(torch.float32)
+        return head_logits(x, self.w, cfg.rms_norm_eps)
 
     def _sync_counters(self) -> None:
         """Device counters for the coming steps.  Tails of equal length stay equal until the next

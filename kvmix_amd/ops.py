@@ -329,6 +329,21 @@ def prefer_single_pass(batch: int, heads: int, kv_heads: int, head_dim: int, wid
         return False
 
 
+def _set_tail(st, prefix: str, tail: torch.Tensor, slot) -> None:
+    """The fields of a tail window and the slot the new token goes to (an int, or a device int64 read by the kernel)."""
+    setattr(st, prefix + "_tail", tail.data_ptr())
+    setattr(st, prefix + "_tail_batch_stride", tail.stride(0))
+    setattr(st, prefix + "_tail_head_stride", tail.stride(1))
+    setattr(st, prefix + "_tail_token_stride", tail.stride(2))
+    setattr(st, prefix + "_tail_slots", tail.shape[2])
+    if torch.is_tensor(slot):
+        if slot.dtype != torch.int64 or slot.numel() != 1 or not slot.is_cuda:
+            raise RuntimeError("a device-side slot must be one int64 element on the GPU")
+        setattr(st, prefix + "_slot_dev", slot.data_ptr())
+    else:
+        setattr(st, prefix + "_slot", int(slot))
+
+
 def rope_append(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, heads: int, kv_heads: int,
                 k_tail: torch.Tensor, v_tail: torch.Tensor, k_slot, v_slot) -> torch.Tensor:
     """Rotary embedding of the new token's query and key heads and the append of its key and value
@@ -362,21 +377,133 @@ def rope_append(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, heads: 
     st.qkv, st.qkv_batch_stride, st.cos, st.sin = qkv.data_ptr(), qkv.stride(0) if B > 1 else total * D, cos.data_ptr(), sin.data_ptr()
     st.q_out, st.q_batch_stride = q_out.data_ptr(), heads * D
     for prefix, tail, slot in (("k", k_tail, k_slot), ("v", v_tail, v_slot)):
-        setattr(st, prefix + "_tail", tail.data_ptr())
-        setattr(st, prefix + "_tail_batch_stride", tail.stride(0))
-        setattr(st, prefix + "_tail_head_stride", tail.stride(1))
-        setattr(st, prefix + "_tail_token_stride", tail.stride(2))
-        setattr(st, prefix + "_tail_slots", tail.shape[2])
-        if torch.is_tensor(slot):
-            if slot.dtype != torch.int64 or slot.numel() != 1 or not slot.is_cuda:
-                raise RuntimeError("a device-side slot must be one int64 element on the GPU")
-            setattr(st, prefix + "_slot_dev", slot.data_ptr())
-        else:
-            setattr(st, prefix + "_slot", int(slot))
+        _set_tail(st, prefix, tail, slot)
     st.batch, st.heads, st.kv_heads, st.D = B, heads, kv_heads, D
     with torch.cuda.device(qkv.device):
         _lib.check(_lib.load().kvmix_rope_append(ctypes.byref(st), _stream(qkv)))
     return q_out
+
+
+@functools.lru_cache(maxsize=None)
+def linear_rows_supported(m: int, k: int, rows: int, epilogue: int = _lib.LINEAR_PLAIN, norm: bool = False,
+                          head_dim: int = 0, kv_rows: int = 0) -> bool:
+    """Whether kvmix_linear_rows takes a projection of these sizes (dense fp16 rows; asks the library)."""
+    import ctypes
+
+    st = _lib.LinearRows()
+    st.m, st.k, st.x_stride, st.w_stride, st.epilogue = m, k, k, k, epilogue
+    st.rows[0], st.out_stride, st.residual_stride = rows, rows, rows
+    st.norm_weight = 16 if norm else None
+    if epilogue == _lib.LINEAR_SWIGLU:
+        st.rows[1] = rows
+    if epilogue == _lib.LINEAR_ROPE_APPEND:
+        st.rows[1] = st.rows[2] = kv_rows
+        st.head_dim = st.k_tail_token_stride = st.v_tail_token_stride = head_dim
+        st.k_tail_slots = st.v_tail_slots = 1
+    return bool(_lib.load().kvmix_linear_rows_supported(ctypes.byref(st)))
+
+
+def _rows2(t: torch.Tensor, what: str) -> torch.Tensor:
+    """[..., n] fp16 as [rows, n] with unit-stride rows."""
+    if t.dtype != torch.float16:
+        raise RuntimeError(f"expected scalar type Half for {what} but found {t.dtype}")
+    t = t.reshape(-1, t.shape[-1])
+    return t if t.stride(1) == 1 and t.stride(0) >= t.shape[1] else t.contiguous()
+
+
+def _linear_descriptor(x, w, split, epilogue, norm_weight, eps):
+    """w: one stacked weight, cut into parts of `split` rows, or a tuple with one weight per part."""
+    st = _lib.LinearRows()
+    x = _rows2(x, "x")
+    ws = w if isinstance(w, (tuple, list)) else (w,)
+    _need_gpu(x, *ws)
+    st.x, st.m, st.k = x.data_ptr(), x.shape[0], x.shape[1]
+    st.x_stride = x.stride(0) if x.shape[0] > 1 else x.shape[1]
+    st.epilogue = epilogue
+    for t in ws:
+        if t.dtype != torch.float16 or t.dim() != 2 or t.shape[1] != x.shape[1] or t.stride(1) != 1 or t.stride(0) != ws[0].stride(0):
+            raise RuntimeError("weights must be fp16 [rows, k] with unit-stride rows and one row stride")
+    st.w_stride = ws[0].stride(0)
+    if len(ws) == 1:
+        if sum(split) != ws[0].shape[0]:
+            raise RuntimeError("the stacked weight must hold the rows of all its parts")
+        at = ws[0].data_ptr()
+        for j, n in enumerate(split):
+            st.w[j], st.rows[j] = at, n
+            at += 2 * n * st.w_stride
+    else:
+        for j, t in enumerate(ws):
+            st.w[j], st.rows[j] = t.data_ptr(), t.shape[0]
+    if norm_weight is not None:
+        if norm_weight.dtype != torch.float16 or norm_weight.numel() != x.shape[1] or not norm_weight.is_contiguous():
+            raise RuntimeError("norm_weight must be k contiguous fp16 values")
+        st.norm_weight, st.norm_eps = norm_weight.data_ptr(), eps
+    return st, x
+
+
+def _linear_launch(st, x) -> None:
+    import ctypes
+
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.load().kvmix_linear_rows(ctypes.byref(st), _stream(x)))
+
+
+def linear_rows(x: torch.Tensor, w: torch.Tensor, norm_weight: torch.Tensor = None, eps: float = 0.0,
+                residual: torch.Tensor = None, fp32: bool = False) -> torch.Tensor:
+    """x @ w.T for a few rows of x (kvmix_linear_rows): x [..., k], w [n, k] fp16 -> [..., n].  norm_weight: x is
+    RMS-normalised first; residual [..., n]: added to the fp16 product; fp32: the fp16 product as fp32."""
+    epilogue = _lib.LINEAR_RESIDUAL if residual is not None else (_lib.LINEAR_FLOAT if fp32 else _lib.LINEAR_PLAIN)
+    n = w.shape[0]
+    st, x2 = _linear_descriptor(x, w, (n,), epilogue, norm_weight, eps)
+    out = torch.empty(x.shape[:-1] + (n,), dtype=torch.float32 if fp32 else torch.float16, device=x.device)
+    if residual is not None:
+        residual = _rows2(residual, "residual")
+        if residual.shape != (x2.shape[0], n):
+            raise RuntimeError("residual must have the shape of the product")
+        st.residual, st.residual_stride = residual.data_ptr(), residual.stride(0) if residual.shape[0] > 1 else n
+    st.out, st.out_stride = out.data_ptr(), n
+    _linear_launch(st, x2)
+    return out
+
+
+def swiglu_rows(x: torch.Tensor, w, norm_weight: torch.Tensor = None, eps: float = 0.0) -> torch.Tensor:
+    """silu(x @ gate.T) * (x @ up.T) for a few rows of x, fp16, in one launch (kvmix_linear_rows); w = the stacked
+    [2 n, k] weight, gate over up, or the pair."""
+    n = w[0].shape[0] if isinstance(w, (tuple, list)) else w.shape[0] // 2
+    st, x2 = _linear_descriptor(x, w, (n, n), _lib.LINEAR_SWIGLU, norm_weight, eps)
+    out = torch.empty(x.shape[:-1] + (n,), dtype=torch.float16, device=x.device)
+    st.out, st.out_stride = out.data_ptr(), n
+    _linear_launch(st, x2)
+    return out
+
+
+def qkv_rope_append(x: torch.Tensor, w, heads: int, kv_heads: int, cos: torch.Tensor, sin: torch.Tensor,
+                    k_tail: torch.Tensor, v_tail: torch.Tensor, k_slot, v_slot, norm_weight: torch.Tensor = None,
+                    eps: float = 0.0) -> torch.Tensor:
+    """The query, key and value projections of one new token per sequence, the rotary embedding of queries and keys and
+    the append to the tail windows, in one launch: rope_append(linear(x)) with the same roundings.
+
+    x [B, (1,) k]; w = the stacked [(heads + 2 kv_heads) D, k] weight or the (query, key, value) weights; cos, sin: D
+    values shared by the sequences, or [B, (1,) D]; tails and slots as in rope_append.
+    Returns the rotated queries [B, heads, 1, D]."""
+    D = k_tail.shape[-1]
+    st, x2 = _linear_descriptor(x, w, (heads * D, kv_heads * D, kv_heads * D), _lib.LINEAR_ROPE_APPEND, norm_weight, eps)
+    B = x2.shape[0]
+    for t in (cos, sin):
+        if t.dtype != torch.float16 or t.numel() not in (D, B * D):
+            raise RuntimeError("qkv_rope_append: cos and sin must hold head_dim fp16 values, shared or per sequence")
+    cos, sin = cos.reshape(-1, D).contiguous(), sin.reshape(-1, D).contiguous()
+    if cos.shape != sin.shape:
+        raise RuntimeError("qkv_rope_append: cos and sin must have the same shape")
+    st.cos, st.sin, st.cos_sin_batch_stride, st.head_dim = cos.data_ptr(), sin.data_ptr(), D if cos.shape[0] > 1 else 0, D
+    for prefix, tail, slot in (("k", k_tail, k_slot), ("v", v_tail, v_slot)):
+        if tail.dtype != torch.float16 or tail.dim() != 4 or tail.shape[:2] != (B, kv_heads) or tail.shape[3] != D or tail.stride(3) != 1:
+            raise RuntimeError("qkv_rope_append: tails must be fp16 [B, kv_heads, slots, D] with unit stride along D")
+        _set_tail(st, prefix, tail, slot)
+    q = torch.empty((B, heads, 1, D), dtype=torch.float16, device=x.device)
+    st.out, st.out_stride = q.data_ptr(), heads * D
+    _linear_launch(st, x2)
+    return q
 
 
 @functools.lru_cache(maxsize=None)

@@ -1,0 +1,107 @@
+"""ops.linear_rows / swiglu_rows / qkv_rope_append (kvmix_linear_rows) against the torch modules they stand for.
+
+Reference: the product in float64 of the fp16 operands, rounded to fp16, then the elementwise work in fp16 tensor
+arithmetic.  The kernel sums in fp32 (error at most k * 2^-24 of the sum of magnitudes), which can turn a rounding to
+fp16 over (2^-10 of the value); with a norm, rms_norm's own fp32 arithmetic can turn over the rounding of an element of
+x as well (at worst of every one: 2^-10 of the sum of magnitudes)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+ULP = 2.0 ** -10
+
+
+def operands(dev, m, k, n):
+    gen = torch.Generator(device="cpu").manual_seed(1000 * m + k + n)
+    r = lambda *s: torch.randn(*s, generator=gen).to(dev).half()  # noqa: E731
+    return r(m, k), (0.03 * r(n, k)).half(), (1 + 0.2 * r(k)).half(), r(m, n)
+
+
+def product(x, w):
+    return (x.double() @ w.double().t()).half(), x.double().abs() @ w.double().abs().t()
+
+
+def within(got, want, bound):
+    assert got.shape == want.shape
+    err = (got.double() - want.double()).abs()
+    assert (err <= bound).all(), float((err - bound).max())
+    assert float(err.norm()) <= ULP / 2 * float(want.double().norm())  # (in the mean: the rounding of the output)
+
+
+# rows of x around the groups of four sequences, k around the chunks of 128 elements and the eight waves, n around the
+# tiles of four rows and the blocks
+@pytest.mark.parametrize("m,k,n", [(1, 128, 1), (1, 1024, 6), (3, 1152, 255), (4, 2048, 1026), (5, 2176, 61), (8, 4096, 300),
+                                   (9, 4096, 130), (16, 4096, 4099), (4, 5632, 513), (16, 6144, 77), (2, 8192, 64),
+                                   (8, 11008, 259), (4, 14336, 65)])
+def test_plain_float_residual(dev, m, k, n):
+    from kvmix_amd import ops
+
+    x, w, _, res = operands(dev, m, k, n)
+    assert ops.linear_rows_supported(m, k, n)
+    y, mag = product(x, w)
+    bound = ULP * y.double().abs() + k * 2.0 ** -24 * mag
+    got = ops.linear_rows(x, w)
+    within(got, y, bound)
+    assert torch.equal(got, ops.linear_rows(x, w))
+    f = ops.linear_rows(x, w, fp32=True)
+    assert f.dtype == torch.float32 and torch.equal(f, got.float())
+    assert torch.equal(ops.linear_rows(x, w, residual=res), res + got)  # the sum in fp16 tensor arithmetic
+    wide = torch.zeros(m, k + 64, device=dev, dtype=torch.float16)      # rows of a larger tensor
+    wide[:, :k] = x
+    assert torch.equal(ops.linear_rows(wide[:, :k], w), got)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 256, 4), (4, 4096, 1001), (7, 2048, 129), (16, 4096, 64), (4, 8192, 31), (8, 6144, 10)])
+def test_norm_and_swiglu(dev, m, k, n):
+    from kvmix_amd import ops
+
+    x, w, nw, _ = operands(dev, m, k, 2 * n)
+    xn = F.rms_norm(x, (k,), nw, 1e-5)
+    y, mag = product(xn, w)
+    got = ops.linear_rows(x, w, nw, 1e-5)
+    within(got, y, ULP * (y.double().abs() + mag))
+    for norm in (None, nw):
+        a = got if norm is not None else ops.linear_rows(x, w)
+        want = F.silu(a[:, :n]) * a[:, n:]
+        s = ops.swiglu_rows(x, w, norm, 1e-5)
+        within(s, want, 4 * ULP * want.double().abs() + 2.0 ** -24)  # expf here and torch's: a rounding of each of two steps
+        assert torch.equal(s, ops.swiglu_rows(x, (w[:n], w[n:]), norm, 1e-5))
+
+
+@pytest.mark.parametrize("m,k,heads,kv,D,per_row", [(1, 256, 2, 1, 64, False), (4, 4096, 32, 8, 128, True), (16, 2048, 3, 3, 128, False),
+                                                    (5, 512, 4, 2, 32, True), (3, 1024, 1, 1, 8, False)])
+def test_qkv_rope_append_is_the_composition(dev, m, k, heads, kv, D, per_row):
+    from kvmix_amd import ops
+
+    x, w, nw, _ = operands(dev, m, k, (heads + 2 * kv) * D)
+    gen = torch.Generator(device="cpu").manual_seed(7)
+    cos, sin = (torch.randn(m if per_row else 1, 1, D, generator=gen).to(dev).half() for _ in range(2))
+    kt, vt = (torch.zeros(m, kv, 6, D, device=dev, dtype=torch.float16) for _ in range(2))
+    slot = torch.tensor([3], device=dev)
+    q = ops.qkv_rope_append(x, w, heads, kv, cos, sin, kt[:, :, 1:], vt, slot, 2, nw, 1e-5)
+    y = ops.linear_rows(x, w, nw, 1e-5).view(m, heads + 2 * kv, D)
+    rot = torch.cat([-y[..., D // 2:], y[..., :D // 2]], -1)
+    want = y * cos + rot * sin
+    assert torch.equal(q[:, :, 0], want[:, :heads])
+    assert torch.equal(kt[:, :, 4], want[:, heads:heads + kv]) and torch.equal(vt[:, :, 2], y[:, heads + kv:])
+    kt[:, :, 4] = 0
+    vt[:, :, 2] = 0
+    assert not kt.any() and not vt.any()
+    ops.qkv_rope_append(x, w, heads, kv, cos, sin, kt, vt, torch.tensor([6], device=dev), torch.tensor([-1], device=dev), nw, 1e-5)
+    assert not kt.any() and not vt.any()  # a device-side slot outside the window writes nothing
+
+
+def test_refusals(dev):
+    from kvmix_amd import ops
+
+    x, w, nw, res = operands(dev, 4, 256, 8)
+    assert not ops.linear_rows_supported(17, 256, 8) and not ops.linear_rows_supported(4, 200, 8)
+    with pytest.raises(RuntimeError):
+        ops.linear_rows(x[:, :200].contiguous(), w[:, :200].contiguous())
+    with pytest.raises(RuntimeError):
+        ops.linear_rows(x, w, residual=res[:2])
+    with pytest.raises(RuntimeError):
+        ops.linear_rows(x.float(), w)
+    with pytest.raises(RuntimeError):
+        ops.qkv_rope_append(x, w, 1, 1, nw[:2], nw[:2], *(torch.zeros(4, 1, 2, 2, device=dev).half() for _ in range(2)), 0, 0)
