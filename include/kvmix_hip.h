@@ -444,6 +444,39 @@ int kvmix_linear_rows_supported(const kvmix_linear_rows_t *step);
 int kvmix_linear_rows(const kvmix_linear_rows_t *step, kvmix_stream_t stream);
 
 /*
+ * Dense attention of a prompt: out = softmax(q k^T * scale + mask) v (the prompt branch of the attention layer,
+ * models/modeling_llama_KVmix.py:252-266, where nobody reads the probabilities).
+ *
+ *   q [batch, heads, q_len, head_dim], k, v [batch, kv_heads, kv_len, head_dim], out [batch, heads, q_len, head_dim]:
+ *   fp16, unit stride along head_dim, strides in elements (of q, k, v multiples of 8, base addresses 16-byte aligned; of
+ *   out multiples of 4); query head h reads kv head h / (heads / kv_heads); head_dim 64 or 128.
+ *   mask: NULL, or an additive mask [mask_batch, mask_heads, q_len, kv_len] of mask_dtype with unit stride along kv_len;
+ *   mask_batch 1 or batch, mask_heads 1 or heads.  Its entries are clamped below at -65504 and rounded to fp16; a row of
+ *   which every entry is at most -65504 (fp16) or -1e30 (fp32) weighs all positions alike.
+ * Logits, softmax and sums are fp32; the probabilities enter the product with v as fp16, with grouped heads as two fp16
+ * parts.  With a mask,
+ * kvmix_prefill_attention_workspace_bytes() of 8-byte aligned scratch (a sixteenth of a half mask).  Other shapes: KVMIX_ERR_UNSUPPORTED (kvmix_prefill_attention_supported tells).
+ */
+typedef struct kvmix_prefill_attn {
+    const void *q;
+    int64_t q_batch_stride, q_head_stride, q_token_stride;
+    const void *k;
+    int64_t k_batch_stride, k_head_stride, k_token_stride;
+    const void *v;
+    int64_t v_batch_stride, v_head_stride, v_token_stride;
+    void *out;
+    int64_t out_batch_stride, out_head_stride, out_token_stride;
+    const void *mask;
+    int64_t mask_batch_stride, mask_head_stride, mask_row_stride, mask_batch, mask_heads;
+    int mask_dtype;
+    int64_t batch, heads, kv_heads, q_len, kv_len, head_dim;
+    float scale;
+} kvmix_prefill_attn_t;
+int64_t kvmix_prefill_attention_workspace_bytes(const kvmix_prefill_attn_t *p);
+int kvmix_prefill_attention_supported(const kvmix_prefill_attn_t *p);
+int kvmix_prefill_attention(const kvmix_prefill_attn_t *p, void *workspace, int64_t workspace_bytes, kvmix_stream_t stream);
+
+/*
  * Measurement support, no counterpart in the reference and not called by any operator: a kernel
  * that only reads, in the access patterns of the GEMV kernels, to establish what streaming rate
  * the GPU reaches without arithmetic (the ceiling the GEMV figures are compared with), and how

@@ -38,6 +38,9 @@ EXPORTS = (
     "kvmix_rope_append",
     "kvmix_linear_rows_supported",
     "kvmix_linear_rows",
+    "kvmix_prefill_attention_workspace_bytes",
+    "kvmix_prefill_attention_supported",
+    "kvmix_prefill_attention",
     "kvmix_probe_stream_read",
 )
 
@@ -106,6 +109,19 @@ class LinearRows(ctypes.Structure):
                 ("k_tail_token_stride", _i64), ("k_tail_slots", _i64), ("k_slot", _i64), ("k_slot_dev", _vp),
                 ("v_tail", _vp), ("v_tail_batch_stride", _i64), ("v_tail_head_stride", _i64),
                 ("v_tail_token_stride", _i64), ("v_tail_slots", _i64), ("v_slot", _i64), ("v_slot_dev", _vp)]
+
+
+class PrefillAttn(ctypes.Structure):
+    """kvmix_prefill_attn_t"""
+    _i64, _i32, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p
+    _fields_ = [
+        ("q", _vp), ("q_batch_stride", _i64), ("q_head_stride", _i64), ("q_token_stride", _i64),
+        ("k", _vp), ("k_batch_stride", _i64), ("k_head_stride", _i64), ("k_token_stride", _i64),
+        ("v", _vp), ("v_batch_stride", _i64), ("v_head_stride", _i64), ("v_token_stride", _i64),
+        ("out", _vp), ("out_batch_stride", _i64), ("out_head_stride", _i64), ("out_token_stride", _i64),
+        ("mask", _vp), ("mask_batch_stride", _i64), ("mask_head_stride", _i64), ("mask_row_stride", _i64), ("mask_batch", _i64),
+        ("mask_heads", _i64), ("mask_dtype", _i32), ("batch", _i64), ("heads", _i64),
+        ("kv_heads", _i64), ("q_len", _i64), ("kv_len", _i64), ("head_dim", _i64), ("scale", ctypes.c_float)]
 
 
 LINEAR_PLAIN, LINEAR_FLOAT, LINEAR_RESIDUAL, LINEAR_SWIGLU, LINEAR_ROPE_APPEND = range(5)
@@ -182,6 +198,12 @@ def load() -> ctypes.CDLL:
     L.kvmix_linear_rows_supported.argtypes = [ctypes.POINTER(LinearRows)]
     L.kvmix_linear_rows.restype = i32
     L.kvmix_linear_rows.argtypes = [ctypes.POINTER(LinearRows), vp]
+    L.kvmix_prefill_attention_workspace_bytes.restype = i64
+    L.kvmix_prefill_attention_workspace_bytes.argtypes = [ctypes.POINTER(PrefillAttn)]
+    L.kvmix_prefill_attention_supported.restype = i32
+    L.kvmix_prefill_attention_supported.argtypes = [ctypes.POINTER(PrefillAttn)]
+    L.kvmix_prefill_attention.restype = i32
+    L.kvmix_prefill_attention.argtypes = [ctypes.POINTER(PrefillAttn), vp, i64, vp]
     L.kvmix_probe_stream_read.restype = i32
     L.kvmix_probe_stream_read.argtypes = [vp, i32, i64, i64, i32, i32, i32, i32, i32, vp, vp]
     _lib = L

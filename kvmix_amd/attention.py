@@ -141,6 +141,31 @@ class KVmixAttention:
             attn_output = out_quant + out_full
         return attn_output, attn_weights
 
+    @staticmethod
+    def _prompt_attention(query_states, key_states, value_states, attention_mask, n_rep):
+        """Attention of a prompt without its probabilities: the library's kernel, or torch's fused routine for what the
+        kernel does not take (head dimensions other than 64 and 128, masks that are neither half nor float) and for
+        calls that something records (gradients, tracing)."""
+        tensors = (query_states, key_states, value_states) + (() if attention_mask is None else (attention_mask,))
+        if ops.plain_call(*tensors):
+            attn_output = ops.prefill_attention(query_states, key_states, value_states, attention_mask)
+            if attn_output is not None:
+                return attn_output
+        mask16 = None
+        if attention_mask is not None:
+            mask16 = attention_mask.clamp(min=torch.finfo(torch.float16).min).to(torch.float16)
+            # A query row whose every position is masked (a left-padding position): the reference adds
+            # the mask to its fp16 logits in the promoted dtype of the two and clamps
+            # (models/modeling_llama_KVmix.py:259-262).  With a half mask every entry of such a row ends
+            # at the lowest finite half, with a float mask of the lowest finite float the logit is
+            # absorbed: the softmax is uniform either way.  The fused routine adds in fp32 and would
+            # keep the logits' differences; a zero query makes them equal.  (A float mask holding
+            # -65504 keeps the differences in the reference too and is left alone.)
+            absorbed = torch.finfo(torch.float16).min if attention_mask.dtype == torch.float16 else -1e30
+            dead = attention_mask.amax(dim=-1, keepdim=True) <= absorbed
+            query_states = query_states.masked_fill(dead, 0)
+        return F.scaled_dot_product_attention(query_states, key_states, value_states, attn_mask=mask16, enable_gqa=n_rep > 1)
+
     # -- the step --------------------------------------------------------------------------
     def forward(self, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor,
                 past_key_value=None, attention_mask: Optional[torch.Tensor] = None, use_cache: bool = True,
@@ -203,27 +228,13 @@ class KVmixAttention:
                                                                          (None,) * 3, prompt=True)
                 k_tail, v_tail = k_tail.contiguous(), v_tail.contiguous()
             if not need_weights and query_states.dtype == torch.float16 and query_states.is_cuda:
-                # nobody reads the probabilities: torch's fused attention, which never holds the
-                # [Q, Q] matrix (fp32 accumulation throughout, where the composition below rounds the
-                # logits and the probabilities to fp16)
-                mask16 = None
-                if attention_mask is not None:
-                    if attention_mask.shape[-2:] != (q_len, kv_seq_len):
-                        raise ValueError(f"Attention mask shape {attention_mask.shape} does not match weights shape "
-                                         f"{(B, nh, q_len, kv_seq_len)}")
-                    mask16 = attention_mask.clamp(min=torch.finfo(torch.float16).min).to(torch.float16)
-                    # A query row whose every position is masked (a left-padding position): the reference adds
-                    # the mask to its fp16 logits in the promoted dtype of the two and clamps
-                    # (models/modeling_llama_KVmix.py:259-262).  With a half mask every entry of such a row ends
-                    # at the lowest finite half, with a float mask of the lowest finite float the logit is
-                    # absorbed: the softmax is uniform either way.  The fused routine adds in fp32 and would
-                    # keep the logits' differences; a zero query makes them equal.  (A float mask holding
-                    # -65504 keeps the differences in the reference too and is left alone.)
-                    absorbed = torch.finfo(torch.float16).min if attention_mask.dtype == torch.float16 else -1e30
-                    dead = attention_mask.amax(dim=-1, keepdim=True) <= absorbed
-                    query_states = query_states.masked_fill(dead, 0)
-                attn_output = F.scaled_dot_product_attention(query_states, key_states, value_states, attn_mask=mask16,
-                                                             enable_gqa=n_rep > 1)
+                # nobody reads the probabilities: attention that never holds the [Q, Q] matrix (fp32
+                # accumulation throughout, where the composition below rounds the logits and the
+                # probabilities to fp16)
+                if attention_mask is not None and attention_mask.shape[-2:] != (q_len, kv_seq_len):
+                    raise ValueError(f"Attention mask shape {attention_mask.shape} does not match weights shape "
+                                     f"{(B, nh, q_len, kv_seq_len)}")
+                attn_output = self._prompt_attention(query_states, key_states, value_states, attention_mask, n_rep)
                 cache = inplace if (use_cache and inplace is not None) else (
                     (kc, k_tail, ks, km, vc, v_tail, vs, vm, kv_seq_len) if use_cache else None)
                 return attn_output, None, cache

@@ -506,6 +506,68 @@ def qkv_rope_append(x: torch.Tensor, w, heads: int, kv_heads: int, cos: torch.Te
     return q
 
 
+def plain_call(*tensors) -> bool:
+    """Whether a call on these tensors is an ordinary one, which a kernel without an autograd formula may serve: no
+    gradient (backward or forward mode) is being recorded, nothing is traced, compiled, transformed or dispatched to a
+    tensor subclass or mode."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    if any(type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter for t in tensors):
+        return False
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _aligned_heads(t: torch.Tensor) -> torch.Tensor:
+    """[B, H, T, D] fp16 as 16-byte pieces can be read from it: unit stride along D, the others multiples of 8."""
+    if t.stride(3) == 1 and t.data_ptr() % 16 == 0 and not any(t.stride(i) % 8 for i in range(3) if t.shape[i] > 1):
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
+def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, attention_mask: torch.Tensor = None):
+    """softmax(q k^T / sqrt(D) + mask) v of a prompt (kvmix_prefill_attention): q [B, nh, Q, D], k, v [B, nkv, T, D] fp16,
+    D 64 or 128, any strides; attention_mask None or [1|B, 1|nh, Q, T] fp32 or fp16, clamped at the lowest half, rows
+    masked everywhere weighing all positions alike.  Returns [B, nh, Q, D] fp16 (stored token by token), or None
+    where the kernel does not take the call."""
+    import ctypes
+
+    if any(t.dim() != 4 or t.dtype != torch.float16 or not t.is_cuda for t in (q, k, v)):
+        return None
+    B, nh, Q, D = q.shape
+    nkv, T = k.shape[1], k.shape[2]
+    if v.shape != k.shape or k.shape[0] != B or k.shape[3] != D or nkv == 0 or nh % nkv or min(B, nh, Q, T) == 0:
+        return None
+    st = _lib.PrefillAttn()
+    if attention_mask is not None:
+        m = attention_mask
+        if m.dim() != 4 or m.dtype not in _DT or m.device != q.device or m.shape[0] not in (1, B) or m.shape[1] not in (1, nh) \
+                or m.shape[2:] != (Q, T):
+            return None
+        if T > 1 and m.stride(3) != 1:
+            m = m.contiguous()
+        st.mask, st.mask_dtype, st.mask_batch, st.mask_heads = m.data_ptr(), _DT[m.dtype], m.shape[0], m.shape[1]
+        st.mask_batch_stride, st.mask_head_stride, st.mask_row_stride = m.stride(0), m.stride(1), m.stride(2)
+    q, k, v = _aligned_heads(q), _aligned_heads(k), _aligned_heads(v)
+    out = torch.empty((B, Q, nh, D), dtype=torch.float16, device=q.device).transpose(1, 2)
+    for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):
+        setattr(st, name, t.data_ptr())
+        setattr(st, name + "_batch_stride", t.stride(0) if t.shape[0] > 1 else 0)
+        setattr(st, name + "_head_stride", t.stride(1) if t.shape[1] > 1 else 0)
+        setattr(st, name + "_token_stride", t.stride(2) if t.shape[2] > 1 else 0)
+    st.batch, st.heads, st.kv_heads, st.q_len, st.kv_len, st.head_dim = B, nh, nkv, Q, T, D
+    st.scale = D ** -0.5
+    L = _lib.load()
+    if not L.kvmix_prefill_attention_supported(ctypes.byref(st)):
+        return None
+    ws_bytes = L.kvmix_prefill_attention_workspace_bytes(ctypes.byref(st))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    with torch.cuda.device(q.device):
+        _lib.check(L.kvmix_prefill_attention(ctypes.byref(st), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q)))
+    return out
+
+
 @functools.lru_cache(maxsize=None)
 def single_pass_supported(head_dim: int, heads_per_kv: int, k_bits: int, k_fmt: int, k_group: int, v_bits: int,
                           v_fmt: int, v_group: int) -> bool:
