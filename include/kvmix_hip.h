@@ -477,6 +477,19 @@ int kvmix_prefill_attention_supported(const kvmix_prefill_attn_t *p);
 int kvmix_prefill_attention(const kvmix_prefill_attn_t *p, void *workspace, int64_t workspace_bytes, kvmix_stream_t stream);
 
 /*
+ * Strided copies, up to sixteen to a launch: outer x inner rows of row_bytes (even; strides in bytes, even; src and dst
+ * must not overlap), as growing a cache by concatenation needs them (models/modeling_llama_KVmix.py:117-118,134-139,
+ * 162-167).  A copy of 2^31 or more 16-byte pieces: KVMIX_ERR_UNSUPPORTED.
+ */
+typedef struct kvmix_copy_rows {
+    const void *src;
+    void *dst;
+    int64_t outer, inner, row_bytes;
+    int64_t src_outer_stride, src_inner_stride, dst_outer_stride, dst_inner_stride;
+} kvmix_copy_rows_t;
+int kvmix_copy_rows(const kvmix_copy_rows_t *items, int count, kvmix_stream_t stream);
+
+/*
  * Measurement support, no counterpart in the reference and not called by any operator: a kernel
  * that only reads, in the access patterns of the GEMV kernels, to establish what streaming rate
  * the GPU reaches without arithmetic (the ceiling the GEMV figures are compared with), and how

@@ -41,6 +41,7 @@ EXPORTS = (
     "kvmix_prefill_attention_workspace_bytes",
     "kvmix_prefill_attention_supported",
     "kvmix_prefill_attention",
+    "kvmix_copy_rows",
     "kvmix_probe_stream_read",
 )
 
@@ -124,6 +125,12 @@ class PrefillAttn(ctypes.Structure):
         ("kv_heads", _i64), ("q_len", _i64), ("kv_len", _i64), ("head_dim", _i64), ("scale", ctypes.c_float)]
 
 
+class CopyRows(ctypes.Structure):
+    """kvmix_copy_rows_t"""
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p)] + [(f, ctypes.c_int64) for f in (
+        "outer", "inner", "row_bytes", "src_outer_stride", "src_inner_stride", "dst_outer_stride", "dst_inner_stride")]
+
+
 LINEAR_PLAIN, LINEAR_FLOAT, LINEAR_RESIDUAL, LINEAR_SWIGLU, LINEAR_ROPE_APPEND = range(5)
 
 
@@ -204,10 +211,23 @@ def load() -> ctypes.CDLL:
     L.kvmix_prefill_attention_supported.argtypes = [ctypes.POINTER(PrefillAttn)]
     L.kvmix_prefill_attention.restype = i32
     L.kvmix_prefill_attention.argtypes = [ctypes.POINTER(PrefillAttn), vp, i64, vp]
+    L.kvmix_copy_rows.restype = i32
+    L.kvmix_copy_rows.argtypes = [ctypes.POINTER(CopyRows), i32, vp]
     L.kvmix_probe_stream_read.restype = i32
     L.kvmix_probe_stream_read.argtypes = [vp, i32, i64, i64, i32, i32, i32, i32, i32, vp, vp]
     _lib = L
     return L
+
+
+def load_host():
+    """The operators' host side (csrc/host.cpp), bound to the library that load() chose."""
+    L = load()
+    try:
+        from . import _host
+    except ImportError as e:
+        raise KVmixLibraryMissing(f"kvmix_amd/_host.so cannot be loaded ({e}); run `python -m kvmix_amd.build_ext` (needs hipcc and g++).") from e
+    _host.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in EXPORTS})
+    return _host
 
 
 def gemv_plan(group: int, bits: int, fmt: int, samples: int, heads_per_kv: int, M: int, K: int, N: int,

@@ -104,6 +104,26 @@ class KVmixAttention:
             vq = (_cat(vq[0], vc, 2), _cat(vq[1], vs, 2), _cat(vq[2], vm, 2))
         return k_tail, kq, v_tail, vq
 
+    def _grown(self, past, key_states, value_states):
+        """The 9-tuple's first eight entries after one call's tokens: appended to the tails, the oldest tail tokens
+        quantized as the policy says, all in new tensors (models/modeling_llama_KVmix.py:117-167).  One launch that
+        moves everything and, when something is flushed, one that quantizes from the old tails to behind the old packed
+        part; torch's cat and the separate quantizers for what those do not take."""
+        kc, k_tail, ks, km, vc, v_tail, vs, vm, _ = past
+        if k_tail is not None and v_tail is not None and self.Vgroup_size == 32:
+            lk, lv, n = k_tail.shape[2], v_tail.shape[2], key_states.shape[2]
+            nk = flush_length(lk + n, self.k_residual_ratio, self.Kgroup_size, self.residual_length)
+            nv = flush_length(lv + n, self.v_residual_ratio, self.Vgroup_size, self.residual_length)
+            # (not a rule that takes the call's own tokens; the reference's 3-bit values do not hold these head sizes)
+            if nk <= lk and nv <= lv and (nv == 0 or self.v_bits != 3):
+                grown = ops.grow_tuple(past, key_states, value_states, nk, nv, self.k_bits, self.Kgroup_size, self.v_bits)
+                if grown is not None:
+                    return grown
+        k_tail = key_states if k_tail is None else torch.cat([k_tail, key_states], dim=2)
+        v_tail = value_states if v_tail is None else torch.cat([v_tail, value_states], dim=2)
+        k_tail, (kc, ks, km), v_tail, (vc, vs, vm) = self._flush(k_tail, (kc, ks, km), v_tail, (vc, vs, vm))
+        return kc, k_tail, ks, km, vc, v_tail, vs, vm
+
     def new_cache(self, capacity: int = 4096, k_fmt: int = ops.FMT_REF, v_fmt: int = ops.FMT_REF) -> PackedKVCache:
         """An empty in-place cache with this layer's bit widths and flush policy; pass it as
         past_key_value from the prompt on (the same object comes back, updated)."""
@@ -193,10 +213,7 @@ class KVmixAttention:
                 kc, k_tail, ks, km, vc, v_tail, vs, vm, kv_seq_len = inplace.as_tuple()
             else:
                 kv_seq_len = key_states.shape[-2] + past_key_value[-1]
-                kc, k_tail, ks, km, vc, v_tail, vs, vm, _ = past_key_value
-                k_tail = key_states if k_tail is None else torch.cat([k_tail, key_states], dim=2)
-                v_tail = value_states if v_tail is None else torch.cat([v_tail, value_states], dim=2)
-                k_tail, (kc, ks, km), v_tail, (vc, vs, vm) = self._flush(k_tail, (kc, ks, km), v_tail, (vc, vs, vm))
+                kc, k_tail, ks, km, vc, v_tail, vs, vm = self._grown(past_key_value, key_states, value_states)
 
             mask_ok = attention_mask is None or (attention_mask.dtype == torch.float32 and attention_mask.dim() == 4
                                                  and attention_mask.shape[1] == 1)

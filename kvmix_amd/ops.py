@@ -22,6 +22,17 @@ from . import _lib
 _DT = {torch.float16: _lib.F16, torch.float32: _lib.F32}
 
 
+_native = None
+
+
+def _host():
+    """The native host side of the operators (csrc/host.cpp)."""
+    global _native
+    if _native is None:
+        _native = _lib.load_host()
+    return _native
+
+
 def _need_gpu(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if not t.is_cuda:
@@ -74,29 +85,7 @@ def quantize_pack_last_dim_cuda(input: torch.Tensor, group_length: int, quant_bi
     Reference: quantize_pack_last_dim_cuda, quant_cuda/csrc/quantization_cuda.cu:631-721.
     Returns (code int32 [B,H,R,S/vpw], scale [B,H,R,S/g], min [B,H,R,S/g]); scale and min have the
     input's dtype.  3-bit uses the reference's 11-codes-per-word layout and needs group_length 11."""
-    if quant_bits == 3 and group_length != 11:
-        raise RuntimeError("For 3-bit quantization, group_length must be 11")
-    if input.dtype not in _DT:
-        raise RuntimeError(f"expected scalar type Float or Half but found {input.dtype}")
-    if input.dim() != 4:
-        raise RuntimeError("input_tensor must be a 4D tensor")
-    _check_bits(quant_bits)
-    B, H, R, S = input.shape
-    if quant_bits == 3:
-        if S % 11 != 0:
-            raise RuntimeError("For 3-bit quantization, steps must be divisible by 11")
-    else:
-        if group_length <= 0 or S % group_length != 0:
-            raise RuntimeError("steps must be divisible by group_length")
-        if S % (32 // quant_bits) != 0:
-            raise RuntimeError("steps must be divisible by (32 / quant_bits)")
-    _need_gpu(input)
-    vpw = _values_per_word(quant_bits)
-    code = torch.empty((B, H, R, S // vpw), dtype=torch.int32, device=input.device)
-    scale = torch.empty((B, H, R, S // group_length), dtype=input.dtype, device=input.device)
-    mn = torch.empty_like(scale)
-    _quantize_into(input, group_length, quant_bits, _lib.FMT_REF, _lib.SCALE_RECIPROCAL, code, scale, mn)
-    return code, scale, mn
+    return _host().quantize_pack_last_dim(input, group_length, quant_bits)
 
 
 def quantize_pack_dense3(input: torch.Tensor, group_length: int = 32):
@@ -105,21 +94,7 @@ def quantize_pack_dense3(input: torch.Tensor, group_length: int = 32):
     scale / rounding arithmetic as quantize_pack_last_dim_cuda.  Pair with
     quantized_gemm(..., bits=3, fmt=FMT_DENSE3).
     Returns (code int32 [B,H,R,3S/32], scale [B,H,R,S/g], min [B,H,R,S/g])."""
-    if input.dtype not in _DT:
-        raise RuntimeError(f"expected scalar type Float or Half but found {input.dtype}")
-    if input.dim() != 4:
-        raise RuntimeError("input_tensor must be a 4D tensor")
-    B, H, R, S = input.shape
-    if group_length <= 0 or group_length % 32 != 0:
-        raise RuntimeError("dense 3-bit needs a group_length that is a multiple of 32")
-    if S % group_length != 0:
-        raise RuntimeError("steps must be divisible by group_length")
-    _need_gpu(input)
-    code = torch.empty((B, H, R, S * 3 // 32), dtype=torch.int32, device=input.device)
-    scale = torch.empty((B, H, R, S // group_length), dtype=input.dtype, device=input.device)
-    mn = torch.empty_like(scale)
-    _quantize_into(input, group_length, 3, _lib.FMT_DENSE3, _lib.SCALE_RECIPROCAL, code, scale, mn)
-    return code, scale, mn
+    return _host().quantize_pack_dense3(input, group_length)
 
 
 FMT_REF = _lib.FMT_REF
@@ -246,18 +221,6 @@ def quantize_kv_flush_batch(flushes) -> None:
         _lib.check(_lib.flush_batch([d[0] for d in ds], [d[1] for d in ds], _stream(ds[0][2][0])))
 
 
-def _batched3(t: torch.Tensor) -> Tuple[torch.Tensor, int, int]:
-    """[B, H, R, S] -> (tensor, batch stride, row stride) with (B, H) collapsible, unit last stride."""
-    B, H, R, S = t.shape
-    ok = (S <= 1 or t.stride(3) == 1) and (B <= 1 or t.stride(0) == H * t.stride(1))
-    ok = ok and (R <= 1 or t.stride(2) >= S) and (H <= 1 or t.stride(1) >= t.stride(2))
-    if not ok:
-        t = t.contiguous()
-    bs = t.stride(1) if B * H > 1 else max(R * max(t.stride(2), S), 1)
-    rs = t.stride(2) if R > 1 else max(S, 1)
-    return t, bs, rs
-
-
 def quantized_gemm(group_size: int, fA: torch.Tensor, qB: torch.Tensor, scales: torch.Tensor,
                    zeros: torch.Tensor, bits: int, fmt: int = _lib.FMT_REF) -> torch.Tensor:
     """out[b,h,m,:] = fA[b,h,m,:] @ dequant(qB[b,h',:,:]) with h' = h // (nh // nh_kv).
@@ -266,45 +229,7 @@ def quantized_gemm(group_size: int, fA: torch.Tensor, qB: torch.Tensor, scales: 
     fA [B,nh,M,K] f16; qB [B,nh_kv,K,N/vpw] i32; scales, zeros [B,nh_kv,K,N/g] f16 -> [B,nh,M,N] f16.
     The packed operands are read in place (views of a larger cache buffer are fine); GQA inputs
     may be passed un-repeated.  `fmt` is an extension (dense 3-bit); the default is the reference's."""
-    if fA.dim() != 4 or qB.dim() != 4:
-        raise RuntimeError("Input tensors must be 4-dimensional")
-    _check_bits(bits)
-    B, nh, M, K = fA.shape
-    nh_kv = qB.shape[1]
-    if nh_kv == 0 or nh % nh_kv != 0:
-        raise RuntimeError("Total heads must be divisible by KV heads")
-    if bits == 3 and fmt == _lib.FMT_REF and group_size != 11:
-        raise RuntimeError("For 3-bit quantization, group size must be 11")
-    if fA.dtype != torch.float16 or scales.dtype != torch.float16 or zeros.dtype != torch.float16:
-        raise RuntimeError("expected scalar type Half for fA, scales and zeros")
-    if qB.dtype != torch.int32:
-        raise RuntimeError("expected scalar type Int for qB")
-    _need_gpu(fA, qB, scales, zeros)
-    if scales.dim() != 4 or zeros.dim() != 4 or scales.shape != zeros.shape:
-        raise RuntimeError("scales and zeros must be 4-dimensional and of equal shape")
-    if qB.shape[0] != B or qB.shape[2] != K or scales.shape[:3] != qB.shape[:3]:
-        raise RuntimeError("shape mismatch between fA, qB and scales")
-    N = zeros.shape[-1] * group_size  # dequantization_gemv_cuda.cu:184
-    L = _lib.load()
-    fA, x_bs, x_rs = _batched3(fA)
-    qB, c_bs, c_rs = _batched3(qB)
-    scales, s_bs, s_rs = _batched3(scales)
-    zeros, z_bs, z_rs = _batched3(zeros)
-    if (z_bs, z_rs) != (s_bs, s_rs):
-        zeros = zeros.contiguous()
-        scales = scales.contiguous()
-        scales, s_bs, s_rs = _batched3(scales)
-        zeros, z_bs, z_rs = _batched3(zeros)
-    out = torch.empty((B, nh, M, N), dtype=torch.float16, device=fA.device)
-    ws_bytes = L.kvmix_gemv_workspace_bytes(B * nh, M, K, N)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=fA.device) if ws_bytes else None
-    with torch.cuda.device(fA.device):
-        _lib.check(L.kvmix_quantized_gemv(
-            group_size, fA.data_ptr(), x_bs, x_rs, qB.data_ptr(), c_bs, c_rs,
-            scales.data_ptr(), zeros.data_ptr(), s_bs, s_rs, bits, fmt, B * nh, nh // nh_kv,
-            M, K, N, out.data_ptr(), M * N, N, ws.data_ptr() if ws is not None else None,
-            ws_bytes, _stream(fA)))
-    return out
+    return _host().quantized_gemm(group_size, fA, qB, scales, zeros, bits, fmt)
 
 
 def prefer_single_pass(batch: int, heads: int, kv_heads: int, head_dim: int, width: int, k_bits: int, k_fmt: int,
@@ -321,12 +246,8 @@ def prefer_single_pass(batch: int, heads: int, kv_heads: int, head_dim: int, wid
         return False
     if k_tokens is None or v_tokens is None or width < max(k_tokens, v_tokens):
         k_tokens = v_tokens = 0
-    step = _lib.attn_step_descriptor(batch, heads, kv_heads, head_dim, k_bits, k_fmt, k_group, k_tokens, v_bits, v_fmt,
-                                     v_group, v_tokens, width - k_tokens, width - v_tokens)
-    try:
-        return _lib.attn_plan(step)["recommended"]
-    except RuntimeError:
-        return False
+    return _host().prefer_single_pass(batch, heads, kv_heads, head_dim, width, k_bits, k_fmt, k_group, v_bits, v_fmt, v_group,
+                                      k_tokens, v_tokens)
 
 
 def _set_tail(st, prefix: str, tail: torch.Tensor, slot) -> None:
@@ -600,106 +521,26 @@ def decode_attention(q: torch.Tensor, k_packed, v_packed, k_tail: torch.Tensor, 
     read when the kernels run (for steps replayed from a captured graph).
     attention_mask: None or fp32 [B,1,1,width].
     Returns (out [B,nh,1,D] fp16, probs [B,nh,1,width] fp16), width = max(Tk + key slots, Tv + value slots)."""
-    import ctypes
-
-    if q.dim() != 4 or q.shape[2] != 1:
-        raise RuntimeError("decode_attention takes one query position: q must be [B, nh, 1, D]")
-    for t in (q, k_tail, v_tail):
-        if t.dtype != torch.float16:
-            raise RuntimeError(f"expected scalar type Half but found {t.dtype}")
-    _need_gpu(q, k_tail, v_tail)
-    _check_bits(k_bits)
-    _check_bits(v_bits)
-    L = _lib.load()
-    B, nh, _, D = q.shape
-    nkv = k_tail.shape[1]
-    if nkv == 0 or nh % nkv != 0:
-        raise RuntimeError("Total heads must be divisible by KV heads")
-    st = _lib.DecodeAttn()
-    q, q_bs, _ = _batched3(q)
-    st.q, st.q_stride = q.data_ptr(), q_bs
-    keep = [q]
-
-    def packed(prefix, triple, tokens_of):
-        if triple is None or triple[0] is None:
-            setattr(st, prefix + "_tokens", 0)
-            return
-        code, scale, zero = triple
-        code, c_bs, c_rs = _batched3(code)
-        scale, s_bs, s_rs = _batched3(scale)
-        zero, z_bs, z_rs = _batched3(zero)
-        if (z_bs, z_rs) != (s_bs, s_rs):
-            scale, zero = scale.contiguous(), zero.contiguous()
-            scale, s_bs, s_rs = _batched3(scale)
-            zero, z_bs, z_rs = _batched3(zero)
-        keep.extend((code, scale, zero))
-        setattr(st, prefix + "_code", code.data_ptr())
-        setattr(st, prefix + "_code_batch_stride", c_bs)
-        setattr(st, prefix + "_code_row_stride", c_rs)
-        setattr(st, prefix + "_scale", scale.data_ptr())
-        setattr(st, prefix + "_zero", zero.data_ptr())
-        setattr(st, prefix + "_sz_batch_stride", s_bs)
-        setattr(st, prefix + "_sz_row_stride", s_rs)
-        setattr(st, prefix + "_tokens", tokens_of(code, zero))
-
-    packed("k", k_packed, lambda code, zero: zero.shape[-1] * k_group)
-    packed("v", v_packed, lambda code, zero: code.shape[2])
-    st.k_bits, st.k_fmt, st.k_group = k_bits, k_fmt, k_group
-    st.v_bits, st.v_fmt, st.v_group = v_bits, v_fmt, v_group
-
-    def tail(prefix, t, length):
-        t, t_bs, t_ts = _batched3(t)
-        keep.append(t)
-        setattr(st, prefix + "_tail", t.data_ptr())
-        setattr(st, prefix + "_tail_batch_stride", t_bs)
-        setattr(st, prefix + "_tail_token_stride", t_ts)
-        setattr(st, prefix + "_tail_slots", t.shape[2])
-        if torch.is_tensor(length):
-            if length.dtype != torch.int64 or length.numel() != 1 or not length.is_cuda:
-                raise RuntimeError("a device-side tail length must be one int64 element on the GPU")
-            setattr(st, prefix + "_tail_len_dev", length.data_ptr())
-        else:
-            setattr(st, prefix + "_tail_len", t.shape[2] if length is None else int(length))
-
-    tail("k", k_tail, k_tail_len)
-    tail("v", v_tail, v_tail_len)
-    width = max(st.k_tokens + st.k_tail_slots, st.v_tokens + st.v_tail_slots)
-    if attention_mask is not None:
-        if attention_mask.dtype != torch.float32 or tuple(attention_mask.shape) != (B, 1, 1, width):
-            raise RuntimeError(f"attention_mask must be fp32 of shape {(B, 1, 1, width)}")
-        if attention_mask.stride(3) != 1:
-            attention_mask = attention_mask.contiguous()
-        keep.append(attention_mask)
-        st.mask, st.mask_stride = attention_mask.data_ptr(), attention_mask.stride(0) if B > 1 else width
-    st.samples, st.heads, st.heads_per_kv, st.D = B * nh, nh, nh // nkv, D
-    out = torch.empty((B, nh, 1, D), dtype=torch.float16, device=q.device)
-    if single_pass:
-        st.out, st.out_stride = out.data_ptr(), D
-        if not L.kvmix_decode_attention_fused_supported(ctypes.byref(st)):
-            raise RuntimeError("the single-pass attention step does not take this layout (head_dim 128, keys 1/2/4-bit or "
-                               "dense 3-bit group 32 or reference 3-bit, values 1/2/4-bit or dense 3-bit group 32)")
-        ws_bytes = L.kvmix_decode_attention_fused_workspace_bytes(ctypes.byref(st))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-        with torch.cuda.device(q.device):
-            _lib.check(L.kvmix_decode_attention_fused(ctypes.byref(st), ws.data_ptr(), ws_bytes, _stream(q)))
-        return out, None
-    probs = torch.empty((B, nh, 1, width), dtype=torch.float16, device=q.device)
-    st.probs, st.probs_stride, st.out, st.out_stride = probs.data_ptr(), width, out.data_ptr(), D
-    ws_bytes = L.kvmix_decode_attention_workspace_bytes(ctypes.byref(st))
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
-    with torch.cuda.device(q.device):
-        _lib.check(L.kvmix_decode_attention(ctypes.byref(st), ws.data_ptr() if ws is not None else None, ws_bytes,
-                                            _stream(q)))
-    return out, probs
+    lengths = []
+    for n in (k_tail_len, v_tail_len):
+        lengths += (-1, n) if torch.is_tensor(n) else (-1 if n is None else int(n), None)
+    return _host().decode_attention(q, k_packed, v_packed, k_tail, v_tail, k_group, k_bits, v_group, v_bits, k_fmt, v_fmt,
+                                    attention_mask, *lengths, single_pass)
 
 
-def _append_checks(input, prev_scale, prev_min):
-    if input.dim() != 4:
-        raise RuntimeError("input_tensor must be a 4D tensor")
-    if input.dtype not in _DT:
-        raise RuntimeError(f"expected scalar type Float or Half but found {input.dtype}")
-    if prev_scale.dtype != input.dtype or prev_min.dtype != input.dtype:
-        raise RuntimeError("previous_scale / previous_min must have the input's dtype")
+def copy_rows(pairs) -> None:
+    """dst.copy_(src) for a sequence of (dst, src) pairs of equal 4-D shape and type on one device, which do not overlap,
+    in one launch per sixteen (kvmix_copy_rows)."""
+    _host().copy_rows(list(pairs))
+
+
+def grow_tuple(past, key_states, value_states, nk: int, nv: int, k_bits: int, k_group: int, v_bits: int):
+    """The first eight entries of the reference's cache tuple after one call's tokens (models/modeling_llama_KVmix.py:
+    117-167), in new tensors: the tails grown by them, the oldest nk key and nv value tokens of the OLD tails quantized to
+    behind the packed part; one launch that moves everything and, when something is flushed, one that quantizes.  Keys in
+    groups of 32 (3 bits: 11), values in groups of 32.  None where the launches do not take the call."""
+    kc, k_tail, ks, km, vc, v_tail, vs, vm, _ = past
+    return _host().grow_tuple(kc, k_tail, ks, km, vc, v_tail, vs, vm, key_states, value_states, nk, nv, k_bits, k_group, v_bits)
 
 
 def process_key_quantization_cuda(input: torch.Tensor, previous_code: torch.Tensor,
@@ -711,31 +552,7 @@ def process_key_quantization_cuda(input: torch.Tensor, previous_code: torch.Tens
     Reference: process_key_quantization_cuda, quant_cuda/csrc/quantization_cuda.cu:298-411.
     The returned scale is (max-min)/qmax rounded to the input dtype (the reference's append
     kernels divide in-kernel, :49-51,:149-151)."""
-    _append_checks(input, previous_scale, previous_min)
-    _check_bits(quant_bits)
-    B, H, D, n = input.shape
-    if quant_bits == 3:
-        if group_length != 11:
-            raise RuntimeError("For 3-bit quantization, group_length must be 11")
-        if n % 11 != 0:
-            raise RuntimeError("new_steps must be divisible by 11 for 3-bit quantization")
-    elif group_length <= 0 or n % group_length != 0:
-        raise RuntimeError("new_steps must be divisible by group_length")
-    _need_gpu(input, previous_code, previous_scale, previous_min)
-    vpw = _values_per_word(quant_bits)
-    if quant_bits != 3 and (group_length % vpw != 0 or n % vpw != 0):
-        raise RuntimeError(_lib.strerror(-9))
-    ow, og = previous_code.shape[3], previous_scale.shape[3]
-    code = torch.empty((B, H, D, ow + n // vpw), dtype=torch.int32, device=input.device)
-    scale = torch.empty((B, H, D, og + n // group_length), dtype=input.dtype, device=input.device)
-    mn = torch.empty_like(scale)
-    code[..., :ow].copy_(previous_code.reshape(B, H, D, ow))
-    scale[..., :og].copy_(previous_scale.reshape(B, H, D, og))
-    mn[..., :og].copy_(previous_min.reshape(B, H, D, og))
-    if n > 0:
-        _quantize_into(input, group_length, quant_bits, _lib.FMT_REF, _lib.SCALE_DIVIDE,
-                       code[..., ow:], scale[..., og:], mn[..., og:])
-    return code, scale, mn
+    return _host().append_keys(input, previous_code, previous_scale, previous_min, group_length, quant_bits)
 
 
 def process_value_quantization_cuda(input: torch.Tensor, previous_code: torch.Tensor,
@@ -747,30 +564,4 @@ def process_value_quantization_cuda(input: torch.Tensor, previous_code: torch.Te
     Reference: process_value_quantization_cuda, quant_cuda/csrc/quantization_cuda.cu:413-537.
     3-bit follows the reference's placeholder branch literally (plain 3*j shifts, so the
     eleventh code of a word keeps only its low two bits)."""
-    _append_checks(input, previous_scale, previous_min)
-    _check_bits(quant_bits)
-    B, H, n, D = input.shape
-    if quant_bits == 3:
-        if group_length != 11:
-            raise RuntimeError("For 3-bit quantization, group_length must be 11")
-        if D % 11 != 0:
-            raise RuntimeError("head_dim must be divisible by 11 for 3-bit quantization")
-    elif group_length <= 0 or D % group_length != 0:
-        raise RuntimeError("head_dim must be divisible by group_length")
-    _need_gpu(input, previous_code, previous_scale, previous_min)
-    vpw = _values_per_word(quant_bits)
-    if quant_bits != 3 and (group_length % vpw != 0 or D % vpw != 0):
-        raise RuntimeError(_lib.strerror(-9))
-    old = previous_code.shape[2]
-    wpt, gpt = D // vpw, D // group_length
-    code = torch.empty((B, H, old + n, wpt), dtype=torch.int32, device=input.device)
-    scale = torch.empty((B, H, old + n, gpt), dtype=input.dtype, device=input.device)
-    mn = torch.empty_like(scale)
-    code[:, :, :old].copy_(previous_code.reshape(B, H, old, wpt))
-    scale[:, :, :old].copy_(previous_scale.reshape(B, H, old, gpt))
-    mn[:, :, :old].copy_(previous_min.reshape(B, H, old, gpt))
-    if n > 0:
-        fmt = _lib.FMT_REF3_WRAP if quant_bits == 3 else _lib.FMT_REF
-        _quantize_into(input, group_length, quant_bits, fmt, _lib.SCALE_DIVIDE,
-                       code[:, :, old:], scale[:, :, old:], mn[:, :, old:])
-    return code, scale, mn
+    return _host().append_values(input, previous_code, previous_scale, previous_min, group_length, quant_bits)
