@@ -186,6 +186,34 @@ class KVmixAttention:
             query_states = query_states.masked_fill(dead, 0)
         return F.scaled_dot_product_attention(query_states, key_states, value_states, attn_mask=mask16, enable_gqa=n_rep > 1)
 
+    def _decode(self, query_states, entries, k_group, k_fmt, v_fmt, attention_mask, need_weights):
+        """Attention over the cache's entries, the call's own tokens among them: (output, probabilities or None)."""
+        kc, k_tail, ks, km, vc, v_tail, vs, vm, kv_seq_len = entries
+        B, nh, q_len, D = query_states.shape
+        nkv = k_tail.shape[1]
+        mask_ok = attention_mask is None or (attention_mask.dtype == torch.float32 and attention_mask.dim() == 4
+                                             and attention_mask.shape[1] == 1)
+        short_tails = max(k_tail.shape[2], v_tail.shape[2]) <= LIBRARY_STEP_MAX_TAIL
+        if q_len == 1 and query_states.dtype == torch.float16 and D % 8 == 0 and mask_ok and short_tails:
+            # the whole step in the library: logits over packed keys and fp16 tail, softmax,
+            # output over packed values and fp16 tail
+            if attention_mask is not None and attention_mask.shape[-2:] != (1, kv_seq_len):
+                raise ValueError(f"Attention mask shape {attention_mask.shape} does not match weights shape "
+                                 f"{(B, nh, 1, kv_seq_len)}")
+            single = (not need_weights) and ops.prefer_single_pass(
+                B, nh, nkv, D, kv_seq_len, self.k_bits, k_fmt, k_group, self.v_bits, v_fmt,
+                self.Vgroup_size, k_tokens=kv_seq_len - k_tail.shape[2], v_tokens=kv_seq_len - v_tail.shape[2])
+            return ops.decode_attention(
+                query_states, (kc, ks, km), (vc, vs, vm), k_tail, v_tail, k_group, self.k_bits, self.Vgroup_size,
+                self.v_bits, k_fmt, v_fmt, attention_mask, single_pass=single)
+        return self._decode_with_torch_glue(query_states, kc, ks, km, k_tail, vc, vs, vm, v_tail, k_group, k_fmt, v_fmt, nh // nkv, attention_mask)
+
+    def attend(self, query_states: torch.Tensor, cache: PackedKVCache, attention_mask: Optional[torch.Tensor] = None,
+               need_weights: bool = True):
+        """The attention of a decode step whose tokens `cache` holds already (a kernel wrote them into its slots:
+        PackedKVCache.next_slots): (attn_output [B,nh,Q,D], attn_weights or None), as forward returns them."""
+        return self._decode(query_states, cache.as_tuple(), cache.Kgroup_size, cache.k_fmt, cache.v_fmt, attention_mask, need_weights)
+
     # -- the step --------------------------------------------------------------------------
     def forward(self, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor,
                 past_key_value=None, attention_mask: Optional[torch.Tensor] = None, use_cache: bool = True,
@@ -215,24 +243,8 @@ class KVmixAttention:
                 kv_seq_len = key_states.shape[-2] + past_key_value[-1]
                 kc, k_tail, ks, km, vc, v_tail, vs, vm = self._grown(past_key_value, key_states, value_states)
 
-            mask_ok = attention_mask is None or (attention_mask.dtype == torch.float32 and attention_mask.dim() == 4
-                                                 and attention_mask.shape[1] == 1)
-            short_tails = max(k_tail.shape[2], v_tail.shape[2]) <= LIBRARY_STEP_MAX_TAIL
-            if q_len == 1 and query_states.dtype == torch.float16 and D % 8 == 0 and mask_ok and short_tails:
-                # the whole step in the library: logits over packed keys and fp16 tail, softmax,
-                # output over packed values and fp16 tail
-                if attention_mask is not None and attention_mask.shape[-2:] != (1, kv_seq_len):
-                    raise ValueError(f"Attention mask shape {attention_mask.shape} does not match weights shape "
-                                     f"{(B, nh, 1, kv_seq_len)}")
-                single = (not need_weights) and ops.prefer_single_pass(
-                    B, nh, key_states.shape[1], D, kv_seq_len, self.k_bits, k_fmt, k_group, self.v_bits, v_fmt,
-                    self.Vgroup_size, k_tokens=kv_seq_len - k_tail.shape[2], v_tokens=kv_seq_len - v_tail.shape[2])
-                attn_output, attn_weights = ops.decode_attention(
-                    query_states, (kc, ks, km), (vc, vs, vm), k_tail, v_tail, k_group, self.k_bits, self.Vgroup_size,
-                    self.v_bits, k_fmt, v_fmt, attention_mask, single_pass=single)
-            else:
-                attn_output, attn_weights = self._decode_with_torch_glue(
-                    query_states, kc, ks, km, k_tail, vc, vs, vm, v_tail, k_group, k_fmt, v_fmt, n_rep, attention_mask)
+            attn_output, attn_weights = self._decode(query_states, (kc, k_tail, ks, km, vc, v_tail, vs, vm, kv_seq_len), k_group, k_fmt, v_fmt,
+                                                     attention_mask, need_weights)
         else:
             # prompt: dense fp16 attention; the cache keeps the oldest tokens quantized
             # (models/modeling_llama_KVmix.py:213-266)

@@ -64,18 +64,23 @@ class _Tail:
         B, H, n, D = new.shape
         if self.buf is None:
             self.buf = torch.zeros((B, H, max(reserve, n), D), dtype=new.dtype, device=new.device)
+        self.room(n).copy_(new)
+        self.len += n
+
+    def room(self, n: int) -> torch.Tensor:
+        """The slots [B,Hkv,n,D] that the next n tokens go to (made first if the buffer's end is reached)."""
         cap = self.buf.shape[2]
         if self.start + self.len + n > cap:
             live = self.view()
             if self.len + n > cap:  # the tail itself has outgrown the buffer: a longer one
-                buf = torch.zeros((B, H, max(2 * cap, self.len + n), D), dtype=new.dtype, device=new.device)
+                B, H, _, D = self.buf.shape
+                buf = torch.zeros((B, H, max(2 * cap, self.len + n), D), dtype=self.buf.dtype, device=self.buf.device)
                 buf[:, :, :self.len].copy_(live)
                 self.buf = buf
             else:  # room at the front: move the live tokens there (regions may overlap)
                 self.buf[:, :, :self.len].copy_(live.clone())
             self.start = 0
-        self.buf[:, :, self.start + self.len:self.start + self.len + n].copy_(new)
-        self.len += n
+        return self.buf[:, :, self.start + self.len:self.start + self.len + n]
 
     def drop_front(self, n: int) -> None:
         self.start += n
@@ -255,6 +260,17 @@ class PackedKVCache:
         fp16 tails for a step whose append is done by the caller on the device (the token goes to
         slot `live tokens` of each window); follow every such step with note_device_append()."""
         return self._k_tail.window(slots), self._v_tail.window(slots), self._k_tail.len, self._v_tail.len
+
+    def next_slots(self, batch: int, kv_heads: int, head_dim: int):
+        """The slots [B,Hkv,1,D] of both tails for a token that a kernel writes itself, when appending it flushes nothing
+        (any more); follow the write with note_device_append().  None: the token has to go through append()."""
+        shape = (batch, kv_heads, head_dim)
+        for t in (self._k_tail, self._v_tail):
+            if t.buf is None or (t.buf.shape[0], t.buf.shape[1], t.buf.shape[3]) != shape or t.buf.dtype != torch.float16:
+                return None
+        if self.flushes_on_next_append():
+            return None
+        return self._k_tail.room(1), self._v_tail.room(1)
 
     def note_device_append(self) -> None:
         """Book-keeping for one token that a device-side step wrote into the tail windows."""

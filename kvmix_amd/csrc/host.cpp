@@ -39,6 +39,7 @@ struct Api {
     decltype(&kvmix_decode_attention_fused) decode_attention_fused;
     decltype(&kvmix_decode_attention_fused_plan) decode_attention_fused_plan;
     decltype(&kvmix_copy_rows) copy_rows;
+    decltype(&kvmix_linear_rows) linear_rows;
 } api;
 
 void bind(const std::unordered_map<std::string, uintptr_t> &at)
@@ -56,6 +57,7 @@ void bind(const std::unordered_map<std::string, uintptr_t> &at)
     KVMIX_BIND(decode_attention_fused);
     KVMIX_BIND(decode_attention_fused_plan);
     KVMIX_BIND(copy_rows);
+    KVMIX_BIND(linear_rows);
 #undef KVMIX_BIND
 }
 
@@ -516,6 +518,130 @@ std::pair<Tensor, OptTensor> decode_attention(const Tensor &q_in, const OptTripl
     return {out, probs};
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// projections of a decode step
+
+// [..., n] fp16 as [rows, n] with unit-stride rows
+Tensor rows2(const Tensor &t, const char *what)
+{
+    if (t.scalar_type() != at::kHalf) fail(std::string("expected scalar type Half for ") + what + " but found " + dtype_name(t));
+    const Tensor r = t.reshape({-1, t.size(-1)});
+    return r.stride(1) == 1 && r.stride(0) >= r.size(1) ? r : r.contiguous();
+}
+
+// ws: one stacked weight, cut into parts of `split` rows, or one weight per part
+Tensor linear_operands(kvmix_linear_rows_t &st, const Tensor &x_in, const std::vector<Tensor> &ws, const std::vector<int64_t> &split, int epilogue,
+                       const OptTensor &norm, double eps)
+{
+    const Tensor x = rows2(x_in, "x");
+    need_gpu({&x});
+    st.x = x.data_ptr(), st.m = x.size(0), st.k = x.size(1);
+    st.x_stride = x.size(0) > 1 ? x.stride(0) : x.size(1);
+    st.epilogue = epilogue;
+    if (ws.empty() || ws.size() > 3) fail("a projection has one to three weights");
+    for (const Tensor &w : ws) {
+        need_gpu({&w});
+        if (w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(1) || w.stride(1) != 1 || w.stride(0) != ws[0].stride(0))
+            fail("weights must be fp16 [rows, k] with unit-stride rows and one row stride");
+    }
+    st.w_stride = ws[0].stride(0);
+    if (ws.size() == 1) {
+        int64_t sum = 0;
+        for (int64_t n : split) sum += n;
+        if (sum != ws[0].size(0)) fail("the stacked weight must hold the rows of all its parts");
+        const char *at = (const char *)ws[0].data_ptr();
+        for (size_t j = 0; j < split.size(); j++) {
+            st.w[j] = at, st.rows[j] = split[j];
+            at += 2 * split[j] * st.w_stride;
+        }
+    } else {
+        for (size_t j = 0; j < ws.size(); j++) st.w[j] = ws[j].data_ptr(), st.rows[j] = ws[j].size(0);
+    }
+    if (norm) {
+        if (norm->scalar_type() != at::kHalf || norm->numel() != x.size(1) || !norm->is_contiguous())
+            fail("norm_weight must be k contiguous fp16 values");
+        st.norm_weight = norm->data_ptr(), st.norm_eps = (float)eps;
+    }
+    return x;
+}
+
+void linear_launch(const kvmix_linear_rows_t &st, const Tensor &x)
+{
+    const c10::DeviceGuard guard(x.device());
+    check(api.linear_rows(&st, stream_of(x)));
+}
+
+Tensor linear_output(const Tensor &x, int64_t n, c10::ScalarType type)
+{
+    std::vector<int64_t> sizes = x.sizes().vec();
+    sizes.back() = n;
+    return at::empty(sizes, x.options().dtype(type).requires_grad(false));
+}
+
+Tensor linear_rows(const Tensor &x_in, const Tensor &w, const OptTensor &norm, double eps, const OptTensor &residual_in, bool fp32)
+{
+    kvmix_linear_rows_t st{};
+    if (w.dim() != 2) fail("weights must be fp16 [rows, k] with unit-stride rows and one row stride");
+    const int64_t n = w.size(0);
+    const Tensor x = linear_operands(st, x_in, {w}, {n}, residual_in ? KVMIX_LINEAR_RESIDUAL : fp32 ? KVMIX_LINEAR_FLOAT : KVMIX_LINEAR_PLAIN, norm, eps);
+    Tensor residual;
+    if (residual_in) {
+        residual = rows2(*residual_in, "residual");
+        if (residual.size(0) != x.size(0) || residual.size(1) != n) fail("residual must have the shape of the product");
+        st.residual = residual.data_ptr(), st.residual_stride = residual.size(0) > 1 ? residual.stride(0) : n;
+    }
+    Tensor out = linear_output(x_in, n, fp32 ? at::kFloat : at::kHalf);
+    st.out = out.data_ptr(), st.out_stride = n;
+    linear_launch(st, x);
+    return out;
+}
+
+Tensor swiglu_rows(const Tensor &x_in, const std::vector<Tensor> &ws, const OptTensor &norm, double eps)
+{
+    kvmix_linear_rows_t st{};
+    if (ws.empty() || ws[0].dim() != 2) fail("weights must be fp16 [rows, k] with unit-stride rows and one row stride");
+    const int64_t n = ws.size() > 1 ? ws[0].size(0) : ws[0].size(0) / 2;
+    const Tensor x = linear_operands(st, x_in, ws, {n, n}, KVMIX_LINEAR_SWIGLU, norm, eps);
+    Tensor out = linear_output(x_in, n, at::kHalf);
+    st.out = out.data_ptr(), st.out_stride = n;
+    linear_launch(st, x);
+    return out;
+}
+
+Tensor qkv_rope_append(const Tensor &x_in, const std::vector<Tensor> &ws, int64_t heads, int64_t kv_heads, const Tensor &cos_in, const Tensor &sin_in,
+                       const Tensor &k_tail, const Tensor &v_tail, int64_t k_slot, const OptTensor &k_slot_dev, int64_t v_slot,
+                       const OptTensor &v_slot_dev, const OptTensor &norm, double eps)
+{
+    kvmix_linear_rows_t st{};
+    const int64_t D = k_tail.size(-1);
+    const Tensor x = linear_operands(st, x_in, ws, {heads * D, kv_heads * D, kv_heads * D}, KVMIX_LINEAR_ROPE_APPEND, norm, eps);
+    const int64_t B = x.size(0);
+    for (const Tensor *t : {&cos_in, &sin_in})
+        if (t->scalar_type() != at::kHalf || (t->numel() != D && t->numel() != B * D) || !t->is_cuda())
+            fail("qkv_rope_append: cos and sin must hold head_dim fp16 values, shared or per sequence");
+    const Tensor cos = cos_in.reshape({-1, D}).contiguous(), sin = sin_in.reshape({-1, D}).contiguous();
+    if (cos.size(0) != sin.size(0)) fail("qkv_rope_append: cos and sin must have the same shape");
+    st.cos = cos.data_ptr(), st.sin = sin.data_ptr(), st.cos_sin_batch_stride = cos.size(0) > 1 ? D : 0, st.head_dim = D;
+    for (const Tensor *t : {&k_tail, &v_tail})
+        if (t->scalar_type() != at::kHalf || !t->is_cuda() || t->dim() != 4 || t->size(0) != B || t->size(1) != kv_heads || t->size(3) != D || t->stride(3) != 1)
+            fail("qkv_rope_append: tails must be fp16 [B, kv_heads, slots, D] with unit stride along D");
+    for (const OptTensor *t : {&k_slot_dev, &v_slot_dev})
+        if (*t && ((*t)->scalar_type() != at::kLong || (*t)->numel() != 1 || !(*t)->is_cuda()))
+            fail("a device-side slot must be one int64 element on the GPU");
+    // (strides of one-element dimensions are whatever the view left there)
+    st.k_tail = k_tail.data_ptr(), st.k_tail_batch_stride = k_tail.stride(0), st.k_tail_head_stride = k_tail.stride(1);
+    st.k_tail_token_stride = std::max(k_tail.stride(2), k_tail.size(2) > 1 ? 0 : D), st.k_tail_slots = k_tail.size(2);
+    st.v_tail = v_tail.data_ptr(), st.v_tail_batch_stride = v_tail.stride(0), st.v_tail_head_stride = v_tail.stride(1);
+    st.v_tail_token_stride = std::max(v_tail.stride(2), v_tail.size(2) > 1 ? 0 : D), st.v_tail_slots = v_tail.size(2);
+    st.k_slot = k_slot, st.v_slot = v_slot;
+    if (k_slot_dev) st.k_slot_dev = k_slot_dev->data_ptr<int64_t>();
+    if (v_slot_dev) st.v_slot_dev = v_slot_dev->data_ptr<int64_t>();
+    Tensor q = empty({B, heads, 1, D}, at::kHalf, x);
+    st.out = q.data_ptr(), st.out_stride = heads * D;
+    linear_launch(st, x);
+    return q;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m)
@@ -530,4 +656,7 @@ PYBIND11_MODULE(_host, m)
     m.def("quantized_gemm", &quantized_gemm);
     m.def("prefer_single_pass", &prefer_single_pass);
     m.def("decode_attention", &decode_attention);
+    m.def("linear_rows", &linear_rows);
+    m.def("swiglu_rows", &swiglu_rows);
+    m.def("qkv_rope_append", &qkv_rope_append);
 }

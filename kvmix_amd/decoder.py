@@ -157,6 +157,17 @@ class Decoder:
         self.caches: List = list(caches) if caches is not None else [None] * cfg.num_layers
         self.position = 0
 
+    def _slots(self, li: int, x: torch.Tensor):
+        """Where layer li's kernels may write the new token's keys and values themselves (an in-place cache that has
+        tokens and does not flush for this one), or None."""
+        from .attention import KVmixAttention
+        from .cache import PackedKVCache
+
+        cache = self.caches[li]
+        if not isinstance(cache, PackedKVCache) or type(self.attention[li]) is not KVmixAttention or cache.kv_seq_len == 0:
+            return None
+        return cache.next_slots(x.shape[0], self.cfg.num_kv_heads, self.cfg.head_dim)
+
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
         """input_ids [B,Q] (prompt when nothing is cached yet, else the new tokens) -> logits of the
         last position [B, vocab] in fp32."""
@@ -176,13 +187,19 @@ class Decoder:
 
             flush_ahead(self.caches)
         for li, lw in enumerate(self.w["layers"]):
-            if _few_rows(x):
-                k, v = (torch.empty((B, cfg.num_kv_heads, 1, cfg.head_dim), dtype=x.dtype, device=x.device) for _ in range(2))
-                q = qkv_of_token(cfg, x, lw, cos, sin, k, v, 0, 0)
+            slots = self._slots(li, x) if _few_rows(x) else None
+            if slots is not None:
+                q = qkv_of_token(cfg, x, lw, cos, sin, slots[0], slots[1], 0, 0)
+                self.caches[li].note_device_append()
+                out, _ = self.attention[li].attend(q, self.caches[li], need_weights=False)
             else:
-                h = rms_norm(x, lw["input_norm"], cfg.rms_norm_eps)
-                q, k, v = project_qkv(cfg, h, lw["wqkv"], cos, sin)
-            out, _, self.caches[li] = self.attention[li](q, k, v, self.caches[li], attention_mask=mask, need_weights=False)
+                if _few_rows(x):
+                    k, v = (torch.empty((B, cfg.num_kv_heads, 1, cfg.head_dim), dtype=x.dtype, device=x.device) for _ in range(2))
+                    q = qkv_of_token(cfg, x, lw, cos, sin, k, v, 0, 0)
+                else:
+                    h = rms_norm(x, lw["input_norm"], cfg.rms_norm_eps)
+                    q, k, v = project_qkv(cfg, h, lw["wqkv"], cos, sin)
+                out, _, self.caches[li] = self.attention[li](q, k, v, self.caches[li], attention_mask=mask, need_weights=False)
             x = add_projection(x, out.transpose(1, 2).reshape(B, Q, cfg.hidden_size), lw["wo"])
             x = add_mlp(x, lw, cfg.rms_norm_eps)
         self.position += Q

@@ -13,7 +13,9 @@ These classes keep that recipe (same class names, same `quant_bits` layout, `con
 on top of the stock `LlamaForCausalLM` / `MistralForCausalLM`: each `self_attn` keeps the stock
 projections and RoPE and hands q, k, v to `KVmixAttention`, and the cache object that travels
 through `generate()` is a `KVmixCache` holding one in-place `PackedKVCache` per layer.  The stock
-model code (embeddings, masks, norms, MLP, sampling) is untouched.
+model code (embeddings, norms, MLP, sampling) is untouched, except that a step of one new token per
+sequence goes through the library's projection kernels where nothing observes or replaces the stock
+modules between them (`_KVmixDecoderLayer`), and gets its mask row from here (`_step_mask`).
 
 Not supported, and refused with an error rather than silently served from a dense cache: beam
 search and assisted decoding (they reorder or crop the cache), other `Cache` classes, attention
@@ -24,14 +26,18 @@ from __future__ import annotations
 from typing import Dict, Optional, Sequence, Union
 
 import torch
+from torch.nn.modules import module as _module
 from transformers import LlamaForCausalLM, MistralForCausalLM
+from transformers.activations import SiLUActivation
 from transformers.cache_utils import Cache, CacheLayerMixin
-from transformers.models.llama.modeling_llama import LlamaAttention
+from transformers.models.llama.modeling_llama import LlamaAttention, LlamaMLP, LlamaRMSNorm
+from transformers.models.llama.modeling_llama import LlamaDecoderLayer as StockLlamaDecoderLayer
 from transformers.models.llama.modeling_llama import apply_rotary_pos_emb as llama_rope
-from transformers.models.mistral.modeling_mistral import MistralAttention
+from transformers.models.mistral.modeling_mistral import MistralAttention, MistralMLP, MistralRMSNorm
+from transformers.models.mistral.modeling_mistral import MistralDecoderLayer as StockMistralDecoderLayer
 from transformers.models.mistral.modeling_mistral import apply_rotary_pos_emb as mistral_rope
 
-from . import ops
+from . import _lib, ops
 from .attention import KVmixAttention
 from .cache import RESIDUAL_RATIO_BY_BITS, PackedKVCache
 
@@ -131,6 +137,16 @@ class KVmixCache(Cache):
         return self.layers[layer_idx].packed.as_tuple()
 
 
+def _additive_mask(attention_mask, dtype):
+    """A mask as the layers take it: additive, in `dtype`."""
+    if attention_mask.dtype == torch.bool:
+        return torch.zeros(attention_mask.shape, dtype=dtype, device=attention_mask.device
+                           ).masked_fill_(~attention_mask, torch.finfo(dtype).min)
+    if attention_mask.dtype != dtype:
+        return attention_mask.clamp(min=torch.finfo(dtype).min).to(dtype)
+    return attention_mask
+
+
 class _KVmixAttentionForward:
     """forward() shared by the Llama and Mistral attention subclasses: the stock projections and
     RoPE, then `KVmixAttention` instead of `past_key_values.update` + the attention interface."""
@@ -165,11 +181,7 @@ class _KVmixAttentionForward:
             # what makes the rows of left-padding positions uniform.  A single-token step adds it to fp32
             # logits (:68-75,189-192), and the library's step takes fp32.
             mask_dtype = query_states.dtype if q_len > 1 else torch.float32
-            if attention_mask.dtype == torch.bool:
-                attention_mask = torch.zeros(attention_mask.shape, dtype=mask_dtype, device=attention_mask.device
-                                             ).masked_fill_(~attention_mask, torch.finfo(mask_dtype).min)
-            elif attention_mask.dtype != mask_dtype:
-                attention_mask = attention_mask.clamp(min=torch.finfo(mask_dtype).min).to(mask_dtype)
+            attention_mask = _additive_mask(attention_mask, mask_dtype)
         packed = None if past_key_values is None else past_key_values.packed(self.layer_idx)
         if packed is not None and q_len == 1 and self.layer_idx == 0:
             # a decode step: what its layers flush are tokens of earlier steps -- all layers' flushes at once,
@@ -192,10 +204,101 @@ class MistralAttention_KVmix(_KVmixAttentionForward, MistralAttention):
     _rope = staticmethod(mistral_rope)
 
 
+def _untouched(module, kind) -> bool:
+    """Whether calling `module` does what the class `kind` does and nothing else (hooks, a replaced forward)."""
+    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__)
+
+
+class _KVmixDecoderLayer:
+    """forward() of the decoder layers: one new token per sequence on a `KVmixCache` takes the projection kernels
+    (kvmix_linear_rows), which stream the weights and take norms, RoPE, the append to the cache, SwiGLU and the residual
+    sums along: four launches and the attention step instead of about forty.  Everything else is the stock layer: prompts,
+    gradients, tracing, autocast, adapters or quantized weights in place of plain fp16 ones, hooks on a module inside."""
+
+    _norm_class = _mlp_class = _kvmix_attention = None
+
+    def _step_weights(self, x):
+        """(q, k, v, o, gate, up, down, input norm, post norm) weights when the layer is the stock one through and
+        through, else None."""
+        m = self._modules
+        attn, ffn, norms = m["self_attn"], m["mlp"], (m["input_layernorm"], m["post_attention_layernorm"])
+        if not (_untouched(attn, self._kvmix_attention) and _untouched(ffn, self._mlp_class)
+                and _untouched(norms[0], self._norm_class) and _untouched(norms[1], self._norm_class)):
+            return None
+        a, f = attn._modules, ffn._modules
+        if not (_untouched(f["act_fn"], SiLUActivation) or _untouched(f["act_fn"], torch.nn.SiLU)):
+            return None
+        weights = []
+        for lin in (a["q_proj"], a["k_proj"], a["v_proj"], a["o_proj"], f["gate_proj"], f["up_proj"], f["down_proj"]):
+            if not _untouched(lin, torch.nn.Linear) or lin._parameters["bias"] is not None:
+                return None
+            weights.append(lin._parameters["weight"])
+        weights += [n._parameters["weight"] for n in norms]
+        for w in weights:
+            if w.dtype != torch.float16 or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16:
+                return None
+        return weights if ops.plain_call(x, *weights) else None
+
+    def _step(self, x, position_embeddings, past_key_values, attention_mask):
+        """The layer's output for one new token per sequence, or None where the kernels do not take it (nothing has been
+        changed then)."""
+        weights = self._step_weights(x)
+        if weights is None or type(self._modules["self_attn"].kvmix) is not KVmixAttention:
+            return None
+        wq, wk, wv, wo, wg, wu, wd, n1, n2 = weights
+        attn, B, hidden = self._modules["self_attn"], x.shape[0], x.shape[2]
+        D = attn.head_dim
+        heads, kv_heads = wq.shape[0] // D, wk.shape[0] // D
+        cos, sin = position_embeddings
+        if cos.dtype != torch.float16 or cos.shape != sin.shape or cos.shape[-1] != D or cos.numel() not in (D, B * D):
+            return None
+        if not (ops.linear_rows_supported(B, hidden, wq.shape[0], _lib.LINEAR_ROPE_APPEND, True, D, wk.shape[0])
+                and ops.linear_rows_supported(B, wo.shape[1], hidden, _lib.LINEAR_RESIDUAL)
+                and ops.linear_rows_supported(B, hidden, wg.shape[0], _lib.LINEAR_SWIGLU, True)):
+            return None
+        if attn.layer_idx == 0:
+            past_key_values.flush_ahead()
+        packed = past_key_values.packed(attn.layer_idx)
+        slots = packed.next_slots(B, kv_heads, D)
+        if slots is None:
+            return None
+        q = ops.qkv_rope_append(x, (wq, wk, wv), heads, kv_heads, cos, sin, slots[0], slots[1], 0, 0, n1,
+                                self._modules["input_layernorm"].variance_epsilon)
+        packed.note_device_append()
+        if attention_mask is not None:
+            attention_mask = _additive_mask(attention_mask, torch.float32)
+        out, _ = attn.kvmix.attend(q, packed, attention_mask, need_weights=False)
+        x = ops.linear_rows(out.view(B, 1, heads * D), wo, residual=x)
+        h = ops.swiglu_rows(x, (wg, wu), n2, self._modules["post_attention_layernorm"].variance_epsilon)
+        if ops.linear_rows_supported(B, wd.shape[1], hidden, _lib.LINEAR_RESIDUAL):
+            return ops.linear_rows(h, wd, residual=x)
+        return x + torch.nn.functional.linear(h, wd)
+
+    def forward(self, hidden_states, *args, **kwargs):
+        cache, rope = kwargs.get("past_key_values"), kwargs.get("position_embeddings")
+        if (not args and hidden_states.dim() == 3 and hidden_states.shape[1] == 1 and hidden_states.is_cuda
+                and hidden_states.dtype == torch.float16 and isinstance(cache, KVmixCache) and rope is not None
+                and cache.get_seq_length(self.self_attn.layer_idx) > 0 and not kwargs.get("output_attentions", False)
+                and not torch.is_autocast_enabled("cuda") and not (_module._global_forward_hooks or _module._global_forward_pre_hooks)):
+            out = self._step(hidden_states, rope, cache, kwargs.get("attention_mask"))
+            if out is not None:
+                return out
+        return super().forward(hidden_states, *args, **kwargs)
+
+
+# (the stock names: they are what device maps know as a unit that is not split)
+class LlamaDecoderLayer(_KVmixDecoderLayer, StockLlamaDecoderLayer):
+    _norm_class, _mlp_class, _kvmix_attention = LlamaRMSNorm, LlamaMLP, LlamaAttention_KVmix
+
+
+class MistralDecoderLayer(_KVmixDecoderLayer, StockMistralDecoderLayer):
+    _norm_class, _mlp_class, _kvmix_attention = MistralRMSNorm, MistralMLP, MistralAttention_KVmix
+
+
 class _KVmixCausalLM:
     """What the two model classes share: converting the attention layers, creating the cache."""
 
-    _attention_class = None
+    _attention_class = _layer_class = None
 
     def _convert(self, config, quant_bits: QuantBits) -> None:
         if getattr(config, "_attn_implementation", "eager") not in (None, "eager"):
@@ -206,7 +309,9 @@ class _KVmixCausalLM:
         self.group_size = int(getattr(config, "group_size", 32))       # Inference-comparision.py:15
         self.residual_length = getattr(config, "residual_length", None)
         for i, layer in enumerate(self.model.layers):
-            layer.self_attn.__class__ = self._attention_class          # same weights, new forward
+            if type(layer) in self._layer_class.__mro__:
+                layer.__class__ = self._layer_class                    # same weights, new forward
+            layer.self_attn.__class__ = self._attention_class
             layer.self_attn._init_kvmix(self.quant_bits[i], self.group_size, self.residual_length)
 
     def new_cache(self, capacity: int = 4096) -> KVmixCache:
@@ -220,6 +325,21 @@ class _KVmixCausalLM:
             raise TypeError(f"{type(self).__name__} needs a KVmixCache as past_key_values, got {type(pkv).__name__}")
         return kwargs
 
+    def _step_mask(self, input_ids, attention_mask, cache):
+        """The additive mask row [B,1,1,length] of a step of one new token per sequence: what the stock model builds from
+        the padding mask (or from none) over some forty small operations, as long as no sliding window cuts the row.
+        Masks in other forms are handed on as they are."""
+        length = cache.get_seq_length() + 1
+        window = getattr(self.config, "sliding_window", None)
+        if length == 1 or not input_ids.is_cuda or input_ids.dim() != 2 or (window is not None and length > window):
+            return attention_mask
+        if attention_mask is None:
+            return torch.zeros((input_ids.shape[0], 1, 1, length), dtype=torch.float32, device=input_ids.device)
+        if attention_mask.dim() != 2 or attention_mask.shape != (input_ids.shape[0], length) or attention_mask.device != input_ids.device:
+            return attention_mask
+        lowest = torch.finfo(self.model.embed_tokens.weight.dtype).min
+        return (attention_mask == 0)[:, None, None, :].to(torch.float32).mul_(lowest)
+
     def forward(self, input_ids=None, attention_mask=None, position_ids=None, past_key_values=None,
                 inputs_embeds=None, labels=None, use_cache=None, **kwargs):
         # a cache is created when the caller asks for one (or leaves it to the config) and is not
@@ -230,6 +350,8 @@ class _KVmixCausalLM:
         if use or past_key_values is not None:
             n = input_ids.shape[1] if input_ids is not None else inputs_embeds.shape[1]
             past_key_values = self._with_cache({"past_key_values": past_key_values}, max(4096, 2 * n))["past_key_values"]
+            if input_ids is not None and n == 1:
+                attention_mask = self._step_mask(input_ids, attention_mask, past_key_values)
         return super().forward(input_ids=input_ids, attention_mask=attention_mask, position_ids=position_ids,
                                past_key_values=past_key_values, inputs_embeds=inputs_embeds, labels=labels,
                                use_cache=use, **kwargs)
@@ -249,7 +371,7 @@ class _KVmixCausalLM:
 
 class LlamaForCausalLM_KVmix(_KVmixCausalLM, LlamaForCausalLM):
     """Drop-in for the reference's class of the same name (models/modeling_llama_KVmix.py:515-537)."""
-    _attention_class = LlamaAttention_KVmix
+    _attention_class, _layer_class = LlamaAttention_KVmix, LlamaDecoderLayer
 
     def __init__(self, config, quant_bits: QuantBits = None, **kwargs):
         super().__init__(config)
@@ -258,7 +380,7 @@ class LlamaForCausalLM_KVmix(_KVmixCausalLM, LlamaForCausalLM):
 
 class MistralForCausalLM_KVmix(_KVmixCausalLM, MistralForCausalLM):
     """Drop-in for the reference's class of the same name (models/modeling_mistral_KVmix.py)."""
-    _attention_class = MistralAttention_KVmix
+    _attention_class, _layer_class = MistralAttention_KVmix, MistralDecoderLayer
 
     def __init__(self, config, quant_bits: QuantBits = None, **kwargs):
         super().__init__(config)

@@ -324,78 +324,17 @@ def linear_rows_supported(m: int, k: int, rows: int, epilogue: int = _lib.LINEAR
     return bool(_lib.load().kvmix_linear_rows_supported(ctypes.byref(st)))
 
 
-def _rows2(t: torch.Tensor, what: str) -> torch.Tensor:
-    """[..., n] fp16 as [rows, n] with unit-stride rows."""
-    if t.dtype != torch.float16:
-        raise RuntimeError(f"expected scalar type Half for {what} but found {t.dtype}")
-    t = t.reshape(-1, t.shape[-1])
-    return t if t.stride(1) == 1 and t.stride(0) >= t.shape[1] else t.contiguous()
-
-
-def _linear_descriptor(x, w, split, epilogue, norm_weight, eps):
-    """w: one stacked weight, cut into parts of `split` rows, or a tuple with one weight per part."""
-    st = _lib.LinearRows()
-    x = _rows2(x, "x")
-    ws = w if isinstance(w, (tuple, list)) else (w,)
-    _need_gpu(x, *ws)
-    st.x, st.m, st.k = x.data_ptr(), x.shape[0], x.shape[1]
-    st.x_stride = x.stride(0) if x.shape[0] > 1 else x.shape[1]
-    st.epilogue = epilogue
-    for t in ws:
-        if t.dtype != torch.float16 or t.dim() != 2 or t.shape[1] != x.shape[1] or t.stride(1) != 1 or t.stride(0) != ws[0].stride(0):
-            raise RuntimeError("weights must be fp16 [rows, k] with unit-stride rows and one row stride")
-    st.w_stride = ws[0].stride(0)
-    if len(ws) == 1:
-        if sum(split) != ws[0].shape[0]:
-            raise RuntimeError("the stacked weight must hold the rows of all its parts")
-        at = ws[0].data_ptr()
-        for j, n in enumerate(split):
-            st.w[j], st.rows[j] = at, n
-            at += 2 * n * st.w_stride
-    else:
-        for j, t in enumerate(ws):
-            st.w[j], st.rows[j] = t.data_ptr(), t.shape[0]
-    if norm_weight is not None:
-        if norm_weight.dtype != torch.float16 or norm_weight.numel() != x.shape[1] or not norm_weight.is_contiguous():
-            raise RuntimeError("norm_weight must be k contiguous fp16 values")
-        st.norm_weight, st.norm_eps = norm_weight.data_ptr(), eps
-    return st, x
-
-
-def _linear_launch(st, x) -> None:
-    import ctypes
-
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.load().kvmix_linear_rows(ctypes.byref(st), _stream(x)))
-
-
 def linear_rows(x: torch.Tensor, w: torch.Tensor, norm_weight: torch.Tensor = None, eps: float = 0.0,
                 residual: torch.Tensor = None, fp32: bool = False) -> torch.Tensor:
     """x @ w.T for a few rows of x (kvmix_linear_rows): x [..., k], w [n, k] fp16 -> [..., n].  norm_weight: x is
     RMS-normalised first; residual [..., n]: added to the fp16 product; fp32: the fp16 product as fp32."""
-    epilogue = _lib.LINEAR_RESIDUAL if residual is not None else (_lib.LINEAR_FLOAT if fp32 else _lib.LINEAR_PLAIN)
-    n = w.shape[0]
-    st, x2 = _linear_descriptor(x, w, (n,), epilogue, norm_weight, eps)
-    out = torch.empty(x.shape[:-1] + (n,), dtype=torch.float32 if fp32 else torch.float16, device=x.device)
-    if residual is not None:
-        residual = _rows2(residual, "residual")
-        if residual.shape != (x2.shape[0], n):
-            raise RuntimeError("residual must have the shape of the product")
-        st.residual, st.residual_stride = residual.data_ptr(), residual.stride(0) if residual.shape[0] > 1 else n
-    st.out, st.out_stride = out.data_ptr(), n
-    _linear_launch(st, x2)
-    return out
+    return _host().linear_rows(x, w, norm_weight, eps, residual, fp32)
 
 
 def swiglu_rows(x: torch.Tensor, w, norm_weight: torch.Tensor = None, eps: float = 0.0) -> torch.Tensor:
     """silu(x @ gate.T) * (x @ up.T) for a few rows of x, fp16, in one launch (kvmix_linear_rows); w = the stacked
     [2 n, k] weight, gate over up, or the pair."""
-    n = w[0].shape[0] if isinstance(w, (tuple, list)) else w.shape[0] // 2
-    st, x2 = _linear_descriptor(x, w, (n, n), _lib.LINEAR_SWIGLU, norm_weight, eps)
-    out = torch.empty(x.shape[:-1] + (n,), dtype=torch.float16, device=x.device)
-    st.out, st.out_stride = out.data_ptr(), n
-    _linear_launch(st, x2)
-    return out
+    return _host().swiglu_rows(x, w if isinstance(w, (tuple, list)) else (w,), norm_weight, eps)
 
 
 def qkv_rope_append(x: torch.Tensor, w, heads: int, kv_heads: int, cos: torch.Tensor, sin: torch.Tensor,
@@ -407,24 +346,11 @@ def qkv_rope_append(x: torch.Tensor, w, heads: int, kv_heads: int, cos: torch.Te
     x [B, (1,) k]; w = the stacked [(heads + 2 kv_heads) D, k] weight or the (query, key, value) weights; cos, sin: D
     values shared by the sequences, or [B, (1,) D]; tails and slots as in rope_append.
     Returns the rotated queries [B, heads, 1, D]."""
-    D = k_tail.shape[-1]
-    st, x2 = _linear_descriptor(x, w, (heads * D, kv_heads * D, kv_heads * D), _lib.LINEAR_ROPE_APPEND, norm_weight, eps)
-    B = x2.shape[0]
-    for t in (cos, sin):
-        if t.dtype != torch.float16 or t.numel() not in (D, B * D):
-            raise RuntimeError("qkv_rope_append: cos and sin must hold head_dim fp16 values, shared or per sequence")
-    cos, sin = cos.reshape(-1, D).contiguous(), sin.reshape(-1, D).contiguous()
-    if cos.shape != sin.shape:
-        raise RuntimeError("qkv_rope_append: cos and sin must have the same shape")
-    st.cos, st.sin, st.cos_sin_batch_stride, st.head_dim = cos.data_ptr(), sin.data_ptr(), D if cos.shape[0] > 1 else 0, D
-    for prefix, tail, slot in (("k", k_tail, k_slot), ("v", v_tail, v_slot)):
-        if tail.dtype != torch.float16 or tail.dim() != 4 or tail.shape[:2] != (B, kv_heads) or tail.shape[3] != D or tail.stride(3) != 1:
-            raise RuntimeError("qkv_rope_append: tails must be fp16 [B, kv_heads, slots, D] with unit stride along D")
-        _set_tail(st, prefix, tail, slot)
-    q = torch.empty((B, heads, 1, D), dtype=torch.float16, device=x.device)
-    st.out, st.out_stride = q.data_ptr(), heads * D
-    _linear_launch(st, x2)
-    return q
+    slots = []
+    for slot in (k_slot, v_slot):
+        slots += (0, slot) if torch.is_tensor(slot) else (int(slot), None)
+    return _host().qkv_rope_append(x, w if isinstance(w, (tuple, list)) else (w,), heads, kv_heads, cos, sin, k_tail, v_tail,
+                                   *slots, norm_weight, eps)
 
 
 def plain_call(*tensors) -> bool:
