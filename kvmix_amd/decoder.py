@@ -250,8 +250,7 @@ class GraphDecoder(Decoder):
         self._stale = True
         self._warm = False
         self._ids = self._logits = None
-        self._pos = self._len = None
-        self._counters = {}
+        self._state = self._pos = self._len = None
         self.graph_steps = self.eager_steps = self.captures = self.flush_steps = 0
 
     # one decode step with static shapes; mutates the device counters
@@ -282,30 +281,26 @@ class GraphDecoder(Decoder):
                                           k_tail_len=klive, v_tail_len=vlive, single_pass=single)
             x = add_projection(x, out.transpose(1, 2).reshape(B, 1, cfg.hidden_size), lw["wo"])
             x = add_mlp(x, lw, cfg.rms_norm_eps)
-        self._pos.add_(1)
-        for slot, live in self._counters.values():
-            slot.add_(1)
-            live.add_(1)
+        self._state.add_(1)
         return head_logits(x, self.w, cfg.rms_norm_eps)
 
     def _sync_counters(self) -> None:
-        """Device counters for the coming steps.  Tails of equal length stay equal until the next
-        flush, so they share one pair of counters (slot of the next token, live slots once it is
-        written): a step then increments a handful of counters instead of two per layer."""
-        dev = self._pos.device
-        self._pos.fill_(self.position)
+        """Device counters for the coming steps: the position and, per tail length, the slot of the next token and the
+        live slots once it is written, in one tensor that a step increments with one launch (tails of equal length stay
+        equal until the next flush)."""
         lengths = []
         for cache in self.caches:
             _, _, nk, nv = cache.tail_windows(self.window)
             lengths.append((nk, nv))
-        for n in {n for pair in lengths for n in pair}:
-            if n not in self._counters:
-                self._counters[n] = (torch.empty(1, dtype=torch.int64, device=dev), torch.empty(1, dtype=torch.int64, device=dev))
-        self._counters = {n: c for n, c in self._counters.items() if any(n in pair for pair in lengths)}
-        for n, (slot, live) in self._counters.items():
-            slot.fill_(n)
-            live.fill_(n + 1)
-        self._len = [(self._counters[nk], self._counters[nv]) for nk, nv in lengths]
+        distinct = sorted({n for pair in lengths for n in pair})
+        values = [self.position] + [v for n in distinct for v in (n, n + 1)]
+        if self._state is None or self._state.numel() != len(values):
+            self._state = torch.empty(len(values), dtype=torch.int64, device=self._ids.device)
+        for i, v in enumerate(values):
+            self._state[i:i + 1].fill_(v)
+        self._pos = self._state[:1]
+        counters = {n: (self._state[2 * i + 1:2 * i + 2], self._state[2 * i + 2:2 * i + 3]) for i, n in enumerate(distinct)}
+        self._len = [(counters[nk], counters[nv]) for nk, nv in lengths]
 
     def _ratio_window(self) -> int:
         """Slots the tail windows need until the next flush under the ratio rule: every tail grows one token a
@@ -326,7 +321,6 @@ class GraphDecoder(Decoder):
         dev = ids.device
         if self._ids is None:
             self._ids = torch.zeros_like(ids)
-            self._pos = torch.zeros(1, dtype=torch.int64, device=dev)
         self._ids.copy_(ids)
         if self.caches[0].residual_length is None:
             self.window = self._ratio_window()
