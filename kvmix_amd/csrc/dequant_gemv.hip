@@ -18,7 +18,8 @@
 //                   waves share a tile and slice K.
 //   gemv_cols_mfma  q.K^T, 1/2/4-bit: matrix cores, one element per lane; GQA (four query heads per
 //                   pass) and 1-bit.
-//   gemv_cols3      q.K^T, the reference's 3-bit format: register streaming, vector ALU.
+//   gemv_cols3      q.K^T, the reference's 3-bit format: register streaming, vector ALU; four query heads per pass over
+//                   whole tiles of 128 words: matrix cores.
 //   gemv_cols       q.K^T, 1/2/4-bit at large batch with long rows, dense 3-bit: vector ALU,
 //                   (scale, zero) staged in LDS.
 //   gemv_rows       p.V for N = 64 / 256 or strided code rows: vector ALU.
@@ -901,6 +902,209 @@ gemv_cols3(GemvArgs a)
                 for (int e = 0; e < PER; e++) op[first + e] = f32_to_h16(flat[e]);
             }
         }
+    }
+}
+
+// ---------------------------------------------------------------------------------------
+// gemv_cols3<1, 2, 8, 4>   four query heads per pass over the reference's 3-bit words, on the matrix cores.
+//   The form above pays four fused multiply-adds per code, one per head, and is bound by them.  Here a lane turns its
+//   words into weights once and v_mfma_f32_4x4x4 (sixteen blocks of 4 heads x 4 lanes, k = four channel rows) multiplies
+//   them by all four heads: A = x of the block's four heads at four rows, B = the lane's own words at those rows, D = the
+//   lane's own outputs for the four heads, so nothing is exchanged between lanes.
+//   The weight scale * code has up to 14 significant bits and goes in as two fp16 operands, both exact: scale / 128 is
+//   split by its bits into parts of 8 and 3 (each times a 3-bit code fits fp16), and with h = 1024 + code * 2^o -- one
+//   v_and_or of the packed field where it lies, o <= 7 -- a part's product is fma(h, part, -1024 part), rounded nowhere.
+//   Three instructions per two codes instead of nine.  2^(o - 7) is taken out of the fp32 sums at the end.  The zero term
+//   is one more product per word.  That needs scale / 128 to be exact and |scale| <= 8188; four rows of which some lane's
+//   scales are not (keys that differ by less than 0.05 or by more than 57000 inside a group) go through plain fp32.
+//   A lane owns two words, a wave 128 (512 bytes of codes per row), 8 rows in flight; ksplit waves share a tile and slice
+//   K where the launch would otherwise have too few of them.
+// Measured: see launch_cols.  Bound now by the 6 vector and 2 matrix instructions per code, word and four rows as they
+// fall between the loads (two waves per SIMD: the fp32 form beside it holds 250 registers).
+// ---------------------------------------------------------------------------------------
+typedef _Float16 cols3_half2 __attribute__((ext_vector_type(2)));
+typedef _Float16 cols3_half4 __attribute__((ext_vector_type(4)));
+typedef float cols3_float4 __attribute__((ext_vector_type(4)));
+
+// code i of a word: in which of the word's 16-bit windows (bits 0, 8, 16, 24 on) it is taken, and its offset there
+__device__ __forceinline__ constexpr int cols3_window(int i) { return i < 3 ? 0 : (i < 6 ? 1 : (i < 8 ? 2 : 3)); }
+__device__ __forceinline__ constexpr int cols3_offset(int i) { return 3 * i - 8 * cols3_window(i); }
+
+template <>
+__global__ void __launch_bounds__(64 * kColsWaves) __attribute__((amdgpu_waves_per_eu(2)))
+gemv_cols3<1, 2, 8, 4>(GemvArgs a)
+{
+    constexpr int VALS = 11, UPL = 2, U = 8, NREP = 4, TU = kWave * UPL, TOT = UPL * VALS;
+    extern __shared__ float xs[];  // x [NREP][K] fp16, then partial sums of a head [waves / 2][TOT][64]
+    uint16_t *xh = reinterpret_cast<uint16_t *>(xs);
+    const int lane = threadIdx.x, wy = threadIdx.y;
+    int64_t bx, hg;
+    xcd_swizzled_block(bx, hg, true);
+    const int64_t sample0 = hg * NREP, m = blockIdx.z, kv = sample0 / a.heads_per_kv;
+    const int K = (int)a.K, nunits = (int)(a.N / VALS);
+    if (nunits < TU) return;  // (never launched so; the same for every thread)
+    const uint16_t *xp = reinterpret_cast<const uint16_t *>(a.x) + sample0 * a.x_bs + m * a.x_rs;
+    for (int i = wy * kWave + lane; i < NREP * K; i += blockDim.y * kWave) xh[i] = xp[(i / K) * a.x_bs + i % K];
+    __syncthreads();
+
+    const int ks = a.ksplit, slice = wy % ks;
+    int t0 = (int)(bx * (blockDim.y / ks) + wy / ks) * TU;
+    if (t0 >= nunits) return;  // (ks > 1: a block is one tile)
+    t0 = t0 + TU <= nunits ? t0 : nunits - TU;
+    const int unit0 = t0 + lane * UPL, kbeg = slice * (K / ks), steps = K / ks / U;
+
+    struct __attribute__((packed, aligned(2))) Half2 {
+        uint16_t v[UPL];
+    };
+    const uint8_t *cb = reinterpret_cast<const uint8_t *>(a.code + kv * a.c_bs);
+    const uint8_t *sb = reinterpret_cast<const uint8_t *>(reinterpret_cast<const uint16_t *>(a.scale) + kv * a.s_bs);
+    const uint8_t *zb = reinterpret_cast<const uint8_t *>(reinterpret_cast<const uint16_t *>(a.zero) + kv * a.s_bs);
+    const uint32_t c_step = (uint32_t)a.c_rs * 4u, s_step = (uint32_t)a.s_rs * 2u;
+    uint32_t co = (uint32_t)unit0 * 4u + (uint32_t)kbeg * c_step, so = (uint32_t)unit0 * 2u + (uint32_t)kbeg * s_step;
+    Words<UPL> cw[U];
+    uint32_t sw[U], zw[U];
+    auto next_row = [&](int u) {
+        cw[u] = ld_stream<Words<UPL>, KVMIX_COLS_NT_CODES>(cb + co);
+        sw[u] = __builtin_bit_cast(uint32_t, ld_stream<Half2, false>(sb + so));
+        zw[u] = __builtin_bit_cast(uint32_t, ld_stream<Half2, false>(zb + so));
+        co += c_step;
+        so += s_step;
+    };
+    cols3_float4 acc[UPL][VALS], zacc[UPL];
+#pragma unroll
+    for (int j = 0; j < UPL; j++) {
+        zacc[j] = cols3_float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < VALS; i++) acc[j][i] = zacc[j];
+    }
+    uint32_t magic = 0x64006400u;
+    asm("" : "+v"(magic));  // (in a register: v_and_or_b32 takes no literal)
+    // rows k .. k + 3, held in registers g .. g + 3
+    auto rows4 = [&](int g, int k) {
+        const cols3_half4 xa = *reinterpret_cast<const cols3_half4 *>(xh + (lane & 3) * K + k);
+        cols3_half2 sp[UPL][2], small[UPL][2];
+        uint32_t inexact = 0, top = 0;
+#pragma unroll
+        for (int j = 0; j < UPL; j++) {
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const uint32_t pair = __builtin_amdgcn_perm(sw[g + 2 * p + 1], sw[g + 2 * p], j ? 0x07060302u : 0x05040100u);
+                sp[j][p] = __builtin_bit_cast(cols3_half2, pair);
+                small[j][p] = sp[j][p] * (_Float16)0.0078125f;
+                inexact |= pair ^ __builtin_bit_cast(uint32_t, small[j][p] * (_Float16)128.0f);
+                const uint32_t size = pair & 0x7fff7fffu;
+                const uint32_t lo = size & 0xffffu, hi = size >> 16;
+                top = top > lo ? top : lo;
+                top = top > hi ? top : hi;
+            }
+        }
+        if (__builtin_expect(__any(inexact != 0 || top > 0x6fffu), 0)) {  // (0x6fff: 8188)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+#pragma unroll
+                for (int j = 0; j < UPL; j++) {
+                    const uint32_t w = cw[g + r].v[j];
+                    const float sc = h16_to_f32((uint16_t)(sw[g + r] >> (16 * j))), ze = h16_to_f32((uint16_t)(zw[g + r] >> (16 * j)));
+                    float x[NREP];
+#pragma unroll
+                    for (int h = 0; h < NREP; h++) {
+                        x[h] = h16_to_f32(xh[h * K + k + r]);
+                        zacc[j][h] = fmaf(x[h], ze, zacc[j][h]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < VALS; i++) {
+                        const float v = sc * ((float)(w & (7u << (3 * i))) * (0.0078125f / (float)(1 << (8 * cols3_window(i)))));
+#pragma unroll
+                        for (int h = 0; h < NREP; h++) acc[j][i][h] = fmaf(x[h], v, acc[j][i][h]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < UPL; j++) {
+            uint32_t win[2][4], z[2];
+            cols3_half2 part[2][2], away[2][2];  // [pair of rows][part of the scale]
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const uint32_t w0 = cw[g + 2 * p].v[j], w1 = cw[g + 2 * p + 1].v[j];
+                win[p][0] = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
+                win[p][1] = __builtin_amdgcn_perm(w1, w0, 0x06050201u);
+                win[p][2] = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
+                win[p][3] = __builtin_amdgcn_perm(w1, w0, 0x0c070c03u);
+                z[p] = __builtin_amdgcn_perm(zw[g + 2 * p + 1], zw[g + 2 * p], j ? 0x07060302u : 0x05040100u);
+                part[p][0] = __builtin_bit_cast(cols3_half2, __builtin_bit_cast(uint32_t, small[j][p]) & 0xfff8fff8u);
+                part[p][1] = small[j][p] - part[p][0];
+#pragma unroll
+                for (int q = 0; q < 2; q++) away[p][q] = part[p][q] * (_Float16)-1024.0f;
+            }
+            zacc[j] = __builtin_amdgcn_mfma_f32_4x4x4f16(xa, __builtin_bit_cast(cols3_half4, ((uint64_t)z[1] << 32) | z[0]), zacc[j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < VALS; i++) {
+                const uint32_t mask = (i == 10 ? 0x00030003u : 0x00070007u) << cols3_offset(i);
+                cols3_half2 h[2];
+#pragma unroll
+                for (int p = 0; p < 2; p++) h[p] = __builtin_bit_cast(cols3_half2, (win[p][cols3_window(i)] & mask) | magic);
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const cols3_half2 b0 = __builtin_elementwise_fma(h[0], part[0][q], away[0][q]);
+                    const cols3_half2 b1 = __builtin_elementwise_fma(h[1], part[1][q], away[1][q]);
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_4x4x4f16(xa, cols3_half4{b0[0], b0[1], b1[0], b1[1]}, acc[j][i], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // (operands of more codes at once would spill)
+            }
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        next_row(u);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll 1
+    for (int st = 0; st < steps - 1; st++) {
+#pragma unroll
+        for (int g = 0; g < U; g += 4) {
+            rows4(g, kbeg + st * U + g);
+#pragma unroll
+            for (int u = 0; u < 4; u++) next_row(g + u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < U; g += 4) rows4(g, kbeg + (steps - 1) * U + g);  // (no row past the slice is ever addressed)
+
+    float *part = xs + NREP * K / 2;
+#pragma unroll
+    for (int h = 0; h < NREP; h++) {  // (one head at a time: all four's sums beside each other would spill)
+        float flat[TOT];
+#pragma unroll
+        for (int j = 0; j < UPL; j++) {
+#pragma unroll
+            for (int i = 0; i < VALS; i++) flat[j * VALS + i] = fmaf(acc[j][i][h], 128.0f / (float)(1 << cols3_offset(i)), zacc[j][h]);
+        }
+        for (int half = ks / 2; half >= 1; half /= 2) {  // the upper half of the waves hands its sums to the lower one
+            if (slice >= half && slice < 2 * half) {
+#pragma unroll
+                for (int e = 0; e < TOT; e++) part[((slice - half) * TOT + e) * kWave + lane] = flat[e];
+            }
+            __syncthreads();
+            if (slice < half) {
+#pragma unroll
+                for (int e = 0; e < TOT; e++) flat[e] += part[(slice * TOT + e) * kWave + lane];
+            }
+            __syncthreads();
+        }
+        if (slice == 0) {
+            uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + (sample0 + h) * a.o_bs + m * a.o_rs + (int64_t)unit0 * VALS;
+#pragma unroll
+            for (int e = 0; e < TOT; e += 2) {
+                const uint32_t pk = f32_to_h16(flat[e]) | ((uint32_t)f32_to_h16(flat[e + 1]) << 16);
+                __builtin_memcpy(op + e, &pk, 4);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -3119,6 +3323,23 @@ struct ColsUpl {
     static constexpr int value = MODE == 3 ? 4 : 1;
 };
 
+static void launch_cols3_heads(GemvArgs &a, int64_t samples, hipStream_t st)
+{
+    const int64_t units = a.N / 11;
+    if (!tile_fits(units, 128)) return;
+    const int64_t tiles = (units + 127) / 128, waves = tiles * (samples / 4) * a.M;
+    int ks = waves < 1024 ? 4 : 1;
+#ifdef KVMIX_EXPERIMENT
+    if (const char *e = getenv("KVMIX_DBG_COLS3_KS")) ks = atoi(e);
+#endif
+    a.ksplit = ks;
+    const size_t x_lds = ((size_t)4 * a.K * 2 + 7) / 8 * 8;
+    const int wpb = ks > 1 ? ks : pick_waves_per_block(tiles);
+    const dim3 grid((unsigned)(ks > 1 ? tiles : (tiles + wpb - 1) / wpb), (unsigned)(samples / 4), (unsigned)a.M);
+    KVMIX_LAUNCH((gemv_cols3<1, 2, 8, 4>), grid, dim3(kWave, wpb), x_lds + (size_t)(ks / 2) * 22 * kWave * sizeof(float), st, a,
+                 "gemv_cols3<1,2,8,4>");
+}
+
 template <int MODE, int RQ, int UPL>
 static void launch_cols_cfg(const GemvArgs &a, int64_t samples, hipStream_t st)
 {
@@ -3374,8 +3595,15 @@ static void launch_cols(GemvArgs &a, int64_t samples, hipStream_t st)
 #ifdef KVMIX_EXPERIMENT
         if (const char *e = getenv("KVMIX_DBG_COLS3_WIDE")) force_wide = atoi(e) == 1 && units >= 256;
 #endif
-        if (heads_per_block(a.heads_per_kv) == 4 && a.K <= 2048)  // GQA: four query heads per pass over the
-            launch_cols3_cfg<2, 2, 4>(a, samples, st);              // words (their x rows must fit into LDS)
+        const bool four_heads = heads_per_block(a.heads_per_kv) == 4 && a.K <= 2048;  // GQA: four query heads per pass
+        // over the words (their x rows must fit into LDS).  On the matrix cores where whole tiles of 128 words cover the row
+        // with at most a quarter of it done twice, in whole steps of eight rows for up to four slices.  Measured per call,
+        // operands from memory, 32 / 8 heads: B = 16, T = 32637 123 -> 86 us (4.5 TB/s), B = 8, T = 8184 30 -> 24.  Not for
+        // 186 words, of which a third would be done twice (B = 64, T = 2046: 36 -> 41).
+        if (four_heads && units >= 128 && a.K % 32 == 0 && 4 * ((units + 127) / 128 * 128) <= 5 * units)
+            launch_cols3_heads(a, samples, st);
+        else if (four_heads)
+            launch_cols3_cfg<2, 2, 4>(a, samples, st);
         else if (force_wide || cols3_whole_rows(units, batch))
             launch_cols3_cfg<1, 4, 1>(a, samples, st);
         else if (units >= 128 && 2 * ((units + 127) / 128) * 128 <= 3 * units && a.K >= 64 &&
