@@ -942,7 +942,7 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
     xcd_swizzled_block(bx, hg, true);
     const int64_t sample0 = hg * NREP, m = blockIdx.z, kv = sample0 / a.heads_per_kv;
     const int K = (int)a.K, nunits = (int)(a.N / VALS);
-    if (nunits < TU) return;  // (never launched so; the same for every thread)
+    if (nunits < TU || K < 32) return;  // (never launched so: a tile wider than the row, fewer rows than the slices' first loads; the same for every thread)
     const uint16_t *xp = reinterpret_cast<const uint16_t *>(a.x) + sample0 * a.x_bs + m * a.x_rs;
     for (int i = wy * kWave + lane; i < NREP * K; i += blockDim.y * kWave) xh[i] = xp[(i / K) * a.x_bs + i % K];
     __syncthreads();
@@ -3326,7 +3326,7 @@ struct ColsUpl {
 static void launch_cols3_heads(GemvArgs &a, int64_t samples, hipStream_t st)
 {
     const int64_t units = a.N / 11;
-    if (!tile_fits(units, 128)) return;
+    if (!tile_fits(units, 128) || !tile_fits(a.K, 32)) return;
     const int64_t tiles = (units + 127) / 128, waves = tiles * (samples / 4) * a.M;
     int ks = waves < 1024 ? 4 : 1;
 #ifdef KVMIX_EXPERIMENT
