@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(kClassWaves * kWave) prefill_mask_classes(Pref
     const int64_t slice = blockIdx.y;
     const int r0 = blockIdx.x * 32, valid = a.q_len - r0 < 32 ? a.q_len - r0 : 32;
     const T *base = (const T *)a.mask + (slice / mask_heads) * a.m_bs + (slice % mask_heads) * a.m_hs;
-    // what the prompt branch takes for a row masked everywhere: see KVmixAttention.forward
+    // what the prompt branch takes for a row masked everywhere: see KVmixAttention._prompt_attention
     const float absorbed = sizeof(T) == 2 ? kHalfLowest : -1e30f;
     for (int t = threadIdx.x; t < a.k_tiles; t += kClassWaves * kWave) tile_bits[t] = 0;
     if (threadIdx.x < 2) row_bits[threadIdx.x] = 0;
