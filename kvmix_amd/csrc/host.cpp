@@ -555,7 +555,12 @@ Tensor linear_operands(kvmix_linear_rows_t &st, const Tensor &x_in, const std::v
             at += 2 * split[j] * st.w_stride;
         }
     } else {
-        for (size_t j = 0; j < ws.size(); j++) st.w[j] = ws[j].data_ptr(), st.rows[j] = ws[j].size(0);
+        // (the epilogues place their outputs by `split`: rows beyond it would be written where no output was made for them)
+        if (ws.size() != split.size()) fail("a projection in parts has one weight per part");
+        for (size_t j = 0; j < ws.size(); j++) {
+            if (ws[j].size(0) != split[j]) fail("each part's weight must hold the rows of that part");
+            st.w[j] = ws[j].data_ptr(), st.rows[j] = split[j];
+        }
     }
     if (norm) {
         if (norm->scalar_type() != at::kHalf || norm->numel() != x.size(1) || !norm->is_contiguous())

@@ -105,3 +105,32 @@ def test_refusals(dev):
         ops.linear_rows(x.float(), w)
     with pytest.raises(RuntimeError):
         ops.qkv_rope_append(x, w, 1, 1, nw[:2], nw[:2], *(torch.zeros(4, 1, 2, 2, device=dev).half() for _ in range(2)), 0, 0)
+
+
+def test_parts_have_the_rows_of_their_heads(dev):
+    """Weights given part by part are held to the heads and to each other before anything is launched: a key weight with
+    more rows than kv_heads * D would write past the tails' heads, a query weight with fewer leave outputs unwritten."""
+    from kvmix_amd import ops
+
+    D, heads, kv = 32, 4, 2
+    x, w, nw, _ = operands(dev, 3, 256, (heads + 2 * kv + 4) * D)
+    cos, sin = (torch.ones(1, 1, D, device=dev).half() for _ in range(2))
+    kt, vt = (torch.zeros(3, kv, 4, D, device=dev).half() for _ in range(2))
+
+    def rows(*parts):
+        return tuple(w[:n * D].contiguous() for n in parts)
+
+    def call(weights):
+        return ops.qkv_rope_append(x, weights, heads, kv, cos, sin, kt, vt, 0, 0, nw, 1e-5)
+
+    for parts in ((heads, kv + 1, kv + 1), (heads, 2 * kv, 2 * kv), (heads, kv, kv + 1), (heads - 2, kv, kv), (2 * heads, kv, kv),
+                  (heads, kv), (heads + 2 * kv - 1, 1)):
+        with pytest.raises(RuntimeError):
+            call(rows(*parts))
+    assert not kt.any() and not vt.any()
+    stacked = torch.cat(rows(heads, kv, kv))
+    want, k_want, v_want = call(stacked), kt.clone(), vt.clone()
+    assert torch.equal(call(rows(heads, kv, kv)), want) and torch.equal(kt, k_want) and torch.equal(vt, v_want)
+    for weights in ((w[:D], w[:2 * D]), (w[:D],) * 3):
+        with pytest.raises(RuntimeError):
+            ops.swiglu_rows(x, weights)
