@@ -85,6 +85,13 @@ void need_half(std::initializer_list<const Tensor *> ts)
         if (t->scalar_type() != at::kHalf) fail("expected scalar type Half but found " + dtype_name(*t));
 }
 
+// what a kernel reads or writes beside `ref` lies where `ref` does
+void need_with(const Tensor &ref, std::initializer_list<const Tensor *> ts)
+{
+    for (const Tensor *t : ts)
+        if (t->device() != ref.device()) fail("expected all tensors on " + ref.device().str() + ", but one is on " + t->device().str());
+}
+
 void check_bits(int64_t bits)
 {
     if (bits < 1 || bits > 4) fail("Supported quantization bits: 1, 2, 3, 4");
@@ -540,7 +547,7 @@ Tensor linear_operands(kvmix_linear_rows_t &st, const Tensor &x_in, const std::v
     st.epilogue = epilogue;
     if (ws.empty() || ws.size() > 3) fail("a projection has one to three weights");
     for (const Tensor &w : ws) {
-        need_gpu({&w});
+        need_with(x, {&w});
         if (w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(1) || w.stride(1) != 1 || w.stride(0) != ws[0].stride(0))
             fail("weights must be fp16 [rows, k] with unit-stride rows and one row stride");
     }
@@ -563,6 +570,7 @@ Tensor linear_operands(kvmix_linear_rows_t &st, const Tensor &x_in, const std::v
         }
     }
     if (norm) {
+        need_with(x, {&*norm});
         if (norm->scalar_type() != at::kHalf || norm->numel() != x.size(1) || !norm->is_contiguous())
             fail("norm_weight must be k contiguous fp16 values");
         st.norm_weight = norm->data_ptr(), st.norm_eps = (float)eps;
@@ -592,6 +600,7 @@ Tensor linear_rows(const Tensor &x_in, const Tensor &w, const OptTensor &norm, d
     Tensor residual;
     if (residual_in) {
         residual = rows2(*residual_in, "residual");
+        need_with(x, {&residual});
         if (residual.size(0) != x.size(0) || residual.size(1) != n) fail("residual must have the shape of the product");
         st.residual = residual.data_ptr(), st.residual_stride = residual.size(0) > 1 ? residual.stride(0) : n;
     }
@@ -621,17 +630,18 @@ Tensor qkv_rope_append(const Tensor &x_in, const std::vector<Tensor> &ws, int64_
     const int64_t D = k_tail.size(-1);
     const Tensor x = linear_operands(st, x_in, ws, {heads * D, kv_heads * D, kv_heads * D}, KVMIX_LINEAR_ROPE_APPEND, norm, eps);
     const int64_t B = x.size(0);
+    need_with(x, {&cos_in, &sin_in, &k_tail, &v_tail});
     for (const Tensor *t : {&cos_in, &sin_in})
-        if (t->scalar_type() != at::kHalf || (t->numel() != D && t->numel() != B * D) || !t->is_cuda())
+        if (t->scalar_type() != at::kHalf || (t->numel() != D && t->numel() != B * D))
             fail("qkv_rope_append: cos and sin must hold head_dim fp16 values, shared or per sequence");
     const Tensor cos = cos_in.reshape({-1, D}).contiguous(), sin = sin_in.reshape({-1, D}).contiguous();
     if (cos.size(0) != sin.size(0)) fail("qkv_rope_append: cos and sin must have the same shape");
     st.cos = cos.data_ptr(), st.sin = sin.data_ptr(), st.cos_sin_batch_stride = cos.size(0) > 1 ? D : 0, st.head_dim = D;
     for (const Tensor *t : {&k_tail, &v_tail})
-        if (t->scalar_type() != at::kHalf || !t->is_cuda() || t->dim() != 4 || t->size(0) != B || t->size(1) != kv_heads || t->size(3) != D || t->stride(3) != 1)
+        if (t->scalar_type() != at::kHalf || t->dim() != 4 || t->size(0) != B || t->size(1) != kv_heads || t->size(3) != D || t->stride(3) != 1)
             fail("qkv_rope_append: tails must be fp16 [B, kv_heads, slots, D] with unit stride along D");
     for (const OptTensor *t : {&k_slot_dev, &v_slot_dev})
-        if (*t && ((*t)->scalar_type() != at::kLong || (*t)->numel() != 1 || !(*t)->is_cuda()))
+        if (*t && ((*t)->scalar_type() != at::kLong || (*t)->numel() != 1 || (*t)->device() != x.device()))
             fail("a device-side slot must be one int64 element on the GPU");
     // (strides of one-element dimensions are whatever the view left there)
     st.k_tail = k_tail.data_ptr(), st.k_tail_batch_stride = k_tail.stride(0), st.k_tail_head_stride = k_tail.stride(1);

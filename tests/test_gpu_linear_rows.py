@@ -134,3 +134,24 @@ def test_parts_have_the_rows_of_their_heads(dev):
     for weights in ((w[:D], w[:2 * D]), (w[:D],) * 3):
         with pytest.raises(RuntimeError):
             ops.swiglu_rows(x, weights)
+
+
+@pytest.mark.parametrize("left", ["x", "w", "norm", "residual", "cos", "sin", "k_tail", "v_tail", "slot"])
+def test_operands_lie_on_one_device(dev, left):
+    """One operand left in host memory (a partly offloaded model) is refused before a kernel sees its address."""
+    from kvmix_amd import ops
+
+    D, heads, kv = 32, 2, 1
+    x, w, nw, res = operands(dev, 2, 256, (heads + 2 * kv) * D)
+    t = {"x": x, "w": w, "norm": nw, "residual": res, "cos": torch.ones(1, 1, D, device=dev).half(), "sin": torch.ones(1, 1, D, device=dev).half(),
+         "k_tail": torch.zeros(2, kv, 3, D, device=dev).half(), "v_tail": torch.zeros(2, kv, 3, D, device=dev).half(), "slot": torch.tensor([1], device=dev)}
+    calls = [(("x", "w", "norm", "cos", "sin", "k_tail", "v_tail", "slot"),
+              lambda t: ops.qkv_rope_append(t["x"], t["w"], heads, kv, t["cos"], t["sin"], t["k_tail"], t["v_tail"], t["slot"], t["slot"], t["norm"], 1e-5)),
+             (("x", "w", "residual"), lambda t: ops.linear_rows(t["x"], t["w"], residual=t["residual"])),
+             (("x", "w", "norm"), lambda t: ops.linear_rows(t["x"], t["w"], t["norm"], 1e-5)),
+             (("x", "w", "norm"), lambda t: ops.swiglu_rows(t["x"], t["w"], t["norm"], 1e-5))]
+    for reads, call in calls:
+        call(t)
+        if left in reads:
+            with pytest.raises(RuntimeError):
+                call({**t, left: t[left].cpu()})
