@@ -380,7 +380,7 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, attenti
     where the kernel does not take the call."""
     import ctypes
 
-    if any(t.dim() != 4 or t.dtype != torch.float16 or not t.is_cuda for t in (q, k, v)):
+    if any(t.dim() != 4 or t.dtype != torch.float16 or not t.is_cuda or t.device != q.device for t in (q, k, v)):
         return None
     B, nh, Q, D = q.shape
     nkv, T = k.shape[1], k.shape[2]
