@@ -396,6 +396,8 @@ int prefill_check(const kvmix_prefill_attn_t *p)
     if (p->heads % p->kv_heads != 0) return KVMIX_ERR_HEADS;
     if (p->head_dim != 64 && p->head_dim != 128) return KVMIX_ERR_UNSUPPORTED;
     if (p->kv_len > kMaxKeyTiles * kPreK || p->q_len > (1 << 24) || p->heads > (1 << 24)) return KVMIX_ERR_UNSUPPORTED;
+    // launches that fit a grid: a block per 128 queries and head, mask slices along y
+    if ((__int128)p->batch * p->heads * ((p->q_len + 32 * kPreWaves - 1) / (32 * kPreWaves)) > 0x7fffffff) return KVMIX_ERR_UNSUPPORTED;
     // 16-byte loads and 8-byte stores
     const int64_t strides[] = {p->q_batch_stride, p->q_head_stride, p->q_token_stride, p->k_batch_stride, p->k_head_stride,
                                p->k_token_stride, p->v_batch_stride, p->v_head_stride, p->v_token_stride};
@@ -406,6 +408,7 @@ int prefill_check(const kvmix_prefill_attn_t *p)
     if (p->mask) {
         if (p->mask_dtype != KVMIX_F16 && p->mask_dtype != KVMIX_F32) return KVMIX_ERR_DTYPE;
         if ((p->mask_batch != 1 && p->mask_batch != p->batch) || (p->mask_heads != 1 && p->mask_heads != p->heads)) return KVMIX_ERR_SHAPE;
+        if ((__int128)p->mask_batch * p->mask_heads > 65535) return KVMIX_ERR_UNSUPPORTED;
         if (p->mask_batch_stride < 0 || p->mask_head_stride < 0 || p->mask_row_stride < 0) return KVMIX_ERR_SHAPE;
     }
     return KVMIX_OK;
@@ -467,11 +470,9 @@ extern "C" int kvmix_prefill_attention(const kvmix_prefill_attn_t *p, void *work
     a.bits = nullptr;
     a.flag_b = a.flag_h = 0;
     const int64_t blocks = p->batch * p->heads * a.q_tiles;
-    if (blocks > 0x7fffffff) return KVMIX_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (p->mask) {
         const int64_t slices = p->mask_batch * p->mask_heads;
-        if (slices > 65535) return KVMIX_ERR_UNSUPPORTED;
         if (!workspace || (uintptr_t)workspace % 8 != 0 || workspace_bytes < kvmix_prefill_attention_workspace_bytes(p)) return KVMIX_ERR_WORKSPACE;
         uint64_t *bits = (uint64_t *)workspace;
         uint8_t *flags = (uint8_t *)workspace + 256 * prefill_flag_bytes(p), *dead = flags + prefill_flag_bytes(p);
