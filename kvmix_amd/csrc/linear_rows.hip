@@ -316,6 +316,7 @@ bool linear_plan(const kvmix_linear_rows_t *p, LinearPlan *pl)
     int64_t pieces = ((units + target - 1) / target + 3) / 4 * 4;
     const int64_t most = (64 << 10) / (kLinWaves * rt * 4 * pl->mg * 4);  // (partial sums in LDS)
     if (pieces > most) pieces = most;
+    if (pieces < 4) pieces = 4;  // (no rows at all: nothing is launched)
     pl->pieces = (int)pieces;
     pl->blocks = (unsigned)((units + pieces - 1) / pieces);
     pl->lds = (size_t)kLinWaves * rt * pieces * 4 * pl->mg * 4;
