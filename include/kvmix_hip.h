@@ -410,8 +410,8 @@ int kvmix_rope_append(const kvmix_rope_append_t *step, kvmix_stream_t stream);
  *                             v_slot of the tail windows, exactly as kvmix_rope_append writes them; cos, sin
  *                             [head_dim] fp16 per sequence, cos_sin_batch_stride elements apart (0: shared)
  * k a multiple of 128, rows 16-byte aligned, m <= 16 and the x rows small enough to stay in registers, else
- * KVMIX_ERR_UNSUPPORTED: kvmix_linear_rows_supported tells (every epilogue takes k <= 4096; the plain ones without a
- * norm k <= 6144, k <= 11264 for m <= 8, k <= 14336 for m <= 4).  Only sizes, strides and the pointers' alignment are
+ * KVMIX_ERR_UNSUPPORTED: kvmix_linear_rows_supported tells (every epilogue takes k <= 4096, the residual one without
+ * a norm only; the plain ones without a norm k <= 6144, k <= 11264 for m <= 8, k <= 14336 for m <= 4).  Only sizes, strides and the pointers' alignment are
  * read there.
  */
 #define KVMIX_LINEAR_PLAIN 0

@@ -303,6 +303,7 @@ bool linear_plan(const kvmix_linear_rows_t *p, LinearPlan *pl)
     pl->mg = p->m <= 4 ? 1 : (p->m <= 8 ? 2 : 4);
     if (!pl->ch || p->m > 16) return false;
     const bool norm = p->norm_weight != nullptr;
+    if (norm && p->epilogue == KVMIX_LINEAR_RESIDUAL) return false;  // (nothing in a decoder layer is both: no such instance)
     if (pl->ch > 8 && (pl->mg > 2 || pair || norm)) return false;
     if ((pl->ch > 6 && pl->mg > 2) || (pl->ch > 11 && pl->mg > 1)) return false;  // (no faster than the library's there)
     if (pl->ch > 6 && norm && pair && pl->mg > 1) return false;
