@@ -595,6 +595,7 @@ Tensor linear_rows(const Tensor &x_in, const Tensor &w, const OptTensor &norm, d
 {
     kvmix_linear_rows_t st{};
     if (w.dim() != 2) fail("weights must be fp16 [rows, k] with unit-stride rows and one row stride");
+    if (residual_in && fp32) fail("a product with a residual is fp16: fp32 cannot be asked for with it");
     const int64_t n = w.size(0);
     const Tensor x = linear_operands(st, x_in, {w}, {n}, residual_in ? KVMIX_LINEAR_RESIDUAL : fp32 ? KVMIX_LINEAR_FLOAT : KVMIX_LINEAR_PLAIN, norm, eps);
     Tensor residual;

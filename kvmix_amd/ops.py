@@ -327,7 +327,8 @@ def linear_rows_supported(m: int, k: int, rows: int, epilogue: int = _lib.LINEAR
 def linear_rows(x: torch.Tensor, w: torch.Tensor, norm_weight: torch.Tensor = None, eps: float = 0.0,
                 residual: torch.Tensor = None, fp32: bool = False) -> torch.Tensor:
     """x @ w.T for a few rows of x (kvmix_linear_rows): x [..., k], w [n, k] fp16 -> [..., n].  norm_weight: x is
-    RMS-normalised first; residual [..., n]: added to the fp16 product; fp32: the fp16 product as fp32."""
+    RMS-normalised first; residual [..., n]: added to the fp16 product (without a norm); fp32: the fp16
+    product as fp32 (without a residual)."""
     return _host().linear_rows(x, w, norm_weight, eps, residual, fp32)
 
 

@@ -155,3 +155,14 @@ def test_operands_lie_on_one_device(dev, left):
         if left in reads:
             with pytest.raises(RuntimeError):
                 call({**t, left: t[left].cpu()})
+
+
+def test_residual_and_fp32_exclude_each_other(dev):
+    """(The residual sum is an fp16 one; as fp32 storage its bytes would be no numbers at all.)  Likewise residual and norm."""
+    from kvmix_amd import ops
+
+    x, w, nw, res = operands(dev, 4, 256, 24)
+    for kw in ({"residual": res, "fp32": True}, {"residual": res, "norm_weight": nw, "eps": 1e-5}):
+        with pytest.raises(RuntimeError):
+            ops.linear_rows(x, w, **kw)
+    assert ops.linear_rows(x, w[:0]).shape == (4, 0) and ops.linear_rows(x[:0], w).shape == (0, 24)
