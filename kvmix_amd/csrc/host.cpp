@@ -448,11 +448,11 @@ bool prefer_single_pass(int64_t batch, int64_t heads, int64_t kv_heads, int64_t 
     return api.decode_attention_fused_plan(&st, &plan) == KVMIX_OK && plan.recommended;
 }
 
-// k_len / v_len: live tail slots (-1: all); *_len_dev: where the kernels read them instead
+// k_len / v_len: live tail slots (none: all); *_len_dev: where the kernels read them instead
 std::pair<Tensor, OptTensor> decode_attention(const Tensor &q_in, const OptTriple &k_packed, const OptTriple &v_packed, const Tensor &k_tail,
                                               const Tensor &v_tail, int64_t k_group, int64_t k_bits, int64_t v_group, int64_t v_bits,
-                                              int64_t k_fmt, int64_t v_fmt, const OptTensor &mask_in, int64_t k_len, const OptTensor &k_len_dev,
-                                              int64_t v_len, const OptTensor &v_len_dev, bool single_pass)
+                                              int64_t k_fmt, int64_t v_fmt, const OptTensor &mask_in, std::optional<int64_t> k_len,
+                                              const OptTensor &k_len_dev, std::optional<int64_t> v_len, const OptTensor &v_len_dev, bool single_pass)
 {
     if (q_in.dim() != 4 || q_in.size(2) != 1) fail("decode_attention takes one query position: q must be [B, nh, 1, D]");
     need_half({&q_in, &k_tail, &v_tail});
@@ -491,9 +491,9 @@ std::pair<Tensor, OptTensor> decode_attention(const Tensor &q_in, const OptTripl
         if (*t && ((*t)->scalar_type() != at::kLong || (*t)->numel() != 1 || !(*t)->is_cuda()))
             fail("a device-side tail length must be one int64 element on the GPU");
     if (k_len_dev) st.k_tail_len_dev = k_len_dev->data_ptr<int64_t>();
-    else st.k_tail_len = k_len < 0 ? st.k_tail_slots : k_len;
+    else st.k_tail_len = k_len.value_or(st.k_tail_slots);
     if (v_len_dev) st.v_tail_len_dev = v_len_dev->data_ptr<int64_t>();
-    else st.v_tail_len = v_len < 0 ? st.v_tail_slots : v_len;
+    else st.v_tail_len = v_len.value_or(st.v_tail_slots);
     const int64_t width = std::max(st.k_tokens + st.k_tail_slots, st.v_tokens + st.v_tail_slots);
     Tensor mask;
     if (mask_in) {

@@ -450,7 +450,7 @@ def decode_attention(q: torch.Tensor, k_packed, v_packed, k_tail: torch.Tensor, 
     Returns (out [B,nh,1,D] fp16, probs [B,nh,1,width] fp16), width = max(Tk + key slots, Tv + value slots)."""
     lengths = []
     for n in (k_tail_len, v_tail_len):
-        lengths += (-1, n) if torch.is_tensor(n) else (-1 if n is None else int(n), None)
+        lengths += (None, n) if torch.is_tensor(n) else (None if n is None else int(n), None)
     return _host().decode_attention(q, k_packed, v_packed, k_tail, v_tail, k_group, k_bits, v_group, v_bits, k_fmt, v_fmt,
                                     attention_mask, *lengths, single_pass)
 
