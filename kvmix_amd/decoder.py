@@ -93,10 +93,15 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return x * cos + rot * sin
 
 
-def _few_rows(x: torch.Tensor) -> bool:
-    """One new token of a few fp16 sequences on the GPU: the projections then go through the library's kernels, which
-    stream the weights and take the normalisation before and the elementwise work after along (kvmix_linear_rows)."""
-    return x.is_cuda and x.dtype == torch.float16 and x.shape[1] == 1
+def _few_rows(x: torch.Tensor, *operands: torch.Tensor) -> bool:
+    """One new token of a few fp16 sequences on the GPU, in a call that nothing records (gradients, tracing, transforms):
+    the projections then go through the library's kernels, which stream the weights and take the normalisation before and
+    the elementwise work after along (kvmix_linear_rows)."""
+    if not (x.is_cuda and x.dtype == torch.float16 and x.shape[1] == 1):
+        return False
+    from . import ops
+
+    return ops.plain_call(x, *operands)
 
 
 def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tensor, sin: torch.Tensor, k_tail: torch.Tensor,
@@ -106,7 +111,8 @@ def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tenso
     from . import _lib, ops
 
     h, kvh = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
-    if ops.linear_rows_supported(x.shape[0], x.shape[2], h, _lib.LINEAR_ROPE_APPEND, True, cfg.head_dim, kvh):
+    if _few_rows(x, lw["wqkv"], lw["input_norm"]) and ops.linear_rows_supported(x.shape[0], x.shape[2], h, _lib.LINEAR_ROPE_APPEND, True,
+                                                                                cfg.head_dim, kvh):
         return ops.qkv_rope_append(x, lw["wqkv"], cfg.num_heads, cfg.num_kv_heads, cos, sin, k_tail, v_tail, k_slot, v_slot,
                                    lw["input_norm"], cfg.rms_norm_eps)
     qkv = F.linear(rms_norm(x, lw["input_norm"], cfg.rms_norm_eps), lw["wqkv"])
@@ -115,7 +121,7 @@ def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tenso
 
 def add_projection(x: torch.Tensor, h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x + h @ w.T"""
-    if _few_rows(x):
+    if _few_rows(x, h, w):
         from . import _lib, ops
 
         if ops.linear_rows_supported(h.shape[0], h.shape[2], w.shape[0], _lib.LINEAR_RESIDUAL):
@@ -126,7 +132,7 @@ def add_projection(x: torch.Tensor, h: torch.Tensor, w: torch.Tensor) -> torch.T
 def add_mlp(x: torch.Tensor, lw: dict, eps: float) -> torch.Tensor:
     """x + mlp(norm(x))"""
     w = lw["w_gate_up"]
-    if _few_rows(x):
+    if _few_rows(x, w, lw["post_norm"]):
         from . import _lib, ops
 
         if ops.linear_rows_supported(x.shape[0], x.shape[2], w.shape[0] // 2, _lib.LINEAR_SWIGLU, True):
@@ -137,7 +143,7 @@ def add_mlp(x: torch.Tensor, lw: dict, eps: float) -> torch.Tensor:
 def head_logits(x: torch.Tensor, weights: dict, eps: float) -> torch.Tensor:
     """x [B,1,hidden] -> logits [B, vocab], fp32 holding the head's output in the weights' type"""
     w = weights["lm_head"]
-    if _few_rows(x):
+    if _few_rows(x, w, weights["norm"]):
         from . import _lib, ops
 
         if ops.linear_rows_supported(x.shape[0], x.shape[2], w.shape[0], _lib.LINEAR_FLOAT, True):
@@ -187,13 +193,14 @@ class Decoder:
 
             flush_ahead(self.caches)
         for li, lw in enumerate(self.w["layers"]):
-            slots = self._slots(li, x) if _few_rows(x) else None
+            one = _few_rows(x, lw["wqkv"], lw["input_norm"])
+            slots = self._slots(li, x) if one else None
             if slots is not None:
                 q = qkv_of_token(cfg, x, lw, cos, sin, slots[0], slots[1], 0, 0)
                 self.caches[li].note_device_append()
                 out, _ = self.attention[li].attend(q, self.caches[li], need_weights=False)
             else:
-                if _few_rows(x):
+                if one:
                     k, v = (torch.empty((B, cfg.num_kv_heads, 1, cfg.head_dim), dtype=x.dtype, device=x.device) for _ in range(2))
                     q = qkv_of_token(cfg, x, lw, cos, sin, k, v, 0, 0)
                 else:

@@ -1,0 +1,67 @@
+"""The decoder stack in calls that something records, and on weights in other layouts than init_weights makes them."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def small(dev, window=32, **kw):
+    from kvmix_amd.decoder import DecoderConfig, init_weights, kvmix_layers
+
+    cfg = DecoderConfig(hidden_size=512, num_layers=2, num_heads=4, num_kv_heads=2, intermediate_size=1024, vocab_size=500)
+    weights = init_weights(cfg, dev, std=0.05, seed=9)
+    gen = torch.Generator(device=dev).manual_seed(1)
+    for lw in weights["layers"] + [weights]:
+        for n in [n for n in lw if "norm" in n]:
+            lw[n].uniform_(0.5, 1.5, generator=gen)
+    layers, caches = kvmix_layers(cfg, [4, 3], [2, 4], residual_length=window, capacity=256)
+    ids = torch.randint(0, 500, (3, 60), generator=gen, device=dev)
+    return cfg, weights, layers, caches, ids
+
+
+def decode(dec, ids, prompt=50):
+    out = [dec.forward(ids[:, :prompt])]
+    for t in range(prompt, ids.shape[1]):
+        out.append(dec.forward(ids[:, t:t + 1]))
+    return torch.stack(out)
+
+
+def test_gradients_of_prompt_and_step(dev):
+    """The head's gradient against its formula, and gradients of whatever lies behind the attention, at a prompt and at steps."""
+    from kvmix_amd.decoder import Decoder
+
+    cfg, weights, layers, caches, ids = small(dev)
+    behind = [weights["lm_head"], weights["norm"]] + [weights["layers"][1][n] for n in ("wo", "post_norm", "w_gate_up", "w_down")]
+    for t in behind:
+        t.requires_grad_(True)
+    dec = Decoder(cfg, weights, layers, caches)
+    for a, b in ((0, 50), (50, 51), (51, 52)):
+        logits = dec.forward(ids[:, a:b])
+        assert logits.requires_grad
+        grads = torch.autograd.grad(logits.sum(), behind)
+        assert all(g is not None and bool(torch.isfinite(g).all()) and float(g.abs().max()) > 0 for g in grads)
+        # d(sum of logits) / d(head row) is the normalised row of x, summed over the sequences, for every token of the vocabulary
+        assert torch.equal(grads[0], grads[0][:1].expand_as(grads[0]))
+        want = logits.detach() @ torch.ones(cfg.vocab_size, 1, device=dev)
+        got = (weights["lm_head"].detach().float() @ grads[0][0].float()).sum()
+        assert float((got - want.sum()).abs()) <= 2e-2 * float(logits.detach().abs().sum()) / cfg.vocab_size ** 0.5
+
+
+def test_forward_mode_and_traces_of_the_pieces(dev):
+    from kvmix_amd.decoder import add_mlp, add_projection, head_logits
+
+    cfg, weights, _, _, _ = small(dev)
+    lw, eps = weights["layers"][0], cfg.rms_norm_eps
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x, x2, t = (torch.randn(3, 1, 512, generator=gen, device=dev).half() for _ in range(3))
+    head_t = 0.05 * torch.randn(500, 512, generator=gen, device=dev).half()
+    _, tangent = torch.func.jvp(lambda w: head_logits(x, {**weights, "lm_head": w}, eps), (weights["lm_head"],), (head_t,))
+    want = F.linear(F.rms_norm(x[:, 0], (512,), weights["norm"], eps), head_t).float()
+    assert float((tangent - want).norm()) <= 1e-2 * float(want.norm())
+    _, tangent = torch.func.jvp(lambda h: add_projection(x, h, lw["wo"]), (x2,), (t,))
+    assert float((tangent - F.linear(t, lw["wo"])).norm()) <= 1e-2 * float(tangent.norm())
+    for f in (lambda x: head_logits(x, weights, eps), lambda x: add_projection(x, x, lw["wo"]), lambda x: add_mlp(x, lw, eps)):
+        traced = torch.jit.trace(f, (x,), check_trace=False)
+        want = f(x2).float()
+        assert float((traced(x2).float() - want).norm()) <= 1e-2 * float(want.norm())
