@@ -93,15 +93,21 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return x * cos + rot * sin
 
 
+def _rows_of_pieces(t: torch.Tensor) -> bool:
+    """fp16 rows that 16-byte pieces can be read from: unit stride along the last dimension, every row on such a piece."""
+    return (t.dtype == torch.float16 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+            and (t.dim() < 2 or (t.dim() == 3 and t.shape[0] == 1) or (t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[-1])))
+
+
 def _few_rows(x: torch.Tensor, *operands: torch.Tensor) -> bool:
-    """One new token of a few fp16 sequences on the GPU, in a call that nothing records (gradients, tracing, transforms):
-    the projections then go through the library's kernels, which stream the weights and take the normalisation before and
-    the elementwise work after along (kvmix_linear_rows)."""
+    """One new token of a few fp16 sequences on the GPU, in a call that nothing records (gradients, tracing, transforms),
+    on operands as the kernels read them: the projections then go through the library's kernels, which stream the weights
+    and take the normalisation before and the elementwise work after along (kvmix_linear_rows)."""
     if not (x.is_cuda and x.dtype == torch.float16 and x.shape[1] == 1):
         return False
     from . import ops
 
-    return ops.plain_call(x, *operands)
+    return ops.plain_call(x, *operands) and all(t.device == x.device and _rows_of_pieces(t) for t in (x, *operands))
 
 
 def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tensor, sin: torch.Tensor, k_tail: torch.Tensor,

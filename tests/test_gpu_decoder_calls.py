@@ -65,3 +65,56 @@ def test_forward_mode_and_traces_of_the_pieces(dev):
         traced = torch.jit.trace(f, (x,), check_trace=False)
         want = f(x2).float()
         assert float((traced(x2).float() - want).norm()) <= 1e-2 * float(want.norm())
+
+
+def misaligned(t):
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:] = t.reshape(-1)
+    return buf[1:].view(t.shape)
+
+
+def transposed(t):
+    return t.t().contiguous().t() if t.dim() == 2 else t
+
+
+def spread(t):
+    return torch.stack([t, t], -1)[..., 0]
+
+
+def sliced(t):  # (rows of a wider matrix: the kernels take these)
+    return torch.cat([t, t[..., :64]], -1)[..., :t.shape[-1]]
+
+
+@pytest.mark.parametrize("layout", [misaligned, transposed, spread, sliced])
+@pytest.mark.parametrize("graph", [False, True])
+def test_weights_in_other_layouts(dev, layout, graph):
+    """Every projection in turn, then all, on weights that hold the same values in another layout; the steps may differ by
+    the order of fp32 sums (nothing is quantized within the window, so no rounding can turn a code over)."""
+    from kvmix_amd.decoder import Decoder, GraphDecoder
+
+    cfg, weights, layers, caches, ids = small(dev, window=96)
+    names = ["input_norm", "wqkv", "wo", "post_norm", "w_gate_up", "w_down"]
+    want = None
+    for change in ([], *([n] for n in names), ["lm_head"], ["norm"], names + ["lm_head", "norm"]):
+        w = {k: layout(v) if k in change else v for k, v in weights.items() if k != "layers"}
+        w["layers"] = [{k: layout(v) if k in change else v for k, v in lw.items()} for lw in weights["layers"]]
+        for c in caches:
+            c.reset()
+        got = decode((GraphDecoder if graph else Decoder)(cfg, w, layers, caches), ids)
+        if want is None:
+            want = got
+        assert float((got - want).norm()) <= (9 * cfg.num_layers + 2) * 2.0 ** -11 * float(want.norm()), change
+
+
+def test_other_rows_of_x(dev):
+    """The functions of a step on an x that is a view: every second row, an odd offset, a transposed one."""
+    from kvmix_amd.decoder import add_mlp, add_projection, head_logits
+
+    cfg, weights, _, _, _ = small(dev)
+    lw, eps = weights["layers"][0], cfg.rms_norm_eps
+    x = torch.randn(3, 1, 512, generator=torch.Generator(device=dev).manual_seed(5), device=dev).half()
+    for f in (lambda x: head_logits(x, weights, eps), lambda x: add_projection(x, x, lw["wo"]), lambda x: add_mlp(x, lw, eps)):
+        want = f(x).float()
+        for view in (misaligned(x), spread(x), torch.cat([x, x], 1)[:, 1:], torch.cat([x, x[..., :1]], -1)[..., :512], x[:1].expand(3, 1, 512)):
+            expect = f(view.contiguous()).float()
+            assert float((f(view).float() - expect).norm()) <= 1e-2 * float(want.norm())
