@@ -70,6 +70,7 @@ void check(int rc)
 
 std::string dtype_name(const Tensor &t)
 {
+    const py::gil_scoped_acquire gil;
     return py::str(py::reinterpret_borrow<py::object>((PyObject *)torch::getTHPDtype(t.scalar_type())));
 }
 
@@ -662,17 +663,20 @@ Tensor qkv_rope_append(const Tensor &x_in, const std::vector<Tensor> &ws, int64_
 
 PYBIND11_MODULE(_host, m)
 {
+    // Allocation and launch run without the interpreter's lock: a launch into a full queue waits, and other Python threads
+    // go on meanwhile.
+    using NoGil = py::call_guard<py::gil_scoped_release>;
     m.def("bind", &bind);
-    m.def("quantize_pack_last_dim", &quantize_pack_last_dim);
-    m.def("quantize_pack_dense3", &quantize_pack_dense3);
-    m.def("append_keys", &append_keys);
-    m.def("append_values", &append_values);
-    m.def("copy_rows", &copy_rows);
-    m.def("grow_tuple", &grow_tuple);
-    m.def("quantized_gemm", &quantized_gemm);
-    m.def("prefer_single_pass", &prefer_single_pass);
-    m.def("decode_attention", &decode_attention);
-    m.def("linear_rows", &linear_rows);
-    m.def("swiglu_rows", &swiglu_rows);
-    m.def("qkv_rope_append", &qkv_rope_append);
+    m.def("quantize_pack_last_dim", &quantize_pack_last_dim, NoGil());
+    m.def("quantize_pack_dense3", &quantize_pack_dense3, NoGil());
+    m.def("append_keys", &append_keys, NoGil());
+    m.def("append_values", &append_values, NoGil());
+    m.def("copy_rows", &copy_rows, NoGil());
+    m.def("grow_tuple", &grow_tuple, NoGil());
+    m.def("quantized_gemm", &quantized_gemm, NoGil());
+    m.def("prefer_single_pass", &prefer_single_pass, NoGil());
+    m.def("decode_attention", &decode_attention, NoGil());
+    m.def("linear_rows", &linear_rows, NoGil());
+    m.def("swiglu_rows", &swiglu_rows, NoGil());
+    m.def("qkv_rope_append", &qkv_rope_append, NoGil());
 }
