@@ -286,3 +286,12 @@ class KVmixAttention:
         return attn_output, attn_weights, cache
 
     __call__ = forward
+
+
+_OWN_CALL = KVmixAttention.__call__
+
+
+def is_plain_attention(attention) -> bool:
+    """Whether a call of `attention` is KVmixAttention.forward and nothing else, so that a caller that has put the tokens
+    into the cache itself may go on with attend()."""
+    return type(attention) is KVmixAttention and KVmixAttention.__call__ is _OWN_CALL and KVmixAttention.forward is _OWN_CALL

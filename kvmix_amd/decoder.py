@@ -172,11 +172,11 @@ class Decoder:
     def _slots(self, li: int, x: torch.Tensor):
         """Where layer li's kernels may write the new token's keys and values themselves (an in-place cache that has
         tokens and does not flush for this one), or None."""
-        from .attention import KVmixAttention
+        from .attention import is_plain_attention
         from .cache import PackedKVCache
 
         cache = self.caches[li]
-        if not isinstance(cache, PackedKVCache) or type(self.attention[li]) is not KVmixAttention or cache.kv_seq_len == 0:
+        if not isinstance(cache, PackedKVCache) or not is_plain_attention(self.attention[li]) or cache.kv_seq_len == 0:
             return None
         return cache.next_slots(x.shape[0], self.cfg.num_kv_heads, self.cfg.head_dim)
 

@@ -23,6 +23,7 @@ implementations other than "eager" (the reference asks for eager too).
 """
 from __future__ import annotations
 
+import sys
 from typing import Dict, Optional, Sequence, Union
 
 import torch
@@ -38,7 +39,7 @@ from transformers.models.mistral.modeling_mistral import MistralDecoderLayer as 
 from transformers.models.mistral.modeling_mistral import apply_rotary_pos_emb as mistral_rope
 
 from . import _lib, ops
-from .attention import KVmixAttention
+from .attention import KVmixAttention, is_plain_attention
 from .cache import RESIDUAL_RATIO_BY_BITS, PackedKVCache
 
 QuantBits = Union[Dict[int, dict], Sequence[dict], None]
@@ -204,9 +205,21 @@ class MistralAttention_KVmix(_KVmixAttentionForward, MistralAttention):
     _rope = staticmethod(mistral_rope)
 
 
+def _ways_in(kind) -> tuple:
+    return tuple(getattr(kind, name, None) for name in ("forward", "__call__", "_rope"))
+
+
+# What a call of the classes a step looks through runs, as their own modules define it (a class whose forward was replaced
+# before this one was imported has no entry): programs replace these on the class as well as on an instance.
+_OWN = {kind: _ways_in(kind) for kind in (LlamaAttention_KVmix, MistralAttention_KVmix, LlamaMLP, MistralMLP, LlamaRMSNorm, MistralRMSNorm,
+                                          StockLlamaDecoderLayer, StockMistralDecoderLayer, SiLUActivation, torch.nn.SiLU, torch.nn.Linear)
+        if getattr(getattr(kind.forward, "__code__", None), "co_filename", None) == getattr(sys.modules[kind.__module__], "__file__", "")}
+
+
 def _untouched(module, kind) -> bool:
     """Whether calling `module` does what the class `kind` does and nothing else (hooks, a replaced forward)."""
-    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__)
+    return (type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__)
+            and _ways_in(kind) == _OWN.get(kind))
 
 
 class _KVmixDecoderLayer:
@@ -215,27 +228,28 @@ class _KVmixDecoderLayer:
     sums along: four launches and the attention step instead of about forty.  Everything else is the stock layer: prompts,
     gradients, tracing, autocast, adapters or quantized weights in place of plain fp16 ones, hooks on a module inside."""
 
-    _norm_class = _mlp_class = _kvmix_attention = None
+    _norm_class = _mlp_class = _kvmix_attention = _stock_class = None
 
     def _step_weights(self, x):
         """(q, k, v, o, gate, up, down, input norm, post norm) weights when the layer is the stock one through and
         through, else None."""
-        m = self._modules
-        attn, ffn, norms = m["self_attn"], m["mlp"], (m["input_layernorm"], m["post_attention_layernorm"])
+        attn, ffn, *norms = (self._modules.get(n) for n in ("self_attn", "mlp", "input_layernorm", "post_attention_layernorm"))
         if not (_untouched(attn, self._kvmix_attention) and _untouched(ffn, self._mlp_class)
-                and _untouched(norms[0], self._norm_class) and _untouched(norms[1], self._norm_class)):
+                and _untouched(norms[0], self._norm_class) and _untouched(norms[1], self._norm_class)
+                and _ways_in(self._stock_class) == _OWN.get(self._stock_class)):
             return None
-        a, f = attn._modules, ffn._modules
-        if not (_untouched(f["act_fn"], SiLUActivation) or _untouched(f["act_fn"], torch.nn.SiLU)):
+        act = ffn._modules.get("act_fn")
+        if not (_untouched(act, SiLUActivation) or _untouched(act, torch.nn.SiLU)):
             return None
         weights = []
-        for lin in (a["q_proj"], a["k_proj"], a["v_proj"], a["o_proj"], f["gate_proj"], f["up_proj"], f["down_proj"]):
-            if not _untouched(lin, torch.nn.Linear) or lin._parameters["bias"] is not None:
-                return None
-            weights.append(lin._parameters["weight"])
-        weights += [n._parameters["weight"] for n in norms]
+        for parent, names in ((attn, ("q_proj", "k_proj", "v_proj", "o_proj")), (ffn, ("gate_proj", "up_proj", "down_proj"))):
+            for lin in (parent._modules.get(n) for n in names):
+                if not _untouched(lin, torch.nn.Linear) or lin.bias is not None:
+                    return None
+                weights.append(lin._parameters.get("weight"))
+        weights += [n._parameters.get("weight") for n in norms]
         for w in weights:
-            if w.dtype != torch.float16 or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16:
+            if w is None or w.dtype != torch.float16 or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16:
                 return None
         return weights if ops.plain_call(x, *weights) else None
 
@@ -243,10 +257,12 @@ class _KVmixDecoderLayer:
         """The layer's output for one new token per sequence, or None where the kernels do not take it (nothing has been
         changed then)."""
         weights = self._step_weights(x)
-        if weights is None or type(self._modules["self_attn"].kvmix) is not KVmixAttention:
+        if weights is None or not is_plain_attention(self._modules["self_attn"].kvmix):
             return None
         wq, wk, wv, wo, wg, wu, wd, n1, n2 = weights
         attn, B, hidden = self._modules["self_attn"], x.shape[0], x.shape[2]
+        if past_key_values.get_seq_length(attn.layer_idx) == 0:
+            return None
         D = attn.head_dim
         heads, kv_heads = wq.shape[0] // D, wk.shape[0] // D
         cos, sin = position_embeddings
@@ -278,7 +294,7 @@ class _KVmixDecoderLayer:
         cache, rope = kwargs.get("past_key_values"), kwargs.get("position_embeddings")
         if (not args and hidden_states.dim() == 3 and hidden_states.shape[1] == 1 and hidden_states.is_cuda
                 and hidden_states.dtype == torch.float16 and isinstance(cache, KVmixCache) and rope is not None
-                and cache.get_seq_length(self.self_attn.layer_idx) > 0 and not kwargs.get("output_attentions", False)
+                and not kwargs.get("output_attentions", False)
                 and not torch.is_autocast_enabled("cuda") and not (_module._global_forward_hooks or _module._global_forward_pre_hooks)):
             out = self._step(hidden_states, rope, cache, kwargs.get("attention_mask"))
             if out is not None:
@@ -288,11 +304,11 @@ class _KVmixDecoderLayer:
 
 # (the stock names: they are what device maps know as a unit that is not split)
 class LlamaDecoderLayer(_KVmixDecoderLayer, StockLlamaDecoderLayer):
-    _norm_class, _mlp_class, _kvmix_attention = LlamaRMSNorm, LlamaMLP, LlamaAttention_KVmix
+    _norm_class, _mlp_class, _kvmix_attention, _stock_class = LlamaRMSNorm, LlamaMLP, LlamaAttention_KVmix, StockLlamaDecoderLayer
 
 
 class MistralDecoderLayer(_KVmixDecoderLayer, StockMistralDecoderLayer):
-    _norm_class, _mlp_class, _kvmix_attention = MistralRMSNorm, MistralMLP, MistralAttention_KVmix
+    _norm_class, _mlp_class, _kvmix_attention, _stock_class = MistralRMSNorm, MistralMLP, MistralAttention_KVmix, StockMistralDecoderLayer
 
 
 class _KVmixCausalLM:

@@ -103,3 +103,55 @@ def test_mask_rows_beyond_the_sliding_window_are_the_stock_ones(dev):
         assert model._step_mask(ids[:, :1], None, cache) is None
     close(long[:, :4], full[:, :4], 2)
     assert float((long[:, -1] - full[:, -1]).norm()) > 0.02 * float(full[:, -1].norm())  # (the window does cut)
+
+
+@pytest.mark.parametrize("family", ["llama", "mistral"])
+def test_replacements_on_the_class_are_used(dev, family, monkeypatch):
+    """A forward replaced on the class of a module inside (not on an instance) is what a step runs, as before a prompt does."""
+    from kvmix_amd import hf
+    from kvmix_amd.attention import KVmixAttention
+
+    model = model_of(family, dev)
+    layer = model.model.layers[0]
+    ids = torch.randint(0, 999, (2, 24), device=dev)
+    kinds = [type(layer.mlp), type(layer.input_layernorm), type(layer.mlp.act_fn), torch.nn.Linear, type(layer.self_attn), type(layer).__mro__[2],
+             KVmixAttention]
+    assert kinds[5] in (hf.StockLlamaDecoderLayer, hf.StockMistralDecoderLayer)
+    with torch.no_grad():
+        want, _ = decode(model, ids, 20)
+        for kind in kinds:
+            seen, own = [], kind.__call__ if kind is KVmixAttention else kind.forward
+            with monkeypatch.context() as m:
+                m.setattr(kind, "__call__" if kind is KVmixAttention else "forward", lambda self, *a, **kw: (seen.append(1), own(self, *a, **kw))[1])
+                got, _ = decode(model, ids, 20)
+            assert len(seen) >= 2 * 5, kind  # (each of the two layers, at the prompt and at four steps)
+            close(got, want, 2)
+        assert torch.equal(decode(model, ids, 20)[0], want)
+
+
+def test_modules_of_other_kinds_inside(dev):
+    """A weight that is a plain tensor, an attention wrapped in a module of its own: the stock layer runs."""
+    model = model_of("llama", dev)
+    ids = torch.randint(0, 999, (2, 24), device=dev)
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, *a, **kw):
+            return self.inner(*a, **kw)
+
+    with torch.no_grad():
+        want, _ = decode(model, ids, 20)
+        lin = model.model.layers[0].mlp.up_proj
+        weight = lin.weight.detach().clone()
+        del lin.weight
+        lin.weight = weight
+        norm = model.model.layers[1].post_attention_layernorm
+        weight = norm.weight.detach().clone()
+        del norm.weight
+        norm.weight = weight
+        close(decode(model, ids, 20)[0], want, 2)
+        model.model.layers[1].self_attn = Wrapped(model.model.layers[1].self_attn)
+        close(decode(model, ids, 20)[0], want, 2)
