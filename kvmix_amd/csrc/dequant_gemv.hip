@@ -911,19 +911,25 @@ gemv_cols3(GemvArgs a)
 //   words into weights once and v_mfma_f32_4x4x4 (sixteen blocks of 4 heads x 4 lanes, k = four channel rows) multiplies
 //   them by all four heads: A = x of the block's four heads at four rows, B = the lane's own words at those rows, D = the
 //   lane's own outputs for the four heads, so nothing is exchanged between lanes.
-//   The weight scale * code has up to 14 significant bits and goes in as two fp16 operands, both exact: scale / 128 is
+//   The weight scale * code has up to 14 significant bits and goes in as two fp16 operands, both exact: the scale is
 //   split by its bits into parts of 8 and 3 (each times a 3-bit code fits fp16), and with h = 1024 + code * 2^o -- one
 //   v_and_or of the packed field where it lies, o <= 7 -- a part's product is fma(h, part, -1024 part), rounded nowhere.
-//   Three instructions per two codes instead of nine.  2^(o - 7) is taken out of the fp32 sums at the end.  The zero term
-//   is one more product per word.  That needs scale / 128 to be exact and |scale| <= 8188; four rows of which some lane's
-//   scales are not (keys that differ by less than 0.05 or by more than 57000 inside a group) go through plain fp32.
+//   Three instructions per two codes instead of nine.  2^o is taken out of the fp32 sums at the end.  The zero term
+//   is one more product per word.  All of it stays finite and exact for every |scale| < 64, subnormal ones included; a
+//   row in which some lane's scale is larger (keys that differ by 448 or more inside a group) goes in as scale / 128
+//   against 128 x.  A row that cannot (a scale of 64 next to one below 2^-7 in the same row, |x| from 512 on against such a
+//   row, scales from 8192 on) and everything that is not finite goes through plain fp32, alone of its four rows.
 //   A lane owns two words, a wave 128 (512 bytes of codes per row), 8 rows in flight; ksplit waves share a tile and slice
 //   K where the launch would otherwise have too few of them.
 // Measured: see launch_cols.  Bound now by the 6 vector and 2 matrix instructions per code, word and four rows as they
-// fall between the loads (two waves per SIMD: the fp32 form beside it holds 250 registers).
+// fall between the loads (150 registers, three waves per SIMD).  B = 16, 32 / 8 heads, T = 32637 in graph replay: 74 us on
+// scales of any size below 64, 86 us where all of them are from 64 to 8192, 105-110 us where a row in four goes through
+// fp32 (98 us before, by the form above, on all of these); against float64, sums over 64 to 128 rows end on another than
+// the nearest fp16 in 0.7-1.8 outputs of a thousand (0.9-3.0 before).
 // ---------------------------------------------------------------------------------------
 typedef _Float16 cols3_half2 __attribute__((ext_vector_type(2)));
 typedef _Float16 cols3_half4 __attribute__((ext_vector_type(4)));
+typedef uint16_t cols3_ushort2 __attribute__((ext_vector_type(2)));
 typedef float cols3_float4 __attribute__((ext_vector_type(4)));
 
 // code i of a word: in which of the word's 16-bit windows (bits 0, 8, 16, 24 on) it is taken, and its offset there
@@ -944,8 +950,13 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
     const int K = (int)a.K, nunits = (int)(a.N / VALS);
     if (nunits < TU || K < 32) return;  // (never launched so: a tile wider than the row, fewer rows than the slices' first loads; the same for every thread)
     const uint16_t *xp = reinterpret_cast<const uint16_t *>(a.x) + sample0 * a.x_bs + m * a.x_rs;
-    for (int i = wy * kWave + lane; i < NREP * K; i += blockDim.y * kWave) xh[i] = xp[(i / K) * a.x_bs + i % K];
-    __syncthreads();
+    int infinite = 0;  // some x is not: a second operand of zero would make a NaN of it
+    for (int i = wy * kWave + lane; i < NREP * K; i += blockDim.y * kWave) {
+        const uint16_t v = xp[(i / K) * a.x_bs + i % K];
+        infinite |= (v & 0x7c00) == 0x7c00;
+        xh[i] = v;
+    }
+    infinite = __syncthreads_or(infinite);
 
     const int ks = a.ksplit, slice = wy % ks;
     int t0 = (int)(bx * (blockDim.y / ks) + wy / ks) * TU;
@@ -982,50 +993,69 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
     // rows k .. k + 3, held in registers g .. g + 3
     auto rows4 = [&](int g, int k) {
         const cols3_half4 xa = *reinterpret_cast<const cols3_half4 *>(xh + (lane & 3) * K + k);
-        cols3_half2 sp[UPL][2], small[UPL][2];
-        uint32_t inexact = 0, top = 0;
+        cols3_half4 xw = xa;  // x of the code products
+        cols3_half2 sp[UPL][2];
+        cols3_ushort2 top = {0, 0};  // the largest |scale| of rows k, k + 2 and of rows k + 1, k + 3
 #pragma unroll
         for (int j = 0; j < UPL; j++) {
+            uint32_t z[2];
 #pragma unroll
             for (int p = 0; p < 2; p++) {
                 const uint32_t pair = __builtin_amdgcn_perm(sw[g + 2 * p + 1], sw[g + 2 * p], j ? 0x07060302u : 0x05040100u);
                 sp[j][p] = __builtin_bit_cast(cols3_half2, pair);
-                small[j][p] = sp[j][p] * (_Float16)0.0078125f;
-                inexact |= pair ^ __builtin_bit_cast(uint32_t, small[j][p] * (_Float16)128.0f);
-                const uint32_t size = pair & 0x7fff7fffu;
-                const uint32_t lo = size & 0xffffu, hi = size >> 16;
-                top = top > lo ? top : lo;
-                top = top > hi ? top : hi;
+                top = __builtin_elementwise_max(top, __builtin_bit_cast(cols3_ushort2, pair & 0x7fff7fffu));
+                z[p] = __builtin_amdgcn_perm(zw[g + 2 * p + 1], zw[g + 2 * p], j ? 0x07060302u : 0x05040100u);
             }
+            zacc[j] = __builtin_amdgcn_mfma_f32_4x4x4f16(xa, __builtin_bit_cast(cols3_half4, ((uint64_t)z[1] << 32) | z[0]), zacc[j], 0, 0, 0);
         }
-        if (__builtin_expect(__any(inexact != 0 || top > 0x6fffu), 0)) {  // (0x6fff: 8188)
+        uint32_t alone = infinite ? 15 : 0;  // rows whose code terms go through fp32
+        if (__builtin_expect(__any(top[0] > 0x53ff || top[1] > 0x53ff), 0)) {  // (0x53ff: the last scale below 64; 0x6fff: below 8192)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
+                const int p = r / 2, e = r % 2;
+                const uint32_t s0 = sw[g + r] & 0x7fffu, s1 = sw[g + r] >> 16 & 0x7fffu;
+                if (__any(s0 > 0x53ffu || s1 > 0x53ffu)) {
+                    const _Float16 xr = xa[r] * (_Float16)128.0f;  // (a scalar: a bit cast of a vector's element reads element 0)
+                    bool bad = s0 > 0x6fffu || s1 > 0x6fffu || (__builtin_bit_cast(uint16_t, xr) & 0x7c00) == 0x7c00;
+                    xw[r] = xr;
+#pragma unroll
+                    for (int j = 0; j < UPL; j++) {
+                        const _Float16 full = sp[j][p][e];
+                        sp[j][p][e] = full * (_Float16)0.0078125f;
+                        bad |= __builtin_bit_cast(uint16_t, full) != __builtin_bit_cast(uint16_t, (_Float16)(sp[j][p][e] * (_Float16)128.0f));
+                    }
+                    if (__any(bad)) alone |= 1u << r;
+                }
+            }
+        }
+        if (__builtin_expect(alone != 0, 0)) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (!(alone >> r & 1)) continue;
+                xw[r] = 0;
 #pragma unroll
                 for (int j = 0; j < UPL; j++) {
+                    sp[j][r / 2][r % 2] = 0;
                     const uint32_t w = cw[g + r].v[j];
-                    const float sc = h16_to_f32((uint16_t)(sw[g + r] >> (16 * j))), ze = h16_to_f32((uint16_t)(zw[g + r] >> (16 * j)));
+                    const float sc = h16_to_f32((uint16_t)(sw[g + r] >> (16 * j)));
                     float x[NREP];
 #pragma unroll
-                    for (int h = 0; h < NREP; h++) {
-                        x[h] = h16_to_f32(xh[h * K + k + r]);
-                        zacc[j][h] = fmaf(x[h], ze, zacc[j][h]);
-                    }
+                    for (int h = 0; h < NREP; h++) x[h] = h16_to_f32(xh[h * K + k + r]);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int i = 0; i < VALS; i++) {
-                        const float v = sc * ((float)(w & (7u << (3 * i))) * (0.0078125f / (float)(1 << (8 * cols3_window(i)))));
+                        const float v = sc * ((float)(w & (7u << (3 * i))) * (1.0f / (float)(1 << (8 * cols3_window(i)))));
 #pragma unroll
                         for (int h = 0; h < NREP; h++) acc[j][i][h] = fmaf(x[h], v, acc[j][i][h]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
             }
-            return;
+            if (alone == 15) return;
         }
 #pragma unroll
         for (int j = 0; j < UPL; j++) {
-            uint32_t win[2][4], z[2];
+            uint32_t win[2][4];
             cols3_half2 part[2][2], away[2][2];  // [pair of rows][part of the scale]
 #pragma unroll
             for (int p = 0; p < 2; p++) {
@@ -1034,13 +1064,11 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
                 win[p][1] = __builtin_amdgcn_perm(w1, w0, 0x06050201u);
                 win[p][2] = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
                 win[p][3] = __builtin_amdgcn_perm(w1, w0, 0x0c070c03u);
-                z[p] = __builtin_amdgcn_perm(zw[g + 2 * p + 1], zw[g + 2 * p], j ? 0x07060302u : 0x05040100u);
-                part[p][0] = __builtin_bit_cast(cols3_half2, __builtin_bit_cast(uint32_t, small[j][p]) & 0xfff8fff8u);
-                part[p][1] = small[j][p] - part[p][0];
+                part[p][0] = __builtin_bit_cast(cols3_half2, __builtin_bit_cast(uint32_t, sp[j][p]) & 0xfff8fff8u);
+                part[p][1] = sp[j][p] - part[p][0];
 #pragma unroll
                 for (int q = 0; q < 2; q++) away[p][q] = part[p][q] * (_Float16)-1024.0f;
             }
-            zacc[j] = __builtin_amdgcn_mfma_f32_4x4x4f16(xa, __builtin_bit_cast(cols3_half4, ((uint64_t)z[1] << 32) | z[0]), zacc[j], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < VALS; i++) {
                 const uint32_t mask = (i == 10 ? 0x00030003u : 0x00070007u) << cols3_offset(i);
@@ -1051,7 +1079,7 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
                 for (int q = 0; q < 2; q++) {
                     const cols3_half2 b0 = __builtin_elementwise_fma(h[0], part[0][q], away[0][q]);
                     const cols3_half2 b1 = __builtin_elementwise_fma(h[1], part[1][q], away[1][q]);
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_4x4x4f16(xa, cols3_half4{b0[0], b0[1], b1[0], b1[1]}, acc[j][i], 0, 0, 0);
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_4x4x4f16(xw, cols3_half4{b0[0], b0[1], b1[0], b1[1]}, acc[j][i], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);  // (operands of more codes at once would spill)
             }
@@ -1082,7 +1110,7 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
 #pragma unroll
         for (int j = 0; j < UPL; j++) {
 #pragma unroll
-            for (int i = 0; i < VALS; i++) flat[j * VALS + i] = fmaf(acc[j][i][h], 128.0f / (float)(1 << cols3_offset(i)), zacc[j][h]);
+            for (int i = 0; i < VALS; i++) flat[j * VALS + i] = fmaf(acc[j][i][h], 1.0f / (float)(1 << cols3_offset(i)), zacc[j][h]);
         }
         for (int half = ks / 2; half >= 1; half /= 2) {  // the upper half of the waves hands its sums to the lower one
             if (slice >= half && slice < 2 * half) {
@@ -3598,7 +3626,7 @@ static void launch_cols(GemvArgs &a, int64_t samples, hipStream_t st)
         const bool four_heads = heads_per_block(a.heads_per_kv) == 4 && a.K <= 2048;  // GQA: four query heads per pass
         // over the words (their x rows must fit into LDS).  On the matrix cores where whole tiles of 128 words cover the row
         // with at most a quarter of it done twice, in whole steps of eight rows for up to four slices.  Measured per call,
-        // operands from memory, 32 / 8 heads: B = 16, T = 32637 123 -> 86 us (4.5 TB/s), B = 8, T = 8184 30 -> 24.  Not for
+        // operands from memory, 32 / 8 heads, whatever the scales: B = 16, T = 32637 123 -> 85 us (4.6 TB/s), B = 8, T = 8184 30 -> 24.  Not for
         // 186 words, of which a third would be done twice (B = 64, T = 2046: 36 -> 41).
         if (four_heads && units >= 128 && a.K % 32 == 0 && 4 * ((units + 127) / 128 * 128) <= 5 * units)
             launch_cols3_heads(a, samples, st);
