@@ -14,6 +14,7 @@ namespace kvmix {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 struct LinearArgs {
     const _Float16 *x, *norm;
@@ -39,6 +40,9 @@ struct LinearArgs {
 enum { kEpiPlain = 0, kEpiFloat = 1, kEpiResidual = 2, kEpiSwiglu = 3, kEpiRope = 4 };
 
 constexpr int kLinWaves = 8;
+
+// Chunks per wave that a kernel of CH of them always has to itself: it is chosen only for more than the next smaller one holds.
+__device__ constexpr int lin_full_chunks(int ch) { return ch <= 2 ? 0 : (ch <= 8 ? ch - 2 : ch - 3); }
 
 __device__ __forceinline__ float lin_rounded(float v)
 {
@@ -89,7 +93,7 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
     extern __shared__ float part[];   // [waves][RT * pieces][MC]
     __shared__ float sq[kLinWaves][MC];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, i = lane & 3, b = lane >> 2;
-    const int chunks = a.k / 128;
+    const int chunks = a.k / 128, wave_s = __builtin_amdgcn_readfirstlane(wave);
     const int64_t units = EPI == kEpiSwiglu ? a.rows0 : (EPI == kEpiRope ? (a.rows0 + a.rows1 + a.rows2) / 2 : a.rows0);
     const int64_t q0 = (int64_t)blockIdx.x * a.pieces;
     const int count = (int)(units - q0 < a.pieces ? units - q0 : a.pieces);
@@ -143,7 +147,7 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
     load(1, wv[1]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < CH; j++) {  // (a chunk past the end repeats the last one's weights and meets x = 0)
+    for (int j = 0; j < CH; j++) {  // (a chunk past the end repeats the last one's weights: both sides are made zero)
         if (wave + kLinWaves * j >= chunks) {
 #pragma unroll
             for (int g = 0; g < MG; g++) xv[g][j] = half8{0, 0, 0, 0, 0, 0, 0, 0};
@@ -191,7 +195,12 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
             for (int g = 0; g < MG; g++) acc[g] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < CH; j++) {
-                const half4 lo = {d[r][j][0], d[r][j][1], d[r][j][2], d[r][j][3]}, hi = {d[r][j][4], d[r][j][5], d[r][j][6], d[r][j][7]};
+                half8 ww = d[r][j];
+                if (j >= lin_full_chunks(CH)) {  // (zero times an infinite weight would be NaN)
+                    const uint32_t keep = wave_s + kLinWaves * j < chunks ? 0xffffffffu : 0;
+                    ww = __builtin_bit_cast(half8, __builtin_bit_cast(uint4v, ww) & keep);
+                }
+                const half4 lo = {ww[0], ww[1], ww[2], ww[3]}, hi = {ww[4], ww[5], ww[6], ww[7]};
 #pragma unroll
                 for (int g = 0; g < MG; g++) {
                     const half8 xx = xv[g][j];

@@ -166,3 +166,23 @@ def test_residual_and_fp32_exclude_each_other(dev):
         with pytest.raises(RuntimeError):
             ops.linear_rows(x, w, **kw)
     assert ops.linear_rows(x, w[:0]).shape == (4, 0) and ops.linear_rows(x[:0], w).shape == (0, 24)
+
+
+@pytest.mark.parametrize("m,k", [(1, 128), (4, 1152), (3, 4224), (9, 2688), (2, 11008)])
+def test_what_is_not_finite(dev, m, k):
+    """Infinities and NaN in any chunk of x or w end in the outputs they belong to, as in the plain product: k around waves
+    whose last chunks lie past the end."""
+    from kvmix_amd import ops
+
+    n = 24
+    x, w, nw, _ = operands(dev, m, k, n)
+    inf = float("inf")
+    for at in (0, k // 2, k - 1):
+        xi, wi = x.clone(), w.clone()
+        wi[5, at], wi[6, at], wi[7, at] = inf, -inf, float("nan")
+        xi[0, k - 1 - at] = -inf
+        got, want = ops.linear_rows(xi, wi).double(), xi.double() @ wi.double().t()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        assert torch.equal(torch.sign(got[torch.isinf(want)]), torch.sign(want[torch.isinf(want)]))
+        fine = torch.isfinite(want)
+        assert float((got - want)[fine].norm()) <= ULP * float(want[fine].norm())
