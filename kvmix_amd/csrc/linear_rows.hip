@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
         for (int j = 0; j < CH; j++) {
             const half8 h = *reinterpret_cast<const half8 *>(a.norm + off[j]);
 #pragma unroll
-            for (int e = 0; e < 8; e++) nw[j][e] = (float)h[e];
+            for (int e = 0; e < 8; e++) nw[j][e] = wave_s + kLinWaves * j < chunks ? (float)h[e] : 0.f;
         }
 #pragma unroll
         for (int g = 0; g < MG; g++) {

@@ -186,3 +186,13 @@ def test_what_is_not_finite(dev, m, k):
         assert torch.equal(torch.sign(got[torch.isinf(want)]), torch.sign(want[torch.isinf(want)]))
         fine = torch.isfinite(want)
         assert float((got - want)[fine].norm()) <= ULP * float(want[fine].norm())
+
+
+@pytest.mark.parametrize("m,k", [(4, 1152), (2, 4224)])
+def test_an_infinite_norm_weight(dev, m, k):
+    from kvmix_amd import ops
+
+    x, w, nw, _ = operands(dev, m, k, 8)
+    nw[k - 1] = float("inf")
+    got, want = ops.linear_rows(x, w, nw, 1e-5), F.rms_norm(x, (k,), nw, 1e-5).double() @ w.double().t()
+    assert torch.isinf(want).all() and torch.equal(got.double(), want)
