@@ -249,8 +249,13 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
             }
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int t, int buf) {
         if (vg < kPreK / 4) {
+            if (__builtin_expect((t + 1) * kPreK > a.kv_len, 0)) {  // (the last value again past the end: weight zero times an infinite one is NaN)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (t * kPreK + 4 * vg + i >= a.kv_len) vr[i] = half8{};
+            }
             const int c = 2 * (vg >> 2) + (vg & 1), at = 8 * ((vg >> 1) & 1);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
@@ -272,7 +277,7 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
     int tile = next_tile(), buf = 0;
     if (tile >= 0) {
         load_tile(tile, 0);
-        store_tile(0);
+        store_tile(tile, 0);
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
@@ -361,7 +366,7 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
             }
         }
         buf ^= 1;
-        if (next >= 0) store_tile(buf);
+        if (next >= 0) store_tile(next, buf);
         __builtin_amdgcn_s_waitcnt(0x0f70);  // the key pieces on their way to LDS (vmcnt 0)
         __syncthreads();
         tile = next;

@@ -119,3 +119,16 @@ def test_prompt_branch_takes_it_only_for_plain_calls(dev):
     assert qg.grad is not None and torch.allclose(out_g.float(), out.float(), rtol=2e-3, atol=2e-3)
     tangent = torch.func.jvp(lambda x: layer._prompt_attention(x.float().half(), k, v, mask, 2), (q,), (torch.zeros_like(q),))[0]
     assert torch.allclose(tangent.float(), out.float(), rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("nh,nkv,T,D", [(2, 2, 70, 128), (4, 1, 129, 64), (2, 2, 64, 128)])
+def test_an_infinite_value_at_the_ragged_end(dev, nh, nkv, T, D):
+    """A value of the last token that is infinite stays infinite in the outputs that weigh it, without a mask."""
+    from kvmix_amd import ops
+
+    q, k, v = operands(dev, 1, nh, nkv, T, T, D)
+    v[0, 0, T - 1, 5], v[0, 0, T - 1, 6] = float("inf"), -float("inf")
+    q[...] = k[:, :, T - 1:].repeat_interleave(nh // nkv, 1) * 0.1  # (every query weighs it)
+    got, want = ops.prefill_attention(q, k, v), reference(q, k, v, None)[0]
+    assert torch.isinf(want).any() and not torch.isnan(want).any()
+    assert torch.equal(torch.isinf(got).cpu(), torch.isinf(want)) and not torch.isnan(got).any()
