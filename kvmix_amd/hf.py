@@ -205,21 +205,17 @@ class MistralAttention_KVmix(_KVmixAttentionForward, MistralAttention):
     _rope = staticmethod(mistral_rope)
 
 
-def _ways_in(kind) -> tuple:
-    return tuple(getattr(kind, name, None) for name in ("forward", "__call__", "_rope"))
-
-
-# What a call of the classes a step looks through runs, as their own modules define it (a class whose forward was replaced
-# before this one was imported has no entry): programs replace these on the class as well as on an instance.
-_OWN = {kind: _ways_in(kind) for kind in (LlamaAttention_KVmix, MistralAttention_KVmix, LlamaMLP, MistralMLP, LlamaRMSNorm, MistralRMSNorm,
-                                          StockLlamaDecoderLayer, StockMistralDecoderLayer, SiLUActivation, torch.nn.SiLU, torch.nn.Linear)
-        if getattr(getattr(kind.forward, "__code__", None), "co_filename", None) == getattr(sys.modules[kind.__module__], "__file__", "")}
-
-
 def _untouched(module, kind) -> bool:
-    """Whether calling `module` does what the class `kind` does and nothing else (hooks, a replaced forward)."""
-    return (type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__)
-            and _ways_in(kind) == _OWN.get(kind))
+    """Whether calling `module` does what the class `kind` does and nothing else (hooks, a forward replaced on the instance)."""
+    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__)
+
+
+def _own_ways(*kinds) -> tuple:
+    """(class, forward, __call__) as the classes' own modules define them; programs replace these on the class as well as on
+    an instance.  (Replaced before this module was imported: an entry that no class matches.)"""
+    def own(kind):
+        return getattr(getattr(kind.forward, "__code__", None), "co_filename", None) == getattr(sys.modules[kind.__module__], "__file__", "")
+    return tuple((kind, kind.forward if own(kind) else None, kind.__call__) for kind in kinds)
 
 
 class _KVmixDecoderLayer:
@@ -228,25 +224,30 @@ class _KVmixDecoderLayer:
     sums along: four launches and the attention step instead of about forty.  Everything else is the stock layer: prompts,
     gradients, tracing, autocast, adapters or quantized weights in place of plain fp16 ones, hooks on a module inside."""
 
-    _norm_class = _mlp_class = _kvmix_attention = _stock_class = None
+    _norm_class = _mlp_class = _kvmix_attention = None
+    _own, _own_rope = (), None
 
     def _step_weights(self, x):
         """(q, k, v, o, gate, up, down, input norm, post norm) weights when the layer is the stock one through and
         through, else None."""
-        attn, ffn, *norms = (self._modules.get(n) for n in ("self_attn", "mlp", "input_layernorm", "post_attention_layernorm"))
+        m = self._modules.get
+        attn, ffn, norms = m("self_attn"), m("mlp"), (m("input_layernorm"), m("post_attention_layernorm"))
         if not (_untouched(attn, self._kvmix_attention) and _untouched(ffn, self._mlp_class)
-                and _untouched(norms[0], self._norm_class) and _untouched(norms[1], self._norm_class)
-                and _ways_in(self._stock_class) == _OWN.get(self._stock_class)):
+                and _untouched(norms[0], self._norm_class) and _untouched(norms[1], self._norm_class)):
             return None
-        act = ffn._modules.get("act_fn")
-        if not (_untouched(act, SiLUActivation) or _untouched(act, torch.nn.SiLU)):
+        for kind, forward, call in self._own:
+            if kind.forward is not forward or kind.__call__ is not call:
+                return None
+        if self._kvmix_attention._rope is not self._own_rope:
+            return None
+        a, f = attn._modules.get, ffn._modules.get
+        if not (_untouched(f("act_fn"), SiLUActivation) or _untouched(f("act_fn"), torch.nn.SiLU)):
             return None
         weights = []
-        for parent, names in ((attn, ("q_proj", "k_proj", "v_proj", "o_proj")), (ffn, ("gate_proj", "up_proj", "down_proj"))):
-            for lin in (parent._modules.get(n) for n in names):
-                if not _untouched(lin, torch.nn.Linear) or lin.bias is not None:
-                    return None
-                weights.append(lin._parameters.get("weight"))
+        for lin in (a("q_proj"), a("k_proj"), a("v_proj"), a("o_proj"), f("gate_proj"), f("up_proj"), f("down_proj")):
+            if not _untouched(lin, torch.nn.Linear) or lin._parameters.get("bias", lin) is not None:
+                return None
+            weights.append(lin._parameters.get("weight"))
         weights += [n._parameters.get("weight") for n in norms]
         for w in weights:
             if w is None or w.dtype != torch.float16 or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16:
@@ -304,11 +305,15 @@ class _KVmixDecoderLayer:
 
 # (the stock names: they are what device maps know as a unit that is not split)
 class LlamaDecoderLayer(_KVmixDecoderLayer, StockLlamaDecoderLayer):
-    _norm_class, _mlp_class, _kvmix_attention, _stock_class = LlamaRMSNorm, LlamaMLP, LlamaAttention_KVmix, StockLlamaDecoderLayer
+    _norm_class, _mlp_class, _kvmix_attention = LlamaRMSNorm, LlamaMLP, LlamaAttention_KVmix
+    _own = _own_ways(StockLlamaDecoderLayer, LlamaAttention_KVmix, LlamaMLP, LlamaRMSNorm, torch.nn.Linear, SiLUActivation, torch.nn.SiLU)
+    _own_rope = staticmethod(llama_rope)
 
 
 class MistralDecoderLayer(_KVmixDecoderLayer, StockMistralDecoderLayer):
-    _norm_class, _mlp_class, _kvmix_attention, _stock_class = MistralRMSNorm, MistralMLP, MistralAttention_KVmix, StockMistralDecoderLayer
+    _norm_class, _mlp_class, _kvmix_attention = MistralRMSNorm, MistralMLP, MistralAttention_KVmix
+    _own = _own_ways(StockMistralDecoderLayer, MistralAttention_KVmix, MistralMLP, MistralRMSNorm, torch.nn.Linear, SiLUActivation, torch.nn.SiLU)
+    _own_rope = staticmethod(mistral_rope)
 
 
 class _KVmixCausalLM:
