@@ -199,6 +199,13 @@ struct Copies {
     std::vector<Tensor> keep;
     Tensor first;
 
+    // whether a copy of this tensor is within the 16-byte pieces that one launch counts (whatever its rows join to)
+    static bool fits(const Tensor &t)
+    {
+        const int64_t row = t.dim() == 4 ? t.size(3) : 1;
+        return row == 0 || t.numel() / row * ((row * (int64_t)t.element_size() + 15) / 16) < (1ll << 31) - 4096;
+    }
+
     void add(const Tensor &dst, const Tensor &from)
     {
         if (from.sizes() != dst.sizes() || from.scalar_type() != dst.scalar_type() || from.dim() != 4)
@@ -244,7 +251,7 @@ void copy_previous(const std::vector<std::pair<Tensor, Tensor>> &pairs)
     Copies c;
     for (const auto &p : pairs) {
         const Tensor src = p.second.reshape(p.first.sizes());
-        if (src.scalar_type() == p.first.scalar_type() && src.device() == p.first.device() && plain(src) && p.first.numel() < (1ll << 32))
+        if (src.scalar_type() == p.first.scalar_type() && src.device() == p.first.device() && plain(src) && Copies::fits(p.first))
             c.add(p.first, src);
         else
             p.first.copy_(src);
@@ -315,7 +322,7 @@ std::optional<Grown> grow_tuple(const OptTensor &kc, const Tensor &k_tail, const
                                 int64_t nk, int64_t nv, int64_t k_bits, int64_t k_group, int64_t v_bits)
 {
     auto takes = [&](const Tensor &t, c10::ScalarType type) {
-        return t.scalar_type() == type && t.dim() == 4 && t.is_cuda() && t.device() == key.device() && plain(t);
+        return t.scalar_type() == type && t.dim() == 4 && t.is_cuda() && t.device() == key.device() && plain(t) && Copies::fits(t);
     };
     for (const Tensor *t : {&k_tail, &v_tail, &key, &value})
         if (!takes(*t, at::kHalf)) return std::nullopt;

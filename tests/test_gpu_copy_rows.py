@@ -65,3 +65,19 @@ def test_growing_the_tuple_matches_concatenation(dev, k_bits, v_bits, window, B,
         flushes += past[0] is None and got[0] is not None or (past[0] is not None and got[0].shape != past[0].shape)
         past = got + (length + n,)
     assert flushes >= 2
+
+
+def test_more_pieces_than_one_launch_counts(dev):
+    """A cache of 2^31 rows (expanded ones here, of one group each) is grown by torch's copies as before: a launch counts
+    fewer sixteen-byte pieces than that."""
+    import KVmix
+
+    shape = (1 << 11, 1 << 10, 1 << 10, 1)
+    code = torch.tensor(0x12345678, dtype=torch.int32, device=dev).expand(shape)
+    scale, zero = (torch.tensor(v, dtype=torch.float16, device=dev).expand(shape) for v in (0.5, -2.0))
+    nothing = torch.empty(shape[:3] + (0,), dtype=torch.float16, device=dev)
+    for got, want in zip(KVmix.process_key_quantization_cuda(nothing, code, scale, zero, 32, 4), (0x12345678, 0.5, -2.0)):
+        assert got.shape == shape and got.is_contiguous()
+        assert all(bool((part == want).all()) for part in got.view(64, -1))
+    del got
+    torch.cuda.empty_cache()
