@@ -168,13 +168,15 @@ __device__ __forceinline__ int value_piece(int d, int c)
 // and the exponentials beside them, so everything else is kept off that path.  The logits are computed transposed
 // (32x32x16, keys as rows): a lane then holds 32 logits of ONE query, the softmax needs a single exchange between the two
 // halves of a wave, and the probabilities are already the right-hand operand of out^T = v^T p^T (the order of the keys
-// inside a product is free: the values are stored in LDS in that order).  The mask's entries are where the logits' sums
-// start from, so a masked tile runs the same code.  Keys go from memory straight to LDS, values through registers
+// inside a product is free: the values are stored in LDS in that order).  The mask's entries are added to the finished
+// logits (sums that start from them round at their size at every step: 2.5 times the error under a mask of -10000).  Keys
+// go from memory straight to LDS, values through registers
 // (transposed on the way), both one tile ahead of the products; two blocks share a CU.  Eight waves on 256 queries read
 // keys and values half as often but lose more to the causal border (T = 2048: 409 against 400 us with split probabilities).
-// Measured (us, causal fp32 mask; torch's fused routine after preparing the mask -> this): B = 4, 32 heads, T = 2048 739 ->
-// 315 (without a mask 667 TFLOP/s); B = 1, T = 4096 927 -> 301; B = 4, T = 512 57 -> 43; 32 / 8 heads: B = 4, T = 2048
-// 6012 -> 340, B = 1, T = 1001 442 -> 61, B = 2, T = 333 207 -> 34.
+// Measured (us per call with the mask's classes, causal fp32 mask; torch's fused routine after preparing the mask -> this):
+// B = 4, 32 heads, T = 2048 739 -> 268 (without a mask 770 TFLOP/s); B = 1, T = 4096 927 -> 283; B = 4, T = 512 57 -> 40;
+// 32 / 8 heads: B = 4, T = 2048 6012 -> 326, B = 1, T = 1001 442 -> 54.  A mask that is mixed in every tile (a bias per
+// distance below the diagonal), B = 2, 32 heads, T = 2048: 283 (504 before).
 template <int D, bool SPLIT>
 __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_attn(PrefillArgs a)
 {
@@ -208,7 +210,6 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
             if (off) qv[ks] = half8{};
         }
     }
-    const int64_t mask_row = b * a.m_bs + head * a.m_hs + (int64_t)row * a.m_rs;
 
     // the key tiles that some query of the block needs, in order
     int window = -kWave;
@@ -289,29 +290,8 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
         const int next = next_tile();
         if (next >= 0) load_tile(next, buf ^ 1);  // (that buffer was last read before the barrier that ended the iteration before)
         if (mine != kTileSkip) {
-            // logits, transposed: a lane has keys 8 (i / 4) + 4 h2 + i % 4 of two times 32 for its one query; the sums
-            // start from the mask's entries (divided by the scale that follows)
+            // logits, transposed: a lane has keys 8 (i / 4) + 4 h2 + i % 4 of two times 32 for its one query
             floatx16 s[2] = {floatx16{}, floatx16{}};
-            if (mine == kTileBinary && k0 + kPreK <= a.kv_len) {
-                const uint32_t word[2] = {(uint32_t)masked, (uint32_t)(masked >> 32)};
-#pragma unroll
-                for (int i = 0; i < 32; i++) {
-                    const int bit = 16 * (i % 4) + 8 * (i / 16) + 2 * (i % 16 / 4);
-                    s[i / 16][i % 16] = word[bit / 32] >> (bit % 32) & 1 ? kHalfLowest * unscale : 0.0f;
-                }
-            } else if (mine != kTilePlain || k0 + kPreK > a.kv_len) {
-#pragma unroll
-                for (int i = 0; i < 32; i++) {
-                    const int key = k0 + 32 * (i / 16) + 8 * (i % 16 / 4) + 4 * h2 + i % 4;
-                    float bias = 0.0f;
-                    if (mine != kTilePlain) {
-                        const int64_t at = mask_row + (key < a.kv_len ? key : 0);
-                        bias = prefill_mask_value(a.mask_f32 ? ((const float *)a.mask)[at] : (float)((const _Float16 *)a.mask)[at]) * unscale;
-                    }
-                    s[i / 16][i % 16] = key < a.kv_len ? bias : -__builtin_inff();
-                    if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // (eight loads in flight: more would spill)
-                }
-            }
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) {
 #pragma unroll
@@ -320,6 +300,37 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
                     s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk, qv[ks], s[t], 0, 0, 0);
                 }
                 if (ks % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (all reads of a tile ahead of its products would spill)
+            }
+            // the mask's entries, divided by the scale that follows, are added to the finished sums: one rounding at their size
+            if (mine == kTileBinary && k0 + kPreK <= a.kv_len) {
+                const uint32_t word[2] = {(uint32_t)masked, (uint32_t)(masked >> 32)};
+#pragma unroll
+                for (int i = 0; i < 32; i++) {
+                    const int bit = 16 * (i % 4) + 8 * (i / 16) + 2 * (i % 16 / 4);
+                    s[i / 16][i % 16] += word[bit / 32] >> (bit % 32) & 1 ? kHalfLowest * unscale : 0.0f;
+                }
+            } else if (mine != kTilePlain) {
+                int r = query;  // (what follows from it is not kept across the tiles)
+                asm volatile("" : "+v"(r));
+                const int64_t mask_row = b * a.m_bs + head * a.m_hs + (int64_t)(r < a.q_len ? r : a.q_len - 1) * a.m_rs;
+                auto add_mask = [&](const auto *entries) {
+#pragma unroll
+                    for (int g = 0; g < 8; g++) {
+                        float v[4];
+                        mask_four(entries + mask_row, k0 + 32 * (g / 4) + 8 * (g % 4) + 4 * h2, a.kv_len, 0.0f, v);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) s[g / 4][4 * (g % 4) + j] += prefill_mask_value(v[j]) * unscale;
+                        __builtin_amdgcn_sched_barrier(0);  // (a load at a time: more would spill, and took longer)
+                    }
+                };
+                if (a.mask_f32) add_mask((const float *)a.mask);
+                else add_mask((const _Float16 *)a.mask);
+            }
+            if (k0 + kPreK > a.kv_len) {
+#pragma unroll
+                for (int i = 0; i < 32; i++) {
+                    if (k0 + 32 * (i / 16) + 8 * (i % 16 / 4) + 4 * h2 + i % 4 >= a.kv_len) s[i / 16][i % 16] = -__builtin_inff();
+                }
             }
             float top = s[0][0];
 #pragma unroll

@@ -132,3 +132,17 @@ def test_an_infinite_value_at_the_ragged_end(dev, nh, nkv, T, D):
     got, want = ops.prefill_attention(q, k, v), reference(q, k, v, None)[0]
     assert torch.isinf(want).any() and not torch.isnan(want).any()
     assert torch.equal(torch.isinf(got).cpu(), torch.isinf(want)) and not torch.isnan(got).any()
+
+
+@pytest.mark.parametrize("nh,nkv", [(8, 8), (8, 2)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_large_entries_of_a_mask_round_once(dev, nh, nkv, dtype):
+    """A mask of -10000 on everything: the sum of logit and entry is rounded at the size of 10000 sqrt(128), 2^-7 in the last
+    place, which is 2.0e-4 (rms) of the logit; with the roundings of probabilities and outputs (2.0 to 2.4e-4) 3.2e-4."""
+    from kvmix_amd import ops
+
+    q, k, v = operands(dev, 1, nh, nkv, 700, 700, 128)
+    mask = torch.full((1, 1, 700, 700), -10000.0, dtype=dtype, device=dev)
+    want = reference(q, k, v, mask)[0]
+    got = ops.prefill_attention(q, k, v, mask).double().cpu()
+    assert float((got - want).norm()) <= 4.5e-4 * float(want.norm())
