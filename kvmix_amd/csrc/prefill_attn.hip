@@ -16,6 +16,7 @@
 namespace kvmix {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2 __attribute__((ext_vector_type(2)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -164,19 +165,21 @@ __device__ __forceinline__ int value_piece(int d, int c)
     return d * 128 + ((c ^ ((d >> 1) & 7)) << 4);
 }
 
-// One block: 128 queries of one head, 32 to a wave, over the key tiles that some of them needs.  Bound by the matrix cores
-// and the exponentials beside them, so everything else is kept off that path.  The logits are computed transposed
+// One block: 128 queries of one head, 32 to a wave, over the key tiles that some of them needs.  Bound by the matrix
+// cores and the exponentials beside them, so everything else is kept off that path.  The logits are computed transposed
 // (32x32x16, keys as rows): a lane then holds 32 logits of ONE query, the softmax needs a single exchange between the two
 // halves of a wave, and the probabilities are already the right-hand operand of out^T = v^T p^T (the order of the keys
 // inside a product is free: the values are stored in LDS in that order).  The mask's entries are added to the finished
 // logits (sums that start from them round at their size at every step: 2.5 times the error under a mask of -10000).  Keys
-// go from memory straight to LDS, values through registers
-// (transposed on the way), both one tile ahead of the products; two blocks share a CU.  Eight waves on 256 queries read
-// keys and values half as often but lose more to the causal border (T = 2048: 409 against 400 us with split probabilities).
-// Measured (us per call with the mask's classes, causal fp32 mask; torch's fused routine after preparing the mask -> this):
-// B = 4, 32 heads, T = 2048 739 -> 268 (without a mask 770 TFLOP/s); B = 1, T = 4096 927 -> 283; B = 4, T = 512 57 -> 40;
-// 32 / 8 heads: B = 4, T = 2048 6012 -> 326, B = 1, T = 1001 442 -> 54.  A mask that is mixed in every tile (a bias per
-// distance below the diagonal), B = 2, 32 heads, T = 2048: 283 (504 before).
+// go from memory straight to LDS, values through registers (transposed on the way), both one tile ahead of the products;
+// two blocks share a CU.  Eight waves on 256 queries read keys and values half as often but lose more to the causal
+// border (T = 2048: 409 against 400 us with split probabilities).  Measured (us per call with the mask's classes, causal
+// fp32 mask; torch's fused routine after preparing the mask -> this): B = 4, 32 heads, T = 2048 739 -> 293 (without a
+// mask 720 TFLOP/s); B = 1, T = 4096 927 -> 285; B = 4, T = 512 57 -> 42; 32 / 8 heads: B = 4, T = 2048 6012 -> 326, B =
+// 1, T = 1001 442 -> 54.  A mask that is mixed in every tile (a bias per distance below the diagonal), B = 2, 32 heads, T
+// = 2048: 273 (504 from sums that start there).  Error against float64 relative to the norm, keys with an outlier
+// channel, causal, T = 300 / 1500 / 2048: 2.35 / 2.37 / 2.41e-4, the routine before 2.36 / 2.39 / 2.42e-4; with the
+// maximum moved from 2^8 on only 2.45 / 2.58 / 2.68e-4 (268 us).
 template <int D, bool SPLIT>
 __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_attn(PrefillArgs a)
 {
@@ -342,9 +345,10 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
                 const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
                 top = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * c;
             }
-            // the maximum is only moved when it has grown by more than 2^8: below that the probabilities stay well
-            // inside fp16's range, and rescaling the 64 sums of a lane costs a quarter of a tile's products
-            if (__any(top > m + 8.0f)) {
+            // With probabilities in two parts the maximum is only moved when it has grown by more than 2^8: below that they
+            // stay well inside fp16's range, and rescaling the 64 sums of a lane costs a quarter of a tile's products.  In
+            // one part the largest has to be exactly one, or its rounding is the largest error of the row.
+            if (__any(top > (SPLIT ? m + 8.0f : m))) {
                 const float grown = fmaxf(m, top);
                 const float shrink = __builtin_amdgcn_exp2f(m - grown);
                 m = grown;
@@ -357,10 +361,14 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     const float p = __builtin_amdgcn_exp2f(fmaf(s[kk / 2][8 * (kk % 2) + i], c, -m));
-                    sum += p;
                     const _Float16 hi = (_Float16)p;
                     ph[kk % 2][i] = hi;
-                    if constexpr (SPLIT) pl[kk % 2][i] = (_Float16)(p - (float)hi);
+                    if constexpr (SPLIT) {
+                        sum += p;
+                        pl[kk % 2][i] = (_Float16)(p - (float)hi);
+                    } else if (i % 2) {  // the sum of what the products weigh with: a common part of the roundings drops out
+                        sum = __builtin_amdgcn_fdot2(half2{ph[kk % 2][i - 1], hi}, half2{(_Float16)1.0f, (_Float16)1.0f}, sum, false);
+                    }
                 }
             };
             probs(0);
@@ -506,7 +514,7 @@ extern "C" int kvmix_prefill_attention(const kvmix_prefill_attn_t *p, void *work
     const dim3 grid((unsigned)blocks), block(kPreWaves * kWave);
     // What the routines that served these calls before held the probabilities in: with one query head per kv head fp16,
     // with grouped heads fp32, here two fp16 parts (their sum is within 2^-22).  The second part costs half as many
-    // products again: B = 4, 32 / 32 heads, T = 2048, causal 315 us without, 398 with it.
+    // products again: B = 4, 32 / 32 heads, T = 2048, causal 293 us without, 328 with it.
     const bool split = a.heads_per_kv > 1;
     if (p->head_dim == 128) split ? prefill_attn<128, true><<<grid, block, 0, st>>>(a) : prefill_attn<128, false><<<grid, block, 0, st>>>(a);
     else split ? prefill_attn<64, true><<<grid, block, 0, st>>>(a) : prefill_attn<64, false><<<grid, block, 0, st>>>(a);

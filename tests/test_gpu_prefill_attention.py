@@ -134,6 +134,27 @@ def test_an_infinite_value_at_the_ragged_end(dev, nh, nkv, T, D):
     assert torch.equal(torch.isinf(got).cpu(), torch.isinf(want)) and not torch.isnan(got).any()
 
 
+@pytest.mark.parametrize("nh,nkv", [(2, 2), (4, 1)])
+def test_a_dominant_key_has_a_weight_of_one(dev, nh, nkv):
+    """Rows that one late key dominates by less than a factor of 2^8: its probability is not rounded and the sum is that of
+    the weights the products see, so that nearly all outputs are the correctly rounded ones (a rounding of that probability
+    to eleven bits would move every third)."""
+    from kvmix_amd import ops
+
+    T, D = 256, 128
+    gen = torch.Generator(device="cpu").manual_seed(3)
+    q, k, v = torch.zeros(1, nh, T, D), torch.zeros(1, nkv, T, D), torch.randn(1, nkv, T, D, generator=gen)
+    q[..., 0] = 16.0
+    q[..., 1] = 16.0 * torch.rand(1, nh, T, generator=gen)
+    k[..., 0] = -60.0
+    k[:, :, 5, 0] = 0.0                              # logit 0 in the first tile
+    k[:, :, 200, 0], k[:, :, 200, 1] = 0.5, 3.3      # up to 5.3 above it in the fourth
+    v[:, :, 5] *= 2.0 ** -9
+    q, k, v = (t.half().to(dev) for t in (q, k, v))
+    got, want = ops.prefill_attention(q, k, v), reference(q, k, v, None)[0]
+    assert float((got.cpu() == want.half()).float().mean()) > 0.9
+
+
 @pytest.mark.parametrize("nh,nkv", [(8, 8), (8, 2)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_large_entries_of_a_mask_round_once(dev, nh, nkv, dtype):
