@@ -94,9 +94,12 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
 
 
 def _rows_of_pieces(t: torch.Tensor) -> bool:
-    """fp16 rows that 16-byte pieces can be read from: unit stride along the last dimension, every row on such a piece."""
-    return (t.dtype == torch.float16 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-            and (t.dim() < 2 or (t.dim() == 3 and t.shape[0] == 1) or (t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[-1])))
+    """fp16 rows that 16-byte pieces can be read from: unit stride along the last dimension, every row on such a piece
+    (rows that follow one another are, at the lengths the kernels take)."""
+    if t.dtype != torch.float16 or t.data_ptr() % 16:
+        return False
+    return t.is_contiguous() or (t.stride(-1) == 1 and (t.dim() < 2 or (t.dim() == 3 and t.shape[0] == 1)
+                                                        or (t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[-1])))
 
 
 def _few_rows(x: torch.Tensor, *operands: torch.Tensor) -> bool:
@@ -107,18 +110,24 @@ def _few_rows(x: torch.Tensor, *operands: torch.Tensor) -> bool:
         return False
     from . import ops
 
-    return ops.plain_call(x, *operands) and all(t.device == x.device and _rows_of_pieces(t) for t in (x, *operands))
+    if not (_rows_of_pieces(x) and ops.plain_call(x, *operands)):
+        return False
+    for t in operands:
+        if t.device != x.device or not _rows_of_pieces(t):
+            return False
+    return True
 
 
 def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tensor, sin: torch.Tensor, k_tail: torch.Tensor,
-                 v_tail: torch.Tensor, k_slot, v_slot) -> torch.Tensor:
+                 v_tail: torch.Tensor, k_slot, v_slot, few_rows: Optional[bool] = None) -> torch.Tensor:
     """One new token: norm, q/k/v projections, RoPE; keys and values to the given slots of the tail windows, the
-    rotated queries [B,nh,1,D] returned."""
+    rotated queries [B,nh,1,D] returned.  few_rows: what _few_rows says of the operands, where the caller has asked."""
     from . import _lib, ops
 
     h, kvh = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
-    if _few_rows(x, lw["wqkv"], lw["input_norm"]) and ops.linear_rows_supported(x.shape[0], x.shape[2], h, _lib.LINEAR_ROPE_APPEND, True,
-                                                                                cfg.head_dim, kvh):
+    if few_rows is None:
+        few_rows = _few_rows(x, lw["wqkv"], lw["input_norm"])
+    if few_rows and ops.linear_rows_supported(x.shape[0], x.shape[2], h, _lib.LINEAR_ROPE_APPEND, True, cfg.head_dim, kvh):
         return ops.qkv_rope_append(x, lw["wqkv"], cfg.num_heads, cfg.num_kv_heads, cos, sin, k_tail, v_tail, k_slot, v_slot,
                                    lw["input_norm"], cfg.rms_norm_eps)
     qkv = F.linear(rms_norm(x, lw["input_norm"], cfg.rms_norm_eps), lw["wqkv"])
@@ -202,13 +211,13 @@ class Decoder:
             one = _few_rows(x, lw["wqkv"], lw["input_norm"])
             slots = self._slots(li, x) if one else None
             if slots is not None:
-                q = qkv_of_token(cfg, x, lw, cos, sin, slots[0], slots[1], 0, 0)
+                q = qkv_of_token(cfg, x, lw, cos, sin, slots[0], slots[1], 0, 0, one)
                 self.caches[li].note_device_append()
                 out, _ = self.attention[li].attend(q, self.caches[li], need_weights=False)
             else:
                 if one:
                     k, v = (torch.empty((B, cfg.num_kv_heads, 1, cfg.head_dim), dtype=x.dtype, device=x.device) for _ in range(2))
-                    q = qkv_of_token(cfg, x, lw, cos, sin, k, v, 0, 0)
+                    q = qkv_of_token(cfg, x, lw, cos, sin, k, v, 0, 0, one)
                 else:
                     h = rms_norm(x, lw["input_norm"], cfg.rms_norm_eps)
                     q, k, v = project_qkv(cfg, h, lw["wqkv"], cos, sin)
