@@ -554,12 +554,13 @@ Tensor linear_operands(kvmix_linear_rows_t &st, const Tensor &x_in, const std::v
     st.x_stride = x.size(0) > 1 ? x.stride(0) : x.size(1);
     st.epilogue = epilogue;
     if (ws.empty() || ws.size() > 3) fail("a projection has one to three weights");
+    auto row_stride = [](const Tensor &w) { return w.size(0) > 1 ? w.stride(0) : w.size(1); };  // (of one row: whatever the view left)
     for (const Tensor &w : ws) {
         need_with(x, {&w});
-        if (w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(1) || w.stride(1) != 1 || w.stride(0) != ws[0].stride(0))
+        if (w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(1) || w.stride(1) != 1 || row_stride(w) != row_stride(ws[0]))
             fail("weights must be fp16 [rows, k] with unit-stride rows and one row stride");
     }
-    st.w_stride = ws[0].stride(0);
+    st.w_stride = row_stride(ws[0]);
     if (ws.size() == 1) {
         int64_t sum = 0;
         for (int64_t n : split) sum += n;

@@ -196,3 +196,12 @@ def test_an_infinite_norm_weight(dev, m, k):
     nw[k - 1] = float("inf")
     got, want = ops.linear_rows(x, w, nw, 1e-5), F.rms_norm(x, (k,), nw, 1e-5).double() @ w.double().t()
     assert torch.isinf(want).all() and torch.equal(got.double(), want)
+
+
+def test_a_weight_of_one_row_with_any_stride(dev):
+    from kvmix_amd import ops
+
+    x, w, _, _ = operands(dev, 3, 256, 2)
+    wide = torch.cat([w, w[:, :3]], 1)[:1, :256]  # (contiguous as torch counts, a stride of 259)
+    assert wide.is_contiguous() and wide.stride(0) == 259
+    assert torch.equal(ops.linear_rows(x, wide), ops.linear_rows(x, w[:1]))
