@@ -252,3 +252,27 @@ def test_single_pass_policy_knows_the_matrix_core_steps():
     from kvmix_amd import _lib
     plan = _lib.attn_plan(_lib.attn_step_descriptor(16, 32, 32, 128, 3, 0, 11, 8063, 4, 0, 32, 8064, 129, 128))
     assert plan["matrix"] and not plan["recommended"]
+
+
+def test_native_policy_fills_the_descriptor_the_plan_query_reads():
+    """ops.prefer_single_pass fills its own kvmix_decode_attn_t (csrc/host.cpp); over layouts, sizes and quantized lengths it is
+    answered as the plan query answers the descriptor of _lib.attn_step_descriptor."""
+    import itertools
+
+    from kvmix_amd import _lib, ops
+
+    seen = set()
+    keys, values = [(1, 0, 32), (2, 0, 32), (3, 0, 11), (3, 1, 32), (4, 0, 32)], [(1, 0, 32), (2, 0, 32), (3, 1, 32), (4, 0, 32)]
+    for (kb, kf, kg), (vb, vf, vg), (B, nh, nkv), T in itertools.product(keys, values, ((1, 32, 32), (4, 32, 8), (16, 32, 32), (64, 12, 12)),
+                                                                         (200, 2304, 8192)):
+        for kt, vt in ((0, 0), ((T - 128) // kg * kg, (T - 128) // vg * vg), ((T - 64) // kg * kg, (T - 160) // vg * vg)):
+            got = ops.prefer_single_pass(B, nh, nkv, 128, T, kb, kf, kg, vb, vf, vg, k_tokens=kt, v_tokens=vt)
+            want = False
+            if ops.single_pass_supported(128, nh // nkv, kb, kf, kg, vb, vf, vg):
+                try:
+                    want = _lib.attn_plan(_lib.attn_step_descriptor(B, nh, nkv, 128, kb, kf, kg, kt, vb, vf, vg, vt, T - kt, T - vt))["recommended"]
+                except RuntimeError:
+                    pass
+            assert got == want, (kb, kf, vb, vf, B, nh, nkv, T, kt, vt)
+            seen.add(got)
+    assert seen == {True, False}
