@@ -118,16 +118,22 @@ def _few_rows(x: torch.Tensor, *operands: torch.Tensor) -> bool:
     return True
 
 
+def _qkv_supported(cfg: DecoderConfig, x: torch.Tensor) -> bool:
+    from . import _lib, ops
+
+    return ops.linear_rows_supported(x.shape[0], x.shape[2], cfg.num_heads * cfg.head_dim, _lib.LINEAR_ROPE_APPEND, True, cfg.head_dim,
+                                     cfg.num_kv_heads * cfg.head_dim)
+
+
 def qkv_of_token(cfg: DecoderConfig, x: torch.Tensor, lw: dict, cos: torch.Tensor, sin: torch.Tensor, k_tail: torch.Tensor,
                  v_tail: torch.Tensor, k_slot, v_slot, few_rows: Optional[bool] = None) -> torch.Tensor:
     """One new token: norm, q/k/v projections, RoPE; keys and values to the given slots of the tail windows, the
     rotated queries [B,nh,1,D] returned.  few_rows: what _few_rows says of the operands, where the caller has asked."""
-    from . import _lib, ops
+    from . import ops
 
-    h, kvh = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
     if few_rows is None:
         few_rows = _few_rows(x, lw["wqkv"], lw["input_norm"])
-    if few_rows and ops.linear_rows_supported(x.shape[0], x.shape[2], h, _lib.LINEAR_ROPE_APPEND, True, cfg.head_dim, kvh):
+    if few_rows and _qkv_supported(cfg, x):
         return ops.qkv_rope_append(x, lw["wqkv"], cfg.num_heads, cfg.num_kv_heads, cos, sin, k_tail, v_tail, k_slot, v_slot,
                                    lw["input_norm"], cfg.rms_norm_eps)
     qkv = F.linear(rms_norm(x, lw["input_norm"], cfg.rms_norm_eps), lw["wqkv"])
@@ -208,7 +214,8 @@ class Decoder:
 
             flush_ahead(self.caches)
         for li, lw in enumerate(self.w["layers"]):
-            one = _few_rows(x, lw["wqkv"], lw["input_norm"])
+            # (rope_append, which serves what kvmix_linear_rows does not take, works on sixteenths of a head)
+            one = _few_rows(x, lw["wqkv"], lw["input_norm"]) and (cfg.head_dim % 16 == 0 or _qkv_supported(cfg, x))
             slots = self._slots(li, x) if one else None
             if slots is not None:
                 q = qkv_of_token(cfg, x, lw, cos, sin, slots[0], slots[1], 0, 0, one)

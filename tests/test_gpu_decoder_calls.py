@@ -118,3 +118,30 @@ def test_other_rows_of_x(dev):
         for view in (misaligned(x), spread(x), torch.cat([x, x], 1)[:, 1:], torch.cat([x, x[..., :1]], -1)[..., :512], x[:1].expand(3, 1, 512)):
             expect = f(view.contiguous()).float()
             assert float((f(view).float() - expect).norm()) <= 1e-2 * float(want.norm())
+
+
+class Dense:
+    """Plain attention over whole keys and values: no limit on head dimensions."""
+
+    def __call__(self, q, k, v, cache, attention_mask=None, need_weights=False):
+        if cache is not None:
+            k, v = torch.cat([cache[0], k], 2), torch.cat([cache[1], v], 2)
+        rep = q.shape[1] // k.shape[1]
+        kk, vv = k.float().repeat_interleave(rep, 1), v.float().repeat_interleave(rep, 1)
+        logits = torch.matmul(q.float(), kk.transpose(2, 3).contiguous()) / q.shape[3] ** 0.5
+        p = torch.softmax(logits if attention_mask is None else logits + attention_mask, -1)
+        return torch.matmul(p, vv).to(q.dtype), None, (k, v)
+
+
+# head dimensions that the projection kernel, rope_append or neither takes
+@pytest.mark.parametrize("hidden,heads,kv_heads", [(320, 8, 4), (128, 16, 8), (240, 5, 5), (512, 4, 2), (360, 15, 3)])
+def test_steps_with_other_head_dimensions(dev, hidden, heads, kv_heads):
+    """Token by token as the prompt of all tokens, on any sizes that torch's products take."""
+    from kvmix_amd.decoder import Decoder, DecoderConfig, init_weights
+
+    cfg = DecoderConfig(hidden_size=hidden, num_layers=2, num_heads=heads, num_kv_heads=kv_heads, intermediate_size=384, vocab_size=100)
+    weights = init_weights(cfg, dev, std=0.05, seed=2)
+    ids = torch.randint(0, 100, (2, 12), generator=torch.Generator().manual_seed(1)).to(dev)
+    got = decode(Decoder(cfg, weights, [Dense(), Dense()]), ids, 6)
+    want = torch.stack([Decoder(cfg, weights, [Dense(), Dense()]).forward(ids[:, :t]) for t in range(6, 13)])
+    assert float((got - want).norm()) <= (9 * cfg.num_layers + 2) * 2.0 ** -11 * float(want.norm())
