@@ -125,12 +125,6 @@ class PrefillAttn(ctypes.Structure):
         ("kv_heads", _i64), ("q_len", _i64), ("kv_len", _i64), ("head_dim", _i64), ("scale", ctypes.c_float)]
 
 
-class CopyRows(ctypes.Structure):
-    """kvmix_copy_rows_t"""
-    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p)] + [(f, ctypes.c_int64) for f in (
-        "outer", "inner", "row_bytes", "src_outer_stride", "src_inner_stride", "dst_outer_stride", "dst_inner_stride")]
-
-
 LINEAR_PLAIN, LINEAR_FLOAT, LINEAR_RESIDUAL, LINEAR_SWIGLU, LINEAR_ROPE_APPEND = range(5)
 
 
@@ -212,7 +206,7 @@ def load() -> ctypes.CDLL:
     L.kvmix_prefill_attention.restype = i32
     L.kvmix_prefill_attention.argtypes = [ctypes.POINTER(PrefillAttn), vp, i64, vp]
     L.kvmix_copy_rows.restype = i32
-    L.kvmix_copy_rows.argtypes = [ctypes.POINTER(CopyRows), i32, vp]
+    L.kvmix_copy_rows.argtypes = [vp, i32, vp]
     L.kvmix_probe_stream_read.restype = i32
     L.kvmix_probe_stream_read.argtypes = [vp, i32, i64, i64, i32, i32, i32, i32, i32, vp, vp]
     _lib = L
