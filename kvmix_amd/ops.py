@@ -356,15 +356,15 @@ def qkv_rope_append(x: torch.Tensor, w, heads: int, kv_heads: int, cos: torch.Te
 
 def plain_call(*tensors) -> bool:
     """Whether a call on these tensors is an ordinary one, which a kernel without an autograd formula may serve: no
-    gradient (backward or forward mode) is being recorded, nothing is traced, compiled, transformed or dispatched to a
-    tensor subclass or mode."""
+    gradient (backward or forward mode) is being recorded, nothing is traced, compiled, transformed, cast (autocast) or
+    dispatched to a tensor subclass or mode."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
     if any(type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter for t in tensors):
         return False
     return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
                 or torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0)
+                or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"))
 
 
 def _aligned_heads(t: torch.Tensor) -> torch.Tensor:

@@ -145,3 +145,24 @@ def test_steps_with_other_head_dimensions(dev, hidden, heads, kv_heads):
     got = decode(Decoder(cfg, weights, [Dense(), Dense()]), ids, 6)
     want = torch.stack([Decoder(cfg, weights, [Dense(), Dense()]).forward(ids[:, :t]) for t in range(6, 13)])
     assert float((got - want).norm()) <= (9 * cfg.num_layers + 2) * 2.0 ** -11 * float(want.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_autocast_is_torchs(dev, dtype):
+    """Under autocast the projections and the prompt's attention are torch's, in the type it casts them to."""
+    from kvmix_amd.attention import KVmixAttention
+    from kvmix_amd.decoder import add_projection, head_logits
+
+    cfg, weights, _, _, _ = small(dev)
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x = torch.randn(3, 1, 512, generator=gen, device=dev).half()
+    q, k, v = (torch.randn(1, 4, 70, 128, generator=gen, device=dev).half() for _ in range(3))
+    mask = torch.full((70, 70), torch.finfo(torch.float32).min, device=dev).triu_(1)[None, None]
+    with torch.autocast("cuda", dtype=dtype):
+        y, want = add_projection(x, x, weights["layers"][0]["wo"]), x + F.linear(x, weights["layers"][0]["wo"])
+        assert y.dtype == want.dtype and torch.equal(y, want)
+        logits = head_logits(x, weights, cfg.rms_norm_eps)
+        assert torch.equal(logits, F.linear(F.rms_norm(x[:, 0], (512,), weights["norm"], cfg.rms_norm_eps), weights["lm_head"]).float())
+        out, _, _ = KVmixAttention(4, 4, residual_length=32)(q, k, v, None, attention_mask=mask, need_weights=False)
+        want = F.scaled_dot_product_attention(q, k, v, attn_mask=mask.clamp(min=-65504.0).half())
+        assert out.dtype == want.dtype and torch.equal(out, want)
