@@ -43,6 +43,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 
 // Switches kept for measurement: with the hint compiled out the HBM counters show the bytes a kernel reads without it.
 #ifndef KVMIX_STREAM_NT
@@ -1380,7 +1381,9 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 // NREP query heads of one kv head reuse the B registers.
 // x*scale is formed once per (row, group) by the lane that loaded that scale (as in
 // gemv_rows) and parked, already split, in the wave's LDS tile in A-operand order.
-// block = (64, KW); grid = (splits, samples/NREP, M); dynamic LDS = KW * NM A tiles,
+// CS blocks may share the columns of a row, 128/CS each (rows_pieces): 16/CS lanes then cover a row's piece and one load
+// instruction reads 4*CS rows.
+// block = (64, KW); grid = (splits * CS, samples/NREP, M); dynamic LDS = KW * NM A tiles,
 // NM = ceil(3*NREP/4).
 // ---------------------------------------------------------------------------------------
 typedef short bf16x4_t __attribute__((ext_vector_type(4)));
@@ -1523,7 +1526,7 @@ constexpr int kRowsMfmaTile = (32 * 17 + 1) * 4 + 4;  // bf16 elements of one A 
 
 constexpr int kRowsMfmaWaves = 16;  // waves per block at most (register budget of 128 per lane)
 
-template <int BITS, int NREP, int DEPTH>
+template <int BITS, int NREP, int DEPTH, int CS>
 __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWaves))
     __attribute__((amdgpu_waves_per_eu(NREP > 1 ? kMfmaHeadsOcc : 4))) gemv_rows_mfma(GemvArgs a)
 {
@@ -1531,12 +1534,14 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     using Elem = typename CodeElem<BITS>::type;
     constexpr int EB = BITS == 30 ? 3 : BITS;   // bytes of a lane's 8 codes
     constexpr int FB = BITS == 30 ? 3 : BITS;   // bits of a code
-    constexpr int LPR = 4;             // groups per row (N = 128)
-    constexpr int EPR = 16;            // lanes (8-code elements) per row
+    constexpr int NC = 128 / CS;       // columns of a block (N = 128)
+    constexpr int LPR = 4 / CS;        // groups per row piece
+    constexpr int EPR = 16 / CS;       // lanes (8-code elements) per row piece
     constexpr int RL = kWave / EPR;    // rows per load instruction (4)
     constexpr int RKB = 4 * RL;        // rows per k-block (16)
-    constexpr int CH = 128;            // rows per chunk: 512 scales = one 128-bit load per lane
+    constexpr int CH = 128;            // rows per chunk: with whole rows 512 scales = one 128-bit load per lane
     constexpr int KB = CH / RKB;       // k-blocks per chunk (8)
+    constexpr bool WHOLE = CS == 1;    // (pieces of rows share their cache lines with other blocks: no streaming hint)
     constexpr int AT = kRowsMfmaTile;  // bf16 elements of one A tile
     constexpr int NP = rows_mfma_parts(NREP); // bf16 parts of x*scale
     constexpr int NM = rows_mfma_sets(NREP);  // MFMAs per B operand
@@ -1548,11 +1553,13 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     const int wy = threadIdx.y;
     const int KW = blockDim.y;
     uint16_t *atile = reinterpret_cast<uint16_t *>(lds) + wy * (NM * AT);
-    float *red = lds;  // [KW][NREP][128], reuses the A tiles after the streaming loop
+    float *red = lds;  // [KW][NREP][NC], reuses the A tiles after the streaming loop
     const int rs = lane / EPR;
     const int wi = lane % EPR;
     int64_t split, hg;
-    xcd_swizzled_block(split, hg, a.heads_per_kv > NREP);
+    xcd_swizzled_block(split, hg, a.heads_per_kv > NREP || CS > 1);
+    const int piece = CS > 1 ? (int)(split % CS) : 0;  // (neighbours on one XCD: its L2 holds the lines they share)
+    split /= CS;
     const int64_t sample0 = hg * NREP;
     const int64_t m = blockIdx.z;
     const int64_t kv = sample0 / a.heads_per_kv;
@@ -1563,11 +1570,11 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     // dense 3-bit: a group is three aligned words; lane j of the group's four loads word
     // min(j, 2), and its 24 bits [24j, 24j+24) are cut out of two neighbours' words in compute()
     // (a dword load at byte 3j instead -- no exchange between lanes -- was measured slower: 33 against 28 us)
-    const uint8_t *cp = reinterpret_cast<const uint8_t *>(a.code + kv * a.c_bs) +
+    const uint8_t *cp = reinterpret_cast<const uint8_t *>(a.code + kv * a.c_bs) + piece * (EPR * EB) +
                         (BITS == 30 ? (wi / 4) * 12 + (wi % 4 < 2 ? wi % 4 : 2) * 4 : wi * EB);
     [[maybe_unused]] const uint32_t sh3 = (uint32_t)(24 * (wi % 4)) % 32u;
-    const uint16_t *sp = reinterpret_cast<const uint16_t *>(a.scale) + kv * a.s_bs;
-    const uint16_t *zp = reinterpret_cast<const uint16_t *>(a.zero) + kv * a.s_bs;
+    const uint16_t *sp = reinterpret_cast<const uint16_t *>(a.scale) + kv * a.s_bs + piece * LPR;
+    const uint16_t *zp = reinterpret_cast<const uint16_t *>(a.zero) + kv * a.s_bs + piece * LPR;
 
     f32x4_t acc[NM][NPOS];
     float zacc[NREP][LPR];
@@ -1581,15 +1588,15 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
 #pragma unroll
         for (int g = 0; g < LPR; g++) zacc[h][g] = 0.f;
     }
-    // staging: this lane owns elements [8*lane, 8*lane+8) of the chunk's [128][4] scale array,
-    // i.e. rows 2*lane and 2*lane+1, all four groups.  Row r of a chunk is k-slot (r%16)/4 of
-    // A-lanes  (r%4)*16 + 4*g + i  in k-block r/16.
+    // staging: this lane owns rows 2*lane and 2*lane+1 of the chunk, all groups of the piece (whole rows: elements
+    // [8*lane, 8*lane+8) of the chunk's [128][4] scale array).  Row r of a chunk is k-slot (r%RKB)/RL of
+    // A-lanes  (r%RL)*EPR + 4*g + i  in k-block r/RKB.
     // A tile: one 8-byte cell (4 k-slots) per (k-block t, lane); the 16 cells of the lanes with
     // the same (t, lane/16) form a row of 17 cells' pitch, and the rows of k-blocks 4..7 are
     // shifted by one more cell.  With that skew the 2-byte staging stores of a wave (same
     // cell column, 32 different rows) fall into 32 different LDS banks, and a wave's 8-byte
     // operand reads stay conflict-free.
-    auto cell = [](int t, int l) { return ((4 * t + l / EPR) * 17 + (l % EPR)) * 4 + (t >> 2) * 4; };
+    auto cell = [](int t, int l) { return ((4 * t + l / 16) * 17 + (l % 16)) * 4 + (t >> 2) * 4; };
     const int row0 = 2 * lane;
     int aoff[2];  // bf16 index of (row0 + e, g = 0, i = 0)
 #pragma unroll
@@ -1612,36 +1619,55 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
         uint16_t v[2];
     };
     // DEPTH chunks are in flight per wave: register set d holds chunk c with c % DEPTH == d
-    Half8 s8[DEPTH], z8[DEPTH];
+    struct __attribute__((packed, aligned(2))) HalfRow {
+        uint16_t v[LPR];
+    };
+    struct HalfRows {
+        HalfRow row[2];
+    };
+    using Scales = std::conditional_t<WHOLE, Half8, HalfRows>;
+    static_assert(sizeof(Scales) == 4 * LPR, "two rows of scales");
+    Scales s8[DEPTH], z8[DEPTH];
     Half2x xh[DEPTH][NREP];
     Elem w[DEPTH][KB][4];
 
     auto chunk_base = [&](int k0) { return k0 + CH <= ke32 ? k0 : max(ke32 - CH, 0); };
     auto load_small = [&](int d, int k0) {
         const uint32_t kr = (uint32_t)(chunk_base(k0) + row0);
-        s8[d] = ld_stream<Half8>(sp + kr * LPR);
-        z8[d] = ld_stream<Half8>(zp + kr * LPR);
+        if constexpr (WHOLE) {
+            s8[d] = ld_stream<Half8>(sp + kr * LPR);
+            z8[d] = ld_stream<Half8>(zp + kr * LPR);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                s8[d].row[q] = ld_stream<HalfRow, false>(sp + (kr + q) * 4);
+                z8[d].row[q] = ld_stream<HalfRow, false>(zp + (kr + q) * 4);
+            }
+        }
 #pragma unroll
         for (int h = 0; h < NREP; h++) xh[d][h] = *reinterpret_cast<const Half2x *>(xp + h * a.x_bs + kr);
     };
     auto load_codes = [&](int d, int k0, int t) {
-        const uint8_t *base = cp + (uint32_t)(chunk_base(k0) + rs) * (EPR * EB);
+        const uint8_t *base = cp + (uint32_t)(chunk_base(k0) + rs) * (16 * EB);
 #pragma unroll
         for (int k = 0; k < 4; k++)
-            w[d][t][k] = ld_stream<Elem>(base + (t * RKB + RL * k) * (EPR * EB));
+            w[d][t][k] = ld_stream<Elem, WHOLE>(base + (t * RKB + RL * k) * (16 * EB));
     };
     auto stage = [&](int d, int k0) {
         const int skip = k0 - chunk_base(k0);  // rows of this chunk that an earlier one covered
+        uint16_t sv[2 * LPR], zv[2 * LPR];
+        __builtin_memcpy(sv, &s8[d], sizeof(sv));
+        __builtin_memcpy(zv, &z8[d], sizeof(zv));
 #pragma unroll
         for (int h = 0; h < NREP; h++) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
+            for (int e = 0; e < 2 * LPR; e++) {
                 const int q = e / LPR, g = e % LPR;
                 const float xv = row0 + q >= skip ? h16_to_f32(xh[d][h].v[q]) : 0.f;
-                zacc[h][g] = fmaf(xv, h16_to_f32(z8[d].v[e]), zacc[h][g]);
+                zacc[h][g] = fmaf(xv, h16_to_f32(zv[e]), zacc[h][g]);
                 // x * scale * 2^90, split into bf16 parts by truncation (three parts: exact)
                 uint32_t part[NP];
-                split_bf16_parts<NP>((xv * 1237940039285380274899124224.0f) * h16_to_f32(s8[d].v[e]), part);
+                split_bf16_parts<NP>((xv * 1237940039285380274899124224.0f) * h16_to_f32(sv[e]), part);
 #pragma unroll
                 for (int pt = 0; pt < NP; pt++) {  // A row NP*h+pt: MFMA (NP*h+pt)/4, lanes 4g + (NP*h+pt)%4
                     const int ar = NP * h + pt;
@@ -1764,15 +1790,15 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
         float z[LPR];
 #pragma unroll
         for (int g = 0; g < LPR; g++) z[g] = zacc[h][g];
-        scatter_reduce<LPR, 8, 0>(z, lane);  // lane bits 3, 2 = group of the lane's codes
+        scatter_reduce<LPR, 2 * LPR, 0>(z, lane);  // lane bits below EPR, above the quad: group of the lane's codes
         z[0] += __shfl_xor(z[0], 1);
         z[0] += __shfl_xor(z[0], 2);
-        z[0] += __shfl_xor(z[0], 16);
-        z[0] += __shfl_xor(z[0], 32);
+#pragma unroll
+        for (int o = EPR; o < kWave; o *= 2) z[0] += __shfl_xor(z[0], o);
         zterm[h] = z[0];
     }
     // code sums: the three parts meet; the 2^-133 of the bf16 patterns, the 2^90 and the
-    // field's bit offset are undone; then the 4 row slots (lane bits 4, 5) are summed
+    // field's bit offset are undone; then the row slots (lane bits from EPR on) are summed
     constexpr int NV = NREP * NPOS;
     float flat[NV];
 #pragma unroll
@@ -1793,8 +1819,12 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
         }
     }
     __syncthreads();  // every wave is done with its A tile: the space becomes `red`
-    constexpr int KEEP = NV / 4;
-    const int first = scatter_reduce<NV, 16, 1>(flat, lane);
+    constexpr int KEEP = NV >= RL ? NV / RL : 1;
+    const int first = scatter_reduce<NV, EPR, 1>(flat, lane);
+    if constexpr (NV < RL) {  // (one step more than there are values to halve: both partners keep the sum)
+        static_assert(2 * NV == RL, "one step");
+        flat[0] += __shfl_xor(flat[0], kWave / 2);
+    }
 #pragma unroll
     for (int i = 0; i < KEEP; i++) {
         const int f = first + i;
@@ -1802,17 +1832,17 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
         float zt = zterm[0];
 #pragma unroll
         for (int hh = 1; hh < NREP; hh++) zt = h == hh ? zterm[hh] : zt;
-        red[(wy * NREP + h) * 128 + wi * NPOS + f % NPOS] = flat[i] + zt;
+        red[(wy * NREP + h) * NC + wi * NPOS + f % NPOS] = flat[i] + zt;
     }
     __syncthreads();
-    for (int t = wy * kWave + lane; t < NREP * 128; t += KW * kWave) {
-        const int h = t / 128, n = t % 128;
+    for (int t = wy * kWave + lane; t < NREP * NC; t += KW * kWave) {
+        const int h = t / NC, n = t % NC;
         float v = 0.f;
-        for (int ww = 0; ww < KW; ww++) v += red[(ww * NREP + h) * 128 + n];
+        for (int ww = 0; ww < KW; ww++) v += red[(ww * NREP + h) * NC + n];
         if (a.splits == 1)
-            a.out[(sample0 + h) * a.o_bs + m * a.o_rs + n] = __float2half_rn(v);
+            a.out[(sample0 + h) * a.o_bs + m * a.o_rs + piece * NC + n] = __float2half_rn(v);
         else
-            a.partial[(((sample0 + h) * a.M + m) * a.splits + split) * a.N + n] = v;
+            a.partial[(((sample0 + h) * a.M + m) * a.splits + split) * a.N + piece * NC + n] = v;
     }
 }
 
@@ -3274,6 +3304,42 @@ static int rows_max_waves(bool mfma, int nrep)
     return nrep > 1 ? kRowsHeadsWaves : (mfma ? kRowsMfmaWaves : kRowsMaxWaves);
 }
 
+// gemv_rows_mfma: blocks that share the columns of an output row, each with 128 / rows_pieces of them.  Launches of few
+// blocks leave CUs idle while the sixteen waves of a block queue for the four SIMDs of theirs: pieces of rows put two or
+// four times as many CUs to work without a reduction behind them, as long as that stays one block per CU (from there on
+// the shorter pieces only cost: B = 8, 32 heads, T = 2048, 2 bits 8.9 us whole, 10.8 in halves).  Measured per call,
+// operands from memory, whole rows -> pieces, us: B = 1, 32 heads, T = 3968, 4 bits 11.9 -> 10.3 (quarters; halves 10.9),
+// 1 bit 9.9 -> 7.3; T = 32640, 2 bits (four blocks along K already) 21.7 -> 20.3 (halves; quarters 27.2); B = 4, T = 2048,
+// 4 bits 10.7 -> 9.4 (halves; quarters 13.8); four query heads of 8 kv heads, B = 1, T = 1024 9.9 -> 7.0.
+static int rows_pieces(int64_t blocks)
+{
+    int cs = 1;
+    while (cs < 4 && 2 * cs * blocks <= 256) cs *= 2;
+    return cs;
+}
+
+template <int MODE, int NREP, int CS>
+static void launch_rows_mfma(const GemvArgs &a, int64_t samples, int waves, hipStream_t st)
+{
+    constexpr int DEPTH = 1;  // chunks in flight per wave (deeper costs occupancy and was slower)
+    const dim3 grid((unsigned)(a.splits * CS), (unsigned)(samples / NREP), (unsigned)a.M), block(kWave, waves);
+    // one A tile per wave and MFMA set; the block reduction (waves*NREP*128 floats) reuses it
+    const size_t lds = (size_t)waves * rows_mfma_sets(NREP) * kRowsMfmaTile * sizeof(uint16_t);
+    if (lds > 64 * 1024 && !t_plan) {
+        // above the default per-block limit: raise it for this kernel, once per device
+        // (the attribute is idempotent: two threads that both find the flag clear set it twice)
+        static std::atomic<bool> raised[kMaxDevices];
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices ||
+            !raised[dev].load(std::memory_order_acquire)) {
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rows_mfma<MODE, NREP, DEPTH, CS>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+            if (dev >= 0 && dev < kMaxDevices) raised[dev].store(true, std::memory_order_release);
+        }
+    }
+    KVMIX_LAUNCH((gemv_rows_mfma<MODE, NREP, DEPTH, CS>), grid, block, lds, st, a, "gemv_rows_mfma<%d,%d,%d>", MODE, NREP, DEPTH);
+}
+
 template <int MODE, int NREP>
 static void launch_rows_n(GemvArgs &a, int64_t samples, hipStream_t st)
 {
@@ -3285,22 +3351,10 @@ static void launch_rows_n(GemvArgs &a, int64_t samples, hipStream_t st)
     const dim3 grid((unsigned)a.splits, (unsigned)(samples / NREP), (unsigned)a.M), block(kWave, p.waves);
     if (mfma) {
         if (!tile_fits(a.K, 128)) return;  // (a chunk past the end is moved back to end at K)
-        // one A tile per wave and MFMA set; the block reduction (waves*NREP*128 floats) reuses it
-        const size_t lds = (size_t)p.waves * rows_mfma_sets(NREP) * kRowsMfmaTile * sizeof(uint16_t);
-        constexpr int DEPTH = 1;  // chunks in flight per wave (deeper costs occupancy and was slower)
-        if (lds > 64 * 1024 && !t_plan) {
-            // above the default per-block limit: raise it for this kernel, once per device
-            // (the attribute is idempotent: two threads that both find the flag clear set it twice)
-            static std::atomic<bool> raised[kMaxDevices];
-            int dev = 0;
-            if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices ||
-                !raised[dev].load(std::memory_order_acquire)) {
-                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rows_mfma<MODE, NREP, DEPTH>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-                if (dev >= 0 && dev < kMaxDevices) raised[dev].store(true, std::memory_order_release);
-            }
-        }
-        KVMIX_LAUNCH((gemv_rows_mfma<MODE, NREP, DEPTH>), grid, block, lds, st, a, "gemv_rows_mfma<%d,%d,%d>", MODE, NREP, DEPTH);
+        const int cs = rows_pieces(samples / NREP * a.M * a.splits);
+        if (cs == 4) launch_rows_mfma<MODE, NREP, 4>(a, samples, p.waves, st);
+        else if (cs == 2) launch_rows_mfma<MODE, NREP, 2>(a, samples, p.waves, st);
+        else launch_rows_mfma<MODE, NREP, 1>(a, samples, p.waves, st);
         if (a.splits > 1) {
             const dim3 g2((unsigned)((a.N + 255) / 256), (unsigned)samples, (unsigned)a.M);
             KVMIX_LAUNCH(reduce_splits, g2, dim3(256), 0, st, a, "reduce_splits");
