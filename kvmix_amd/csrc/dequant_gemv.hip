@@ -1370,12 +1370,28 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 //   B   <-> codes: v_perm_b32 puts byte b of two rows' elements into the low bytes of the two
 //           halves of a register and one v_and_b32 isolates a field of both.  An 8-bit
 //           pattern p in the low byte of a bf16 IS the number p * 2^-133 (subnormals and the
-//           first binade share one ulp), so the masked register is a bf16 pair with no
-//           shift and no conversion; a field at bit offset o simply counts 2^o-fold.
-//   A   <-> x*scale*2^90 split into three bf16 (8 significant bits each: the product of two
+//           first binade share one ulp; in an fp16 it is p * 2^-24), so the masked register is a bf16 pair
+//           with no shift and no conversion; a field at bit offset o simply counts 2^o-fold.
+//   A   <-> one head: x*scale*2^90 split into three bf16 (8 significant bits each: the product of two
 //           fp16 has at most 22, so the split is exact).  2^90 keeps every product far above
-//           the fp32 subnormals and below overflow for any fp16 x and scale.  The 3*NREP
-//           (head, part) rows are packed four to an MFMA; unused rows are zero.
+//           the fp32 subnormals and below overflow for any fp16 x and scale.
+//           Four heads: x*scale in two fp16 parts, each one packed multiplication of two rows -- hi = x*scale
+//           rounded, lo = fma(x, scale, -hi), together exact as long as lo does not reach below fp16's smallest step.
+//           For that x and scale are first multiplied by powers of two, one per head and one per group, that put
+//           x below 2^7 and scale below 2^8: a product is then off by at most 2^-25 where the largest of its
+//           (head, group) may be 2^15.  They start where probabilities and ordinary scales need them (x < 2,
+//           scale < 8: an error of 2^-36 per product) and are lowered, with the sums so far, when a chunk holds
+//           something larger.  Against the three bf16 parts (12 rows, three MFMAs per B operand) this is 8
+//           rows, two MFMAs, a third of the LDS stores and a fifth of the arithmetic of forming them.
+//           The (part, head) rows are packed four to an MFMA; unused rows are zero.
+//           Measured, four query heads per kv head, operands from memory, bf16 -> fp16 parts (and blocks of
+//           eight waves instead of four), us: B = 16, 8 kv heads, T = 32640, 2 bits 72.8 -> 57; T = 8064, 4 bits
+//           27.8 -> 25; B = 4, T = 32640, 1 bit 25.5 -> 22.3; B = 8, T = 8064, dense 3-bit 18.7 -> 17.1.  Outputs
+//           that are not the fp16 nearest to the exact sum, of 1000, bf16 -> fp16 parts: T = 1000 / 16000 / 32000,
+//           2 bits 5.5 / 4.7 / 4.9 -> 3.3 / 3.9 / 4.3; T = 4000 / 16000, 4 bits 4.0 / 4.5 -> 3.4 / 4.1.  One
+//           head stays on bf16: there the three rows share one MFMA, and the narrower loads and the one more
+//           shift per byte cost more (B = 16, 32 heads, T = 8064, 2 bits 38.2 -> 39.9; B = 64, T = 3968, 1 bit 56.5
+//           -> 64.0).  Bound by the vector ALU (400 instructions per 128 rows) beside the MFMAs.
 //   D   <-> lane l accumulates, for each of its 8 code positions p, partial sums of output
 //           column 8*(l%16)+p over its rows, one per A row; the parts are added at the end.
 // NREP query heads of one kv head reuse the B registers.
@@ -1469,6 +1485,16 @@ __device__ __forceinline__ uint32_t field_operand_top(uint32_t t, int f)
     const uint32_t mask = ((1u << (BITS * (f + 1))) - 1u) * 0x00010001u;
     return sh > 0 ? (t << sh) & (mask << sh) : t & mask;
 }
+// Field f alone, UP bits further up: the operand for x * scale in fp16 parts, of eleven bits where a bf16 part has eight.
+// With the fields 0..f together their products have up to nineteen bits and the matrix cores drop the lowest where they
+// align four of them (2-bit p.V, T = 16000: 8.1 of 1000 outputs were not the fp16 nearest to the exact sum, 4.7 with
+// bf16 parts); alone they have thirteen and nothing is dropped (3.9).
+template <int BITS, int UP>
+__device__ __forceinline__ uint32_t field_alone_top(uint32_t t, int f)
+{
+    const int sh = UP + field_shift<BITS>(f);
+    return (t << sh) & ((((1u << BITS) - 1u) << (BITS * f + sh)) * 0x00010001u);
+}
 // sum of field f alone, counting 2^(BITS * f + field_shift(f))-fold
 template <int BITS>
 __device__ __forceinline__ float field_sum_top(float cur, float prev, int f)
@@ -1484,25 +1510,18 @@ __device__ __forceinline__ constexpr int field_offset_top(int f)
     return BITS * f + field_shift<BITS>(f);
 }
 
-// bf16 parts x*scale*2^90 is split into: three (24 significant bits hold the product of two fp16 exactly).  One
-// query head: its three rows fit one MFMA.  Four heads per pass: twelve rows, three MFMAs per B operand.
-// KVMIX_HEADS_PARTS = 2 (measurement only; p.V kernel) rounds the second part to nearest instead -- every product off
-// by up to 2^-17 of itself, eight rows, two MFMAs per B operand, a third of the staging gone: 2-bit p.V at B = 16,
-// 32 / 8 heads, T = 32768 70 -> 55 us.  Not shipped: where the code term and the zero term of an output nearly cancel
-// (a peaked probability row on a value near zero) that error took a 4-bit case at K = 128 from 0.65 to 1.4 times the
-// GEMV tolerance (tests/test_gpu_gemv.py holds the case).
+// parts of x*scale.  p.V with one query head and q.K^T: three bf16 (24 significant bits hold the product of two fp16
+// exactly).  p.V with four heads per pass: two fp16.  (Two bf16 parts, the second rounded to nearest, leave every product
+// off by up to 2^-17 of itself: where the code term and the zero term of an output nearly cancel that took a 4-bit case
+// at K = 128 from 0.65 to 1.4 times the GEMV tolerance; tests/test_gpu_gemv.py holds the case.)
 // (What the matrix cores keep of a sum of such products, and what the p.V kernels do about it: field_operand_top.)
-#ifndef KVMIX_HEADS_PARTS
-#define KVMIX_HEADS_PARTS 3
-#endif
-constexpr int rows_mfma_parts(int nrep) { return nrep > 1 ? KVMIX_HEADS_PARTS : 3; }   // p.V
+constexpr int rows_mfma_parts(int nrep) { return nrep > 1 ? 2 : 3; }                    // p.V: fp16 / bf16
 constexpr int cols_mfma_parts(int) { return 3; }                                        // q.K^T
 constexpr int mfma_sets(int parts, int nrep) { return (parts * nrep + 3) / 4; }
 constexpr int rows_mfma_sets(int nrep) { return mfma_sets(rows_mfma_parts(nrep), nrep); }
 constexpr int cols_mfma_sets(int nrep) { return mfma_sets(cols_mfma_parts(nrep), nrep); }
 // v (= x*scale*2^90) as NP bf16, part i in the high half of part[i]: all but the last by truncation (the
-// remainders are exact); the last holds what is left exactly when NP = 3 and is rounded to nearest otherwise
-// (a carry into the exponent is the next power of two, as it should be; v is far from overflow)
+// remainders are exact); the last holds what is left exactly when NP = 3
 template <int NP>
 __device__ __forceinline__ void split_bf16_parts(float v, uint32_t *part)
 {
@@ -1511,7 +1530,8 @@ __device__ __forceinline__ void split_bf16_parts(float v, uint32_t *part)
         part[i] = __float_as_uint(v) & 0xffff0000u;
         v -= __uint_as_float(part[i]);
     }
-    part[NP - 1] = NP >= 3 ? __float_as_uint(v) : __float_as_uint(v) + 0x8000u;
+    static_assert(NP == 3, "the last part is exact");
+    part[NP - 1] = __float_as_uint(v);
 }
 // the sum over the parts' accumulators of head h at code position p
 template <int NP, int NM, int NPOS>
@@ -1522,12 +1542,20 @@ __device__ __forceinline__ float parts_sum(const f32x4_t (&acc)[NM][NPOS], int h
     for (int i = 1; i < NP; i++) s += acc[(NP * h + i) / 4][p][(NP * h + i) % 4];
     return s;
 }
+// 2^n in both halves, -14 <= n <= 15
+__device__ __forceinline__ half2_t half_power(int n)
+{
+    return __builtin_bit_cast(half2_t, (uint32_t)((n + 15) << 10) * 0x00010001u);
+}
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef uint16_t ushort2_t __attribute__((ext_vector_type(2)));
 constexpr int kRowsMfmaTile = (32 * 17 + 1) * 4 + 4;  // bf16 elements of one A tile (32 skewed rows), 8-byte multiple
 
-constexpr int kRowsMfmaWaves = 16;  // waves per block at most (register budget of 128 per lane)
+constexpr int kRowsMfmaWaves = 16;      // waves per block at most (register budget of 128 per lane)
+constexpr int kRowsMfmaHeadsWaves = 8;  // ... four heads per pass (256)
 
 template <int BITS, int NREP, int DEPTH, int CS>
-__global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWaves))
+__global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMfmaWaves))
     __attribute__((amdgpu_waves_per_eu(NREP > 1 ? kMfmaHeadsOcc : 4))) gemv_rows_mfma(GemvArgs a)
 {
     // BITS = 30: dense 3-bit stream, a lane's 8 codes are 3 bytes
@@ -1541,9 +1569,11 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     constexpr int RKB = 4 * RL;        // rows per k-block (16)
     constexpr int CH = 128;            // rows per chunk: with whole rows 512 scales = one 128-bit load per lane
     constexpr int KB = CH / RKB;       // k-blocks per chunk (8)
+    constexpr bool HALVES = NREP > 1;  // x*scale in two fp16 parts instead of three bf16 parts
+    constexpr int NP = rows_mfma_parts(NREP);
+    constexpr int TOP = HALVES ? 3 : 0;  // bits the codes' patterns are moved up by in a half's eleven
     constexpr bool WHOLE = CS == 1;    // (pieces of rows share their cache lines with other blocks: no streaming hint)
     constexpr int AT = kRowsMfmaTile;  // bf16 elements of one A tile
-    constexpr int NP = rows_mfma_parts(NREP); // bf16 parts of x*scale
     constexpr int NM = rows_mfma_sets(NREP);  // MFMAs per B operand
     constexpr int NPOS = 8;            // code positions per lane
     constexpr int FPB = 8 / FB;        // whole fields per byte window
@@ -1576,6 +1606,14 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     const uint16_t *sp = reinterpret_cast<const uint16_t *>(a.scale) + kv * a.s_bs + piece * LPR;
     const uint16_t *zp = reinterpret_cast<const uint16_t *>(a.zero) + kv * a.s_bs + piece * LPR;
 
+    // powers of two that x and scale are multiplied by, and the largest values (two halves each) they are good for
+    int x_pow[NREP], s_pow[LPR];
+    uint32_t x_limit[NREP], s_limit[LPR];
+#pragma unroll
+    for (int h = 0; h < NREP; h++) x_pow[h] = 6, x_limit[h] = ((16 << 10) - 1) * 0x00010001u;  // |x| < 2: probabilities
+#pragma unroll
+    for (int g = 0; g < LPR; g++) s_pow[g] = 5, s_limit[g] = ((18 << 10) - 1) * 0x00010001u;  // |scale| < 8
+    const int own_group = wi / 4;
     f32x4_t acc[NM][NPOS];
     float zacc[NREP][LPR];
 #pragma unroll
@@ -1588,20 +1626,22 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
 #pragma unroll
         for (int g = 0; g < LPR; g++) zacc[h][g] = 0.f;
     }
-    // staging: this lane owns rows 2*lane and 2*lane+1 of the chunk, all groups of the piece (whole rows: elements
-    // [8*lane, 8*lane+8) of the chunk's [128][4] scale array).  Row r of a chunk is k-slot (r%RKB)/RL of
-    // A-lanes  (r%RL)*EPR + 4*g + i  in k-block r/RKB.
-    // A tile: one 8-byte cell (4 k-slots) per (k-block t, lane); the 16 cells of the lanes with
-    // the same (t, lane/16) form a row of 17 cells' pitch, and the rows of k-blocks 4..7 are
-    // shifted by one more cell.  With that skew the 2-byte staging stores of a wave (same
-    // cell column, 32 different rows) fall into 32 different LDS banks, and a wave's 8-byte
-    // operand reads stay conflict-free.
-    auto cell = [](int t, int l) { return ((4 * t + l / 16) * 17 + (l % 16)) * 4 + (t >> 2) * 4; };
-    const int row0 = 2 * lane;
-    int aoff[2];  // bf16 index of (row0 + e, g = 0, i = 0)
+    // staging: row r of a chunk is k-slot (r%RKB)/RL of A-lanes  (r%RL)*EPR + 4*g + i  in k-block r/RKB.  This lane owns
+    // two rows of the chunk, all groups of the piece.  One head: rows 2*lane and 2*lane+1 (whole rows: elements
+    // [8*lane, 8*lane+8) of the chunk's [128][4] scale array, one load).  Several heads: rows RL apart, neighbouring
+    // k-slots of the same A-lanes, so that a part's two products leave with one store.
+    // A tile: one 8-byte cell (4 k-slots) per (k-block t, lane); the cells of 16 lanes form a row of 17 cells' pitch, and
+    // with one head the rows of k-blocks 4..7 are shifted by one more cell.  With that skew the staging stores of a wave
+    // (same cell column, 32 different rows: of 2 bytes, or of 4 to both pairs of k-slots) fall into different LDS
+    // banks, and a wave's 8-byte operand reads stay conflict-free.
+    constexpr int SKEW = HALVES ? 0 : 4;
+    auto cell = [](int t, int l) { return ((4 * t + l / 16) * 17 + (l % 16)) * 4 + (t >> 2) * SKEW; };
+    constexpr int ROW_STEP = HALVES ? RL : 1;
+    const int row0 = HALVES ? lane / RL * (2 * RL) + lane % RL : 2 * lane;
+    int aoff[2];  // element of (row0 + e * ROW_STEP, g = 0, i = 0)
 #pragma unroll
     for (int e = 0; e < 2; e++) {
-        const int r = row0 + e;
+        const int r = row0 + e * ROW_STEP;
         aoff[e] = cell(r / RKB, (r % RL) * EPR) + (r % RKB) / RL;
     }
 
@@ -1615,37 +1655,38 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     if (a.K < CH) return;  // (never launched so: a chunk longer than K would leave the operand; the same for every thread)
     const int stride = KW * CH;
     const int kfirst = (int)kbeg + __builtin_amdgcn_readfirstlane(wy) * CH;
+    struct __attribute__((packed, aligned(2))) HalfRow {
+        uint16_t v[LPR];
+    };
+    struct __attribute__((packed, aligned(2))) HalfRows {
+        HalfRow row[2];
+    };
     struct __attribute__((packed, aligned(2))) Half2x {
         uint16_t v[2];
     };
     // DEPTH chunks are in flight per wave: register set d holds chunk c with c % DEPTH == d
-    struct __attribute__((packed, aligned(2))) HalfRow {
-        uint16_t v[LPR];
-    };
-    struct HalfRows {
-        HalfRow row[2];
-    };
-    using Scales = std::conditional_t<WHOLE, Half8, HalfRows>;
-    static_assert(sizeof(Scales) == 4 * LPR, "two rows of scales");
-    Scales s8[DEPTH], z8[DEPTH];
+    HalfRows s8[DEPTH], z8[DEPTH];
     Half2x xh[DEPTH][NREP];
     Elem w[DEPTH][KB][4];
 
     auto chunk_base = [&](int k0) { return k0 + CH <= ke32 ? k0 : max(ke32 - CH, 0); };
     auto load_small = [&](int d, int k0) {
         const uint32_t kr = (uint32_t)(chunk_base(k0) + row0);
-        if constexpr (WHOLE) {
-            s8[d] = ld_stream<Half8>(sp + kr * LPR);
-            z8[d] = ld_stream<Half8>(zp + kr * LPR);
+        if constexpr (WHOLE && !HALVES) {
+            s8[d] = ld_stream<HalfRows>(sp + kr * 4);
+            z8[d] = ld_stream<HalfRows>(zp + kr * 4);
         } else {
 #pragma unroll
             for (int q = 0; q < 2; q++) {
-                s8[d].row[q] = ld_stream<HalfRow, false>(sp + (kr + q) * 4);
-                z8[d].row[q] = ld_stream<HalfRow, false>(zp + (kr + q) * 4);
+                s8[d].row[q] = ld_stream<HalfRow, WHOLE>(sp + (kr + q * ROW_STEP) * 4);
+                z8[d].row[q] = ld_stream<HalfRow, WHOLE>(zp + (kr + q * ROW_STEP) * 4);
             }
         }
 #pragma unroll
-        for (int h = 0; h < NREP; h++) xh[d][h] = *reinterpret_cast<const Half2x *>(xp + h * a.x_bs + kr);
+        for (int h = 0; h < NREP; h++) {
+            if constexpr (HALVES) xh[d][h] = Half2x{xp[h * a.x_bs + kr], xp[h * a.x_bs + kr + ROW_STEP]};
+            else xh[d][h] = *reinterpret_cast<const Half2x *>(xp + h * a.x_bs + kr);
+        }
     };
     auto load_codes = [&](int d, int k0, int t) {
         const uint8_t *base = cp + (uint32_t)(chunk_base(k0) + rs) * (16 * EB);
@@ -1655,32 +1696,98 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
     };
     auto stage = [&](int d, int k0) {
         const int skip = k0 - chunk_base(k0);  // rows of this chunk that an earlier one covered
-        uint16_t sv[2 * LPR], zv[2 * LPR];
-        __builtin_memcpy(sv, &s8[d], sizeof(sv));
-        __builtin_memcpy(zv, &z8[d], sizeof(zv));
+        if constexpr (HALVES) {
+            const uint32_t keep = (row0 >= skip ? 0xffffu : 0u) | (row0 + ROW_STEP >= skip ? 0xffff0000u : 0u);
+            uint32_t xp2[NREP], sp2[LPR], over = 0;
+            auto excess = [&](uint32_t v, uint32_t limit) {
+                over |= __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(ushort2_t, v & 0x7fff7fffu),
+                                                                                   __builtin_bit_cast(ushort2_t, limit)));
+            };
 #pragma unroll
-        for (int h = 0; h < NREP; h++) {
+            for (int h = 0; h < NREP; h++) {
+                xp2[h] = (xh[d][h].v[0] | (uint32_t)xh[d][h].v[1] << 16) & keep;
+                excess(xp2[h], x_limit[h]);
+            }
+#pragma unroll
+            for (int g = 0; g < LPR; g++) {
+                sp2[g] = s8[d].row[0].v[g] | (uint32_t)s8[d].row[1].v[g] << 16;
+                excess(sp2[g], s_limit[g]);
+            }
+            if (__builtin_expect(__ballot(over != 0) != 0, 0)) {  // larger than the scaling allows: smaller powers from here on
+                auto wave_max = [&](uint32_t v) {
+                    v &= 0x7fff7fffu;
+                    v = max(v & 0xffffu, v >> 16);
+#pragma unroll
+                    for (int o = 1; o < kWave; o *= 2) v = max(v, (uint32_t)__shfl_xor((int)v, o));
+                    return (int)__builtin_amdgcn_readfirstlane(v);
+                };
+                int down = 0;  // of the lane's own group
+#pragma unroll
+                for (int g = 0; g < LPR; g++) {
+                    const int sb = min(s_pow[g], 22 - (wave_max(sp2[g]) >> 10));
+                    down = own_group == g ? sb - s_pow[g] : down;
+                    s_pow[g] = sb;
+                    s_limit[g] = (((23 - sb) << 10) - 1) * 0x00010001u;
+                }
+#pragma unroll
+                for (int h = 0; h < NREP; h++) {
+                    const int xb = min(x_pow[h], 21 - (wave_max(xp2[h]) >> 10));
+                    const float f = ldexpf(1.0f, xb - x_pow[h] + down);
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+#pragma unroll
+                        for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
+                    }
+                    x_pow[h] = xb;
+                    x_limit[h] = (((22 - xb) << 10) - 1) * 0x00010001u;
+                }
+            }
+            half2_t ss[LPR];
+#pragma unroll
+            for (int g = 0; g < LPR; g++) ss[g] = __builtin_bit_cast(half2_t, sp2[g]) * half_power(s_pow[g]);
+#pragma unroll
+            for (int h = 0; h < NREP; h++) {
+                const half2_t x = __builtin_bit_cast(half2_t, xp2[h]), xs = x * half_power(x_pow[h]);
+#pragma unroll
+                for (int g = 0; g < LPR; g++) {
+#pragma unroll
+                    for (int q = 0; q < 2; q++) zacc[h][g] = fmaf((float)x[q], h16_to_f32(z8[d].row[q].v[g]), zacc[h][g]);
+                    const half2_t hi = xs * ss[g], lo = __builtin_elementwise_fma(xs, ss[g], -hi);
+                    // A rows h (first part) and NREP + h (second): MFMA row / 4, lanes 4g + row % 4
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const int ar = NREP * i + h;
+                        *reinterpret_cast<uint32_t *>(atile + (ar / 4) * AT + aoff[0] + g * 16 + (ar % 4) * 4) = __builtin_bit_cast(uint32_t, i ? lo : hi);
+                    }
+                }
+            }
+        } else {
 #pragma unroll
             for (int e = 0; e < 2 * LPR; e++) {
                 const int q = e / LPR, g = e % LPR;
-                const float xv = row0 + q >= skip ? h16_to_f32(xh[d][h].v[q]) : 0.f;
-                zacc[h][g] = fmaf(xv, h16_to_f32(zv[e]), zacc[h][g]);
+                const float xv = row0 + q >= skip ? h16_to_f32(xh[d][0].v[q]) : 0.f;
+                zacc[0][g] = fmaf(xv, h16_to_f32(z8[d].row[q].v[g]), zacc[0][g]);
                 // x * scale * 2^90, split into bf16 parts by truncation (three parts: exact)
                 uint32_t part[NP];
-                split_bf16_parts<NP>((xv * 1237940039285380274899124224.0f) * h16_to_f32(sv[e]), part);
+                split_bf16_parts<NP>((xv * 1237940039285380274899124224.0f) * h16_to_f32(s8[d].row[q].v[g]), part);
 #pragma unroll
-                for (int pt = 0; pt < NP; pt++) {  // A row NP*h+pt: MFMA (NP*h+pt)/4, lanes 4g + (NP*h+pt)%4
-                    const int ar = NP * h + pt;
-                    atile[(ar / 4) * AT + aoff[q] + g * 16 + (ar % 4) * 4] = (uint16_t)(part[pt] >> 16);
-                }
+                for (int pt = 0; pt < NP; pt++) atile[aoff[q] + g * 16 + pt * 4] = (uint16_t)(part[pt] >> 16);  // A row pt: lanes 4g + pt
             }
         }
     };
     auto compute = [&](int d, int t) {
-        bf16x4_t av[NM];
+        uint2 av[NM];
 #pragma unroll
-        for (int q = 0; q < NM; q++)
-            av[q] = *reinterpret_cast<const bf16x4_t *>(atile + q * AT + cell(t, lane));
+        for (int q = 0; q < NM; q++) av[q] = *reinterpret_cast<const uint2 *>(atile + q * AT + cell(t, lane));
+        auto multiply = [&](uint32_t b01, uint32_t b23, int p) {
+#pragma unroll
+            for (int q = 0; q < NM; q++) {
+                if constexpr (HALVES)
+                    acc[q][p] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, av[q]), __builtin_bit_cast(half4_t, make_uint2(b01, b23)), acc[q][p], 0, 0, 0);
+                else
+                    acc[q][p] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(bf16x4_t, av[q]), __builtin_bit_cast(bf16x4_t, make_uint2(b01, b23)), acc[q][p], 0, 0, 0);
+            }
+        };
         if constexpr (BITS == 30) {
             // the lane's 24 bits hold code i at bit 3i.  Codes 0,1 are bits 0..5 of byte 0 and codes 6,7 bits
             // 2..7 of byte 2; codes 2,3 and 4,5 are bits 2..7 of byte 0 and bits 0..5 of byte 1 of the stream
@@ -1705,19 +1812,13 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
                 const uint32_t *src = from_u ? u : v;
                 const uint32_t t01 = __builtin_amdgcn_perm(src[1], src[0], sel);
                 const uint32_t t23 = __builtin_amdgcn_perm(src[3], src[2], sel);
-                // bit offset of the pair's first field in its byte: 0 or 2; a pair at 0 is moved up by two (see
-                // field_operand_top: its first field would have five leading zeros)
-                constexpr bool UP = KVMIX_ROWS_FIELDS_TOP;
-                const uint32_t s01 = UP && mm % 2 == 0 ? t01 << 2 : t01, s23 = UP && mm % 2 == 0 ? t23 << 2 : t23;
-                const int o0 = UP || mm % 2 != 0 ? 2 : 0;
+                // the pair's fields lie at bit 0 or 2 of the byte: all to bits TOP + 2 and up (see field_operand_top)
+                const int up = (mm % 2 == 0 ? 2 : 0) + TOP;
+                const uint32_t s01 = t01 << up, s23 = t23 << up;
 #pragma unroll
                 for (int f = 0; f < 2; f++) {
-                    const uint32_t mask = 0x00070007u << (o0 + 3 * f);
-                    const bf16x4_t bv = __builtin_bit_cast(bf16x4_t, make_uint2(s01 & mask, s23 & mask));
-#pragma unroll
-                    for (int q = 0; q < NM; q++)
-                        acc[q][mm * 2 + f] =
-                            __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(av[q], bv, acc[q][mm * 2 + f], 0, 0, 0);
+                    const uint32_t mask = 0x00070007u << (TOP + 2 + 3 * f);
+                    multiply(s01 & mask, s23 & mask, mm * 2 + f);
                 }
             }
         } else {
@@ -1729,13 +1830,8 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
                 const uint32_t t23 = perm_elems(w[d][t][3], w[d][t][2], sel);
 #pragma unroll
                 for (int f = 0; f < FPB; f++) {
-                    const bf16x4_t bv = __builtin_bit_cast(
-                        bf16x4_t, KVMIX_ROWS_FIELDS_TOP ? make_uint2(field_operand_top<FB>(t01, f), field_operand_top<FB>(t23, f))
-                                                        : make_uint2(field_operand<FB>(t01, f), field_operand<FB>(t23, f)));
-#pragma unroll
-                    for (int q = 0; q < NM; q++)
-                        acc[q][b * FPB + f] =
-                            __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(av[q], bv, acc[q][b * FPB + f], 0, 0, 0);
+                    if constexpr (HALVES) multiply(field_alone_top<FB, TOP>(t01, f), field_alone_top<FB, TOP>(t23, f), b * FPB + f);
+                    else multiply(field_operand_top<FB>(t01, f), field_operand_top<FB>(t23, f), b * FPB + f);
                 }
             }
         }
@@ -1797,25 +1893,29 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsHeadsWaves : kRowsMfmaWa
         for (int o = EPR; o < kWave; o *= 2) z[0] += __shfl_xor(z[0], o);
         zterm[h] = z[0];
     }
-    // code sums: the three parts meet; the 2^-133 of the bf16 patterns, the 2^90 and the
+    // code sums: the two parts meet; the 2^-24 of the patterns, the powers of x and scale and the
     // field's bit offset are undone; then the row slots (lane bits from EPR on) are summed
     constexpr int NV = NREP * NPOS;
     float flat[NV];
+    int own_pow = s_pow[0];
+#pragma unroll
+    for (int g = 1; g < LPR; g++) own_pow = own_group == g ? s_pow[g] : own_pow;
 #pragma unroll
     for (int h = 0; h < NREP; h++) {
         float sums[NPOS];
 #pragma unroll
-        for (int p = 0; p < NPOS; p++)
-            sums[p] = parts_sum<NP>(acc, h, p);
+        for (int p = 0; p < NPOS; p++) {
+            sums[p] = acc[h / 4][p][h % 4];
+#pragma unroll
+            for (int i = 1; i < NP; i++) sums[p] += acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4];
+        }
 #pragma unroll
         for (int p = 0; p < NPOS; p++) {
-            // (bit offset code p's field counts with: dense 3-bit 2 5 2 5 2 5 2 5 -- in its byte 0 3 2 5 0 3 2 5, the pairs at
-            // 0 moved up by two --, else see field_offset_top)
-            const int off = BITS == 30 ? 3 * (p % 2) + (KVMIX_ROWS_FIELDS_TOP ? 2 : 2 * ((p / 2) % 2)) : (KVMIX_ROWS_FIELDS_TOP ? field_offset_top<FB>(p % FPB) : FB * (p % FPB));
-            const float sum = BITS == 30 ? sums[p]
-                              : KVMIX_ROWS_FIELDS_TOP ? field_sum_top<FB>(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB)
-                                                      : field_sum(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
-            flat[h * NPOS + p] = sum * __uint_as_float((uint32_t)(127 + 43 - off) << 23);
+            // (bit offset code p's field counts with: dense 3-bit 2 5 2 5 2 5 2 5, else see field_offset_top)
+            const int off = TOP + (BITS == 30 ? 2 + 3 * (p % 2) : field_offset_top<FB>(p % FPB));
+            const float sum = BITS == 30 || HALVES ? sums[p] : field_sum_top<FB>(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
+            if constexpr (HALVES) flat[h * NPOS + p] = ldexpf(sum, 24 - off - x_pow[h] - own_pow);
+            else flat[h * NPOS + p] = sum * __uint_as_float((uint32_t)(127 + 43 - off) << 23);
         }
     }
     __syncthreads();  // every wave is done with its A tile: the space becomes `red`
@@ -3240,11 +3340,11 @@ struct RowsPlan {
 };
 
 // How gemv_rows covers K for `batch_rows` = samples*M independent outputs.
-// (blocks of at most four waves are the multi-head kernels, which hold two waves per SIMD:
+// (blocks of at most eight waves are the multi-head kernels, which hold two waves per SIMD:
 // they get half as many waves, again one resident round)
 static RowsPlan plan_rows(int64_t batch_rows, int64_t K, int64_t N, int max_waves)
 {
-    const int64_t target = max_waves <= kRowsHeadsWaves ? kTargetWaves / kHeadsWaveDiv : kTargetWaves;
+    const int64_t target = max_waves <= kRowsMfmaHeadsWaves ? kTargetWaves / kHeadsWaveDiv : kTargetWaves;
     RowsPlan p{4, 1, K > 0 ? K : 1};
     if (!rows_shape_ok(N) || batch_rows <= 0 || K <= 0) return p;
     const int64_t chunk = 512 / (N / 32);            // rows one wave takes per step
@@ -3301,7 +3401,7 @@ static bool rows_use_mfma(int mode, int64_t N, int64_t K, int64_t c_rs)
 }
 static int rows_max_waves(bool mfma, int nrep)
 {
-    return nrep > 1 ? kRowsHeadsWaves : (mfma ? kRowsMfmaWaves : kRowsMaxWaves);
+    return nrep > 1 ? (mfma ? kRowsMfmaHeadsWaves : kRowsHeadsWaves) : (mfma ? kRowsMfmaWaves : kRowsMaxWaves);
 }
 
 // gemv_rows_mfma: blocks that share the columns of an output row, each with 128 / rows_pieces of them.  Launches of few
@@ -3754,7 +3854,9 @@ extern "C" size_t kvmix_gemv_workspace_bytes(int64_t samples, int64_t M, int64_t
     const RowsPlan p1 = plan_rows(samples * M, K, N, kRowsMaxWaves);
     const RowsPlan p8 = plan_rows(samples * M, K, N, kRowsMfmaWaves);
     const RowsPlan p4 = plan_rows((samples + 3) / 4 * M, K, N, kRowsHeadsWaves);
+    const RowsPlan p4m = plan_rows((samples + 3) / 4 * M, K, N, kRowsMfmaHeadsWaves);
     int splits = p1.splits > p4.splits ? p1.splits : p4.splits;
+    splits = p4m.splits > splits ? p4m.splits : splits;
     splits = p8.splits > splits ? p8.splits : splits;
     return splits > 1 ? (size_t)(samples * M) * (size_t)splits * (size_t)N * sizeof(float) : 0;
 }

@@ -56,3 +56,41 @@ def test_against_float64(dev, bits, B, nh, nkv, M, K):
     got = KVmix.quantized_gemm(32, *(t.to(dev) for t in ops), 3 if bits == 30 else bits, *((1,) if bits == 30 else ())).double().cpu()
     want, size = exact(bits, *ops)
     assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + K * 2.0 ** -23 * size + 2.0 ** -25).all()
+
+
+@pytest.mark.gpu
+# x of any size, heads of one kv head far apart; scales beyond what the first powers of two are good for, groups far apart, a
+# row larger than all before it in the last chunk
+@pytest.mark.parametrize("kind", ["normal", "large", "heads apart", "groups apart", "rising", "tiny"])
+@pytest.mark.parametrize("bits", [1, 2, 4, 30])
+def test_two_fp16_parts_of_four_heads(dev, bits, kind):
+    """x * scale in two fp16 parts after powers of two per (head, group): beside the bound above a product is off by at most
+    2^-25 of what the powers leave, for x of at most X in its head 2^-25 max(1, X) / 2^6, times max(2^-5, 2^-7 S) for
+    scales of at most S in its group, and that 2^bits - 1 times."""
+    import KVmix
+
+    B, nh, nkv, M, K = 2, 8, 2, 1, 1111
+    x, code, scale, zero = operands(bits, B, nh, nkv, M, K, 7 * bits)
+    gen = torch.Generator().manual_seed(bits)
+    if kind != "tiny":
+        x = torch.randn(x.shape, generator=gen).half()
+    if kind == "large":
+        x, scale = x * 6, scale * 20
+    if kind == "heads apart":
+        x = x * (10.0 ** torch.arange(-4, 4)).half()[None, :, None, None]
+    if kind == "groups apart":
+        scale = scale * torch.tensor([1e-4, 1.0, 30.0, 300.0]).half()
+    if kind == "rising":
+        x[..., -1], scale[:, :, -1] = 30.0, 90.0
+        x[..., 300], scale[:, :, 5] = 9.0, 20.0
+    if kind == "tiny":
+        x, scale, zero = x * 2.0 ** -6, scale * 2.0 ** -10, zero * 2.0 ** -10
+    ops = (x, code, scale, zero)
+    got = KVmix.quantized_gemm(32, *(t.to(dev) for t in ops), 3 if bits == 30 else bits, *((1,) if bits == 30 else ())).double().cpu()
+    want, size = exact(bits, *ops)
+    X = x.double().abs().amax(-1, keepdim=True).clamp(min=1.0)
+    S = (scale.double().abs().amax(2, keepdim=True) * 2.0 ** -7).clamp(min=2.0 ** -5).repeat_interleave(4, 1).repeat_interleave(32, -1)
+    parts = K * (2 ** (3 if bits == 30 else bits) - 1) * 2.0 ** -31 * X * S
+    finite = want.abs() < 65504
+    assert finite.float().mean() > 0.5
+    assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + K * 2.0 ** -23 * size + parts + 2.0 ** -25)[finite].all()
