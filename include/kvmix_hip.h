@@ -330,6 +330,18 @@ int kvmix_decode_attention_fused(const kvmix_decode_attn_t *step, void *workspac
                                  kvmix_stream_t stream);
 
 /*
+ * The same with the probabilities: `probs` [samples, width] (stride `probs_stride`) receives fp16(softmax) of every
+ * position, zero past the live ones, as kvmix_decode_attention returns them; the output is formed from the unrounded
+ * ones, as in kvmix_decode_attention_fused.  Slabs only (the vector-ALU kind), and a second kernel that merges them and
+ * turns the logits they left in `probs` into probabilities.  Takes what kvmix_decode_attention_fused takes.
+ * ..._recommended: 1 where this is faster than the launches of kvmix_decode_attention (measured); reads the sizes only.
+ */
+size_t kvmix_decode_attention_fused_weights_workspace_bytes(const kvmix_decode_attn_t *step);
+int kvmix_decode_attention_fused_weights_recommended(const kvmix_decode_attn_t *step);
+int kvmix_decode_attention_fused_weights(const kvmix_decode_attn_t *step, void *workspace, size_t workspace_bytes,
+                                         kvmix_stream_t stream);
+
+/*
  * How kvmix_decode_attention_fused would run a step of these sizes: which positions go through the matrix-core
  * kernel, how the rest is cut into slabs, and the launches' geometry.  No counterpart in the reference; it needs no
  * GPU and launches nothing (for the dispatch tests, for callers that choose between the two step forms, and for

@@ -34,6 +34,9 @@ EXPORTS = (
     "kvmix_decode_attention_fused_supported",
     "kvmix_decode_attention_fused_workspace_bytes",
     "kvmix_decode_attention_fused",
+    "kvmix_decode_attention_fused_weights_workspace_bytes",
+    "kvmix_decode_attention_fused_weights_recommended",
+    "kvmix_decode_attention_fused_weights",
     "kvmix_decode_attention_fused_plan",
     "kvmix_rope_append",
     "kvmix_linear_rows_supported",
@@ -191,6 +194,12 @@ def load() -> ctypes.CDLL:
     L.kvmix_decode_attention_fused_workspace_bytes.argtypes = [ctypes.POINTER(DecodeAttn)]
     L.kvmix_decode_attention_fused.restype = i32
     L.kvmix_decode_attention_fused.argtypes = [ctypes.POINTER(DecodeAttn), vp, sz, vp]
+    L.kvmix_decode_attention_fused_weights_workspace_bytes.restype = sz
+    L.kvmix_decode_attention_fused_weights_workspace_bytes.argtypes = [ctypes.POINTER(DecodeAttn)]
+    L.kvmix_decode_attention_fused_weights_recommended.restype = i32
+    L.kvmix_decode_attention_fused_weights_recommended.argtypes = [ctypes.POINTER(DecodeAttn)]
+    L.kvmix_decode_attention_fused_weights.restype = i32
+    L.kvmix_decode_attention_fused_weights.argtypes = [ctypes.POINTER(DecodeAttn), vp, sz, vp]
     L.kvmix_decode_attention_fused_plan.restype = i32
     L.kvmix_decode_attention_fused_plan.argtypes = [ctypes.POINTER(DecodeAttn), ctypes.POINTER(AttnPlan)]
     L.kvmix_rope_append.restype = i32

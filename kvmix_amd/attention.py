@@ -200,12 +200,12 @@ class KVmixAttention:
             if attention_mask is not None and attention_mask.shape[-2:] != (1, kv_seq_len):
                 raise ValueError(f"Attention mask shape {attention_mask.shape} does not match weights shape "
                                  f"{(B, nh, 1, kv_seq_len)}")
-            single = (not need_weights) and ops.prefer_single_pass(
+            single = ops.prefer_single_pass(
                 B, nh, nkv, D, kv_seq_len, self.k_bits, k_fmt, k_group, self.v_bits, v_fmt,
-                self.Vgroup_size, k_tokens=kv_seq_len - k_tail.shape[2], v_tokens=kv_seq_len - v_tail.shape[2])
+                self.Vgroup_size, kv_seq_len - k_tail.shape[2], kv_seq_len - v_tail.shape[2], need_weights)
             return ops.decode_attention(
                 query_states, (kc, ks, km), (vc, vs, vm), k_tail, v_tail, k_group, self.k_bits, self.Vgroup_size,
-                self.v_bits, k_fmt, v_fmt, attention_mask, single_pass=single)
+                self.v_bits, k_fmt, v_fmt, attention_mask, single_pass=single, weights=need_weights)
         return self._decode_with_torch_glue(query_states, kc, ks, km, k_tail, vc, vs, vm, v_tail, k_group, k_fmt, v_fmt, nh // nkv, attention_mask)
 
     def attend(self, query_states: torch.Tensor, cache: PackedKVCache, attention_mask: Optional[torch.Tensor] = None,

@@ -82,6 +82,68 @@ __global__ void __launch_bounds__(kFusedD) attn_fused_merge(const float *ws_o, c
     out[sample * o_bs + c] = f32_to_h16(L > 0.f ? o / L : 0.f);
 }
 
+// The merge of a step that also returns its probabilities: grid = (samples, parts of a row), 256 threads.  Every block forms
+// the row's maximum and sum from the slabs' (at most width / 512 of them), the first merges the outputs, and each turns its
+// part of the row, in which the slabs left the fp16 logits, into fp16(exp(x - maximum) / sum) in place, x the logit scaled
+// and masked as the slabs took it.  Positions past the live ones get zero.  Sums without a live position or with a NaN
+// are divided by as they are, as in attn_tail_softmax.
+// Bound by its chain of a few short phases; a part is eight entries per thread.  Measured, step with probabilities, four
+// launches of kvmix_decode_attention -> slabs and this, operands from memory, us: 32 / 8 heads, B = 1, T = 1036, 4 bits 31.1 ->
+// 16.2; T = 4000, 32 heads 28.2 -> 18.2; B = 4, T = 512, 4-bit keys, dense 3-bit values 30.7 -> 17.3.
+constexpr int kWeightsThreads = 256, kWeightsPart = 8 * kWeightsThreads;
+__global__ void __launch_bounds__(kWeightsThreads) attn_fused_merge_weights(FusedArgs a, int64_t width)
+{
+    __shared__ float scratch[2][kWeightsThreads / kWave];
+    const int64_t sample = blockIdx.x;
+    const int tid = threadIdx.x;
+    const float *ml = a.ws_ml + sample * a.slabs * 2;
+    int64_t k_len = a.k_len_dev ? *a.k_len_dev : a.k_len;
+    k_len = k_len < 0 ? 0 : (k_len > a.k_slots ? a.k_slots : k_len);
+    const int64_t live = a.k_tokens + k_len;
+
+    float M = -INFINITY;
+    for (int s = tid; s < a.slabs; s += kWeightsThreads) M = fmaxf(M, ml[2 * s]);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+    if (tid % kWave == 0) scratch[0][tid / kWave] = M;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWeightsThreads / kWave; w++) M = fmaxf(M, scratch[0][w]);
+    float L = 0.f;
+    for (int s = tid; s < a.slabs; s += kWeightsThreads) L = fmaf(ml[2 * s + 1], ml[2 * s] == -INFINITY ? 0.f : expf(ml[2 * s] - M), L);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) L += __shfl_xor(L, o);
+    if (tid % kWave == 0) scratch[1][tid / kWave] = L;
+    __syncthreads();
+    L = scratch[1][0];
+#pragma unroll
+    for (int w = 1; w < kWeightsThreads / kWave; w++) L += scratch[1][w];
+
+    uint16_t *row = a.probs + sample * a.p_bs;
+    const float *mrow = a.mask ? a.mask + (sample / a.heads) * a.mask_bs : nullptr;
+    const int64_t i0 = (int64_t)blockIdx.y * kWeightsPart + tid * 8;
+    auto probability = [&](int64_t i, uint16_t logit) -> uint16_t {
+        if (i >= live) return 0;
+        float x = h16_to_f32(logit) * a.inv_sqrt_d;
+        if (mrow) x = fmaxf(x + mrow[i], kLowest);
+        return f32_to_h16((x == -INFINITY ? 0.f : expf(x - M)) / L);
+    };
+    if (i0 + 8 <= width) {
+        F8 h = *reinterpret_cast<const F8 *>(row + i0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) h.v[i] = probability(i0 + i, h.v[i]);
+        *reinterpret_cast<F8 *>(row + i0) = h;
+    } else {
+        for (int64_t i = i0; i < width; i++) row[i] = probability(i, row[i]);
+    }
+    if (blockIdx.y != 0 || tid >= kFusedD) return;
+    const float *op = a.ws_o + sample * a.slabs * kFusedD + tid;
+    float o = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < a.slabs; s++) o = fmaf(op[(int64_t)s * kFusedD], ml[2 * s] == -INFINITY ? 0.f : expf(ml[2 * s] - M), o);
+    a.out[sample * a.o_bs + tid] = f32_to_h16(o / L);
+}
+
 }  // namespace kvmix
 
 using namespace kvmix;
@@ -158,9 +220,11 @@ static bool coop_ok(int km, int64_t pairs)
     return km == 3 ? pairs >= 128 : true;
 }
 
-static FusedLayout fused_layout(const kvmix_decode_attn_t *p)
+// (weights: the matrix-core tiles keep their logits in registers, so a step that returns probabilities runs on slabs)
+static FusedLayout fused_layout(const kvmix_decode_attn_t *p, bool weights = false)
 {
     FusedLayout l{false, false, 0, fused_slabs(p), 0, fused_slab(p)};
+    if (weights) return l;
     const int km = fused_key_mode(p), vm = fused_value_mode(p);
     const int vbits = vm == 3 ? 3 : vm;
     // positions quantized on both sides, in whole words of the keys and whole groups of the values; tiles of 1024
@@ -287,18 +351,16 @@ extern "C" int kvmix_decode_attention_fused_plan(const kvmix_decode_attn_t *p, k
     return KVMIX_OK;
 }
 
-extern "C" int kvmix_decode_attention_fused(const kvmix_decode_attn_t *p, void *workspace, size_t workspace_bytes,
-                                            kvmix_stream_t stream)
+static int fused_step(const kvmix_decode_attn_t *p, bool weights, void *workspace, hipStream_t st)
 {
-    const int chk = fused_check(p, true);
-    if (chk != KVMIX_OK || p->samples == 0) return chk;
     const int k_mode = fused_key_mode(p), v_mode = fused_value_mode(p);
-    const FusedLayout lay = fused_layout(p);
+    const FusedLayout lay = fused_layout(p, weights);
     const int64_t slabs = lay.slabs();
     const int64_t kv_samples = p->samples / p->heads_per_kv;
-    if (!workspace || workspace_bytes < kvmix_decode_attention_fused_workspace_bytes(p)) return KVMIX_ERR_WORKSPACE;
 
     FusedArgs a;
+    a.probs = weights ? (uint16_t *)p->probs : nullptr;
+    a.p_bs = p->probs_stride;
     a.q = (const uint16_t *)p->q;
     a.k_code = p->k_code;
     a.k_scale = (const uint16_t *)p->k_scale;
@@ -346,7 +408,6 @@ extern "C" int kvmix_decode_attention_fused(const kvmix_decode_attn_t *p, void *
     a.heads = p->heads;
     a.inv_sqrt_d = 1.0f / sqrtf((float)p->D);
 
-    hipStream_t st = (hipStream_t)stream;
     // one query head per block: the heads that share a kv head re-read its slab through L2 (two heads
     // per block need more registers than a 512-thread block has)
     a.head_groups = p->heads_per_kv;
@@ -370,8 +431,54 @@ extern "C" int kvmix_decode_attention_fused(const kvmix_decode_attn_t *p, void *
         hipLaunchKernelGGL(attn_fused_slab<1>, grid, dim3(kFusedThreads), 0, st, a);
         rc = launch_status();
     }
-    if (rc != KVMIX_OK || (slabs == 1 && !lay.mfma)) return rc;  // a single slab of attn_fused_slab is normalised and stored by that kernel
+    if (rc != KVMIX_OK) return rc;
+    if (weights) {
+        const int64_t width = fused_width(p);
+        hipLaunchKernelGGL(attn_fused_merge_weights, dim3((unsigned)p->samples, (unsigned)((width + kWeightsPart - 1) / kWeightsPart)),
+                           dim3(kWeightsThreads), 0, st, a, width);
+        return launch_status();
+    }
+    if (slabs == 1 && !lay.mfma) return rc;  // a single slab of attn_fused_slab is normalised and stored by that kernel
     hipLaunchKernelGGL(attn_fused_merge, dim3((unsigned)p->samples), dim3(kFusedD), 0, st, a.ws_o, a.ws_ml, (int)slabs,
                        (uint16_t *)p->out, p->out_stride);
     return launch_status();
+}
+
+extern "C" int kvmix_decode_attention_fused(const kvmix_decode_attn_t *p, void *workspace, size_t workspace_bytes,
+                                            kvmix_stream_t stream)
+{
+    const int chk = fused_check(p, true);
+    if (chk != KVMIX_OK || p->samples == 0) return chk;
+    if (!workspace || workspace_bytes < kvmix_decode_attention_fused_workspace_bytes(p)) return KVMIX_ERR_WORKSPACE;
+    return fused_step(p, false, workspace, (hipStream_t)stream);
+}
+
+extern "C" size_t kvmix_decode_attention_fused_weights_workspace_bytes(const kvmix_decode_attn_t *p)
+{
+    if (!p || p->samples <= 0 || !kvmix_decode_attention_fused_supported(p)) return 0;
+    return (size_t)p->samples * (size_t)fused_layout(p, true).slabs() * (kFusedD + 2) * sizeof(float);
+}
+
+extern "C" int kvmix_decode_attention_fused_weights(const kvmix_decode_attn_t *p, void *workspace, size_t workspace_bytes,
+                                                    kvmix_stream_t stream)
+{
+    const int chk = fused_check(p, true);
+    if (chk != KVMIX_OK || p->samples == 0) return chk;
+    if (!p->probs) return KVMIX_ERR_NULL;
+    if (p->probs_stride < fused_width(p) || (fused_width(p) + kWeightsPart - 1) / kWeightsPart > 65535) return KVMIX_ERR_SHAPE;
+    if (!workspace || workspace_bytes < kvmix_decode_attention_fused_weights_workspace_bytes(p)) return KVMIX_ERR_WORKSPACE;
+    return fused_step(p, true, workspace, (hipStream_t)stream);
+}
+
+// Which form of a step with probabilities is faster (operands from memory, four launches -> slabs, us): the slabs up to 450 000
+// (query head x position) entries, 300 000 with the reference's 3-bit keys, which the slabs take as vector arithmetic
+// throughout.  33 000 entries (1 x 1036, 32 / 8 heads, 4 bits) 31.1 -> 16.2; 128 000 (1 x 4000, 4 bits) 28.2 -> 18.2;
+// 256 000: 1 x 8000, 2 bits 29.0 -> 20.9, 1 x 8000, 32 / 8 heads, 4 bits 37.3 -> 20.0, 4 x 2000, 3-bit keys 29.2 -> 25.5; 307 000
+// (32 x 300) 49.0 -> 34.3; level at 512 000: 4 x 4000, 2 bits 34.6 -> 34.2, 8 x 2000, 32 / 8 heads 35.7 -> 35.2.
+constexpr int64_t kSmallWeightsEntries = 450000, kSmallWeightsEntriesRef3 = 300000;
+extern "C" int kvmix_decode_attention_fused_weights_recommended(const kvmix_decode_attn_t *p)
+{
+    if (fused_check(p, false) != KVMIX_OK || p->samples == 0) return 0;
+    const bool ref3 = p->k_tokens > 0 && fused_key_mode(p) == 3;
+    return p->samples * fused_width(p) <= (ref3 ? kSmallWeightsEntriesRef3 : kSmallWeightsEntries) ? 1 : 0;
 }

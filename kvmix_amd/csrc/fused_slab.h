@@ -21,6 +21,8 @@ struct FusedArgs {
     int64_t o_bs;
     float *ws_o;              // [samples, slabs, D]
     float *ws_ml;             // [samples, slabs, 2]: slab maximum, slab sum
+    uint16_t *probs;          // optional [samples, width]: the fp16 logits of the live positions, for attn_fused_merge_weights
+    int64_t p_bs;
     int64_t q_bs, kc_bs, kc_rs, ksz_bs, ksz_rs, vc_bs, vc_rs, vsz_bs, vsz_rs;
     int64_t kt_bs, kt_ts, vt_bs, vt_ts, mask_bs;
     int64_t k_tokens, v_tokens, k_slots, v_slots, k_len, v_len;
@@ -349,8 +351,10 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
     __syncthreads();
 
     const float *mrow = a.mask ? a.mask + (sample0 / a.heads) * a.mask_bs : nullptr;
-    auto finish = [&](float dot, int64_t pos) {  // fp16 logit -> scaled, masked fp32 value
-        float x = h16_to_f32(f32_to_h16(dot)) * a.inv_sqrt_d;
+    auto finish = [&](float dot, int64_t pos, int h) {  // fp16 logit -> scaled, masked fp32 value
+        const uint16_t logit = f32_to_h16(dot);
+        if (a.probs) a.probs[(sample0 + h) * a.p_bs + pos] = logit;
+        float x = h16_to_f32(logit) * a.inv_sqrt_d;
         if (mrow) x = fmaxf(x + mrow[pos], kLowest);
         return x;
     };
@@ -373,7 +377,7 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
                 float dot = 0.f;
 #pragma unroll
                 for (int w = 0; w < (SlabCfg<KL>::kWaves); w++) dot += red[(w * NREP + h) * (SlabCfg<KL>::kRedStride) + at];
-                lg[idx] = finish(dot, t0 + pos);
+                lg[idx] = finish(dot, t0 + pos, h);
             }
         }
     }
@@ -399,7 +403,7 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
             if (in && sub == 0) {
                 const int64_t pos = a.k_tokens + j;
 #pragma unroll
-                for (int h = 0; h < NREP; h++) lg[h * S + (int)(pos - t0)] = finish(dot[h], pos);
+                for (int h = 0; h < NREP; h++) lg[h * S + (int)(pos - t0)] = finish(dot[h], pos, h);
             }
         }
     }
@@ -484,10 +488,10 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
         float o = 0.f;
 #pragma unroll
         for (int w = 0; w < (SlabCfg<KL>::kWaves); w++) o += red[(w * NREP + h) * kFusedD + c];
-        if (a.slabs == 1) a.out[(sample0 + h) * a.o_bs + c] = f32_to_h16(l_h[h] > 0.f ? o / l_h[h] : 0.f);
+        if (a.slabs == 1 && !a.probs) a.out[(sample0 + h) * a.o_bs + c] = f32_to_h16(l_h[h] > 0.f ? o / l_h[h] : 0.f);
         else a.ws_o[((sample0 + h) * a.slabs + a.slab0 + slab) * kFusedD + c] = o;
     }
-    if (tid == 0 && a.slabs > 1) {
+    if (tid == 0 && (a.slabs > 1 || a.probs)) {
 #pragma unroll
         for (int h = 0; h < NREP; h++) {
             a.ws_ml[((sample0 + h) * a.slabs + a.slab0 + slab) * 2 + 0] = m_h[h];

@@ -38,6 +38,9 @@ struct Api {
     decltype(&kvmix_decode_attention_fused_workspace_bytes) decode_attention_fused_workspace_bytes;
     decltype(&kvmix_decode_attention_fused) decode_attention_fused;
     decltype(&kvmix_decode_attention_fused_plan) decode_attention_fused_plan;
+    decltype(&kvmix_decode_attention_fused_weights_workspace_bytes) decode_attention_fused_weights_workspace_bytes;
+    decltype(&kvmix_decode_attention_fused_weights_recommended) decode_attention_fused_weights_recommended;
+    decltype(&kvmix_decode_attention_fused_weights) decode_attention_fused_weights;
     decltype(&kvmix_copy_rows) copy_rows;
     decltype(&kvmix_linear_rows) linear_rows;
 } api;
@@ -56,6 +59,9 @@ void bind(const std::unordered_map<std::string, uintptr_t> &at)
     KVMIX_BIND(decode_attention_fused_workspace_bytes);
     KVMIX_BIND(decode_attention_fused);
     KVMIX_BIND(decode_attention_fused_plan);
+    KVMIX_BIND(decode_attention_fused_weights_workspace_bytes);
+    KVMIX_BIND(decode_attention_fused_weights_recommended);
+    KVMIX_BIND(decode_attention_fused_weights);
     KVMIX_BIND(copy_rows);
     KVMIX_BIND(linear_rows);
 #undef KVMIX_BIND
@@ -433,7 +439,7 @@ Tensor quantized_gemm(int64_t group, const Tensor &fA, const Tensor &qB, const T
 }
 
 bool prefer_single_pass(int64_t batch, int64_t heads, int64_t kv_heads, int64_t D, int64_t width, int64_t k_bits, int64_t k_fmt, int64_t k_group,
-                        int64_t v_bits, int64_t v_fmt, int64_t v_group, int64_t k_tokens, int64_t v_tokens)
+                        int64_t v_bits, int64_t v_fmt, int64_t v_group, int64_t k_tokens, int64_t v_tokens, bool weights)
 {
     kvmix_decode_attn_t st{};
     const bool ref3 = k_bits == 3 && k_fmt == KVMIX_FMT_REF;
@@ -452,6 +458,7 @@ bool prefer_single_pass(int64_t batch, int64_t heads, int64_t kv_heads, int64_t 
     st.k_tail_slots = st.k_tail_len = width - k_tokens, st.v_tail_slots = st.v_tail_len = width - v_tokens;
     st.k_tail_token_stride = st.v_tail_token_stride = D;
     st.k_tail_batch_stride = st.k_tail_slots * D, st.v_tail_batch_stride = st.v_tail_slots * D;
+    if (weights) return api.decode_attention_fused_weights_recommended(&st);
     kvmix_attn_plan_t plan;
     return api.decode_attention_fused_plan(&st, &plan) == KVMIX_OK && plan.recommended;
 }
@@ -460,7 +467,8 @@ bool prefer_single_pass(int64_t batch, int64_t heads, int64_t kv_heads, int64_t 
 std::pair<Tensor, OptTensor> decode_attention(const Tensor &q_in, const OptTriple &k_packed, const OptTriple &v_packed, const Tensor &k_tail,
                                               const Tensor &v_tail, int64_t k_group, int64_t k_bits, int64_t v_group, int64_t v_bits,
                                               int64_t k_fmt, int64_t v_fmt, const OptTensor &mask_in, std::optional<int64_t> k_len,
-                                              const OptTensor &k_len_dev, std::optional<int64_t> v_len, const OptTensor &v_len_dev, bool single_pass)
+                                              const OptTensor &k_len_dev, std::optional<int64_t> v_len, const OptTensor &v_len_dev, bool single_pass,
+                                              bool weights)
 {
     if (q_in.dim() != 4 || q_in.size(2) != 1) fail("decode_attention takes one query position: q must be [B, nh, 1, D]");
     need_half({&q_in, &k_tail, &v_tail});
@@ -518,6 +526,15 @@ std::pair<Tensor, OptTensor> decode_attention(const Tensor &q_in, const OptTripl
         if (!api.decode_attention_fused_supported(&st))
             fail("the single-pass attention step does not take this layout (head_dim 128, keys 1/2/4-bit or dense 3-bit group 32 or "
                  "reference 3-bit, values 1/2/4-bit or dense 3-bit group 32)");
+        if (weights) {
+            Tensor probs = empty({B, nh, 1, width}, at::kHalf, q_in);
+            st.probs = probs.data_ptr(), st.probs_stride = width;
+            const size_t bytes = api.decode_attention_fused_weights_workspace_bytes(&st);
+            const Tensor ws = empty({(int64_t)bytes}, at::kByte, q_in);
+            const c10::DeviceGuard guard(q_in.device());
+            check(api.decode_attention_fused_weights(&st, ws.data_ptr(), bytes, stream_of(q_in)));
+            return {out, probs};
+        }
         const size_t bytes = api.decode_attention_fused_workspace_bytes(&st);
         const Tensor ws = empty({(int64_t)bytes}, at::kByte, q_in);
         const c10::DeviceGuard guard(q_in.device());

@@ -234,8 +234,8 @@ def quantized_gemm(group_size: int, fA: torch.Tensor, qB: torch.Tensor, scales: 
 
 def prefer_single_pass(batch: int, heads: int, kv_heads: int, head_dim: int, width: int, k_bits: int, k_fmt: int,
                        k_group: int, v_bits: int, v_fmt: int, v_group: int, k_tokens: int = None,
-                       v_tokens: int = None) -> bool:
-    """Policy for callers that do not need the probabilities: whether the single-pass step is both
+                       v_tokens: int = None, weights: bool = False) -> bool:
+    """Policy for callers that do not need the probabilities (weights: that do): whether the single-pass step is both
     available for this layout and the faster of the two at this size.  The library holds the measured rule
     (kvmix_decode_attention_fused_plan: `recommended`); k_tokens / v_tokens are the quantized lengths, where the
     caller knows them (they decide whether a large step can use the matrix cores; without them a step is
@@ -247,7 +247,7 @@ def prefer_single_pass(batch: int, heads: int, kv_heads: int, head_dim: int, wid
     if k_tokens is None or v_tokens is None or width < max(k_tokens, v_tokens):
         k_tokens = v_tokens = 0
     return _host().prefer_single_pass(batch, heads, kv_heads, head_dim, width, k_bits, k_fmt, k_group, v_bits, v_fmt, v_group,
-                                      k_tokens, v_tokens)
+                                      k_tokens, v_tokens, weights)
 
 
 def _set_tail(st, prefix: str, tail: torch.Tensor, slot) -> None:
@@ -432,14 +432,14 @@ def single_pass_supported(head_dim: int, heads_per_kv: int, k_bits: int, k_fmt: 
 def decode_attention(q: torch.Tensor, k_packed, v_packed, k_tail: torch.Tensor, v_tail: torch.Tensor,
                      k_group: int, k_bits: int, v_group: int, v_bits: int, k_fmt: int = _lib.FMT_REF,
                      v_fmt: int = _lib.FMT_REF, attention_mask=None, k_tail_len=None, v_tail_len=None,
-                     single_pass: bool = False):
+                     single_pass: bool = False, weights: bool = False):
     """One decode step of attention over the packed cache plus its fp16 tails, in four or five
     launches (no reference operator: it is what models/modeling_llama_KVmix.py:180-211 composes
     from quantized_gemm, matmul, cat and softmax).
 
     single_pass=True runs the step as one pass over the positions instead (two launches, logits and
-    probabilities stay on chip); no probabilities are returned (probs is None) and the roundings
-    after the softmax are not the reference's (see the header).  Layouts the single-pass kernels do
+    probabilities stay on chip); no probabilities are returned (probs is None; weights=True: they are, at
+    the price of writing the logits) and the roundings after the softmax are not the reference's (see the header).  Layouts the single-pass kernels do
     not take raise RuntimeError; `single_pass_supported` tells beforehand.
 
     q [B,nh,1,D] fp16; k_packed = (code [B,Hkv,D,Tk/vpw], scale, min) or None; v_packed =
@@ -452,7 +452,7 @@ def decode_attention(q: torch.Tensor, k_packed, v_packed, k_tail: torch.Tensor, 
     for n in (k_tail_len, v_tail_len):
         lengths += (None, n) if torch.is_tensor(n) else (None if n is None else int(n), None)
     return _host().decode_attention(q, k_packed, v_packed, k_tail, v_tail, k_group, k_bits, v_group, v_bits, k_fmt, v_fmt,
-                                    attention_mask, *lengths, single_pass)
+                                    attention_mask, *lengths, single_pass, weights)
 
 
 def copy_rows(pairs) -> None:
