@@ -502,6 +502,15 @@ typedef struct kvmix_copy_rows {
 int kvmix_copy_rows(const kvmix_copy_rows_t *items, int count, kvmix_stream_t stream);
 
 /*
+ * A cache grown by concatenation: `copies` as kvmix_copy_rows takes them, and what is quantized to behind them -- `keys` and
+ * `values` as kvmix_quant_pack_kv_flush takes them, either of which may be NULL (`values` alone quantizes any fp16 rows, as
+ * kvmix_quant_pack_last_dim does) -- in one launch where the sizes and formats allow it.  The copies must not overlap
+ * what the quantizers read or write.
+ */
+int kvmix_grow(const kvmix_copy_rows_t *copies, int count, const kvmix_key_flush_t *keys, const kvmix_value_flush_t *values,
+               kvmix_stream_t stream);
+
+/*
  * Measurement support, no counterpart in the reference and not called by any operator: a kernel
  * that only reads, in the access patterns of the GEMV kernels, to establish what streaming rate
  * the GPU reaches without arithmetic (the ceiling the GEMV figures are compared with), and how

@@ -45,6 +45,7 @@ EXPORTS = (
     "kvmix_prefill_attention_supported",
     "kvmix_prefill_attention",
     "kvmix_copy_rows",
+    "kvmix_grow",
     "kvmix_probe_stream_read",
 )
 
@@ -216,6 +217,8 @@ def load() -> ctypes.CDLL:
     L.kvmix_prefill_attention.argtypes = [ctypes.POINTER(PrefillAttn), vp, i64, vp]
     L.kvmix_copy_rows.restype = i32
     L.kvmix_copy_rows.argtypes = [vp, i32, vp]
+    L.kvmix_grow.restype = i32
+    L.kvmix_grow.argtypes = [vp, i32, ctypes.POINTER(KeyFlush), ctypes.POINTER(ValueFlush), vp]
     L.kvmix_probe_stream_read.restype = i32
     L.kvmix_probe_stream_read.argtypes = [vp, i32, i64, i64, i32, i32, i32, i32, i32, vp, vp]
     _lib = L

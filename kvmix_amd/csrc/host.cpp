@@ -42,6 +42,7 @@ struct Api {
     decltype(&kvmix_decode_attention_fused_weights_recommended) decode_attention_fused_weights_recommended;
     decltype(&kvmix_decode_attention_fused_weights) decode_attention_fused_weights;
     decltype(&kvmix_copy_rows) copy_rows;
+    decltype(&kvmix_grow) grow;
     decltype(&kvmix_linear_rows) linear_rows;
 } api;
 
@@ -63,6 +64,7 @@ void bind(const std::unordered_map<std::string, uintptr_t> &at)
     KVMIX_BIND(decode_attention_fused_weights_recommended);
     KVMIX_BIND(decode_attention_fused_weights);
     KVMIX_BIND(copy_rows);
+    KVMIX_BIND(grow);
     KVMIX_BIND(linear_rows);
 #undef KVMIX_BIND
 }
@@ -235,6 +237,28 @@ struct Copies {
         items.push_back(it);
     }
 
+    // rows [from_row, from_row + rows) of `from` (its last dimension `cols`) to rows [row, ..) of `out`, a fresh [B, H, ., .]
+    // tensor, from column 0 on; the caller has seen that their sizes and types match
+    void add_rows(const Tensor &out, int64_t row, const Tensor &from, int64_t from_row, int64_t rows, int64_t cols)
+    {
+        if (rows == 0 || cols == 0) return;
+        if (!first.defined()) first = out;
+        const int64_t B = from.size(0), H = from.size(1), es = from.element_size();
+        const bool ok = (cols <= 1 || from.stride(3) == 1) && (B <= 1 || H <= 1 || from.stride(0) == H * from.stride(1));
+        Tensor copied;
+        if (!ok) copied = from.narrow(2, from_row, rows).contiguous();
+        const Tensor &src = ok ? from : copied;
+        if (!ok) from_row = 0;
+        kvmix_copy_rows_t it;
+        it.src = (const char *)src.data_ptr() + from_row * src.stride(2) * es;
+        it.dst = (char *)out.data_ptr() + row * out.stride(2) * es;
+        it.outer = B * H, it.inner = rows, it.row_bytes = cols * es;
+        it.src_outer_stride = es * src.stride(H > 1 ? 1 : 0), it.src_inner_stride = es * src.stride(2);
+        it.dst_outer_stride = es * out.stride(1), it.dst_inner_stride = es * out.stride(2);
+        items.push_back(it);
+        if (!ok) keep.push_back(std::move(copied));
+    }
+
     void run()
     {
         if (items.empty()) return;
@@ -265,6 +289,39 @@ void copy_previous(const std::vector<std::pair<Tensor, Tensor>> &pairs)
     c.run();
 }
 
+// Previous parts of a grown cache that one launch moves, quantizing x to behind them (rows of 16-bit values): of the
+// expected shape and type, on x's device, in a call that nothing records.
+bool grows_in_one(const Tensor &x, const Tensor &code0, const Tensor &scale0, const Tensor &mn0, int64_t R, int64_t words, int64_t groups)
+{
+    auto takes = [&](const Tensor &t, c10::ScalarType type, int64_t cols) {
+        return t.scalar_type() == type && t.device() == x.device() && t.dim() == 4 && t.size(0) == x.size(0) && t.size(1) == x.size(1) &&
+               t.size(2) == R && t.size(3) == cols && plain(t) && Copies::fits(t);
+    };
+    return x.scalar_type() == at::kHalf && x.numel() > 0 && takes(code0, at::kInt, words) && takes(scale0, at::kHalf, groups) &&
+           takes(mn0, at::kHalf, groups);
+}
+
+// the launch: code, scale and mn are fresh; x's results go to behind `words` / `groups` columns (dim 3) or `rows` rows (dim 2)
+void grow_rows(const Tensor &x, const Tensor &code0, const Tensor &scale0, const Tensor &mn0, const Tensor &code, const Tensor &scale, const Tensor &mn,
+               int64_t group, int64_t bits, int fmt, int64_t code_at, int64_t scale_at)
+{
+    Copies c;
+    c.items.reserve(3);
+    c.add_rows(code, 0, code0, 0, code0.size(2), code0.size(3));
+    c.add_rows(scale, 0, scale0, 0, scale0.size(2), scale0.size(3));
+    c.add_rows(mn, 0, mn0, 0, mn0.size(2), mn0.size(3));
+    const Rows r = rows3(x);
+    kvmix_value_flush_t vf{};
+    vf.x = r.t.data_ptr(), vf.outer = x.size(0) * x.size(1), vf.inner = x.size(2), vf.steps = x.size(3);
+    vf.x_outer_stride = r.outer, vf.x_inner_stride = r.inner;
+    vf.group = (int)group, vf.bits = (int)bits, vf.fmt = fmt, vf.scale_mode = KVMIX_SCALE_DIVIDE;
+    vf.code = (uint32_t *)code.data_ptr() + code_at, vf.code_outer_stride = code.stride(1), vf.code_inner_stride = code.stride(2);
+    vf.scale = (char *)scale.data_ptr() + 2 * scale_at, vf.zero = (char *)mn.data_ptr() + 2 * scale_at;
+    vf.sz_outer_stride = scale.stride(1), vf.sz_inner_stride = scale.stride(2);
+    const c10::DeviceGuard guard(x.device());
+    check(api.grow(c.items.data(), (int)c.items.size(), nullptr, &vf, stream_of(x)));
+}
+
 void append_checks(const Tensor &x, const Tensor &scale, const Tensor &mn, int64_t bits)
 {
     if (x.dim() != 4) fail("input_tensor must be a 4D tensor");
@@ -289,6 +346,10 @@ Triple append_keys(const Tensor &x, const Tensor &code0, const Tensor &scale0, c
     const int64_t ow = code0.size(3), og = scale0.size(3);
     Tensor code = empty({B, H, D, ow + n / vpw}, at::kInt, x), scale = empty({B, H, D, og + n / group}, x.scalar_type(), x);
     Tensor mn = at::empty_like(scale);
+    if (grows_in_one(x, code0, scale0, mn0, D, ow, og)) {
+        grow_rows(x, code0, scale0, mn0, code, scale, mn, group, bits, KVMIX_FMT_REF, ow, og);
+        return {code, scale, mn};
+    }
     copy_previous({{code.narrow(3, 0, ow), code0}, {scale.narrow(3, 0, og), scale0}, {mn.narrow(3, 0, og), mn0}});
     if (n > 0)
         quantize_into(x, group, bits, KVMIX_FMT_REF, KVMIX_SCALE_DIVIDE, code.narrow(3, ow, n / vpw), scale.narrow(3, og, n / group),
@@ -312,6 +373,11 @@ Triple append_values(const Tensor &x, const Tensor &code0, const Tensor &scale0,
     const int64_t old = code0.size(2);
     Tensor code = empty({B, H, old + n, D / vpw}, at::kInt, x), scale = empty({B, H, old + n, D / group}, x.scalar_type(), x);
     Tensor mn = at::empty_like(scale);
+    if (grows_in_one(x, code0, scale0, mn0, old, D / vpw, D / group)) {
+        grow_rows(x, code0, scale0, mn0, code, scale, mn, group, bits, bits == 3 ? KVMIX_FMT_REF3_WRAP : KVMIX_FMT_REF, old * (D / vpw),
+                  old * (D / group));
+        return {code, scale, mn};
+    }
     copy_previous({{code.narrow(2, 0, old), code0}, {scale.narrow(2, 0, old), scale0}, {mn.narrow(2, 0, old), mn0}});
     if (n > 0)
         quantize_into(x, group, bits, bits == 3 ? KVMIX_FMT_REF3_WRAP : KVMIX_FMT_REF, KVMIX_SCALE_DIVIDE, code.narrow(2, old, n),
@@ -343,57 +409,66 @@ std::optional<Grown> grow_tuple(const OptTensor &kc, const Tensor &k_tail, const
     if (kc.has_value() != ks.has_value() || kc.has_value() != km.has_value() || vc.has_value() != vs.has_value() ||
         vc.has_value() != vm.has_value())
         return std::nullopt;
+    // the previous packed parts must be what their new tensors continue
+    auto shaped = [&](const OptTensor &t, int64_t rows, int64_t cols) {
+        return !t || (t->size(0) == B && t->size(1) == H && (rows < 0 || t->size(2) == rows) && (cols < 0 || t->size(3) == cols));
+    };
+    const bool even_k = shaped(kc, D, -1) && shaped(ks, D, -1) && shaped(km, D, -1);
+    const bool even_v = shaped(vc, -1, D * v_bits / 32) && shaped(vs, -1, D / 32) && shaped(vm, -1, D / 32);
+    if ((nk > 0 && !even_k) || (nv > 0 && !even_v)) fail("copy_rows: source and destination must be 4-D and of equal shape and type");
     Copies c;
+    c.items.reserve(10);
     auto tail = [&](const Tensor &old, const Tensor &fresh, int64_t drop) {
         const int64_t keep = old.size(2) - drop;
         Tensor out = empty({B, H, keep + n, D}, at::kHalf, key);
-        c.add(out.narrow(2, 0, keep), old.narrow(2, drop, keep));
-        c.add(out.narrow(2, keep, n), fresh);
+        c.add_rows(out, 0, old, drop, keep, D);
+        c.add_rows(out, keep, fresh, 0, n, D);
         return out;
     };
     const Tensor new_k = tail(k_tail, key, nk), new_v = tail(v_tail, value, nv);
-    auto grown = [&](const OptTensor &old, c10::ScalarType type, int64_t rows, int64_t cols, int64_t dim, Tensor &behind) {
+    // (behind: where the flush writes, the columns or rows past the old part)
+    auto grown = [&](const OptTensor &old, c10::ScalarType type, int64_t rows, int64_t cols, int64_t dim, void *&behind) {
         const int64_t have = old ? old->size(dim) : 0;
         Tensor out = dim == 3 ? empty({B, H, rows, have + cols}, type, key) : empty({B, H, have + rows, cols}, type, key);
-        if (have) c.add(out.narrow(dim, 0, have), *old);
-        behind = out.narrow(dim, have, dim == 3 ? cols : rows);
-        return OptTensor(out);
+        if (have) c.add_rows(out, 0, *old, 0, dim == 3 ? rows : have, dim == 3 ? have : cols);
+        behind = (char *)out.data_ptr() + have * (dim == 3 ? 1 : cols) * (int64_t)out.element_size();
+        return OptTensor(std::move(out));
     };
     Grown g(kc, new_k, ks, km, vc, new_v, vs, vm);
     kvmix_key_flush_t kf{};
     kvmix_value_flush_t vf{};
     kf.group = (int)k_group, kf.bits = (int)k_bits, kf.fmt = KVMIX_FMT_REF, kf.scale_mode = KVMIX_SCALE_RECIPROCAL;
     vf.group = 32, vf.bits = (int)v_bits, vf.fmt = KVMIX_FMT_REF, vf.scale_mode = KVMIX_SCALE_RECIPROCAL;
-    Tensor code, scale, zero, from_k, vcode, vscale, vzero;
+    Tensor from_k;
     Rows from_v;
+    void *behind = nullptr;
     if (nk > 0) {
-        std::get<0>(g) = grown(kc, at::kInt, D, nk / codes_per_word(k_bits), 3, code);
-        std::get<2>(g) = grown(ks, at::kHalf, D, nk / k_group, 3, scale);
-        std::get<3>(g) = grown(km, at::kHalf, D, nk / k_group, 3, zero);
+        std::get<0>(g) = grown(kc, at::kInt, D, nk / codes_per_word(k_bits), 3, behind);
+        kf.code = (uint32_t *)behind;
+        std::get<2>(g) = grown(ks, at::kHalf, D, nk / k_group, 3, kf.scale);
+        std::get<3>(g) = grown(km, at::kHalf, D, nk / k_group, 3, kf.zero);
+        const Tensor &code = *std::get<0>(g), &scale = *std::get<2>(g);
         from_k = k_tail.narrow(2, 0, nk);
         if (from_k.stride(3) != 1 || (B > 1 && from_k.stride(0) != H * from_k.stride(1))) from_k = from_k.contiguous();
         kf.k = from_k.data_ptr(), kf.outer = B * H, kf.n = nk, kf.D = D;
         kf.k_outer_stride = from_k.stride(1), kf.k_token_stride = from_k.stride(2);
-        kf.code = (uint32_t *)code.data_ptr(), kf.code_outer_stride = code.stride(1), kf.code_inner_stride = code.stride(2);
-        kf.scale = scale.data_ptr(), kf.zero = zero.data_ptr();
+        kf.code_outer_stride = code.stride(1), kf.code_inner_stride = code.stride(2);
         kf.sz_outer_stride = scale.stride(1), kf.sz_inner_stride = scale.stride(2);
     }
     if (nv > 0) {
-        std::get<4>(g) = grown(vc, at::kInt, nv, D * v_bits / 32, 2, vcode);
-        std::get<6>(g) = grown(vs, at::kHalf, nv, D / 32, 2, vscale);
-        std::get<7>(g) = grown(vm, at::kHalf, nv, D / 32, 2, vzero);
+        std::get<4>(g) = grown(vc, at::kInt, nv, D * v_bits / 32, 2, behind);
+        vf.code = (uint32_t *)behind;
+        std::get<6>(g) = grown(vs, at::kHalf, nv, D / 32, 2, vf.scale);
+        std::get<7>(g) = grown(vm, at::kHalf, nv, D / 32, 2, vf.zero);
+        const Tensor &vcode = *std::get<4>(g), &vscale = *std::get<6>(g);
         from_v = rows3(v_tail.narrow(2, 0, nv));
         vf.x = from_v.t.data_ptr(), vf.outer = B * H, vf.inner = nv, vf.steps = D;
         vf.x_outer_stride = from_v.outer, vf.x_inner_stride = from_v.inner;
-        vf.code = (uint32_t *)vcode.data_ptr(), vf.code_outer_stride = vcode.stride(1), vf.code_inner_stride = vcode.stride(2);
-        vf.scale = vscale.data_ptr(), vf.zero = vzero.data_ptr();
+        vf.code_outer_stride = vcode.stride(1), vf.code_inner_stride = vcode.stride(2);
         vf.sz_outer_stride = vscale.stride(1), vf.sz_inner_stride = vscale.stride(2);
     }
-    c.run();
-    if (nk > 0 || nv > 0) {
-        const c10::DeviceGuard guard(key.device());
-        check(api.quant_pack_kv_flush(&kf, &vf, stream_of(key)));
-    }
+    const c10::DeviceGuard guard(key.device());
+    check(api.grow(c.items.data(), (int)c.items.size(), nk > 0 ? &kf : nullptr, nv > 0 ? &vf : nullptr, stream_of(key)));
     return g;
 }
 

@@ -20,7 +20,7 @@
 //   quant_key_tokens_slab  the same for D = 128 with aligned rows: a block takes a chunk of groups of 64
 //                        channels through LDS and writes each channel row's results as contiguous pieces.
 
-#include "kvmix_common.h"
+#include "copy_rows.h"
 
 #include <vector>
 
@@ -346,9 +346,8 @@ struct __attribute__((packed, aligned(2))) Half11 {
 };
 
 template <int P, bool WRAP>
-__global__ void __launch_bounds__(256) quant_rows_ref3_f16(QuantArgs a, uint32_t words_per_row, int64_t total_words)
+__device__ __forceinline__ void rows_ref3_f16_body(const QuantArgs &a, uint32_t words_per_row, int64_t total_words, int64_t first)
 {
-    const int64_t first = (int64_t)blockIdx.x * (256 * P) + threadIdx.x;
     Half11 raw[P];
     int64_t o[P], i[P];
     uint32_t wr[P];
@@ -391,6 +390,12 @@ __global__ void __launch_bounds__(256) quant_rows_ref3_f16(QuantArgs a, uint32_t
             ((__half *)a.zero)[o[p] * a.s_os + i[p] * a.s_is + wr[p]] = __float2half_rn(mn);
         }
     }
+}
+
+template <int P, bool WRAP>
+__global__ void __launch_bounds__(256) quant_rows_ref3_f16(QuantArgs a, uint32_t words_per_row, int64_t total_words)
+{
+    rows_ref3_f16_body<P, WRAP>(a, words_per_row, total_words, (int64_t)blockIdx.x * (256 * P) + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -676,6 +681,27 @@ __global__ void __launch_bounds__(256) quant_kv_flush(FlushItem f)
 {
     __shared__ __attribute__((aligned(16))) uint16_t tile[kKeySlabTile];
     flush_block<false>(f, blockIdx.x, tile);
+}
+
+// What growing a cache by concatenation moves and what it quantizes to behind that, in one launch: nothing of either is
+// read by the other.  The quantizer's blocks come first (they are the longer chains), the copies' behind them.
+// Bound by HBM where the copies are large (both append operators on 2304 cached tokens, batch 4, 78 MB: 28.2 -> 16.1 us per
+// call, with the host's share, against copies and quantizers one after the other), by latency where everything is small
+// (a step on the 9-tuple that flushes 32 tokens onto 992, 8 kv heads: 40.5 -> 26.0 us).
+__global__ void __launch_bounds__(256) grow_kv_flush(CopyArgs c, FlushItem f)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t tile[kKeySlabTile];
+    if (blockIdx.x < f.blocks) flush_block<false>(f, blockIdx.x, tile);
+    else copy_block(c, blockIdx.x - f.blocks);
+}
+
+// ... with rows in the reference's 3-bit words
+constexpr int kGrowRef3Pieces = 2;
+__global__ void __launch_bounds__(256) grow_rows_ref3(CopyArgs c, QuantArgs a, uint32_t words_per_row, int64_t total_words, unsigned blocks)
+{
+    if (blockIdx.x < blocks)
+        rows_ref3_f16_body<kGrowRef3Pieces, false>(a, words_per_row, total_words, (int64_t)blockIdx.x * (256 * kGrowRef3Pieces) + threadIdx.x);
+    else copy_block(c, blockIdx.x - blocks);
 }
 
 // The flushes of up to kFlushBatch layers in one launch (kvmix_quant_pack_kv_flush_batch): first the key blocks of all
@@ -994,7 +1020,8 @@ struct FlushSetup {
     bool kempty, vempty, vfast, fused;
     int vpw;
 };
-static int setup_flush(const kvmix_key_flush_t *kf, const kvmix_value_flush_t *vf, FlushSetup &fs, bool batched = false)
+// either: also where only one half has something to do and that half's blocks may run beside others
+static int setup_flush(const kvmix_key_flush_t *kf, const kvmix_value_flush_t *vf, FlushSetup &fs, bool batched = false, bool either = false)
 {
     if (!kf || !vf) return KVMIX_ERR_NULL;
     FlushItem &f = fs.item;
@@ -1008,14 +1035,14 @@ static int setup_flush(const kvmix_key_flush_t *kf, const kvmix_value_flush_t *v
                         vf->code_inner_stride, vf->scale, vf->zero, vf->sz_outer_stride, vf->sz_inner_stride, f.va, fs.vpw,
                         fs.vempty, fs.vfast);
     if (rc != KVMIX_OK) return rc;  // (nothing was launched: both halves are checked first)
-    fs.fused = !(fs.kempty || fs.vempty || !fs.vfast);
+    fs.fused = either ? !(fs.kempty && fs.vempty) && (fs.vempty || fs.vfast) : !(fs.kempty || fs.vempty || !fs.vfast);
     if (!fs.fused) return KVMIX_OK;
     // key slab path: D = 128, token rows 16-byte aligned
-    f.k_tiled = key_rows_tileable(f.ka);
-    f.k_threads = f.k_groups * kf->outer * kf->D;
+    f.k_tiled = !fs.kempty && key_rows_tileable(f.ka);
+    f.k_threads = fs.kempty ? 0 : f.k_groups * kf->outer * kf->D;
     const int64_t k_blocks = f.k_tiled ? key_slab_units(f.kmode, kf->outer, f.k_groups) : (f.k_threads + 255) / 256;
-    f.v_groups_per_row = f.va.steps / 32;
-    f.v_total_groups = f.va.outer * f.va.inner * f.v_groups_per_row;
+    f.v_groups_per_row = fs.vempty ? 0 : f.va.steps / 32;
+    f.v_total_groups = fs.vempty ? 0 : f.va.outer * f.va.inner * f.v_groups_per_row;
     // A flush alone is a latency-bound launch and wants many small threads (four to a group); in a batch of layers
     // the value half is a streaming kernel and takes the prompt quantizer's form, a thread per group (measured, the
     // 32 flushes of a step in four launches: 222.8 -> 206.7 us).
@@ -1094,4 +1121,51 @@ extern "C" int kvmix_quant_pack_kv_flush_batch(const kvmix_key_flush_t *const *k
         b.count++;
     }
     return flush_launch();
+}
+
+// a value half from this many groups on streams in a launch of its own (the quantizer for large inputs)
+constexpr int64_t kGrowMaxGroups = (int64_t)64 * kRowsPieces * 2048;
+
+extern "C" int kvmix_grow(const kvmix_copy_rows_t *copies, int count, const kvmix_key_flush_t *keys, const kvmix_value_flush_t *values,
+                          kvmix_stream_t stream)
+{
+    const int chk = copy_check(copies, count);
+    if (chk != KVMIX_OK) return chk;
+    if (!keys && !values) return kvmix_copy_rows(copies, count, stream);
+    // (an absent half: nothing of it)
+    kvmix_key_flush_t no_keys{};
+    kvmix_value_flush_t no_values{};
+    no_keys.group = no_values.group = 32, no_keys.bits = no_values.bits = 4;
+    no_keys.fmt = no_values.fmt = KVMIX_FMT_REF, no_keys.scale_mode = no_values.scale_mode = KVMIX_SCALE_RECIPROCAL;
+    const kvmix_key_flush_t *kf = keys ? keys : &no_keys;
+    const kvmix_value_flush_t *vf = values ? values : &no_values;
+    FlushSetup fs;
+    const int rc = setup_flush(kf, vf, fs, false, true);
+    if (rc != KVMIX_OK) return rc;
+    hipStream_t st = (hipStream_t)stream;
+    CopyArgs c;
+    c.count = 0;
+    c.first[0] = 0;
+    int moved = 0;
+    for (int i = 0; i < count; i++) moved += copy_is_empty(copies[i]) ? 0 : 1;
+    const QuantArgs &a = fs.item.va;
+    // rows in the reference's 3-bit words (the wrapping form of the append operator is the general quantizer's)
+    const bool ref3 = fs.kempty && !fs.vempty && a.bits == 3 && a.fmt == KVMIX_FMT_REF && a.outer * a.inner * (a.steps / 11) < (1ll << 30);
+    const bool one = moved <= kCopyItems && moved > 0 && (ref3 || (fs.fused && (fs.vempty || fs.item.v_total_groups < kGrowMaxGroups)));
+    if (!one) {
+        const int crc = kvmix_copy_rows(copies, count, stream);
+        if (crc != KVMIX_OK) return crc;
+        if (fs.kempty || fs.vempty || !fs.vfast) return launch_flush_halves(kf, fs, st);
+        return kvmix_quant_pack_kv_flush(kf, vf, stream);
+    }
+    for (int i = 0; i < count; i++)
+        if (!copy_is_empty(copies[i])) copy_add(c, copies[i]);
+    if (ref3) {
+        const int64_t words = a.steps / 11, total = a.outer * a.inner * words;
+        const unsigned blocks = (unsigned)((total + 256 * kGrowRef3Pieces - 1) / (256 * kGrowRef3Pieces));
+        hipLaunchKernelGGL(grow_rows_ref3, dim3(blocks + c.first[c.count]), dim3(256), 0, st, c, a, (uint32_t)words, total, blocks);
+    } else {
+        hipLaunchKernelGGL(grow_kv_flush, dim3(fs.item.blocks + c.first[c.count]), dim3(256), 0, st, c, fs.item);
+    }
+    return launch_status();
 }
