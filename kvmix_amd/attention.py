@@ -124,6 +124,20 @@ class KVmixAttention:
         k_tail, (kc, ks, km), v_tail, (vc, vs, vm) = self._flush(k_tail, (kc, ks, km), v_tail, (vc, vs, vm))
         return kc, k_tail, ks, km, vc, v_tail, vs, vm
 
+    def _prompt_entries(self, key_states, value_states):
+        """The 9-tuple's first eight entries after a prompt (models/modeling_llama_KVmix.py:219-251): its oldest tokens
+        quantized, the rest as tails of their own."""
+        nk = flush_length(key_states.shape[2], self.k_residual_ratio, self.Kgroup_size, self.residual_length, True)
+        nv = flush_length(value_states.shape[2], self.v_residual_ratio, self.Vgroup_size, self.residual_length, True)
+        if nk > 0 and nv > 0 and self.Vgroup_size == 32 and self.v_bits != 3:
+            # (the prompt is the old tail, nothing is appended to it)
+            past = (None, key_states, None, None, None, value_states, None, None, 0)
+            grown = ops.grow_tuple(past, key_states[:, :, :0], value_states[:, :, :0], nk, nv, self.k_bits, self.Kgroup_size, self.v_bits)
+            if grown is not None:
+                return grown
+        k_tail, (kc, ks, km), v_tail, (vc, vs, vm) = self._flush(key_states, (None,) * 3, value_states, (None,) * 3, prompt=True)
+        return kc, k_tail.contiguous(), ks, km, vc, v_tail.contiguous(), vs, vm
+
     def new_cache(self, capacity: int = 4096, k_fmt: int = ops.FMT_REF, v_fmt: int = ops.FMT_REF) -> PackedKVCache:
         """An empty in-place cache with this layer's bit widths and flush policy; pass it as
         past_key_value from the prompt on (the same object comes back, updated)."""
@@ -253,9 +267,7 @@ class KVmixAttention:
                 if use_cache:
                     inplace.append(key_states, value_states, prompt=True)
             elif use_cache:
-                k_tail, (kc, ks, km), v_tail, (vc, vs, vm) = self._flush(key_states, (None,) * 3, value_states,
-                                                                         (None,) * 3, prompt=True)
-                k_tail, v_tail = k_tail.contiguous(), v_tail.contiguous()
+                kc, k_tail, ks, km, vc, v_tail, vs, vm = self._prompt_entries(key_states, value_states)
             if not need_weights and query_states.dtype == torch.float16 and query_states.is_cuda:
                 # nobody reads the probabilities: attention that never holds the [Q, Q] matrix (fp32
                 # accumulation throughout, where the composition below rounds the logits and the

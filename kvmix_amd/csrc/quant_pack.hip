@@ -714,6 +714,7 @@ constexpr int kFlushBatch = 8;
 #define KVMIX_FLUSH_STREAM_GROUPS 16384
 #endif
 constexpr int64_t kFlushStreamGroups = KVMIX_FLUSH_STREAM_GROUPS;  // value groups of a pair from which on its half streams
+constexpr int64_t kFlushStreamAlone = 1 << 18;  // ... of one pair from which on it takes the batched kernel
 struct FlushBatchArgs {
     FlushItem item[kFlushBatch];
     unsigned k_first[kFlushBatch + 1];  // first key block of item i among the launch's key blocks
@@ -1073,6 +1074,10 @@ extern "C" int kvmix_quant_pack_kv_flush(const kvmix_key_flush_t *kf, const kvmi
     if (rc != KVMIX_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
     if (!fs.fused) return launch_flush_halves(kf, fs, st);
+    // What a long prompt brings streams, as the flushes of many layers do: the batched kernel with one pair.  Measured (us,
+    // with the allocation of the results, this kernel -> the batched one): 4 x 32 heads x 1920 tokens, 4/2 bits 52.1 -> 42.7, 16 x
+    // 32 x 992, 1/1 bits 96.6 -> 73.7, 8 x 32 x 1920, 3/4 bits 111.7 -> 87.3; 1 x 32 x 3968 (508 000 groups) 30.8 -> 25.9.
+    if (fs.item.v_total_groups >= kFlushStreamAlone) return kvmix_quant_pack_kv_flush_batch(&kf, &vf, 1, stream);
     hipLaunchKernelGGL(quant_kv_flush, dim3(fs.item.blocks), dim3(256), 0, st, fs.item);
     return launch_status();
 }
@@ -1123,8 +1128,8 @@ extern "C" int kvmix_quant_pack_kv_flush_batch(const kvmix_key_flush_t *const *k
     return flush_launch();
 }
 
-// a value half from this many groups on streams in a launch of its own (the quantizer for large inputs)
-constexpr int64_t kGrowMaxGroups = (int64_t)64 * kRowsPieces * 2048;
+// a value half from this many groups on streams in a launch of its own
+constexpr int64_t kGrowMaxGroups = kFlushStreamAlone;
 
 extern "C" int kvmix_grow(const kvmix_copy_rows_t *copies, int count, const kvmix_key_flush_t *keys, const kvmix_value_flush_t *values,
                           kvmix_stream_t stream)

@@ -64,3 +64,21 @@ def test_steps_on_the_tuple(dev, B, H, D, kb, vb, rk, rv):
             if a is not None:
                 bits(a, b)
     assert (False, False) in flushed and len(flushed) >= 2
+
+
+# flush and tails in one launch and, from 2^18 value groups on, in two; nothing to flush on one side; a head dimension of 64
+@pytest.mark.parametrize("B,H,T,D,R", [(1, 4, 400, 128, 128), (2, 3, 333, 64, None), (2, 32, 1100, 128, 64), (1, 2, 129, 128, 128), (1, 1, 40, 128, 128)])
+@pytest.mark.parametrize("kb,vb", [(4, 2), (3, 4), (1, 1)])
+def test_prompts_on_the_tuple(dev, B, H, T, D, R, kb, vb):
+    from kvmix_amd.attention import KVmixAttention
+
+    gen = torch.Generator(device=dev).manual_seed(T)
+    layer = KVmixAttention(kb, vb, residual_length=R)
+    k, v = (torch.randn(B, T, H, D, generator=gen, device=dev).half().transpose(1, 2) for _ in range(2))
+    for key, value in ((k, v), (k.contiguous(), v.contiguous())):
+        kt, kq, vt, vq = layer._flush(key, (None,) * 3, value, (None,) * 3, prompt=True)
+        for a, b in zip(layer._prompt_entries(key, value), (kq[0], kt, kq[1], kq[2], vq[0], vt, vq[1], vq[2])):
+            assert (a is None) == (b is None)
+            if a is not None:
+                bits(a, b)
+                assert a.is_contiguous()
