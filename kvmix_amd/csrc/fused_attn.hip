@@ -37,7 +37,7 @@ constexpr int kSlabG32 = SlabCfg<kKeyLanes>::kSlabG32;
 constexpr int kSlabRef3 = SlabCfg<kKeyLanes>::kSlabRef3;
 
 template <int NREP>
-__global__ void __launch_bounds__(kFusedThreads) attn_fused_slab(FusedArgs a)
+__global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(4))) attn_fused_slab(FusedArgs a)
 {
     __shared__ float smem[SlabCfg<kKeyLanes>::lds_floats(NREP)];
     attn_fused_slab_body<NREP, kKeyLanes>(a, blockIdx.x, gridDim.x, threadIdx.x, smem);
@@ -58,8 +58,7 @@ __global__ void __launch_bounds__(kFusedD) attn_fused_merge(const float *ws_o, c
     // the row maximum: every thread takes a share of the slabs, then the block combines
     float M = -INFINITY;
     for (int s = c; s < slabs; s += kFusedD) M = fmaxf(M, ml[2 * s]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+    M = wave_reduce<true>(M);
     if (c % kWave == 0) part[c / kWave] = M;
     __syncthreads();
     M = fmaxf(part[0], part[1]);
@@ -103,16 +102,14 @@ __global__ void __launch_bounds__(kWeightsThreads) attn_fused_merge_weights(Fuse
 
     float M = -INFINITY;
     for (int s = tid; s < a.slabs; s += kWeightsThreads) M = fmaxf(M, ml[2 * s]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+    M = wave_reduce<true>(M);
     if (tid % kWave == 0) scratch[0][tid / kWave] = M;
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kWeightsThreads / kWave; w++) M = fmaxf(M, scratch[0][w]);
     float L = 0.f;
     for (int s = tid; s < a.slabs; s += kWeightsThreads) L = fmaf(ml[2 * s + 1], ml[2 * s] == -INFINITY ? 0.f : expf(ml[2 * s] - M), L);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) L += __shfl_xor(L, o);
+    L = wave_reduce<false>(L);
     if (tid % kWave == 0) scratch[1][tid / kWave] = L;
     __syncthreads();
     L = scratch[1][0];
@@ -120,7 +117,7 @@ __global__ void __launch_bounds__(kWeightsThreads) attn_fused_merge_weights(Fuse
     for (int w = 1; w < kWeightsThreads / kWave; w++) L += scratch[1][w];
 
     uint16_t *row = a.probs + sample * a.p_bs;
-    const float *mrow = a.mask ? a.mask + (sample / a.heads) * a.mask_bs : nullptr;
+    const float *mrow = a.mask ? a.mask + (uint32_t)sample / (uint32_t)a.heads * a.mask_bs : nullptr;
     const int64_t i0 = (int64_t)blockIdx.y * kWeightsPart + tid * 8;
     auto probability = [&](int64_t i, uint16_t logit) -> uint16_t {
         if (i >= live) return 0;

@@ -126,16 +126,28 @@ __device__ __forceinline__ int fold_lanes(float *v, int lane, int &left)
         constexpr int H = NV / 2;
         const bool up = (lane & FIRST) != 0;
 #pragma unroll
-        for (int i = 0; i < H; i++) {
-            const float keep = up ? v[H + i] : v[i];
-            const float send = up ? v[i] : v[H + i];
-            v[i] = keep + __shfl_xor(send, FIRST);
-        }
+        for (int i = 0; i < H; i++) v[i] = halving_sum<FIRST>(v[i], v[H + i], lane);
         return (up ? H : 0) + fold_lanes<H, FIRST * 2, LAST>(v, lane, left);
     } else {
 #pragma unroll
-        for (int i = 0; i < NV; i++) v[i] += __shfl_xor(v[i], FIRST);
+        for (int i = 0; i < NV; i++) v[i] = halving_sum<FIRST>(v[i], v[i], lane);
         return fold_lanes<NV, FIRST * 2, LAST>(v, lane, left);
+    }
+}
+
+// The same from bit FIRST down to LAST, over counts that stay even: most of the values meet in the cheap upper steps.
+template <int NV, int FIRST, int LAST>
+__device__ __forceinline__ int fold_lanes_down(float *v, int lane)
+{
+    if constexpr (FIRST < LAST) {
+        return 0;
+    } else {
+        constexpr int H = NV / 2;
+        static_assert(NV % 2 == 0, "an even count");
+        const bool up = (lane & FIRST) != 0;
+#pragma unroll
+        for (int i = 0; i < H; i++) v[i] = halving_sum<FIRST>(v[i], v[H + i], lane);
+        return (up ? H : 0) + fold_lanes_down<H, FIRST / 2, LAST>(v, lane);
     }
 }
 
@@ -192,15 +204,17 @@ __device__ __forceinline__ void slab_key_partials(const FusedArgs &a, int64_t kv
     }
     if (units > 0) {
         const int64_t word0 = MODE == 3 ? first / 11 : (MODE == 30 ? first / 32 * 3 : first * MODE / 32);
-        const uint32_t *codes = a.k_code + kv * a.kc_bs + word0;
-        const int64_t sz0 = kv * a.ksz_bs + first / UNIT;
+        // (a lane's first row once; the others a distance further on that is the same for all lanes)
+        const uint32_t *codes = a.k_code + kv * a.kc_bs + word0 + dg * a.kc_rs;
+        const int64_t sz0 = kv * a.ksz_bs + first / UNIT + dg * a.ksz_rs;
 #pragma unroll
-        for (int d = dg; d < kFusedD; d += 32) {
+        for (int i32 = 0; i32 < kFusedD / 32; i32++) {
+            const int d = dg + 32 * i32;
             Words<WORDS> w;
             uint16_t sc[NSZ], zr[NSZ];
-            const uint32_t *cp = codes + (int64_t)d * a.kc_rs;
-            const uint16_t *sp = a.k_scale + sz0 + (int64_t)d * a.ksz_rs;
-            const uint16_t *zp = a.k_zero + sz0 + (int64_t)d * a.ksz_rs;
+            const uint32_t *cp = codes + i32 * (32 * a.kc_rs);
+            const uint16_t *sp = a.k_scale + sz0 + i32 * (32 * a.ksz_rs);
+            const uint16_t *zp = a.k_zero + sz0 + i32 * (32 * a.ksz_rs);
             if (MODE != 3 || units == NSZ) {
                 w = *reinterpret_cast<const Words<WORDS> *>(cp);
                 if (MODE == 3) {
@@ -263,6 +277,14 @@ __device__ __forceinline__ void slab_key_partials(const FusedArgs &a, int64_t kv
     }
 }
 
+// in ? a : b without a branch around what forms them
+__device__ __forceinline__ int64_t pick(bool in, int64_t a, int64_t b)
+{
+    uint32_t lo = (uint32_t)a, hi = (uint32_t)(a >> 32);
+    asm volatile("" : "+v"(lo), "+v"(hi));
+    return (int64_t)((uint64_t)(in ? hi : (uint32_t)(b >> 32)) << 32 | (in ? lo : (uint32_t)b));
+}
+
 // acc[h][i] += sum over the slab's quantized value tokens of p[h][t] * value[t][32 * grp + i]:
 // four lanes share a token (one group of 32 head dimensions each), a block covers
 // (SlabCfg<KL>::kThreads) / 4 tokens per step.  Every load is unconditional (a token past the end is
@@ -273,19 +295,22 @@ __device__ __forceinline__ void slab_value_quant(const FusedArgs &a, int64_t kv,
 {
     constexpr int GW = MODE == 3 ? 3 : MODE;  // words per group of 32 codes
     const int grp = tid % 4, tok = tid / 4;
-    const uint32_t *codes = a.v_code + kv * a.vc_bs + grp * GW;
-    const int64_t sz = kv * a.vsz_bs + grp;
+    // (a lane's first token, and the last there is: what stands in past the end)
+    constexpr int ROWS = SlabCfg<KL>::kThreads / 4;
+    const int n = (int)(t_end - t0);
+    const int64_t code0 = kv * a.vc_bs + t0 * a.vc_rs + grp * GW, code_last = code0 + (n - 1) * a.vc_rs, code_lane = code0 + tok * a.vc_rs;
+    const int64_t sz0 = kv * a.vsz_bs + t0 * a.vsz_rs + grp, sz_last = sz0 + (n - 1) * a.vsz_rs, sz_lane = sz0 + tok * a.vsz_rs;
     float zacc[NREP];
 #pragma unroll
     for (int h = 0; h < NREP; h++) zacc[h] = 0.f;
 #pragma unroll
     for (int it = 0; it < STEPS; it++) {
-        const int at = tok + it * ((SlabCfg<KL>::kThreads) / 4);
-        const bool in = t0 + at < t_end;
-        const int64_t t = in ? t0 + at : t_end - 1;
-        const Words<GW> g = *reinterpret_cast<const Words<GW> *>(codes + t * a.vc_rs);
-        const float s = h16_to_f32(a.v_scale[sz + t * a.vsz_rs]);
-        const float z = h16_to_f32(a.v_zero[sz + t * a.vsz_rs]);
+        const int at = tok + it * ROWS;
+        const bool in = at < n;
+        const Words<GW> g = *reinterpret_cast<const Words<GW> *>(a.v_code + pick(in, code_lane + it * (ROWS * a.vc_rs), code_last));
+        const int64_t sz_at = pick(in, sz_lane + it * (ROWS * a.vsz_rs), sz_last);
+        const float s = h16_to_f32(a.v_scale[sz_at]);
+        const float z = h16_to_f32(a.v_zero[sz_at]);
 #pragma unroll
         for (int h = 0; h < NREP; h++) {
             const float ph = in ? p[h * a.slab + at] : 0.f;
@@ -303,11 +328,7 @@ __device__ __forceinline__ void slab_value_quant(const FusedArgs &a, int64_t kv,
 template <int KL>
 __device__ __forceinline__ float fused_block_reduce(float v, bool is_max, float *scratch, int tid)
 {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const float other = __shfl_xor(v, o);
-        v = is_max ? fmaxf(v, other) : v + other;
-    }
+    v = is_max ? wave_reduce<true>(v) : wave_reduce<false>(v);
     __syncthreads();  // (scratch may still be read from the previous reduction)
     if (tid % kWave == 0) scratch[tid / kWave] = v;
     __syncthreads();
@@ -317,6 +338,11 @@ __device__ __forceinline__ float fused_block_reduce(float v, bool is_max, float 
     return r;
 }
 
+// What bounds a slab of a small step is its chain of phases, each a few hundred instructions on two waves per SIMD.  64-bit
+// divisions and row addresses, lane exchanges through the LDS and a round trip to memory per 32 tail tokens made up a sixth of
+// it: single-pass steps with and without them, operands from memory, us: 32 heads, B = 4, T = 512 12.7 -> 10.9, T = 570 (3-bit
+// keys) 16.1 -> 13.9; 32 / 8 heads, B = 1, T = 1036 14.0 -> 12.0; B = 32, T = 300 28.3 -> 25.5.  (Touching what the later phases
+// read at the start, so that they find it in the L2: 1 us slower.)
 // One slab: block `launch` of `n_blocks` (slabs x head groups x kv heads), (SlabCfg<KL>::kThreads) threads (numbered
 // by `tid`), SlabCfg<KL>::lds_floats(NREP) floats of LDS at `smem`.  Every thread of the block must call it (block barriers).
 template <int NREP, int KL>
@@ -332,11 +358,13 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
     // logical order is slab-fastest, then query head, then kv head: the slabs of one row of scales
     // (neighbours share 128-byte lines) and the query heads of one kv head meet in one L2.
     // (one-dimensional numbering: slabs x head groups x kv heads blocks)
-    const int64_t per = n_blocks / 8, rem = n_blocks % 8, xcd = launch % 8;
-    const int64_t logical = xcd * per + (xcd < rem ? xcd : rem) + launch / 8;
-    const int slab = (int)(logical % a.launch_slabs);
-    const int head_group = (int)((logical / a.launch_slabs) % a.head_groups);
-    const int64_t kv = logical / ((int64_t)a.launch_slabs * a.head_groups);
+    // (32-bit: a launch has fewer than 2^31 blocks, and 64-bit divisions were a microsecond of every block)
+    const uint32_t per = (uint32_t)n_blocks / 8, rem = (uint32_t)n_blocks % 8, xcd = (uint32_t)launch % 8;
+    const uint32_t logical = xcd * per + (xcd < rem ? xcd : rem) + (uint32_t)launch / 8;
+    const uint32_t row = logical / (uint32_t)a.launch_slabs;
+    const int slab = (int)(logical - row * (uint32_t)a.launch_slabs);
+    const int head_group = (int)(row % (uint32_t)a.head_groups);
+    const int64_t kv = row / (uint32_t)a.head_groups;
     const int64_t sample0 = kv * a.heads_per_kv + (int64_t)head_group * NREP;
     const int S = a.slab;
     const int64_t t0 = a.t_begin + (int64_t)slab * S, t1 = t0 + S;
@@ -350,7 +378,7 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
     for (int i = tid; i < NREP * S; i += (SlabCfg<KL>::kThreads)) lg[i] = -INFINITY;
     __syncthreads();
 
-    const float *mrow = a.mask ? a.mask + (sample0 / a.heads) * a.mask_bs : nullptr;
+    const float *mrow = a.mask ? a.mask + (uint32_t)sample0 / (uint32_t)a.heads * a.mask_bs : nullptr;
     auto finish = [&](float dot, int64_t pos, int h) {  // fp16 logit -> scaled, masked fp32 value
         const uint16_t logit = f32_to_h16(dot);
         if (a.probs) a.probs[(sample0 + h) * a.p_bs + pos] = logit;
@@ -369,11 +397,10 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
         default: slab_key_partials<3, NREP, KL>(a, kv, t0, qs, red, tid); break;
         }
         __syncthreads();
-        const int lpp = a.k_mode == 3 ? 44 : 32;
         for (int idx = tid; idx < NREP * S; idx += (SlabCfg<KL>::kThreads)) {
-            const int h = idx / S, pos = idx % S;
+            const int h = NREP == 1 ? 0 : idx / S, pos = NREP == 1 ? idx : idx % S;
             if (t0 + pos < a.k_tokens) {
-                const int at = (pos / lpp) * (lpp + 1) + pos % lpp;
+                const int at = pos + (a.k_mode == 3 ? pos / 44 : pos / 32);  // (a pad behind a lane's positions)
                 float dot = 0.f;
 #pragma unroll
                 for (int w = 0; w < (SlabCfg<KL>::kWaves); w++) dot += red[(w * NREP + h) * (SlabCfg<KL>::kRedStride) + at];
@@ -386,24 +413,34 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
         const int sub = tid % 16, grp = tid / 16;
         const int64_t j_begin = t0 > a.k_tokens ? t0 - a.k_tokens : 0;
         const int64_t j_end = t1 - a.k_tokens < k_len ? t1 - a.k_tokens : k_len;
-        const uint16_t *kt = a.k_tail + kv * a.kt_bs + sub * 8;
-        for (int64_t j0 = j_begin; j0 < j_end; j0 += (SlabCfg<KL>::kThreads) / 16) {
-            const int64_t j = j0 + grp;
-            const bool in = j < j_end;
-            const F8 kk = *reinterpret_cast<const F8 *>(kt + (in ? j : j_begin) * a.kt_ts);
-            float dot[NREP];
+        // (four tokens of a lane group are in flight: one after the other each was a round trip to memory)
+        constexpr int GROUPS = SlabCfg<KL>::kThreads / 16, AHEAD = 4;
+        const int count = (int)(j_end - j_begin);
+        const int64_t first = kv * a.kt_bs + j_begin * a.kt_ts + sub * 8, lane_first = first + grp * a.kt_ts;
+        for (int j0 = 0; j0 < count; j0 += GROUPS * AHEAD) {
+            F8 kk[AHEAD];
 #pragma unroll
-            for (int h = 0; h < NREP; h++) {
-                dot[h] = 0.f;
+            for (int u = 0; u < AHEAD; u++)  // (the first stands in past the end)
+                kk[u] = *reinterpret_cast<const F8 *>(a.k_tail + pick(j0 + u * GROUPS + grp < count, lane_first + (j0 + u * GROUPS) * a.kt_ts, first));
 #pragma unroll
-                for (int i = 0; i < 8; i++) dot[h] = fmaf(qs[h * kFusedD + sub * 8 + i], h16_to_f32(kk.v[i]), dot[h]);
+            for (int u = 0; u < AHEAD; u++) {
+                const int j = j0 + u * GROUPS + grp;
+                float dot[NREP];
 #pragma unroll
-                for (int o = 8; o >= 1; o >>= 1) dot[h] += __shfl_xor(dot[h], o);
-            }
-            if (in && sub == 0) {
-                const int64_t pos = a.k_tokens + j;
+                for (int h = 0; h < NREP; h++) {
+                    dot[h] = 0.f;
 #pragma unroll
-                for (int h = 0; h < NREP; h++) lg[h * S + (int)(pos - t0)] = finish(dot[h], pos, h);
+                    for (int i = 0; i < 8; i++) dot[h] = fmaf(qs[h * kFusedD + sub * 8 + i], h16_to_f32(kk[u].v[i]), dot[h]);
+                    dot[h] += row_ror<8>(dot[h]);
+                    dot[h] += row_ror<4>(dot[h]);
+                    dot[h] += row_ror<2>(dot[h]);
+                    dot[h] += row_ror<1>(dot[h]);
+                }
+                if (j < count && sub == 0) {
+                    const int64_t pos = a.k_tokens + j_begin + j;
+#pragma unroll
+                    for (int h = 0; h < NREP; h++) lg[h * S + (int)(pos - t0)] = finish(dot[h], pos, h);
+                }
             }
         }
     }
@@ -478,7 +515,7 @@ __device__ __forceinline__ void attn_fused_slab_body(const FusedArgs &a, int64_t
     __syncthreads();  // (red still holds the key partials that step 1a read)
 #pragma unroll
     for (int h = 0; h < NREP; h++) {
-        const int at = scatter_reduce<32, 4, 1>(acc[h], lane);  // every lane ends with two head dimensions
+        const int at = fold_lanes_down<32, 32, 4>(acc[h], lane);  // every lane ends with two head dimensions
         red[(wave * NREP + h) * kFusedD + (lane % 4) * 32 + at] = acc[h][0];
         red[(wave * NREP + h) * kFusedD + (lane % 4) * 32 + at + 1] = acc[h][1];
     }

@@ -95,6 +95,47 @@ __device__ __forceinline__ float scale_for_output(float range, float scale_div, 
     return scale_mode == KVMIX_SCALE_RECIPROCAL ? range * inv_qmax : scale_div;
 }
 
+// v of the lane N further on in its row of sixteen (cyclically)
+template <int N>
+__device__ __forceinline__ float row_ror(float v)
+{
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, true));
+}
+
+// One halving step over the lanes that differ in bit B: the lane with the bit clear gets lo summed over the pair, its partner
+// hi.  The upper two bits by row swaps (no LDS, no selects), bit 8 by DPP.
+template <int B>
+__device__ __forceinline__ float halving_sum(float lo, float hi, int lane)
+{
+    if constexpr (B == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else if constexpr (B == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        const bool up = (lane & B) != 0;
+        const float keep = up ? hi : lo, send = up ? lo : hi;
+        if constexpr (B == 8) return keep + row_ror<8>(send);
+        else return keep + __shfl_xor(send, B);
+    }
+}
+
+// Sum or maximum over a wave, in all lanes: rows of sixteen by DPP (each step leaves a period half as long), rows by swaps.
+template <bool MAX>
+__device__ __forceinline__ float wave_reduce(float v)
+{
+    auto both = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+    v = both(v, row_ror<8>(v));
+    v = both(v, row_ror<4>(v));
+    v = both(v, row_ror<2>(v));
+    v = both(v, row_ror<1>(v));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = both(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return both(__uint_as_float(w[0]), __uint_as_float(w[1]));
+}
+
 // Halving butterfly over lanes.  v[0..NV) of every lane are summed across the lanes whose
 // indices differ in the bits {FIRST, 2*FIRST, ...} (UP = 1: up to bit 32; UP = 0: FIRST, FIRST/2,
 // ... down to bit 1).  A step halves what a lane holds: the lane with the step's bit clear
@@ -109,11 +150,7 @@ __device__ __forceinline__ int scatter_reduce(float *v, int lane)
         constexpr int H = NV / 2;
         const bool up = (lane & FIRST) != 0;
 #pragma unroll
-        for (int i = 0; i < H; i++) {
-            const float keep = up ? v[H + i] : v[i];
-            const float send = up ? v[i] : v[H + i];
-            v[i] = keep + __shfl_xor(send, FIRST);
-        }
+        for (int i = 0; i < H; i++) v[i] = halving_sum<FIRST>(v[i], v[H + i], lane);
         return (up ? H : 0) + scatter_reduce<H, UP ? FIRST * 2 : FIRST / 2, UP>(v, lane);
     }
 }

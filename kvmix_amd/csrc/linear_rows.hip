@@ -51,26 +51,6 @@ __device__ __forceinline__ float lin_rounded(float v)
     return h16_to_f32((uint16_t)bits);
 }
 
-// lanes below the middle of each pair of N-lane rows: the sum over the pair of `lo`, lanes above it: of `hi`
-__device__ __forceinline__ float halving_sum32(float lo, float hi)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-__device__ __forceinline__ float halving_sum16(float lo, float hi)
-{
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// v of the lane N further on in its row of sixteen (cyclically)
-template <int N>
-__device__ __forceinline__ float dpp_row_ror(float v)
-{
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, true));
-}
-
 // Bound by HBM and, for the small ones, by what a launch costs before its bytes count.  A block takes `pieces` outputs
 // (rows of w, or pairs of rows for the epilogues that combine two) and its eight waves slice K by 128-element chunks,
 // round-robin, so that the block reads whole contiguous rows.  A wave keeps its slice of all x rows in registers for its
@@ -211,9 +191,9 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
             // sum over the sixteen blocks (lane bits 2..5): two halving steps leave one row per lane, two plain ones finish
 #pragma unroll
             for (int g = 0; g < MG; g++) {
-                float v = halving_sum16(halving_sum32(acc[g][0], acc[g][2]), halving_sum32(acc[g][1], acc[g][3]));
-                v += dpp_row_ror<8>(v);
-                v += dpp_row_ror<4>(v);
+                float v = halving_sum<16>(halving_sum<32>(acc[g][0], acc[g][2], lane), halving_sum<32>(acc[g][1], acc[g][3], lane), lane);
+                v += row_ror<8>(v);
+                v += row_ror<4>(v);
                 if ((lane & 12) == 0)
                     part[((int64_t)(wave * RT + r) * a.pieces + 4 * t + (lane >> 5) * 2 + (lane >> 4 & 1)) * MC + g * 4 + i] = v;
             }
