@@ -50,12 +50,8 @@ constexpr int kAttnRowEntries = 16384;  // longest row the softmax keeps in regi
 template <int THREADS>
 __device__ __forceinline__ float block_reduce(float v, bool is_max, float *scratch)
 {
-    // THREADS / 64 waves; xor-shuffles inside the wave, then one value per wave through LDS
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        const float other = __shfl_xor(v, o);
-        v = is_max ? fmaxf(v, other) : v + other;
-    }
+    // THREADS / 64 waves; lane exchanges inside the wave, then one value per wave through LDS
+    v = is_max ? wave_reduce<true>(v) : wave_reduce<false>(v);
     const int wave = threadIdx.x / kWave;
     __syncthreads();  // (scratch may still be read from an earlier reduction)
     if (threadIdx.x % kWave == 0) scratch[wave] = v;
@@ -77,7 +73,7 @@ __global__ void __launch_bounds__(THREADS) attn_tail_softmax(AttnArgs a)
     constexpr int kAttnThreads = THREADS, kAttnGroups = THREADS / 16, kRowVecs = kAttnRowEntries / (THREADS * 8);
     __shared__ float scratch[kAttnThreads / kWave];
     const int64_t sample = blockIdx.x;
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int tid = threadIdx.x;
     uint16_t *row = a.probs + sample * a.p_bs;
     // (a device-side counter that ran past the window is cut to it: nothing is read out of bounds)
@@ -107,8 +103,10 @@ __global__ void __launch_bounds__(THREADS) attn_tail_softmax(AttnArgs a)
         }
 #pragma unroll
         for (int t = 0; t < kTailUnroll; t++) {
-#pragma unroll
-            for (int o = 8; o >= 1; o >>= 1) dot[t] += __shfl_xor(dot[t], o);
+            dot[t] += row_ror<8>(dot[t]);
+            dot[t] += row_ror<4>(dot[t]);
+            dot[t] += row_ror<2>(dot[t]);
+            dot[t] += row_ror<1>(dot[t]);
             const int64_t j = j0 + kAttnGroups * t + tid / 16;
             if (sub == 0 && j < a.k_slots) row[a.k_tokens + j] = j < k_len ? f32_to_h16(dot[t]) : (uint16_t)0xfc00u;  // -inf
         }
@@ -118,7 +116,7 @@ __global__ void __launch_bounds__(THREADS) attn_tail_softmax(AttnArgs a)
     __syncthreads();
 
     // 2. softmax of the row in fp32: x = fp32(logit) / sqrt(D) (+ mask, clamped to the lowest finite value)
-    const float *mrow = a.mask ? a.mask + (sample / a.heads) * a.mask_bs : nullptr;
+    const float *mrow = a.mask ? a.mask + (int64_t)((uint32_t)sample / (uint32_t)a.heads) * a.mask_bs : nullptr;
     auto value = [&](int64_t i, uint16_t h) {
         float x = h16_to_f32(h) * a.inv_sqrt_d;
         if (mrow) x = fmaxf(x + mrow[i], -3.4028234663852886e38f);
@@ -191,7 +189,7 @@ __global__ void __launch_bounds__(THREADS) attn_tail_output(AttnArgs a)
     constexpr int kAttnGroups = THREADS / 16;
     __shared__ float part[kAttnGroups][129];
     const int64_t sample = blockIdx.x;
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int tid = threadIdx.x;
     const int sub = tid % 16, grp = tid / 16;
     int64_t v_len = a.v_len_dev ? *a.v_len_dev : a.v_len;

@@ -437,13 +437,15 @@ __device__ __forceinline__ void accumulate_heads(const uint32_t *w, const float 
 constexpr int kXcds = 8;
 __device__ __forceinline__ void xcd_swizzled_block(int64_t &bx, int64_t &by, bool enable)
 {
-    const int64_t nx = gridDim.x, n = nx * (int64_t)gridDim.y;
-    const int64_t l = (int64_t)blockIdx.y * nx + blockIdx.x;
-    const int64_t xcd = l % kXcds, slot = l / kXcds;
-    const int64_t per = n / kXcds, rem = n % kXcds;
-    const int64_t j = enable ? xcd * per + (xcd < rem ? xcd : rem) + slot : l;
-    bx = j % nx;
+    // (32-bit: a launch has fewer than 2^31 blocks along x and y, since each block has outputs of its own; the 64-bit divisions
+    // were 280 scalar instructions before a block's first load)
+    const uint32_t nx = gridDim.x, n = nx * gridDim.y;
+    const uint32_t l = blockIdx.y * nx + blockIdx.x;
+    const uint32_t xcd = l % kXcds, slot = l / kXcds;
+    const uint32_t per = n / kXcds, rem = n % kXcds;
+    const uint32_t j = enable ? xcd * per + (xcd < rem ? xcd : rem) + slot : l;
     by = j / nx;
+    bx = j - (uint32_t)by * nx;
 }
 
 // LDS traffic between lanes of ONE wave: the wave's instructions execute in order, so a
@@ -497,7 +499,7 @@ __global__ void __launch_bounds__(64 * kColsWaves) gemv_cols(GemvArgs a)
     int64_t bx, sample;
     xcd_swizzled_block(bx, sample, true);
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int K = (int)a.K;
     const int nunits = (int)(a.N / VALS);
     if (nunits < TU) return;                    // (never launched so: a tile wider than the row would leave the operand)
@@ -682,7 +684,7 @@ gemv_cols3(GemvArgs a)
     xcd_swizzled_block(bx, hg, true);
     const int64_t sample0 = hg * NREP;
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample0 / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample0 / (uint32_t)a.heads_per_kv;
     const int K = (int)a.K;
     const int nunits = (int)(a.N / VALS);
     if (nunits < TU) return;  // (never launched so: a tile wider than the row would leave the operand; the same for every thread)
@@ -947,7 +949,7 @@ gemv_cols3<1, 2, 8, 4>(GemvArgs a)
     const int lane = threadIdx.x, wy = threadIdx.y;
     int64_t bx, hg;
     xcd_swizzled_block(bx, hg, true);
-    const int64_t sample0 = hg * NREP, m = blockIdx.z, kv = sample0 / a.heads_per_kv;
+    const int64_t sample0 = hg * NREP, m = blockIdx.z, kv = (uint32_t)sample0 / (uint32_t)a.heads_per_kv;
     const int K = (int)a.K, nunits = (int)(a.N / VALS);
     if (nunits < TU || K < 32) return;  // (never launched so: a tile wider than the row, fewer rows than the slices' first loads; the same for every thread)
     const uint16_t *xp = reinterpret_cast<const uint16_t *>(a.x) + sample0 * a.x_bs + m * a.x_rs;
@@ -1183,7 +1185,7 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
     xcd_swizzled_block(split, hg, a.heads_per_kv > NREP);
     const int64_t sample0 = hg * NREP;
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample0 / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample0 / (uint32_t)a.heads_per_kv;
     const int64_t kbeg = split * a.rows_per_split;
     const int64_t kend = kbeg + a.rows_per_split < a.K ? kbeg + a.rows_per_split : a.K;
 
@@ -1592,7 +1594,7 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
     split /= CS;
     const int64_t sample0 = hg * NREP;
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample0 / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample0 / (uint32_t)a.heads_per_kv;
     const int64_t kbeg = split * a.rows_per_split;
     const int64_t kend = kbeg + a.rows_per_split < a.K ? kbeg + a.rows_per_split : a.K;
 
@@ -1993,7 +1995,7 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     xcd_swizzled_block(bx, hg, true);
     const int64_t sample0 = hg * NREP;
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample0 / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample0 / (uint32_t)a.heads_per_kv;
     const int K = (int)a.K;
     const int ngroups = (int)(a.N / 32);
     // a.splits tiles per wave: tiles (bx*splits + j)*nw + wy, j = 0..splits-1 -- the block's
@@ -2230,7 +2232,7 @@ gemv_cols_mfma2(GemvArgs a)
     int64_t bx, sample;
     xcd_swizzled_block(bx, sample, true);
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int K = (int)a.K;
     const int ngroups = (int)(a.N / 32);
     // ks > 1 (small problems): ks neighbouring waves share a tile and slice its K rows
@@ -2702,7 +2704,7 @@ __device__ __forceinline__ void attn_slab_mfma_body(const AttnSlabArgs &a, int64
     uint8_t *mine = reinterpret_cast<uint8_t *>(lds) + wy * kSlabLds;
     uint16_t *atile = reinterpret_cast<uint16_t *>(mine);
     float *pbuf = reinterpret_cast<float *>(mine + kSlabKeyBytes);  // [1024] probabilities of the slab
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int ngroups = (int)(a.tokens / 32);
     const int tile = COOP ? (int)bx : (int)bx * nw + wy;
     if (ngroups < TG) return;  // (never launched so: a slab longer than the row would leave the operands)
@@ -2860,7 +2862,7 @@ __device__ __forceinline__ void attn_slab_mfma_body(const AttnSlabArgs &a, int64
         }
         wave_lds_fence();
         const int q = lane / 4;
-        const float *mrow = a.mask ? a.mask + (sample / a.heads) * a.mask_bs : nullptr;
+        const float *mrow = a.mask ? a.mask + (int64_t)((uint32_t)sample / (uint32_t)a.heads) * a.mask_bs : nullptr;
         if constexpr (COOP) {
             // every wave has the sums of its rows for all 1024 positions: they meet in LDS (the waves' pbuf areas,
             // in position order), then wave w finishes positions [256 w, 256 w + 256) as a slab of its own
@@ -2988,7 +2990,7 @@ __device__ __forceinline__ void attn_slab_ref3_body(const AttnSlabArgs &a, int64
     float *xs = reinterpret_cast<float *>(mine);                                  // [128] query * 2^90
     uint16_t *atile = reinterpret_cast<uint16_t *>(mine + K * 4);
     float *pbuf = reinterpret_cast<float *>(mine + K * 4 + kSlabRef3ABytes);      // [1408] probabilities of the slab
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int nwords = (int)(a.tokens / VALS);
     const int tile = COOP ? (int)bx : (int)bx * nw + wy;
     if (nwords < TW) return;  // (never launched so: a slab longer than the row would leave the operands)
@@ -3079,7 +3081,7 @@ __device__ __forceinline__ void attn_slab_ref3_body(const AttnSlabArgs &a, int64
         for (int u = 0; u < U; u++) compute_row(u);
 
         // the logits of this lane's 22 positions: fp16 rounding, 1/sqrt(D), mask as in the reference
-        const float *mrow = a.mask ? a.mask + (sample / a.heads) * a.mask_bs + (int64_t)w_first * VALS : nullptr;
+        const float *mrow = a.mask ? a.mask + (int64_t)((uint32_t)sample / (uint32_t)a.heads) * a.mask_bs + (int64_t)w_first * VALS : nullptr;
         if constexpr (COOP) {
             // the waves' sums over their rows meet in LDS (the waves' pbuf areas, in position order); then wave w
             // finishes three of the tile's eleven 128-position chunks as a slab of its own: chunks 3 w .. 3 w + 2,
@@ -3178,9 +3180,9 @@ attn_step_mfma(AttnSlabArgs m, fused::FusedArgs f, unsigned mfma_blocks, unsigne
     if (blockIdx.x < mfma_blocks) {
         // consecutive logical blocks on one XCD (xcd_swizzled_block, for a part of a one-dimensional grid; the XCD
         // of a block is its index in the whole launch modulo 8, and the tiles come first)
-        const int64_t n = mfma_blocks, l = blockIdx.x;
-        const int64_t xcd = l % kXcds, slot = l / kXcds, per = n / kXcds, rem = n % kXcds;
-        const int64_t j = xcd * per + (xcd < rem ? xcd : rem) + slot;
+        const uint32_t n = mfma_blocks, l = blockIdx.x;
+        const uint32_t xcd = l % kXcds, slot = l / kXcds, per = n / kXcds, rem = n % kXcds;
+        const uint32_t j = xcd * per + (xcd < rem ? xcd : rem) + slot;
         if constexpr (KBITS == 3)
             attn_slab_ref3_body<VMODE, COOP>(m, j % mfma_nx, j / mfma_nx, lds);
         else
@@ -3234,7 +3236,7 @@ __global__ void __launch_bounds__(GenericCfg<MODE>::THREADS) gemv_generic(GemvAr
     const bool live = u < units;
     const int64_t sample = blockIdx.y;
     const int64_t m = blockIdx.z;
-    const int64_t kv = sample / a.heads_per_kv;
+    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
     const int64_t grp = (u * VALS) / a.group;
     const __half *xp = a.x + sample * a.x_bs + m * a.x_rs;
     const uint32_t *cp = a.code + kv * a.c_bs + u * WORDS;

@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
         if constexpr (EPI == kEpiSwiglu) {
             return (r ? a.w1 : a.w0) + q * a.w_rs;
         } else if constexpr (EPI == kEpiRope) {
-            const int64_t head = q / a.half;
+            const int64_t head = (uint32_t)q / (uint32_t)a.half;  // (rows of 256 bytes and more: fewer than 2^31)
             int64_t row = head * 2 * a.half + (q - head * a.half) + (r ? a.half : 0);
             if (row < a.rows0) return a.w0 + row * a.w_rs;
             row -= a.rows0;
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(kLinWaves * kWave) linear_rows(LinearArgs a)
             ((uint16_t *)a.out)[m * a.out_rs + q] = f32_to_h16(act * up);
         } else {
             const int D = 2 * a.half;
-            const int64_t head = q / a.half;
+            const int64_t head = (uint32_t)q / (uint32_t)a.half;  // (rows of 256 bytes and more: fewer than 2^31)
             const int d = (int)(q - head * a.half);
             float x1 = lin_rounded(s[0]), x2 = lin_rounded(s[1]);
             const int64_t heads = a.rows0 / D, kv = a.rows1 / D;

@@ -213,11 +213,11 @@ __global__ void __launch_bounds__(kPreWaves * kWave) __attribute__((amdgpu_waves
     // after head left a last head whose long tiles ran on alone: B = 4, 32 heads, T = 2048 260 -> 239 us, a bias per distance
     // 248 -> 173.  Without a mask all blocks are alike, and the query tiles of one head after the other share more (363 against
     // 377 us).
-    const int64_t n = gridDim.x, l = blockIdx.x, xcd = l % 8, per = n / 8, rem = n % 8, heads = n / a.q_tiles, nth = l % heads;
-    const int64_t job = xcd * per + (xcd < rem ? xcd : rem) + l / 8;
-    const int qt = a.q_tiles - 1 - (int)(a.flags ? l / heads : job % a.q_tiles);
-    const int64_t bh = !a.flags ? job / a.q_tiles : heads % 8 == 0 ? nth % 8 * (heads / 8) + nth / 8 : nth;
-    const int b = (int)(bh / a.heads), head = (int)(bh % a.heads);
+    const uint32_t n = gridDim.x, l = blockIdx.x, xcd = l % 8, per = n / 8, rem = n % 8, q_tiles = a.q_tiles, heads = n / q_tiles, nth = l % heads;
+    const uint32_t job = xcd * per + (xcd < rem ? xcd : rem) + l / 8;
+    const int qt = (int)(q_tiles - 1 - (a.flags ? l / heads : job % q_tiles));
+    const uint32_t bh = !a.flags ? job / q_tiles : heads % 8 == 0 ? nth % 8 * (heads / 8) + nth / 8 : nth;
+    const int b = (int)(bh / (uint32_t)a.heads), head = (int)(bh % (uint32_t)a.heads);
     const _Float16 *kp = a.k + b * a.k_bs + (head / a.heads_per_kv) * a.k_hs;
     const _Float16 *vp = a.v + b * a.v_bs + (head / a.heads_per_kv) * a.v_hs;
     const int64_t slice = (int64_t)b * a.flag_b + (int64_t)head * a.flag_h;
