@@ -98,6 +98,7 @@ constexpr int kMfma1MaxWaves = kTargetWaves;    // one-element matrix-core q.K^T
 constexpr int kMfma2ResidentWaves = 3072;   // gemv_cols_mfma2: 3 waves on each of 1024 SIMDs
 constexpr int64_t kMfma2WideMinCodes = 6144;    // gemv_cols_mfma2: rows from this many codes on may take the wide tiles
 constexpr int64_t kMfma2WideMaxWaves = 2048;    // ... in launches of up to this many of them (one round, two waves per SIMD)
+constexpr int kColsHeadsKsplitWaves = 2048; // gemv_cols_mfma, four heads: four waves share a tile while that keeps the launch to this many waves (one resident round)
 constexpr int kMfma2KsplitWaves = 1536;     // gemv_cols_mfma2: waves share a tile (slicing K) while that keeps the launch below this many waves
 #ifndef KVMIX_ROWS_CHUNKS_PER_WAVE
 #define KVMIX_ROWS_CHUNKS_PER_WAVE 8
@@ -1518,7 +1519,7 @@ __device__ __forceinline__ constexpr int field_offset_top(int f)
 // at K = 128 from 0.65 to 1.4 times the GEMV tolerance; tests/test_gpu_gemv.py holds the case.)
 // (What the matrix cores keep of a sum of such products, and what the p.V kernels do about it: field_operand_top.)
 constexpr int rows_mfma_parts(int nrep) { return nrep > 1 ? 2 : 3; }                    // p.V: fp16 / bf16
-constexpr int cols_mfma_parts(int) { return 3; }                                        // q.K^T
+constexpr int cols_mfma_parts(int nrep) { return nrep > 1 ? 2 : 3; }                    // q.K^T: the same
 constexpr int mfma_sets(int parts, int nrep) { return (parts * nrep + 3) / 4; }
 constexpr int rows_mfma_sets(int nrep) { return mfma_sets(rows_mfma_parts(nrep), nrep); }
 constexpr int cols_mfma_sets(int nrep) { return mfma_sets(cols_mfma_parts(nrep), nrep); }
@@ -1534,15 +1535,6 @@ __device__ __forceinline__ void split_bf16_parts(float v, uint32_t *part)
     }
     static_assert(NP == 3, "the last part is exact");
     part[NP - 1] = __float_as_uint(v);
-}
-// the sum over the parts' accumulators of head h at code position p
-template <int NP, int NM, int NPOS>
-__device__ __forceinline__ float parts_sum(const f32x4_t (&acc)[NM][NPOS], int h, int p)
-{
-    float s = acc[(NP * h) / 4][p][(NP * h) % 4];
-#pragma unroll
-    for (int i = 1; i < NP; i++) s += acc[(NP * h + i) / 4][p][(NP * h + i) % 4];
-    return s;
 }
 // 2^n in both halves, -14 <= n <= 15
 __device__ __forceinline__ half2_t half_power(int n)
@@ -1963,13 +1955,19 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
 //   eight-byte cells at a pitch of 33: staging stores and operand reads are bank-conflict
 //   free).  A chunk that would cross K is moved back to end at K and its repeated rows meet
 //   x == 0 (the host gives this kernel K >= 32).  Loads rotate as in gemv_rows_mfma.
+//   Four heads: two fp16 parts after powers of two, as in gemv_rows_mfma (one per group of 32 codes, one per head), 8 A
+//   rows instead of 12 and with them two MFMAs per field instead of three.  16 x 8 kv heads, four heads each, us: 8064 tokens in 4 bits 27.0 -> 24.5, 32000 in 2 bits 94 -> 85 (issue of MFMAs and of the operands' VALU work, not
+//   memory: 3.4 and 2.3 TB/s); outputs that are not the fp16 nearest to the exact sum: 1.5 -> 1.1 of 1000.
+//   Launches of few tiles: the waves of a block share one (ksplit), each takes consecutive chunks of its rows and
+//   their sums meet in the A tiles in the order of the rows: 8 kv heads of 1024 tokens, K = 128, 13.0 -> 7.1 us (a wave
+//   walks one chunk instead of four: the launch is latency alone).
 //   The last tile of a row is shifted left to end at N (N >= 512, a multiple of 32).
 //   A wave walks `splits` tiles one after the other with the load pipeline running across
 //   them.  block = (64, 2..4) waves on neighbouring tiles; grid = (tiles/(waves*splits),
 //   samples/NREP, M), XCD-swizzled; dynamic LDS = waves * (NM tiles of kColsMfmaTile bf16 +
 //   NREP*16 floats).
 // ---------------------------------------------------------------------------------------
-constexpr int kColsMfmaTile = 16 * 33 * 4;  // bf16 elements: 16 rows of 33 four-element cells
+constexpr int kColsMfmaTile = 16 * 33 * 4;  // 2-byte elements: 16 rows of 33 four-element cells
 
 template <int BITS, int NREP>
 __global__ void __launch_bounds__(64 * kColsWaves)
@@ -1979,8 +1977,10 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     constexpr int CH = 32;             // rows per chunk
     constexpr int KB = CH / 4;         // MFMA k-steps per chunk
     constexpr int AT = kColsMfmaTile;
+    constexpr bool HALVES = NREP > 1;  // x*scale in two fp16 parts instead of three bf16 parts (see gemv_rows_mfma)
     constexpr int NP = cols_mfma_parts(NREP);
     constexpr int NM = cols_mfma_sets(NREP);
+    constexpr int TOP = HALVES ? 3 : 0;
     constexpr int NPOS = 8;
     constexpr int FPB = 8 / BITS;
     constexpr int TG = 16;             // groups per tile
@@ -2001,12 +2001,17 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     // a.splits tiles per wave: tiles (bx*splits + j)*nw + wy, j = 0..splits-1 -- the block's
     // waves sit on neighbouring tiles at any time.  A tile past N is redirected to the last
     // one (recomputed, stored twice with identical values): uniform control flow, no branches.
+    // a.ksplit > 1: the block's waves share one tile, each with some of its chunks (and there is one tile per block).
     const int tpw = a.splits;
-    const int tile0 = (int)bx * tpw * nw + wy;
+    const bool shared = a.ksplit > 1;
+    const int tile0 = shared ? (int)bx : (int)bx * tpw * nw + wy;
     if (ngroups < TG || K < CH) return;  // (never launched so: a tile wider than the row, a chunk longer than K)
-    if (tile0 * TG >= ngroups) return;  // (no block barrier below)
+    if (tile0 * TG >= ngroups) return;  // (a whole block where its waves share the tile)
     const int nch = (K + CH - 1) / CH;
-    const int items = tpw * nch;        // (tile, chunk) pairs of this wave, in order
+    // (tile, chunk) pairs of this wave, in order; a wave of a shared tile may have none
+    const int per = shared ? (nch + nw - 1) / nw : 0;
+    const int begin = shared ? (wy * per < nch ? wy * per : nch) : 0;
+    const int items = shared ? (begin + per < nch ? begin + per : nch) : tpw * nch;
 
     const uint16_t *xp = reinterpret_cast<const uint16_t *>(a.x) + sample0 * a.x_bs + m * a.x_rs;
     const Elem *cbase = reinterpret_cast<const Elem *>(a.code + kv * a.c_bs) + lane;
@@ -2017,6 +2022,12 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     const uint16_t *sbase = reinterpret_cast<const uint16_t *>(a.scale) + kv * a.s_bs + 8 * par;
     const uint16_t *zbase = reinterpret_cast<const uint16_t *>(a.zero) + kv * a.s_bs + 8 * par;
 
+    // powers of two that x (per head) and scale (per group) are multiplied by, and the largest values they are good for:
+    // two halves each, x_limit of one head, s_limit of two of the groups that the lane stages
+    int x_pow[NREP], own_pow;  // own_pow: of the scales of the group whose outputs this lane holds
+    uint32_t x_limit[NREP], s_limit[4];
+#pragma unroll
+    for (int h = 0; h < NREP; h++) x_pow[h] = 3, x_limit[h] = ((19 << 10) - 1) * 0x00010001u;  // |x| < 16
     f32x4_t acc[NM][NPOS];
     float zacc[NREP][8];
     auto clear = [&]() {
@@ -2030,6 +2041,9 @@ __global__ void __launch_bounds__(64 * kColsWaves)
 #pragma unroll
             for (int j = 0; j < 8; j++) zacc[h][j] = 0.f;
         }
+        own_pow = 5;  // (a tile's groups owe nothing to those of the tile before)
+#pragma unroll
+        for (int g = 0; g < 4; g++) s_limit[g] = ((18 << 10) - 1) * 0x00010001u;  // |scale| < 8
     };
     clear();
 
@@ -2065,6 +2079,72 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     auto stage = [&](int it) {
         const int k0 = chunk_k0(it);
         const int skip = k0 - chunk_base(k0);  // rows of this chunk that an earlier one covered
+        if constexpr (HALVES) {
+            uint32_t x2[NREP], s2[4], over = 0;
+            __builtin_memcpy(s2, &s8, 16);
+            auto excess = [&](uint32_t v, uint32_t limit) {
+                over |= __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(ushort2_t, v & 0x7fff7fffu),
+                                                                                   __builtin_bit_cast(ushort2_t, limit)));
+            };
+#pragma unroll
+            for (int h = 0; h < NREP; h++) {
+                x2[h] = srow >= skip ? xh[h] * 0x00010001u : 0u;
+                excess(x2[h], x_limit[h]);
+            }
+#pragma unroll
+            for (int g = 0; g < 4; g++) excess(s2[g], s_limit[g]);
+            if (__builtin_expect(__ballot(over != 0) != 0, 0)) {  // larger than the scaling allows: smaller powers from here on
+                auto exponent = [&](uint32_t v, int apart) {  // of the largest fp16 value among every apart-th lane's
+                    v &= 0x7fffu;
+                    for (int o = apart; o < kWave; o *= 2) v = max(v, (uint32_t)__shfl_xor((int)v, o));
+                    return (int)(v >> 10);
+                };
+                const int had = own_pow;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int sh = 16 * (j % 2);
+                    const int sb = min(22 - (int)((s_limit[j / 2] >> sh & 0xffffu) >> 10), 22 - exponent(s2[j / 2] >> sh, 2));
+                    s_limit[j / 2] = (s_limit[j / 2] & ~(0xffffu << sh)) | (uint32_t)(((23 - sb) << 10) - 1) << sh;
+                    const int of_group = __shfl(sb, lane / 32);  // (lane 0 stages groups 0..7, lane 1 groups 8..15)
+                    if (lane / 4 % 8 == j) own_pow = of_group;
+                }
+#pragma unroll
+                for (int h = 0; h < NREP; h++) {
+                    const int xb = min(x_pow[h], 21 - (int)__builtin_amdgcn_readfirstlane(exponent(x2[h], 1)));
+                    const float f = ldexpf(1.0f, xb - x_pow[h] + own_pow - had);
+#pragma unroll
+                    for (int i = 0; i < NP; i++) {
+#pragma unroll
+                        for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
+                    }
+                    x_pow[h] = xb;
+                    x_limit[h] = (((22 - xb) << 10) - 1) * 0x00010001u;
+                }
+            }
+            half2_t ss[4];
+#pragma unroll
+            for (int g = 0; g < 4; g++) ss[g] = __builtin_bit_cast(half2_t, s2[g]) * __builtin_bit_cast(half2_t, 0x97ff97ffu - s_limit[g]);  // 2^n: (n + 15) << 10, and the limit is ((23 - n) << 10) - 1
+#pragma unroll
+            for (int h = 0; h < NREP; h++) {
+                const half2_t x = __builtin_bit_cast(half2_t, x2[h]), xs = x * half_power(x_pow[h]);
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const half2_t hi = xs * ss[g], lo = __builtin_elementwise_fma(xs, ss[g], -hi);
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const int j = 2 * g + e;
+                        zacc[h][j] = fmaf((float)x[e], h16_to_f32(z8.v[j]), zacc[h][j]);
+                        // A rows h (first part) and NREP + h (second): MFMA row / 4, lanes 4j + row % 4
+#pragma unroll
+                        for (int i = 0; i < NP; i++) {
+                            const int ar = NREP * i + h;
+                            atile[(ar / 4) * AT + aoff + (4 * j + ar % 4) * 4] = __builtin_bit_cast(uint16_t, i ? lo[e] : hi[e]);
+                        }
+                    }
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int h = 0; h < NREP; h++) {
             const float xv = srow >= skip ? h16_to_f32(xh[h]) : 0.f;
@@ -2072,8 +2152,8 @@ __global__ void __launch_bounds__(64 * kColsWaves)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 zacc[h][j] = fmaf(xv, h16_to_f32(z8.v[j]), zacc[h][j]);
-                uint32_t part[NP];
-                split_bf16_parts<NP>(x2 * h16_to_f32(s8.v[j]), part);  // (three parts: exact)
+                uint32_t part[3];
+                split_bf16_parts<3>(x2 * h16_to_f32(s8.v[j]), part);  // (three parts: exact)
 #pragma unroll
                 for (int pt = 0; pt < NP; pt++) {  // A row NP*h+pt: MFMA (NP*h+pt)/4, lanes 4g + (NP*h+pt)%4
                     const int ar = NP * h + pt;
@@ -2083,9 +2163,9 @@ __global__ void __launch_bounds__(64 * kColsWaves)
         }
     };
     auto compute = [&](int t) {
-        bf16x4_t av[NM];
+        uint2 av[NM];
 #pragma unroll
-        for (int q = 0; q < NM; q++) av[q] = *reinterpret_cast<const bf16x4_t *>(atile + q * AT + cell(t, lane));
+        for (int q = 0; q < NM; q++) av[q] = *reinterpret_cast<const uint2 *>(atile + q * AT + cell(t, lane));
 #pragma unroll
         for (int b = 0; b < BITS; b++) {
             const uint32_t sel = 0x0c000c00u | (uint32_t)b | ((uint32_t)(4 + b) << 16);
@@ -2093,12 +2173,17 @@ __global__ void __launch_bounds__(64 * kColsWaves)
             const uint32_t t23 = __builtin_amdgcn_perm((uint32_t)w[t][3], (uint32_t)w[t][2], sel);
 #pragma unroll
             for (int f = 0; f < FPB; f++) {
-                const bf16x4_t bv =
-                    __builtin_bit_cast(bf16x4_t, make_uint2(field_operand<BITS>(t01, f), field_operand<BITS>(t23, f)));
+                const uint2 bv = HALVES ? make_uint2(field_alone_top<BITS, TOP>(t01, f), field_alone_top<BITS, TOP>(t23, f))
+                                        : make_uint2(field_operand<BITS>(t01, f), field_operand<BITS>(t23, f));
 #pragma unroll
-                for (int q = 0; q < NM; q++)
-                    acc[q][b * FPB + f] =
-                        __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(av[q], bv, acc[q][b * FPB + f], 0, 0, 0);
+                for (int q = 0; q < NM; q++) {
+                    if constexpr (HALVES)
+                        acc[q][b * FPB + f] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, av[q]), __builtin_bit_cast(half4_t, bv),
+                                                                                 acc[q][b * FPB + f], 0, 0, 0);
+                    else
+                        acc[q][b * FPB + f] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(bf16x4_t, av[q]), __builtin_bit_cast(bf16x4_t, bv),
+                                                                                     acc[q][b * FPB + f], 0, 0, 0);
+                }
             }
         }
     };
@@ -2123,14 +2208,27 @@ __global__ void __launch_bounds__(64 * kColsWaves)
         for (int h = 0; h < NREP; h++) {
             const float zt = zl[h * TG + lane / 4];
             Out8 o;
-            float sums[NPOS];
-#pragma unroll
-            for (int p = 0; p < NPOS; p++)
-                sums[p] = parts_sum<NP>(acc, h, p);
+            float sums[NPOS], value[NPOS];
 #pragma unroll
             for (int p = 0; p < NPOS; p++) {
-                const float sum = field_sum(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
-                o.v[p] = f32_to_h16(fmaf(sum, __uint_as_float((uint32_t)(127 + 43 - BITS * (p % FPB)) << 23), zt));
+                sums[p] = acc[h / 4][p][h % 4];
+#pragma unroll
+                for (int i = 1; i < NP; i++) sums[p] += acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4];
+            }
+#pragma unroll
+            for (int p = 0; p < NPOS; p++) {
+                if constexpr (HALVES) {
+                    value[p] = ldexpf(sums[p], 24 - TOP - field_offset_top<BITS>(p % FPB) - x_pow[h] - own_pow) + zt;
+                } else {
+                    const float sum = field_sum(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
+                    value[p] = fmaf(sum, __uint_as_float((uint32_t)(127 + 43 - BITS * (p % FPB)) << 23), zt);
+                }
+                o.v[p] = f32_to_h16(value[p]);
+            }
+            if (shared) {  // (over the wave's own A tile, which it has read)
+#pragma unroll
+                for (int p = 0; p < NPOS; p++) reinterpret_cast<float *>(atile)[(h * NPOS + p) * kWave + lane] = value[p];
+                continue;
             }
             uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + (sample0 + h) * a.o_bs + m * a.o_rs + col;
             *reinterpret_cast<Out8 *>(op) = o;
@@ -2139,20 +2237,22 @@ __global__ void __launch_bounds__(64 * kColsWaves)
         clear();
     };
 
-    load_small(0);
+    load_small(begin < items ? begin : nch - 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < KB; t++) {
-        load_codes(0, t);
+        load_codes(begin < items ? begin : nch - 1, t);
         __builtin_amdgcn_sched_barrier(0);
     }
-    // some A rows are never written: clear the tile once -- behind the first loads, whose latency
+    // three parts leave A rows that are never written: clear the tile once -- behind the first loads, whose latency
     // covers it (every wave of a launch starts at the same time)
-    for (int i = lane; i < NM * AT / 2; i += kWave) reinterpret_cast<uint32_t *>(atile)[i] = 0u;
+    if constexpr (!HALVES) {
+        for (int i = lane; i < NM * AT / 2; i += kWave) reinterpret_cast<uint32_t *>(atile)[i] = 0u;
+    }
     wave_lds_fence();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
-    for (int it = 0; it < items; it++) {
+    for (int it = begin; it < items; it++) {
         const int nx = it + 1 < items ? it + 1 : it;  // (past the end: the same item again)
         stage(it);
         wave_lds_fence();
@@ -2165,7 +2265,24 @@ __global__ void __launch_bounds__(64 * kColsWaves)
             __builtin_amdgcn_sched_barrier(0);
         }
         wave_lds_fence();  // the next chunk overwrites the tile
-        if (it % nch == nch - 1) finish_tile(it);
+        if (!shared && it % nch == nch - 1) finish_tile(it);
+    }
+    if (!shared) return;
+    // the waves' sums meet: a wave takes every nw-th head (and output), in the order of the chunks
+    finish_tile(0);
+    __syncthreads();
+    constexpr int PITCH = NM * AT + NREP * TG * 2;  // halves between two waves' tiles
+    const int64_t col = (int64_t)tile_g0(0) * 32 + lane * 8;
+    for (int h = wy; h < NREP; h += nw) {
+        Out8 o;
+#pragma unroll
+        for (int p = 0; p < NPOS; p++) {
+            float v = 0.f;
+            for (int ww = 0; ww < nw; ww++)
+                v += reinterpret_cast<const float *>(reinterpret_cast<uint16_t *>(lds) + ww * PITCH)[(h * NPOS + p) * kWave + lane];
+            o.v[p] = f32_to_h16(v);
+        }
+        *reinterpret_cast<Out8 *>(reinterpret_cast<uint16_t *>(a.out) + (sample0 + h) * a.o_bs + m * a.o_rs + col) = o;
     }
 }
 
@@ -3586,10 +3703,22 @@ static void launch_cols_mfma(GemvArgs &a, int64_t samples, hipStream_t st)
     int64_t tpw = batch * tiles / target;
     tpw = tpw < 1 ? 1 : (tpw > 8 ? 8 : tpw);
     const int64_t slots = (tiles + tpw - 1) / tpw;  // waves per output row
-    const int wpb = pick_waves_per_block(slots);
+    const size_t lds_wave = cols_mfma_sets(NREP) * kColsMfmaTile * sizeof(uint16_t) + NREP * 16 * sizeof(float);
     a.splits = (int)tpw;
+    // Few tiles: the waves of a block share one.  Four heads of a kv head, K = 128, us: 8 kv heads of 1024 tokens 11.3 with
+    // a wave per tile, 9.7 with two, 7.7 with four; 32 of 8064 (512 tiles: the most the rule takes) 13.1, 13.9, 12.8; 128
+    // of 8064 24.0, 36, 42.  (Two waves are never better than both others.)
+    const int64_t chunks = (a.K + 31) / 32;
+    a.ksplit = NREP > 1 && chunks > 1 && batch * tiles * kColsWaves <= kColsHeadsKsplitWaves ? (int)(chunks < kColsWaves ? chunks : kColsWaves) : 1;
+    if (a.ksplit > 1) {
+        a.splits = 1;
+        const dim3 grid((unsigned)tiles, (unsigned)(samples / NREP), (unsigned)a.M);
+        KVMIX_LAUNCH((gemv_cols_mfma<BITS, NREP>), grid, dim3(kWave, a.ksplit), a.ksplit * lds_wave, st, a, "gemv_cols_mfma<%d,%d>", BITS, NREP);
+        return;
+    }
+    const int wpb = pick_waves_per_block(slots);
     const dim3 grid((unsigned)((slots + wpb - 1) / wpb), (unsigned)(samples / NREP), (unsigned)a.M);
-    const size_t lds = (size_t)wpb * (cols_mfma_sets(NREP) * kColsMfmaTile * sizeof(uint16_t) + NREP * 16 * sizeof(float));
+    const size_t lds = (size_t)wpb * lds_wave;
     KVMIX_LAUNCH((gemv_cols_mfma<BITS, NREP>), grid, dim3(kWave, wpb), lds, st, a, "gemv_cols_mfma<%d,%d>", BITS, NREP);
 }
 
