@@ -1956,16 +1956,17 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
 //   free).  A chunk that would cross K is moved back to end at K and its repeated rows meet
 //   x == 0 (the host gives this kernel K >= 32).  Loads rotate as in gemv_rows_mfma.
 //   Four heads: two fp16 parts after powers of two, as in gemv_rows_mfma (one per group of 32 codes, one per head), 8 A
-//   rows instead of 12 and with them two MFMAs per field instead of three.  16 x 8 kv heads, four heads each, us: 8064 tokens in 4 bits 27.0 -> 24.5, 32000 in 2 bits 94 -> 85 (issue of MFMAs and of the operands' VALU work, not
-//   memory: 3.4 and 2.3 TB/s); outputs that are not the fp16 nearest to the exact sum: 1.5 -> 1.1 of 1000.
+//   rows instead of 12 and with them two MFMAs per field instead of three.  16 x 8 kv heads, four heads each, us: 8064
+//   tokens in 4 bits 27.0 -> 24.5, 32000 in 2 bits 94 -> 85 (issue of MFMAs and of the operands' VALU work, not memory:
+//   3.4 and 2.3 TB/s); outputs that are not the fp16 nearest to the exact sum: 1.5 -> 1.1 of 1000.
 //   Launches of few tiles: the waves of a block share one (ksplit), each takes consecutive chunks of its rows and
 //   their sums meet in the A tiles in the order of the rows: 8 kv heads of 1024 tokens, K = 128, 13.0 -> 7.1 us (a wave
 //   walks one chunk instead of four: the launch is latency alone).
 //   The last tile of a row is shifted left to end at N (N >= 512, a multiple of 32).
 //   A wave walks `splits` tiles one after the other with the load pipeline running across
 //   them.  block = (64, 2..4) waves on neighbouring tiles; grid = (tiles/(waves*splits),
-//   samples/NREP, M), XCD-swizzled; dynamic LDS = waves * (NM tiles of kColsMfmaTile bf16 +
-//   NREP*16 floats).
+//   samples/NREP, M), XCD-swizzled; dynamic LDS = waves * (NM tiles of kColsMfmaTile elements
+//   + NREP*16 floats).  Shared tiles: grid = (tiles, samples/NREP, M), block = (64, ksplit).
 // ---------------------------------------------------------------------------------------
 constexpr int kColsMfmaTile = 16 * 33 * 4;  // 2-byte elements: 16 rows of 33 four-element cells
 
