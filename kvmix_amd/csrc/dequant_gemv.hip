@@ -91,7 +91,7 @@ constexpr int kCols3HeadsOcc = KVMIX_COLS3_HEADS_OCC;   // waves per SIMD the co
 #define KVMIX_MFMA_HEADS_OCC 2
 #endif
 constexpr int kMfmaHeadsOcc = KVMIX_MFMA_HEADS_OCC;   // ... gemv_rows_mfma / gemv_cols_mfma, four heads
-constexpr int kMfma2Occ = 2;                // ... gemv_cols_mfma2 (at least; it comes out at three)
+constexpr int kMfma2Occ = 2;                // ... gemv_cols_mfma2 (at least; it comes out at three; plain tiles of 1 bit fit four)
 constexpr int kHeadsWaveDiv = 2;            // p.V, four heads per pass: half as many waves wanted
 constexpr int kMfma2MaxWaves = kTargetWaves;    // two-element matrix-core q.K^T kernel up to this many tiles
 constexpr int kMfma1MaxWaves = kTargetWaves;    // one-element matrix-core q.K^T kernel (one head) below this many tiles
@@ -436,17 +436,20 @@ __device__ __forceinline__ void accumulate_heads(const uint32_t *w, const float 
 // one cache row (they share the 128-byte lines that straddle tile borders) and query heads
 // of one kv head (they read the same packed data) then meet in one L2.
 constexpr int kXcds = 8;
+template <typename Index = uint32_t>
 __device__ __forceinline__ void xcd_swizzled_block(int64_t &bx, int64_t &by, bool enable)
 {
     // (32-bit: a launch has fewer than 2^31 blocks along x and y, since each block has outputs of its own; the 64-bit divisions
-    // were 280 scalar instructions before a block's first load)
-    const uint32_t nx = gridDim.x, n = nx * gridDim.y;
-    const uint32_t l = blockIdx.y * nx + blockIdx.x;
-    const uint32_t xcd = l % kXcds, slot = l / kXcds;
-    const uint32_t per = n / kXcds, rem = n % kXcds;
-    const uint32_t j = enable ? xcd * per + (xcd < rem ? xcd : rem) + slot : l;
-    by = j / nx;
-    bx = j - (uint32_t)by * nx;
+    // were 280 scalar instructions before a block's first load.  gemv_cols and gemv_rows keep them: without, the compiler
+    // gives their load loops up to 20 registers more, and some lose the fourth wave per SIMD.)
+    const Index nx = gridDim.x, n = nx * (Index)gridDim.y;
+    const Index l = (Index)blockIdx.y * nx + blockIdx.x;
+    const Index xcd = l % kXcds, slot = l / kXcds;
+    const Index per = n / kXcds, rem = n % kXcds;
+    const Index j = enable ? xcd * per + (xcd < rem ? xcd : rem) + slot : l;
+    const Index y = j / nx;
+    by = y;
+    bx = j - y * nx;
 }
 
 // LDS traffic between lanes of ONE wave: the wave's instructions execute in order, so a
@@ -498,9 +501,9 @@ __global__ void __launch_bounds__(64 * kColsWaves) gemv_cols(GemvArgs a)
     const int rq = lane / GL;
     const int gl = lane % GL;
     int64_t bx, sample;
-    xcd_swizzled_block(bx, sample, true);
+    xcd_swizzled_block<int64_t>(bx, sample, true);
     const int64_t m = blockIdx.z;
-    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
+    const int64_t kv = sample / a.heads_per_kv;
     const int K = (int)a.K;
     const int nunits = (int)(a.N / VALS);
     if (nunits < TU) return;                    // (never launched so: a tile wider than the row would leave the operand)
@@ -1183,10 +1186,10 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
     // (measured: with one query head per kv head nothing is shared between blocks and the
     // launch order is 3 us faster at B=16, T=8k; with GQA the heads of a kv head want one L2)
     int64_t split, hg;
-    xcd_swizzled_block(split, hg, a.heads_per_kv > NREP);
+    xcd_swizzled_block<int64_t>(split, hg, a.heads_per_kv > NREP);
     const int64_t sample0 = hg * NREP;
     const int64_t m = blockIdx.z;
-    const int64_t kv = (uint32_t)sample0 / (uint32_t)a.heads_per_kv;
+    const int64_t kv = sample0 / a.heads_per_kv;
     const int64_t kbeg = split * a.rows_per_split;
     const int64_t kend = kbeg + a.rows_per_split < a.K ? kbeg + a.rows_per_split : a.K;
 
@@ -2322,7 +2325,7 @@ constexpr size_t cols_mfma2_lds(bool wide)  // bytes per wave: the A tile + the 
 // NTC: the codes are loaded non-temporally (the host asks for it while the launch is no more than a few rounds of
 // resident waves: measured faster up to 8k waves, slower at 16k, where rows of neighbouring tiles meet in the L2)
 template <int BITS, bool NTC, bool WIDE>
-__global__ void __launch_bounds__(64 * kColsWaves) __attribute__((amdgpu_waves_per_eu(kMfma2Occ)))
+__global__ void __launch_bounds__(64 * kColsWaves) __attribute__((amdgpu_waves_per_eu(BITS == 1 && !WIDE ? 4 : kMfma2Occ)))
 gemv_cols_mfma2(GemvArgs a)
 {
     static_assert(BITS == 4 || BITS == 2 || BITS == 1, "per sub-piece a dword (4, 2 bits) or a ushort (1 bit) per lane");
@@ -3354,7 +3357,7 @@ __global__ void __launch_bounds__(GenericCfg<MODE>::THREADS) gemv_generic(GemvAr
     const bool live = u < units;
     const int64_t sample = blockIdx.y;
     const int64_t m = blockIdx.z;
-    const int64_t kv = (uint32_t)sample / (uint32_t)a.heads_per_kv;
+    const int64_t kv = sample / a.heads_per_kv;
     const int64_t grp = (u * VALS) / a.group;
     const __half *xp = a.x + sample * a.x_bs + m * a.x_rs;
     const uint32_t *cp = a.code + kv * a.c_bs + u * WORDS;

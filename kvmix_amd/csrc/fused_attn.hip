@@ -469,9 +469,9 @@ extern "C" int kvmix_decode_attention_fused_weights(const kvmix_decode_attn_t *p
 
 // Which form of a step with probabilities is faster (operands from memory, four launches -> slabs, us): the slabs up to 450 000
 // (query head x position) entries, 300 000 with the reference's 3-bit keys, which the slabs take as vector arithmetic
-// throughout.  33 000 entries (1 x 1036, 32 / 8 heads, 4 bits) 31.1 -> 16.2; 128 000 (1 x 4000, 4 bits) 28.2 -> 18.2;
-// 256 000: 1 x 8000, 2 bits 29.0 -> 20.9, 1 x 8000, 32 / 8 heads, 4 bits 37.3 -> 20.0, 4 x 2000, 3-bit keys 29.2 -> 25.5; 307 000
-// (32 x 300) 49.0 -> 34.3; level at 512 000: 4 x 4000, 2 bits 34.6 -> 34.2, 8 x 2000, 32 / 8 heads 35.7 -> 35.2.
+// throughout.  256 000 entries: 1 x 8000, 2 bits 26.4 -> 17.5; 1 x 8000, 32 / 8 heads, 4 bits 27.9 -> 17.2; 4 x 2000, 3-bit keys
+// 30.3 -> 25.1; 333 000: 4 x 2600, 4 bits 33.4 -> 26.9, 2 bits, 32 / 8 heads 29.0 -> 22.7; 410 000: 8 x 1600, 32 / 8 heads 25.7 -> 26.2;
+// 435 000: 4 x 3400, 2 bits 31.4 -> 28.6, 4 bits, 32 / 8 heads 30.5 -> 26.8; level at 512 000: 4 x 4000, 2 bits 34.6 -> 34.2.
 constexpr int64_t kSmallWeightsEntries = 450000, kSmallWeightsEntriesRef3 = 300000;
 extern "C" int kvmix_decode_attention_fused_weights_recommended(const kvmix_decode_attn_t *p)
 {
