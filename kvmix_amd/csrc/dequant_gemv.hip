@@ -1385,9 +1385,11 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 //           rounded, lo = fma(x, scale, -hi), together exact as long as lo does not reach below fp16's smallest step.
 //           For that x and scale are first multiplied by powers of two, one per head and one per group, that put
 //           x below 2^7 and scale below 2^8: a product is then off by at most 2^-25 where the largest of its
-//           (head, group) may be 2^15.  They start where probabilities and ordinary scales need them (x < 2,
-//           scale < 8: an error of 2^-36 per product) and are lowered, with the sums so far, when a chunk holds
-//           something larger.  Against the three bf16 parts (12 rows, three MFMAs per B operand) this is 8
+//           (head, group) is 2^9 to 2^15.  The powers follow the data (kPartsTop): powers good for x < 2 and scale < 8
+//           that stay there unless something is larger leave every product off by 2^-36, which for the flat rows of a long
+//           context over small values (T = 32000, 4 bits, values of deviation 0.03 / 0.01) is 66 / 121 of 1000
+//           outputs off the nearest fp16, where three exact parts leave 8.0 / 4.2 and this 8.3 / 4.9.
+//           Against the three bf16 parts (12 rows, three MFMAs per B operand) this is 8
 //           rows, two MFMAs, a third of the LDS stores and a fifth of the arithmetic of forming them.
 //           The (part, head) rows are packed four to an MFMA; unused rows are zero.
 //           Measured, four query heads per kv head, operands from memory, bf16 -> fp16 parts (and blocks of
@@ -1516,8 +1518,8 @@ __device__ __forceinline__ constexpr int field_offset_top(int f)
     return BITS * f + field_shift<BITS>(f);
 }
 
-// parts of x*scale.  p.V with one query head and q.K^T: three bf16 (24 significant bits hold the product of two fp16
-// exactly).  p.V with four heads per pass: two fp16.  (Two bf16 parts, the second rounded to nearest, leave every product
+// parts of x*scale.  One query head: three bf16 (24 significant bits hold the product of two fp16 exactly).  Four heads
+// per pass: two fp16.  (Two bf16 parts, the second rounded to nearest, leave every product
 // off by up to 2^-17 of itself: where the code term and the zero term of an output nearly cancel that took a 4-bit case
 // at K = 128 from 0.65 to 1.4 times the GEMV tolerance; tests/test_gpu_gemv.py holds the case.)
 // (What the matrix cores keep of a sum of such products, and what the p.V kernels do about it: field_operand_top.)
@@ -1546,6 +1548,38 @@ __device__ __forceinline__ half2_t half_power(int n)
 }
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef uint16_t ushort2_t __attribute__((ext_vector_type(2)));
+
+// The powers of two 2^n that x and scale are multiplied by before they are split into fp16 parts, and the largest magnitude
+// (two halves of it) each is good for.  They follow the data: all start at 2^15, where a product is off by 2^-55 at most (2^25
+// of them with codes of 15 do not show in the smallest fp16), and the first value that a power is too large for takes it
+// down to that value's own size.  The first chunk does as a rule; a later one only when it holds something kPartsRoom binades
+// larger.  So a product is off by at most 2^-34 of what the largest x of its head and the largest scale of its group make.
+constexpr int kPartsTop = 15, kPartsXBelow = 7, kPartsSBelow = 8;  // x * 2^n < 2^7, scale * 2^n < 2^8
+constexpr int kPartsRoom = 2;
+__device__ __forceinline__ uint32_t parts_limit(int n, int below) { return (uint32_t)(((15 + below - n) << 10) - 1) * 0x00010001u; }
+// n for values of at most `largest` (an fp16 magnitude): with room for larger ones where that does not cost small ones bits
+__device__ __forceinline__ int parts_power(int n, uint32_t largest, int below)
+{
+    const int fits = 14 + below - (int)(largest >> 10);
+    return n <= fits ? n : max(fits - kPartsRoom, min(fits, 0));
+}
+__device__ __forceinline__ uint32_t max_halves(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushort2_t, a), __builtin_bit_cast(ushort2_t, b)));
+}
+// the maximum of each half over the lanes that differ in bits FROM and up, in all of them
+template <int FROM>
+__device__ __forceinline__ uint32_t wave_max_halves(uint32_t v)
+{
+    v = max_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true));
+    v = max_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, true));
+    v = max_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, true));
+    if constexpr (FROM == 1) v = max_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, true));
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max_halves(r[0], r[1]);
+    const auto w = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return max_halves(w[0], w[1]);
+}
 constexpr int kRowsMfmaTile = (32 * 17 + 1) * 4 + 4;  // bf16 elements of one A tile (32 skewed rows), 8-byte multiple
 
 constexpr int kRowsMfmaWaves = 16;      // waves per block at most (register budget of 128 per lane)
@@ -1607,9 +1641,9 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
     int x_pow[NREP], s_pow[LPR];
     uint32_t x_limit[NREP], s_limit[LPR];
 #pragma unroll
-    for (int h = 0; h < NREP; h++) x_pow[h] = 6, x_limit[h] = ((16 << 10) - 1) * 0x00010001u;  // |x| < 2: probabilities
+    for (int h = 0; h < NREP; h++) x_pow[h] = kPartsTop, x_limit[h] = parts_limit(kPartsTop, kPartsXBelow);
 #pragma unroll
-    for (int g = 0; g < LPR; g++) s_pow[g] = 5, s_limit[g] = ((18 << 10) - 1) * 0x00010001u;  // |scale| < 8
+    for (int g = 0; g < LPR; g++) s_pow[g] = kPartsTop, s_limit[g] = parts_limit(kPartsTop, kPartsSBelow);
     const int own_group = wi / 4;
     f32x4_t acc[NM][NPOS];
     float zacc[NREP][LPR];
@@ -1710,33 +1744,39 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
                 sp2[g] = s8[d].row[0].v[g] | (uint32_t)s8[d].row[1].v[g] << 16;
                 excess(sp2[g], s_limit[g]);
             }
-            if (__builtin_expect(__ballot(over != 0) != 0, 0)) {  // larger than the scaling allows: smaller powers from here on
-                auto wave_max = [&](uint32_t v) {
-                    v &= 0x7fff7fffu;
-                    v = max(v & 0xffffu, v >> 16);
-#pragma unroll
-                    for (int o = 1; o < kWave; o *= 2) v = max(v, (uint32_t)__shfl_xor((int)v, o));
-                    return (int)__builtin_amdgcn_readfirstlane(v);
+            if (__builtin_expect(__ballot(over != 0) != 0, 0)) {  // larger than a power allows: a smaller one from here on
+                // (two groups or two heads in the halves of a register)
+                auto largest_of = [&](uint32_t u, uint32_t v) {
+                    const uint32_t both = max_halves(__builtin_amdgcn_perm(v, u, 0x05040100u) & 0x7fff7fffu, __builtin_amdgcn_perm(v, u, 0x07060302u) & 0x7fff7fffu);
+                    return (uint32_t)__builtin_amdgcn_readfirstlane(wave_max_halves<1>(both));
                 };
-                int down = 0;  // of the lane's own group
+                int down = 0, x_down[NREP];  // down: of the lane's own group
 #pragma unroll
                 for (int g = 0; g < LPR; g++) {
-                    const int sb = min(s_pow[g], 22 - (wave_max(sp2[g]) >> 10));
-                    down = own_group == g ? sb - s_pow[g] : down;
-                    s_pow[g] = sb;
-                    s_limit[g] = (((23 - sb) << 10) - 1) * 0x00010001u;
+                    const uint32_t largest = largest_of(sp2[g & ~1], sp2[g | 1 < LPR ? g | 1 : g]);
+                    const int n = parts_power(s_pow[g], largest >> 16 * (g % 2) & 0xffffu, kPartsSBelow);
+                    down = own_group == g ? n - s_pow[g] : down;
+                    s_pow[g] = n;
+                    s_limit[g] = parts_limit(n, kPartsSBelow);
                 }
 #pragma unroll
                 for (int h = 0; h < NREP; h++) {
-                    const int xb = min(x_pow[h], 21 - (wave_max(xp2[h]) >> 10));
-                    const float f = ldexpf(1.0f, xb - x_pow[h] + down);
+                    const uint32_t largest = largest_of(xp2[h & ~1], xp2[h | 1]);
+                    const int n = parts_power(x_pow[h], largest >> 16 * (h % 2) & 0xffffu, kPartsXBelow);
+                    x_down[h] = n - x_pow[h];
+                    x_pow[h] = n;
+                    x_limit[h] = parts_limit(n, kPartsXBelow);
+                }
+                if (k0 != kfirst) {  // (nothing is summed before the first chunk)
 #pragma unroll
-                    for (int i = 0; i < 2; i++) {
+                    for (int h = 0; h < NREP; h++) {
+                        const float f = ldexpf(1.0f, x_down[h] + down);
 #pragma unroll
-                        for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
+                        for (int i = 0; i < 2; i++) {
+#pragma unroll
+                            for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
+                        }
                     }
-                    x_pow[h] = xb;
-                    x_limit[h] = (((22 - xb) << 10) - 1) * 0x00010001u;
                 }
             }
             half2_t ss[LPR];
@@ -1959,11 +1999,13 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
 //   free).  A chunk that would cross K is moved back to end at K and its repeated rows meet
 //   x == 0 (the host gives this kernel K >= 32).  Loads rotate as in gemv_rows_mfma.
 //   Four heads: two fp16 parts after powers of two, as in gemv_rows_mfma (one per group of 32 codes, one per head), 8 A
-//   rows instead of 12 and with them two MFMAs per field instead of three.  16 x 8 kv heads, four heads each, us: 8064
-//   tokens in 4 bits 27.0 -> 24.5, 32000 in 2 bits 94 -> 85 (issue of MFMAs and of the operands' VALU work, not memory:
-//   3.4 and 2.3 TB/s); outputs that are not the fp16 nearest to the exact sum: 1.5 -> 1.1 of 1000.
+//   rows instead of 12 and with them two MFMAs per field instead of three.  The powers follow the data anew in every tile
+//   (outputs that two tiles form come out the same).  16 x 8 kv heads, four heads each, us: 8064 tokens in 4 bits 23.6 ->
+//   21.6, 32000 in 2 bits 86 -> 79 (issue of MFMAs and of the operands' VALU work, not memory); outputs that are not the
+//   fp16 nearest to the exact sum, of 1000: 1.8 -> 1.2, keys and queries a hundredth of that size 0.9 -> 0.6 (12 with
+//   powers that only follow large values, which are 2 to 4 us faster at 32000 tokens).
 //   Launches of few tiles: the waves of a block share one (ksplit), each takes consecutive chunks of its rows and
-//   their sums meet in the A tiles in the order of the rows: 8 kv heads of 1024 tokens, K = 128, 13.0 -> 7.1 us (a wave
+//   their sums meet in the A tiles in the order of the rows: 8 kv heads of 1024 tokens, K = 128, 13.0 -> 7.8 us (a wave
 //   walks one chunk instead of four: the launch is latency alone).
 //   The last tile of a row is shifted left to end at N (N >= 512, a multiple of 32).
 //   A wave walks `splits` tiles one after the other with the load pipeline running across
@@ -2030,8 +2072,6 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     // two halves each, x_limit of one head, s_limit of two of the groups that the lane stages
     int x_pow[NREP], own_pow;  // own_pow: of the scales of the group whose outputs this lane holds
     uint32_t x_limit[NREP], s_limit[4];
-#pragma unroll
-    for (int h = 0; h < NREP; h++) x_pow[h] = 3, x_limit[h] = ((19 << 10) - 1) * 0x00010001u;  // |x| < 16
     f32x4_t acc[NM][NPOS];
     float zacc[NREP][8];
     auto clear = [&]() {
@@ -2045,9 +2085,12 @@ __global__ void __launch_bounds__(64 * kColsWaves)
 #pragma unroll
             for (int j = 0; j < 8; j++) zacc[h][j] = 0.f;
         }
-        own_pow = 5;  // (a tile's groups owe nothing to those of the tile before)
+        // (a tile owes nothing to the one before: outputs that two tiles form come out the same)
 #pragma unroll
-        for (int g = 0; g < 4; g++) s_limit[g] = ((18 << 10) - 1) * 0x00010001u;  // |scale| < 8
+        for (int h = 0; h < NREP; h++) x_pow[h] = kPartsTop, x_limit[h] = parts_limit(kPartsTop, kPartsXBelow);
+        own_pow = kPartsTop;
+#pragma unroll
+        for (int g = 0; g < 4; g++) s_limit[g] = parts_limit(kPartsTop, kPartsSBelow);
     };
     clear();
 
@@ -2097,32 +2140,46 @@ __global__ void __launch_bounds__(64 * kColsWaves)
             }
 #pragma unroll
             for (int g = 0; g < 4; g++) excess(s2[g], s_limit[g]);
-            if (__builtin_expect(__ballot(over != 0) != 0, 0)) {  // larger than the scaling allows: smaller powers from here on
-                auto exponent = [&](uint32_t v, int apart) {  // of the largest fp16 value among every apart-th lane's
-                    v &= 0x7fffu;
-                    for (int o = apart; o < kWave; o *= 2) v = max(v, (uint32_t)__shfl_xor((int)v, o));
-                    return (int)(v >> 10);
-                };
+            if (__builtin_expect(__ballot(over != 0) != 0, 0)) {  // larger than a power allows: a smaller one from here on
+                // (limits instead of powers: a group keeps its limit unless something is above it, see parts_power)
+                constexpr uint32_t kMantissa = 0x03ff03ffu, kRoom = kPartsRoom * 0x04000400u, kZero = ((15 + kPartsSBelow) << 10) * 0x00010001u - 0x00010001u;
                 const int had = own_pow;
+                int x_down[NREP];
+                uint32_t own_limit = 0;  // of the group of the lane's outputs: lanes 0 and 1 stage groups 0..7 and 8..15
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int sh = 16 * (j % 2);
-                    const int sb = min(22 - (int)((s_limit[j / 2] >> sh & 0xffffu) >> 10), 22 - exponent(s2[j / 2] >> sh, 2));
-                    s_limit[j / 2] = (s_limit[j / 2] & ~(0xffffu << sh)) | (uint32_t)(((23 - sb) << 10) - 1) << sh;
-                    const int of_group = __shfl(sb, lane / 32);  // (lane 0 stages groups 0..7, lane 1 groups 8..15)
-                    if (lane / 4 % 8 == j) own_pow = of_group;
-                }
+                for (int g = 0; g < 4; g++) {
+                    const uint32_t largest = wave_max_halves<2>(s2[g] & 0x7fff7fffu) | kMantissa, room = largest + kRoom;
+                    const uint32_t with_room = max_halves(largest, __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(ushort2_t, room), __builtin_bit_cast(ushort2_t, kZero))));
+                    uint32_t limit = 0;
 #pragma unroll
-                for (int h = 0; h < NREP; h++) {
-                    const int xb = min(x_pow[h], 21 - (int)__builtin_amdgcn_readfirstlane(exponent(x2[h], 1)));
-                    const float f = ldexpf(1.0f, xb - x_pow[h] + own_pow - had);
-#pragma unroll
-                    for (int i = 0; i < NP; i++) {
-#pragma unroll
-                        for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
+                    for (int e = 0; e < 2; e++) {
+                        const uint32_t half = 0xffffu << 16 * e;
+                        limit |= (largest & half) > (s_limit[g] & half) ? with_room & half : s_limit[g] & half;
                     }
-                    x_pow[h] = xb;
-                    x_limit[h] = (((22 - xb) << 10) - 1) * 0x00010001u;
+                    s_limit[g] = limit;
+                    const uint32_t of0 = __builtin_amdgcn_readlane(limit, 0), of1 = __builtin_amdgcn_readlane(limit, 1);
+                    own_limit = lane / 8 % 4 == g ? (lane < 32 ? of0 : of1) : own_limit;
+                }
+                own_pow = 14 + kPartsSBelow - (int)((lane / 4 % 2 ? own_limit >> 16 : own_limit & 0xffffu) >> 10);
+#pragma unroll
+                for (int h = 0; h < NREP; h++) {  // (two heads in the halves of a register)
+                    const uint32_t pair = __builtin_amdgcn_perm(x2[h | 1], x2[h & ~1], 0x05040100u) & 0x7fff7fffu;
+                    const uint32_t largest = (uint32_t)__builtin_amdgcn_readfirstlane(wave_max_halves<2>(pair));
+                    const int n = parts_power(x_pow[h], largest >> 16 * (h % 2) & 0xffffu, kPartsXBelow);
+                    x_down[h] = n - x_pow[h];
+                    x_pow[h] = n;
+                    x_limit[h] = parts_limit(n, kPartsXBelow);
+                }
+                if (shared ? it != begin : k0 != 0) {  // (nothing is summed before a tile's first chunk)
+#pragma unroll
+                    for (int h = 0; h < NREP; h++) {
+                        const float f = ldexpf(1.0f, x_down[h] + own_pow - had);
+#pragma unroll
+                        for (int i = 0; i < NP; i++) {
+#pragma unroll
+                            for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
+                        }
+                    }
                 }
             }
             half2_t ss[4];

@@ -98,8 +98,8 @@ def test_pv_with_probability_rows(oracle, dev, bits, nkv):
     zero term sum p*zero of an output are large and of opposite sign where the values straddle zero, and the kernels
     form the two separately (the reference adds code*scale + zero per element first), so an output in which they
     cancel shows every bit the code term has lost.  Two things keep it whole: x*scale goes to the matrix cores as
-    three bf16 parts that hold the product exactly (two parts, measured faster for four heads per pass, are off by
-    up to 2^-17 of every product: 1.4 times the tolerance here), and the code fields of the low nibble of a byte are
+    three bf16 parts that hold the product exactly (one head) or two fp16 parts that are off by 2^-34 of the largest
+    product (four heads; two bf16 parts are off by up to 2^-17 of every product: 1.4 times the tolerance here), and the code fields of the low nibble of a byte are
     moved up before they become operands -- the matrix cores align the four products of a sum by the operands'
     exponent fields, which all byte patterns share, so a pattern with leading zeros leaves that many fewer bits for
     a sum that one product dominates (with the fields in place: 1.7 times the tolerance on a 2-bit output of
