@@ -1394,9 +1394,11 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 //           The (part, head) rows are packed four to an MFMA; unused rows are zero.
 //           Measured, four query heads per kv head, operands from memory, bf16 -> fp16 parts (and blocks of
 //           eight waves instead of four), us: B = 16, 8 kv heads, T = 32640, 2 bits 72.8 -> 57; T = 8064, 4 bits
-//           27.8 -> 25; B = 4, T = 32640, 1 bit 25.5 -> 22.3; B = 8, T = 8064, dense 3-bit 18.7 -> 17.1.  Outputs
-//           that are not the fp16 nearest to the exact sum, of 1000, bf16 -> fp16 parts: T = 1000 / 16000 / 32000,
-//           2 bits 5.5 / 4.7 / 4.9 -> 3.3 / 3.9 / 4.3; T = 4000 / 16000, 4 bits 4.0 / 4.5 -> 3.4 / 4.1.  One
+//           27.8 -> 25.7, 1 bit 28.6 -> 20.5, dense 3-bit 30.1 -> 24.6; B = 8, T = 8064, dense 3-bit 21.1 -> 18.6.
+//           Outputs that are not the fp16 nearest to the exact sum, of 1000, bf16 -> fp16 parts, T = 1000 / 4000 / 16000 /
+//           32640: 1 bit 3.4 / 3.3 / 7.0 / 6.9 -> 2.0 / 2.4 / 4.6 / 4.4, 2 bits 5.3 / 4.9 / 10.4 / 10.0 -> 3.5 / 4.4 / 7.9 / 8.0, 4 bits
+//           5.7 / 4.9 / 10.6 / 10.0 -> 3.7 / 4.5 / 8.5 / 10.8, dense 3-bit 5.0 / 4.8 / 8.8 / 8.1 -> 3.6 / 4.8 / 9.0 / 9.3 (5.9 and 11.0 at
+//           4000 and 16000 with the lower field of a byte three bits below the upper).  One
 //           head stays on bf16: there the three rows share one MFMA, and the narrower loads and the one more
 //           shift per byte cost more (B = 16, 32 heads, T = 8064, 2 bits 38.2 -> 39.9; B = 64, T = 3968, 1 bit 56.5
 //           -> 64.0).  Bound by the vector ALU (400 instructions per 128 rows) beside the MFMAs.
@@ -1849,13 +1851,23 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
                 const uint32_t *src = from_u ? u : v;
                 const uint32_t t01 = __builtin_amdgcn_perm(src[1], src[0], sel);
                 const uint32_t t23 = __builtin_amdgcn_perm(src[3], src[2], sel);
-                // the pair's fields lie at bit 0 or 2 of the byte: all to bits TOP + 2 and up (see field_operand_top)
-                const int up = (mm % 2 == 0 ? 2 : 0) + TOP;
-                const uint32_t s01 = t01 << up, s23 = t23 << up;
+                // the pair's fields lie at bit 0 or 2 of the byte: to bits 2 and 5 of a bf16's eight, and each to the top
+                // of a half's eleven (see field_operand_top)
+                const int at = mm % 2 == 0 ? 0 : 2;
+                if constexpr (HALVES) {
 #pragma unroll
-                for (int f = 0; f < 2; f++) {
-                    const uint32_t mask = 0x00070007u << (TOP + 2 + 3 * f);
-                    multiply(s01 & mask, s23 & mask, mm * 2 + f);
+                    for (int f = 0; f < 2; f++) {
+                        const int up = TOP + 5 - (at + 3 * f);
+                        const uint32_t mask = 0x00070007u << (TOP + 5);
+                        multiply((t01 << up) & mask, (t23 << up) & mask, mm * 2 + f);
+                    }
+                } else {
+                    const uint32_t s01 = t01 << (2 - at), s23 = t23 << (2 - at);
+#pragma unroll
+                    for (int f = 0; f < 2; f++) {
+                        const uint32_t mask = 0x00070007u << (2 + 3 * f);
+                        multiply(s01 & mask, s23 & mask, mm * 2 + f);
+                    }
                 }
             }
         } else {
@@ -1948,8 +1960,8 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
         }
 #pragma unroll
         for (int p = 0; p < NPOS; p++) {
-            // (bit offset code p's field counts with: dense 3-bit 2 5 2 5 2 5 2 5, else see field_offset_top)
-            const int off = TOP + (BITS == 30 ? 2 + 3 * (p % 2) : field_offset_top<FB>(p % FPB));
+            // (bit offset code p's field counts with: dense 3-bit 2 5 2 5 2 5 2 5, in a half 8 throughout, else see field_offset_top)
+            const int off = TOP + (BITS == 30 ? (HALVES ? 5 : 2 + 3 * (p % 2)) : field_offset_top<FB>(p % FPB));
             const float sum = BITS == 30 || HALVES ? sums[p] : field_sum_top<FB>(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
             if constexpr (HALVES) flat[h * NPOS + p] = ldexpf(sum, 24 - off - x_pow[h] - own_pow);
             else flat[h * NPOS + p] = sum * __uint_as_float((uint32_t)(127 + 43 - off) << 23);
