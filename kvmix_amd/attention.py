@@ -200,7 +200,7 @@ class KVmixAttention:
             query_states = query_states.masked_fill(dead, 0)
         return F.scaled_dot_product_attention(query_states, key_states, value_states, attn_mask=mask16, enable_gqa=n_rep > 1)
 
-    def _decode(self, query_states, entries, k_group, k_fmt, v_fmt, attention_mask, need_weights):
+    def _decode(self, query_states, entries, k_group, k_fmt, v_fmt, attention_mask, need_weights, allow_single_pass):
         """Attention over the cache's entries, the call's own tokens among them: (output, probabilities or None)."""
         kc, k_tail, ks, km, vc, v_tail, vs, vm, kv_seq_len = entries
         B, nh, q_len, D = query_states.shape
@@ -214,7 +214,7 @@ class KVmixAttention:
             if attention_mask is not None and attention_mask.shape[-2:] != (1, kv_seq_len):
                 raise ValueError(f"Attention mask shape {attention_mask.shape} does not match weights shape "
                                  f"{(B, nh, 1, kv_seq_len)}")
-            single = ops.prefer_single_pass(
+            single = allow_single_pass and ops.prefer_single_pass(
                 B, nh, nkv, D, kv_seq_len, self.k_bits, k_fmt, k_group, self.v_bits, v_fmt,
                 self.Vgroup_size, kv_seq_len - k_tail.shape[2], kv_seq_len - v_tail.shape[2], need_weights)
             return ops.decode_attention(
@@ -223,23 +223,27 @@ class KVmixAttention:
         return self._decode_with_torch_glue(query_states, kc, ks, km, k_tail, vc, vs, vm, v_tail, k_group, k_fmt, v_fmt, nh // nkv, attention_mask)
 
     def attend(self, query_states: torch.Tensor, cache: PackedKVCache, attention_mask: Optional[torch.Tensor] = None,
-               need_weights: bool = True):
+               need_weights: bool = True, allow_single_pass: bool = True):
         """The attention of a decode step whose tokens `cache` holds already (a kernel wrote them into its slots:
         PackedKVCache.next_slots): (attn_output [B,nh,Q,D], attn_weights or None), as forward returns them."""
-        return self._decode(query_states, cache.as_tuple(), cache.Kgroup_size, cache.k_fmt, cache.v_fmt, attention_mask, need_weights)
+        return self._decode(query_states, cache.as_tuple(), cache.Kgroup_size, cache.k_fmt, cache.v_fmt, attention_mask, need_weights,
+                            allow_single_pass)
 
     # -- the step --------------------------------------------------------------------------
     def forward(self, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor,
                 past_key_value=None, attention_mask: Optional[torch.Tensor] = None, use_cache: bool = True,
-                need_weights: bool = True):
+                need_weights: bool = True, allow_single_pass: bool = True):
         """query_states [B,nh,Q,D], key/value_states [B,Hkv,Q,D] (fp16, after RoPE).
         past_key_value: None (prompt), the reference's 9-tuple (a new tuple is returned, grown by
         concatenation as the reference does), or a PackedKVCache (updated in place and returned;
         an empty one means prompt).
-        need_weights=False lets a single-token step run as one pass over the positions where that
-        is the faster form; no probabilities exist then and attn_weights is None (the output differs
-        from the other form by the reference's roundings after the softmax, about 2^-10 of the
-        largest value).
+        A single-token step runs as one pass over the positions where that is the faster form, with the
+        probabilities (small steps: ops.prefer_single_pass(weights=True)) and without.  Its output then differs
+        from the other form's, the launches of ops.decode_attention, by the reference's roundings after the
+        softmax, which it leaves out: the probabilities it multiplies are fp32, quantized and fp16 part are added
+        in fp32 (about 2^-10 of the largest value; the returned fp16 probabilities times the values are that far
+        from it too).  allow_single_pass=False keeps the launches that round as the reference does at every size.
+        need_weights=False: no probabilities exist in a single pass and attn_weights is None.
         Returns (attn_output [B,nh,Q,D] fp16, attn_weights fp16 or None, past_key_value or None)."""
         B, nh, q_len, D = query_states.shape
         n_rep = nh // key_states.shape[1]
@@ -258,7 +262,7 @@ class KVmixAttention:
                 kc, k_tail, ks, km, vc, v_tail, vs, vm = self._grown(past_key_value, key_states, value_states)
 
             attn_output, attn_weights = self._decode(query_states, (kc, k_tail, ks, km, vc, v_tail, vs, vm, kv_seq_len), k_group, k_fmt, v_fmt,
-                                                     attention_mask, need_weights)
+                                                     attention_mask, need_weights, allow_single_pass)
         else:
             # prompt: dense fp16 attention; the cache keeps the oldest tokens quantized
             # (models/modeling_llama_KVmix.py:213-266)

@@ -90,3 +90,33 @@ def test_lengths_from_the_device_and_windows_past_them(dev):
     out, probs = ops.decode_attention(q, None, None, kt, vt, 32, 4, 32, 4, k_tail_len=n, v_tail_len=n, single_pass=True, weights=True)
     bad = out.isnan().any(-1).squeeze(-1)
     assert bad.tolist() == [[False, True, False, False], [False] * 4] and probs[0, 1, 0, :70].isnan().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("inplace", [False, True])
+def test_a_caller_keeps_the_launches_that_round_as_the_reference_does(dev, inplace):
+    """forward with its defaults takes the single pass here; with allow_single_pass=False its output is the four launches' bit
+    by bit: the halves of the output rounded and added as halves."""
+    from kvmix_amd import ops
+    from kvmix_amd.attention import KVmixAttention
+
+    gen = torch.Generator(device=dev).manual_seed(11)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=dev).half()
+    layer = KVmixAttention(4, 2, residual_length=64)
+    k, v = rand(2, 2, 501, 128), rand(2, 2, 501, 128)
+    past = layer.new_cache(1024) if inplace else None
+    *_, past = layer(rand(2, 8, 501, 128), k, v, past, need_weights=False)
+    q, k1, v1 = rand(2, 8, 1, 128), rand(2, 2, 1, 128), rand(2, 2, 1, 128)
+    out, probs, grown = layer(q, k1, v1, past, allow_single_pass=False)
+    kc, kt, ks, km, vc, vt, vs, vm, width = grown.as_tuple() if inplace else grown
+    assert ops.prefer_single_pass(2, 8, 2, 128, width, 4, 0, 32, 2, 0, 32, width - kt.shape[2], width - vt.shape[2], True)
+    step = lambda single: ops.decode_attention(q, (kc, ks, km), (vc, vs, vm), kt, vt, 32, 4, 32, 2, single_pass=single, weights=single)
+    want, wp = step(False)
+    assert torch.equal(out, want) and torch.equal(probs, wp)
+    tq = width - vt.shape[2]
+    halves = ops.quantized_gemm(32, probs[..., :tq], vc, vs, vm, 2).float()
+    tail = torch.matmul(probs[..., tq:].double().reshape(2, 2, 4, -1), vt.double()).reshape(out.shape)
+    assert ((out.double() - (halves + tail.half().float()).half().double()).abs() <= 2.0 ** -10 * tail.abs() + 2.0 ** -10 * out.double().abs() + 2.0 ** -24).all()
+    if inplace:
+        assert torch.equal(layer.attend(q, grown, allow_single_pass=False)[0], want)
+        assert torch.equal(layer.attend(q, grown)[0], step(True)[0])
