@@ -261,8 +261,8 @@ extern "C" size_t kvmix_decode_attention_fused_workspace_bytes(const kvmix_decod
 }
 
 // the argument checks of kvmix_decode_attention_fused; `pointers`: also that the operands are there (the plan query
-// passes sizes only)
-static int fused_check(const kvmix_decode_attn_t *p, bool pointers)
+// passes sizes only); `weights`: of the step that returns its probabilities, whose launch has other blocks
+static int fused_check(const kvmix_decode_attn_t *p, bool pointers, bool weights = false)
 {
     if (!p) return KVMIX_ERR_NULL;
     if (p->samples < 0 || p->D <= 0 || p->k_tokens < 0 || p->v_tokens < 0 || p->k_tail_slots < 0 || p->v_tail_slots < 0 ||
@@ -295,8 +295,7 @@ static int fused_check(const kvmix_decode_attn_t *p, bool pointers)
         if (pointers && (!p->v_code || !p->v_scale || !p->v_zero)) return KVMIX_ERR_NULL;
         if (p->v_code_row_stride < kFusedD * p->v_bits / 32 || p->v_sz_row_stride < kFusedD / 32) return KVMIX_ERR_SHAPE;
     }
-    const FusedLayout lay = fused_layout(p);
-    const int64_t slabs = lay.slabs();
+    const int64_t slabs = fused_layout(p, weights).slabs();
     if (slabs > 0x7fffffff || slabs * p->samples > 0x7fffffff) return KVMIX_ERR_SHAPE;  // (blocks of one launch)
     return KVMIX_OK;
 }
@@ -459,7 +458,7 @@ extern "C" size_t kvmix_decode_attention_fused_weights_workspace_bytes(const kvm
 extern "C" int kvmix_decode_attention_fused_weights(const kvmix_decode_attn_t *p, void *workspace, size_t workspace_bytes,
                                                     kvmix_stream_t stream)
 {
-    const int chk = fused_check(p, true);
+    const int chk = fused_check(p, true, true);
     if (chk != KVMIX_OK || p->samples == 0) return chk;
     if (!p->probs) return KVMIX_ERR_NULL;
     if (p->probs_stride < fused_width(p) || (fused_width(p) + kWeightsPart - 1) / kWeightsPart > 65535) return KVMIX_ERR_SHAPE;
@@ -475,7 +474,7 @@ extern "C" int kvmix_decode_attention_fused_weights(const kvmix_decode_attn_t *p
 constexpr int64_t kSmallWeightsEntries = 450000, kSmallWeightsEntriesRef3 = 300000;
 extern "C" int kvmix_decode_attention_fused_weights_recommended(const kvmix_decode_attn_t *p)
 {
-    if (fused_check(p, false) != KVMIX_OK || p->samples == 0) return 0;
+    if (fused_check(p, false, true) != KVMIX_OK || p->samples == 0) return 0;
     const bool ref3 = p->k_tokens > 0 && fused_key_mode(p) == 3;
     return p->samples * fused_width(p) <= (ref3 ? kSmallWeightsEntriesRef3 : kSmallWeightsEntries) ? 1 : 0;
 }

@@ -25,6 +25,24 @@ def test_steps_it_is_chosen_for():
     assert not chosen(8, 32, 32, 8192) and not chosen(1, 32, 32, 10000, 3) and not chosen(1, 36, 12, 100)  # (three heads per kv head)
 
 
+def test_more_blocks_than_a_launch_holds_are_refused():
+    """The slabs of a step with probabilities are shorter than the tiles without: 1025 and 2049 a row here.  (No probabilities
+    are passed, so that nothing is launched whatever the check says.)"""
+    import ctypes
+
+    L = _lib.load()
+
+    def code(samples):
+        st = _lib.attn_step_descriptor(samples // 32, 32, 32, 128, 4, 0, 32, 1 << 20, 4, 0, 32, 1 << 20, 16, 16)
+        for name in ("q", "out", "k_tail", "v_tail", "k_code", "k_scale", "k_zero", "v_code", "v_scale", "v_zero"):
+            setattr(st, name, 4096)
+        assert _lib.attn_plan(st)["matrix"]
+        return L.kvmix_decode_attention_fused_weights(ctypes.byref(st), None, 0, None)
+
+    null, shape = -7, -8
+    assert code(32 * 1000) == null and code(32 * 48000) == shape
+
+
 @pytest.mark.gpu
 # one slab, two with a ragged last, the longest; GQA; no quantized part; left-padded masks; a row masked everywhere
 @pytest.mark.parametrize("B,nh,nkv,T,tail", [(2, 4, 4, 40, 40), (1, 8, 2, 512, 32), (1, 8, 2, 1037, 45), (2, 4, 4, 2100, 52), (1, 16, 2, 3000, 24), (1, 32, 32, 8001, 33)])
