@@ -466,15 +466,24 @@ extern "C" int kvmix_decode_attention_fused_weights(const kvmix_decode_attn_t *p
     return fused_step(p, true, workspace, (hipStream_t)stream);
 }
 
-// Which form of a step with probabilities is faster (operands from memory, four launches -> slabs, us): the slabs up to 450 000
-// (query head x position) entries, 300 000 with the reference's 3-bit keys, which the slabs take as vector arithmetic
-// throughout.  256 000 entries: 1 x 8000, 2 bits 26.4 -> 17.5; 1 x 8000, 32 / 8 heads, 4 bits 27.9 -> 17.2; 4 x 2000, 3-bit keys
-// 30.3 -> 25.1; 333 000: 4 x 2600, 4 bits 33.4 -> 26.9, 2 bits, 32 / 8 heads 29.0 -> 22.7; 410 000: 8 x 1600, 32 / 8 heads 25.7 -> 26.2;
-// 435 000: 4 x 3400, 2 bits 31.4 -> 28.6, 4 bits, 32 / 8 heads 30.5 -> 26.8; level at 512 000: 4 x 4000, 2 bits 34.6 -> 34.2.
-constexpr int64_t kSmallWeightsEntries = 450000, kSmallWeightsEntriesRef3 = 300000;
+// Which form of a step with probabilities is faster (32 query heads, operands from memory, four launches -> slabs, us): the slabs
+// up to 450 000 (query head x position) entries, 300 000 with the reference's 3-bit keys, which the slabs take as vector
+// arithmetic throughout.  4 x 3400: 4 bits 40.5 -> 36.1, 32 / 8 heads 33.2 -> 27.8, 2 bits 33.3 -> 30.6; 16 x 800: 40.4 -> 35.8, 33.3 ->
+// 30.4, 36.0 -> 32.2; 32 x 400: 61.7 -> 36.3, 52.5 -> 30.3, 51.3 -> 32.2; 8 x 1200, 3-bit keys 30.6 -> 26.6.
+// From 129 to 256 rows the launches with a block per row are one round, at most a block to a CU, and the line lies lower.  8 x
+// T, 4 bits: T = 1171 32.1 -> 31.1, 1367 33.7 -> 33.9, 1562 34.5 -> 36.2 (2 bits 30.2 -> 31.3); 32 / 8 heads, 2 bits: 1600 28.1 -> 26.0, 1750
+// 29.5 -> 30.5; dense 3-bit values, with one head per kv head: 6 x 1302 33.6 -> 33.2, 6 x 1562 35.4 -> 37.5, 8 x 976 30.3 -> 27.7, 8 x 1171
+// 34.7 -> 36.4, 8 x 1562 37.9 -> 42.2 (to either side of those rows: 4 x 3125 42.4 -> 40.7, 10 x 1250 46.9 -> 42.9).
+constexpr int64_t kWeightsEntries = 450000, kWeightsEntriesRef3 = 300000;
+constexpr int64_t kWeightsEntriesOneRound = 350000, kWeightsEntriesOneRoundGrouped = 420000, kWeightsEntriesOneRoundDense3 = 260000;
 extern "C" int kvmix_decode_attention_fused_weights_recommended(const kvmix_decode_attn_t *p)
 {
     if (fused_check(p, false, true) != KVMIX_OK || p->samples == 0) return 0;
-    const bool ref3 = p->k_tokens > 0 && fused_key_mode(p) == 3;
-    return p->samples * fused_width(p) <= (ref3 ? kSmallWeightsEntriesRef3 : kSmallWeightsEntries) ? 1 : 0;
+    int64_t most = p->k_tokens > 0 && fused_key_mode(p) == 3 ? kWeightsEntriesRef3 : kWeightsEntries;
+    if (p->samples > 128 && p->samples <= 256) {
+        const bool dense3 = p->v_tokens > 0 && fused_value_mode(p) == 3;
+        const int64_t round = p->heads_per_kv > 1 ? kWeightsEntriesOneRoundGrouped : dense3 ? kWeightsEntriesOneRoundDense3 : kWeightsEntriesOneRound;
+        if (round < most) most = round;
+    }
+    return p->samples * fused_width(p) <= most ? 1 : 0;
 }

@@ -25,6 +25,20 @@ def test_steps_it_is_chosen_for():
     assert not chosen(8, 32, 32, 8192) and not chosen(1, 32, 32, 10000, 3) and not chosen(1, 36, 12, 100)  # (three heads per kv head)
 
 
+@pytest.mark.parametrize("batch,kv_heads,vb,fmt,taken,left", [
+    (8, 32, 4, 0, 1360, 1562), (8, 8, 2, 0, 1600, 1750), (8, 32, 3, 1, 976, 1171), (5, 32, 4, 0, 2180, 2500),  # (129 to 256 rows: one round)
+    (4, 32, 3, 1, 3400, 3700), (9, 32, 3, 1, 1500, 1700), (32, 32, 2, 0, 430, 450), (1, 8, 4, 0, 14000, 15000)])
+def test_sides_of_the_rule(batch, kv_heads, vb, fmt, taken, left):
+    import ctypes
+
+    def chosen(width):
+        tokens = width // 352 * 352
+        st = _lib.attn_step_descriptor(batch, 32, kv_heads, 128, 4, 0, 32, tokens, vb, fmt, 32, tokens, width - tokens, width - tokens)
+        return _lib.load().kvmix_decode_attention_fused_weights_recommended(ctypes.byref(st))
+
+    assert chosen(taken) and not chosen(left)
+
+
 def test_more_blocks_than_a_launch_holds_are_refused():
     """The slabs of a step with probabilities are shorter than the tiles without: 1025 and 2049 a row here.  (No probabilities
     are passed, so that nothing is launched whatever the check says.)"""
