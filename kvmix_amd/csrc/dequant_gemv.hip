@@ -1475,9 +1475,6 @@ __device__ __forceinline__ float field_sum(float cur, float prev, int f)
 // the accumulator is the smaller addend; once it dominates, the sum is exact and rounded to nearest.  With the
 // fields in place a 2-bit p.V carries 18 bits of a dominant product, a 4-bit one 20, which shows where the code
 // term and the zero term of an output cancel).
-#ifndef KVMIX_ROWS_FIELDS_TOP
-#define KVMIX_ROWS_FIELDS_TOP 1
-#endif
 // bits the fields 0..f are moved up by: the fields of the low nibble by four, so that one shifted copy of the
 // register serves them all and no operand of a dominant product has more than three leading zeros (1-bit codes;
 // two for 2-bit codes, none for 4-bit codes) where in place it has up to seven (six, four)
@@ -2776,12 +2773,11 @@ __device__ __forceinline__ void slab_value_phase(const AttnSlabArgs &a, int64_t 
                 const uint32_t *src = from_u ? u : v;
                 const uint32_t t01 = __builtin_amdgcn_perm(src[1], src[0], sel);
                 const uint32_t t23 = __builtin_amdgcn_perm(src[3], src[2], sel);
-                constexpr bool UP = KVMIX_ROWS_FIELDS_TOP;  // (a pair at bit 0 is moved up by two, as in gemv_rows_mfma)
-                const uint32_t s01 = UP && mm % 2 == 0 ? t01 << 2 : t01, s23 = UP && mm % 2 == 0 ? t23 << 2 : t23;
-                const int o0 = UP || mm % 2 != 0 ? 2 : 0;
+                // (a pair at bit 0 is moved up by two, as in gemv_rows_mfma with one head)
+                const uint32_t s01 = mm % 2 == 0 ? t01 << 2 : t01, s23 = mm % 2 == 0 ? t23 << 2 : t23;
 #pragma unroll
                 for (int f = 0; f < 2; f++) {
-                    const uint32_t mask = 0x00070007u << (o0 + 3 * f);
+                    const uint32_t mask = 0x00070007u << (2 + 3 * f);
                     const bf16x4_t bv = __builtin_bit_cast(bf16x4_t, make_uint2(s01 & mask, s23 & mask));
                     acc[mm * 2 + f] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(av, bv, acc[mm * 2 + f], 0, 0, 0);
                 }
@@ -2794,9 +2790,7 @@ __device__ __forceinline__ void slab_value_phase(const AttnSlabArgs &a, int64_t 
                 const uint32_t t23 = perm_elems(w[t][3], w[t][2], sel);
 #pragma unroll
                 for (int f = 0; f < FPB; f++) {
-                    const bf16x4_t bv = __builtin_bit_cast(
-                        bf16x4_t, KVMIX_ROWS_FIELDS_TOP ? make_uint2(field_operand_top<FB>(t01, f), field_operand_top<FB>(t23, f))
-                                                        : make_uint2(field_operand<FB>(t01, f), field_operand<FB>(t23, f)));
+                    const bf16x4_t bv = __builtin_bit_cast(bf16x4_t, make_uint2(field_operand_top<FB>(t01, f), field_operand_top<FB>(t23, f)));
                     acc[b * FPB + f] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(av, bv, acc[b * FPB + f], 0, 0, 0);
                 }
             }
@@ -2842,10 +2836,8 @@ __device__ __forceinline__ void slab_value_phase(const AttnSlabArgs &a, int64_t 
     for (int p = 0; p < NPOS; p++) sums[p] = (acc[p][0] + acc[p][1]) + acc[p][2];
 #pragma unroll
     for (int p = 0; p < NPOS; p++) {
-        const int off = BITS == 30 ? 3 * (p % 2) + (KVMIX_ROWS_FIELDS_TOP ? 2 : 2 * ((p / 2) % 2)) : (KVMIX_ROWS_FIELDS_TOP ? field_offset_top<FB>(p % FPB) : FB * (p % FPB));
-        const float sum = BITS == 30 ? sums[p]
-                          : KVMIX_ROWS_FIELDS_TOP ? field_sum_top<FB>(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB)
-                                                  : field_sum(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
+        const int off = BITS == 30 ? 2 + 3 * (p % 2) : field_offset_top<FB>(p % FPB);
+        const float sum = BITS == 30 ? sums[p] : field_sum_top<FB>(sums[p], sums[p > 0 ? p - 1 : 0], p % FPB);
         flat[p] = sum * __uint_as_float((uint32_t)(127 + 43 - off) << 23);
     }
     const int first = scatter_reduce<NPOS, 16, 1>(flat, lane);  // two of the lane's eight columns are left
