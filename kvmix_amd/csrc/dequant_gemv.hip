@@ -1584,7 +1584,7 @@ constexpr int kRowsMfmaTile = (32 * 17 + 1) * 4 + 4;  // bf16 elements of one A 
 constexpr int kRowsMfmaWaves = 16;      // waves per block at most (register budget of 128 per lane)
 constexpr int kRowsMfmaHeadsWaves = 8;  // ... four heads per pass (256)
 
-template <int BITS, int NREP, int DEPTH, int CS>
+template <int BITS, int NREP, int CS>
 __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMfmaWaves))
     __attribute__((amdgpu_waves_per_eu(NREP > 1 ? kMfmaHeadsOcc : 4))) gemv_rows_mfma(GemvArgs a)
 {
@@ -1599,6 +1599,7 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
     constexpr int RKB = 4 * RL;        // rows per k-block (16)
     constexpr int CH = 128;            // rows per chunk: with whole rows 512 scales = one 128-bit load per lane
     constexpr int KB = CH / RKB;       // k-blocks per chunk (8)
+    constexpr int DEPTH = 1;           // chunks in flight per wave (deeper costs occupancy and was slower)
     constexpr bool HALVES = NREP > 1;  // x*scale in two fp16 parts instead of three bf16 parts
     constexpr int NP = rows_mfma_parts(NREP);
     constexpr int TOP = HALVES ? 3 : 0;  // bits the codes' patterns are moved up by in a half's eleven
@@ -3605,7 +3606,6 @@ static int rows_pieces(int64_t blocks)
 template <int MODE, int NREP, int CS>
 static void launch_rows_mfma(const GemvArgs &a, int64_t samples, int waves, hipStream_t st)
 {
-    constexpr int DEPTH = 1;  // chunks in flight per wave (deeper costs occupancy and was slower)
     const dim3 grid((unsigned)(a.splits * CS), (unsigned)(samples / NREP), (unsigned)a.M), block(kWave, waves);
     // one A tile per wave and MFMA set; the block reduction (waves*NREP*128 floats) reuses it
     const size_t lds = (size_t)waves * rows_mfma_sets(NREP) * kRowsMfmaTile * sizeof(uint16_t);
@@ -3616,12 +3616,12 @@ static void launch_rows_mfma(const GemvArgs &a, int64_t samples, int waves, hipS
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices ||
             !raised[dev].load(std::memory_order_acquire)) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rows_mfma<MODE, NREP, DEPTH, CS>),
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rows_mfma<MODE, NREP, CS>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
             if (dev >= 0 && dev < kMaxDevices) raised[dev].store(true, std::memory_order_release);
         }
     }
-    KVMIX_LAUNCH((gemv_rows_mfma<MODE, NREP, DEPTH, CS>), grid, block, lds, st, a, "gemv_rows_mfma<%d,%d,%d>", MODE, NREP, DEPTH);
+    KVMIX_LAUNCH((gemv_rows_mfma<MODE, NREP, CS>), grid, block, lds, st, a, "gemv_rows_mfma<%d,%d,%d>", MODE, NREP, CS);
 }
 
 template <int MODE, int NREP>

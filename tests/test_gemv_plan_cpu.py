@@ -37,8 +37,8 @@ def test_config0_single_layer_b1_t4096():
     qk = plan(4, REF, 1, 32, 1, 3968, 128, "qk")
     assert qk["kernel"].startswith("gemv_cols_mfma2<4,")
     pv = plan(4, REF, 1, 32, 1, 3968, 128, "pv")
-    # 32 slices: one block of sixteen waves each, no second launch for a reduction
-    assert pv["kernel"] == "gemv_rows_mfma<4,1,1>" and pv["block"] == (64, 16, 1) and pv["launches"] == 1
+    # 32 slices: four blocks of sixteen waves each, with a quarter of the columns, no second launch for a reduction
+    assert pv["kernel"] == "gemv_rows_mfma<4,1,4>" and pv["grid"][:2] == (4, 32) and pv["block"] == (64, 16, 1) and pv["launches"] == 1
 
 
 def test_config1_mixed_bits_b8_t8192():
@@ -87,7 +87,8 @@ def test_config3_sweep_t4096_residual32(bits, batch):
     else:
         # non-temporal code loads (second argument) for 2-bit launches of up to three resident rounds of waves
         assert qk.startswith(f"gemv_cols_mfma2<{bits},{int(bits == 2 and batch <= 64)},")
-    assert plan(bits, REF, batch, 32, 1, 4064, 128, "pv")["kernel"] == f"gemv_rows_mfma<{bits},1,1>"
+    # (one sequence: four blocks share the columns of a row)
+    assert plan(bits, REF, batch, 32, 1, 4064, 128, "pv")["kernel"] == f"gemv_rows_mfma<{bits},1,{4 if batch == 1 else 1}>"
 
 
 def test_only_odd_shapes_reach_the_generic_kernel():

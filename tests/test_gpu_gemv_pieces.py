@@ -25,6 +25,11 @@ def test_launches_that_leave_cus_idle_are_cut_along_the_columns():
     assert plan(1, 2048, 1, 4064)["grid"][:2] == (1, 2048)
 
 
+def test_the_plan_names_the_kernel_with_its_pieces():
+    assert [plan(2, samples, 1, 2048)["kernel"] for samples in (32, 128, 256)] == [f"gemv_rows_mfma<2,1,{n}>" for n in (4, 2, 1)]
+    assert plan(30, 32, 4, 1024)["kernel"] == "gemv_rows_mfma<30,4,4>"
+
+
 def operands(bits, B, nh, nkv, M, K, seed):
     gen = torch.Generator().manual_seed(seed)
     words = 12 if bits == 30 else 4 * bits
