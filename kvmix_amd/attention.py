@@ -107,8 +107,8 @@ class KVmixAttention:
     def _grown(self, past, key_states, value_states):
         """The 9-tuple's first eight entries after one call's tokens: appended to the tails, the oldest tail tokens
         quantized as the policy says, all in new tensors (models/modeling_llama_KVmix.py:117-167).  One launch that
-        moves everything and, when something is flushed, one that quantizes from the old tails to behind the old packed
-        part; torch's cat and the separate quantizers for what those do not take."""
+        moves everything and quantizes what is flushed from the old tails to behind the old packed
+        part; torch's cat and the separate quantizers for what that does not take."""
         kc, k_tail, ks, km, vc, v_tail, vs, vm, _ = past
         if k_tail is not None and v_tail is not None and self.Vgroup_size == 32:
             lk, lv, n = k_tail.shape[2], v_tail.shape[2], key_states.shape[2]

@@ -929,9 +929,9 @@ gemv_cols3(GemvArgs a)
 //   A lane owns two words, a wave 128 (512 bytes of codes per row), 8 rows in flight; ksplit waves share a tile and slice
 //   K where the launch would otherwise have too few of them.
 // Measured: see launch_cols.  Bound now by the 6 vector and 2 matrix instructions per code, word and four rows as they
-// fall between the loads (150 registers, three waves per SIMD).  B = 16, 32 / 8 heads, T = 32637 in graph replay: 74 us on
-// scales of any size below 64, 86 us where all of them are from 64 to 8192, 105-110 us where a row in four goes through
-// fp32 (98 us before, by the form above, on all of these); against float64, sums over 64 to 128 rows end on another than
+// fall between the loads (166 registers, three waves per SIMD).  B = 16, 32 / 8 heads, T = 32637 in graph replay: 86 us on
+// scales of any size below 64, 94 us where all of them are from 64 to 8192 (72 to 78 us for the first under the profiler,
+// which on another box gave 74, 86, 105-110 where a row in four goes through fp32, and 98 by the form above on all of these); against float64, sums over 64 to 128 rows end on another than
 // the nearest fp16 in 0.7-1.8 outputs of a thousand (0.9-3.0 before).
 // ---------------------------------------------------------------------------------------
 typedef _Float16 cols3_half2 __attribute__((ext_vector_type(2)));
@@ -1388,13 +1388,15 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 //           (head, group) is 2^9 to 2^15.  The powers follow the data (kPartsTop): powers good for x < 2 and scale < 8
 //           that stay there unless something is larger leave every product off by 2^-36, which for the flat rows of a long
 //           context over small values (T = 32000, 4 bits, values of deviation 0.03 / 0.01) is 66 / 121 of 1000
-//           outputs off the nearest fp16, where three exact parts leave 8.0 / 4.2 and this 8.3 / 4.9.
+//           outputs off the nearest fp16, where three exact parts leave 8.0 / 4.2 and this 8.3 / 4.9 (the measured error
+//           of flat rows lies this far apart from one draw of values to the next: 6.7 / 3.0 and 6.1 / 2.8 on another).
 //           Against the three bf16 parts (12 rows, three MFMAs per B operand) this is 8
 //           rows, two MFMAs, a third of the LDS stores and a fifth of the arithmetic of forming them.
 //           The (part, head) rows are packed four to an MFMA; unused rows are zero.
 //           Measured, four query heads per kv head, operands from memory, bf16 -> fp16 parts (and blocks of
-//           eight waves instead of four), us: B = 16, 8 kv heads, T = 32640, 2 bits 72.8 -> 57; T = 8064, 4 bits
-//           27.8 -> 25.7, 1 bit 28.6 -> 20.5, dense 3-bit 30.1 -> 24.6; B = 8, T = 8064, dense 3-bit 21.1 -> 18.6.
+//           eight waves instead of four), us: B = 16, 8 kv heads, T = 32640, 2 bits 72.3 -> 58.8, 4 bits
+//           78.5 -> 71.7, dense 3-bit 83 -> 70; T = 8064, 1 bit 29.5 -> 21.6, 4 bits 30.0 -> 26.4, dense 3-bit 32.3 -> 26.5;
+//           B = 4, T = 2048, 4 bits (and column pieces) 11.0 -> 8.3.
 //           Outputs that are not the fp16 nearest to the exact sum, of 1000, bf16 -> fp16 parts, T = 1000 / 4000 / 16000 /
 //           32640: 1 bit 3.4 / 3.3 / 7.0 / 6.9 -> 2.0 / 2.4 / 4.6 / 4.4, 2 bits 5.3 / 4.9 / 10.4 / 10.0 -> 3.5 / 4.4 / 7.9 / 8.0, 4 bits
 //           5.7 / 4.9 / 10.6 / 10.0 -> 3.7 / 4.5 / 8.5 / 10.8, dense 3-bit 5.0 / 4.8 / 8.8 / 8.1 -> 3.6 / 4.8 / 9.0 / 9.3 (5.9 and 11.0 at
@@ -2010,12 +2012,12 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
 //   x == 0 (the host gives this kernel K >= 32).  Loads rotate as in gemv_rows_mfma.
 //   Four heads: two fp16 parts after powers of two, as in gemv_rows_mfma (one per group of 32 codes, one per head), 8 A
 //   rows instead of 12 and with them two MFMAs per field instead of three.  The powers follow the data anew in every tile
-//   (outputs that two tiles form come out the same).  16 x 8 kv heads, four heads each, us: 8064 tokens in 4 bits 23.6 ->
-//   21.6, 32000 in 2 bits 86 -> 79 (issue of MFMAs and of the operands' VALU work, not memory); outputs that are not the
+//   (outputs that two tiles form come out the same).  16 x 8 kv heads, four heads each, operands from memory, us: 8064 tokens in 2 bits
+//   24.8 -> 21.7, 4 bits 27.9 -> 24.8, 32000 in 2 bits 91 -> 83, 4 bits 98 -> 95.5 (issue of MFMAs and of the operands' VALU work, not memory); outputs that are not the
 //   fp16 nearest to the exact sum, of 1000: 1.8 -> 1.2, keys and queries a hundredth of that size 0.9 -> 0.6 (12 with
 //   powers that only follow large values, which are 2 to 4 us faster at 32000 tokens).
 //   Launches of few tiles: the waves of a block share one (ksplit), each takes consecutive chunks of its rows and
-//   their sums meet in the A tiles in the order of the rows: 8 kv heads of 1024 tokens, K = 128, 13.0 -> 7.8 us (a wave
+//   their sums meet in the A tiles in the order of the rows: 8 kv heads of 1024 tokens, K = 128, 4 bits 13.1 -> 8.0 us (a wave
 //   walks one chunk instead of four: the launch is latency alone).
 //   The last tile of a row is shifted left to end at N (N >= 512, a multiple of 32).
 //   A wave walks `splits` tiles one after the other with the load pipeline running across

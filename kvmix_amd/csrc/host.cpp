@@ -385,8 +385,9 @@ Triple append_values(const Tensor &x, const Tensor &code0, const Tensor &scale0,
     return {code, scale, mn};
 }
 
-// The 9-tuple after one call's tokens: everything moved by one launch into new tensors, what the policy flushes (nk, nv
-// tokens of the OLD tails) quantized by another from the old tails to behind the old packed part.  The caller has checked
+// The 9-tuple after one call's tokens: everything moved into new tensors, and what the policy flushes (nk, nv tokens of the
+// OLD tails) quantized from the old tails to behind the old packed part, in one launch (kvmix_grow; two or three where the
+// value half streams or the formats are not the fused kernel's).  The caller has checked
 // that nk and nv fit the old tails and that the flush kernels take the groups and widths.  None: torch's composition.
 using Grown = std::tuple<OptTensor, Tensor, OptTensor, OptTensor, OptTensor, Tensor, OptTensor, OptTensor>;
 std::optional<Grown> grow_tuple(const OptTensor &kc, const Tensor &k_tail, const OptTensor &ks, const OptTensor &km, const OptTensor &vc,

@@ -464,8 +464,8 @@ def copy_rows(pairs) -> None:
 def grow_tuple(past, key_states, value_states, nk: int, nv: int, k_bits: int, k_group: int, v_bits: int):
     """The first eight entries of the reference's cache tuple after one call's tokens (models/modeling_llama_KVmix.py:
     117-167), in new tensors: the tails grown by them, the oldest nk key and nv value tokens of the OLD tails quantized to
-    behind the packed part; one launch that moves everything and, when something is flushed, one that quantizes.  Keys in
-    groups of 32 (3 bits: 11), values in groups of 32.  None where the launches do not take the call."""
+    behind the packed part, in one launch (kvmix_grow; more for the values of a long prompt).  Keys in
+    groups of 32 (3 bits: 11), values in groups of 32.  None where that does not take the call."""
     kc, k_tail, ks, km, vc, v_tail, vs, vm, _ = past
     return _host().grow_tuple(kc, k_tail, ks, km, vc, v_tail, vs, vm, key_states, value_states, nk, nv, k_bits, k_group, v_bits)
 
