@@ -1395,11 +1395,11 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 //           The (part, head) rows are packed four to an MFMA; unused rows are zero.
 //           Measured, four query heads per kv head, operands from memory, bf16 -> fp16 parts (and blocks of
 //           eight waves instead of four), us: B = 16, 8 kv heads, T = 32640, 2 bits 72.3 -> 58.8, 4 bits
-//           78.5 -> 71.7, dense 3-bit 83 -> 70; T = 8064, 1 bit 29.5 -> 21.6, 4 bits 30.0 -> 26.4, dense 3-bit 32.3 -> 26.5;
-//           B = 4, T = 2048, 4 bits (and column pieces) 11.0 -> 8.3.
+//           78.5 -> 72.3, dense 3-bit 83 -> 72; T = 8064, 1 bit 29.5 -> 21.6, 4 bits 30.0 -> 26.6, dense 3-bit 32.3 -> 26.6;
+//           B = 4, T = 2048, 4 bits (and column pieces) 11.0 -> 8.6.
 //           Outputs that are not the fp16 nearest to the exact sum, of 1000, bf16 -> fp16 parts, T = 1000 / 4000 / 16000 /
 //           32640: 1 bit 3.4 / 3.3 / 7.0 / 6.9 -> 2.0 / 2.4 / 4.6 / 4.4, 2 bits 5.3 / 4.9 / 10.4 / 10.0 -> 3.5 / 4.4 / 7.9 / 8.0, 4 bits
-//           5.7 / 4.9 / 10.6 / 10.0 -> 3.7 / 4.5 / 8.5 / 10.8, dense 3-bit 5.0 / 4.8 / 8.8 / 8.1 -> 3.6 / 4.8 / 9.0 / 9.3 (5.9 and 11.0 at
+//           5.7 / 4.9 / 10.6 / 10.0 -> 3.7 / 4.5 / 8.6 / 8.8, dense 3-bit 5.0 / 4.8 / 8.8 / 8.1 -> 3.6 / 4.8 / 8.8 / 8.4 (5.9 and 11.0 at
 //           4000 and 16000 with the lower field of a byte three bits below the upper).  One
 //           head stays on bf16: there the three rows share one MFMA, and the narrower loads and the one more
 //           shift per byte cost more (B = 16, 32 heads, T = 8064, 2 bits 38.2 -> 39.9; B = 64, T = 3968, 1 bit 56.5
@@ -1581,6 +1581,13 @@ __device__ __forceinline__ uint32_t wave_max_halves(uint32_t v)
     const auto w = __builtin_amdgcn_permlane32_swap(v, v, false, false);
     return max_halves(w[0], w[1]);
 }
+// Sums of an eleven-bit part times codes of three or four bits round from the first products on, where those of an eight-bit
+// part stay exact for thousands of them.  After this many chunks of a wave they are put by and begin anew, so that a long row
+// rounds no more than it did with three bf16 parts: outputs off the nearest fp16 at T = 32640, of 1000, 4 bits 10.8 -> 8.8 (bf16
+// parts 10.0), dense 3-bit 9.3 -> 8.4 (8.1).  32 registers and 0.2 us of a small launch (B = 4, 8 kv heads, T = 2048 8.3 -> 8.6;
+// B = 16, T = 32640 4 bits 71.7 -> 72.3, dense 3-bit 70.3 -> 72.2).  Codes of one and two bits need none of it (4.4 and 8.0, bf16 parts 6.9
+// and 10.0), and it would cost them 2 to 4 %.
+constexpr int kPartsTogether = 6;
 constexpr int kRowsMfmaTile = (32 * 17 + 1) * 4 + 4;  // bf16 elements of one A tile (32 skewed rows), 8-byte multiple
 
 constexpr int kRowsMfmaWaves = 16;      // waves per block at most (register budget of 128 per lane)
@@ -1604,6 +1611,7 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
     constexpr int DEPTH = 1;           // chunks in flight per wave (deeper costs occupancy and was slower)
     constexpr bool HALVES = NREP > 1;  // x*scale in two fp16 parts instead of three bf16 parts
     constexpr int NP = rows_mfma_parts(NREP);
+    constexpr bool PUT_BY = HALVES && FB >= 3;  // (kPartsTogether)
     constexpr int TOP = HALVES ? 3 : 0;  // bits the codes' patterns are moved up by in a half's eleven
     constexpr bool WHOLE = CS == 1;    // (pieces of rows share their cache lines with other blocks: no streaming hint)
     constexpr int AT = kRowsMfmaTile;  // bf16 elements of one A tile
@@ -1648,6 +1656,12 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
     for (int g = 0; g < LPR; g++) s_pow[g] = kPartsTop, s_limit[g] = parts_limit(kPartsTop, kPartsSBelow);
     const int own_group = wi / 4;
     f32x4_t acc[NM][NPOS];
+    [[maybe_unused]] float whole[NREP][NPOS];  // the parts' sums of kPartsTogether chunks each
+#pragma unroll
+    for (int h = 0; h < NREP; h++) {
+#pragma unroll
+        for (int p = 0; p < NPOS; p++) whole[h][p] = 0.f;
+    }
     float zacc[NREP][LPR];
 #pragma unroll
     for (int q = 0; q < NM; q++) {
@@ -1778,6 +1792,10 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
 #pragma unroll
                             for (int p = 0; p < NPOS; p++) acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4] *= f;
                         }
+                        if constexpr (PUT_BY) {
+#pragma unroll
+                            for (int p = 0; p < NPOS; p++) whole[h][p] *= f;
+                        }
                     }
                 }
             }
@@ -1904,8 +1922,20 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
         for (int i = lane; i < NM * AT / 2; i += kWave) reinterpret_cast<uint32_t *>(atile)[i] = 0u;
         wave_lds_fence();
         __builtin_amdgcn_sched_barrier(0);
+        [[maybe_unused]] int walked = 0;
 #pragma unroll 1
         for (int k0 = kfirst; k0 < ke32; k0 += DEPTH * stride) {
+            if constexpr (PUT_BY) {
+                if (++walked > kPartsTogether) {
+                    walked = 1;
+#pragma unroll
+                    for (int p = 0; p < NPOS; p++) {
+#pragma unroll
+                        for (int h = 0; h < 4; h++) whole[h][p] += acc[0][p][h] + acc[1][p][h];
+                        acc[0][p] = acc[1][p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                    }
+                }
+            }
 #pragma unroll
             for (int d = 0; d < DEPTH; d++) {
                 const int kc = k0 + d * stride, kn = kc + DEPTH * stride;
@@ -1957,6 +1987,7 @@ __global__ void __launch_bounds__(64 * (NREP > 1 ? kRowsMfmaHeadsWaves : kRowsMf
             sums[p] = acc[h / 4][p][h % 4];
 #pragma unroll
             for (int i = 1; i < NP; i++) sums[p] += acc[(NREP * i + h) / 4][p][(NREP * i + h) % 4];
+            if constexpr (PUT_BY) sums[p] += whole[h][p];
         }
 #pragma unroll
         for (int p = 0; p < NPOS; p++) {
