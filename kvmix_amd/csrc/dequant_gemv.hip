@@ -1386,10 +1386,10 @@ __global__ void __launch_bounds__(NREP > 1 ? 64 * kRowsHeadsWaves : 64 * kRowsMa
 //           For that x and scale are first multiplied by powers of two, one per head and one per group, that put
 //           x below 2^7 and scale below 2^8: a product is then off by at most 2^-25 where the largest of its
 //           (head, group) is 2^9 to 2^15.  The powers follow the data (kPartsTop): powers good for x < 2 and scale < 8
-//           that stay there unless something is larger leave every product off by 2^-36, which for the flat rows of a long
-//           context over small values (T = 32000, 4 bits, values of deviation 0.03 / 0.01) is 66 / 121 of 1000
-//           outputs off the nearest fp16, where three exact parts leave 8.0 / 4.2 and this 8.3 / 4.9 (the measured error
-//           of flat rows lies this far apart from one draw of values to the next: 6.7 / 3.0 and 6.1 / 2.8 on another).
+//           that stay there unless something is larger leave every product off by 2^-36, which for the rows of a long
+//           context over small values (T = 32640, 4 bits, values of deviation 0.03 / 0.01) is 65 / 124 of 1000 outputs off
+//           the nearest fp16 under softmax rows and 129 / 168 under flat ones, where three exact parts leave 4.3 / 2.6 and
+//           6.7 / 3.0, and this 3.9 / 2.2 and 6.1 / 2.6.
 //           Against the three bf16 parts (12 rows, three MFMAs per B operand) this is 8
 //           rows, two MFMAs, a third of the LDS stores and a fifth of the arithmetic of forming them.
 //           The (part, head) rows are packed four to an MFMA; unused rows are zero.
