@@ -129,6 +129,8 @@ class KVmixAttention:
         quantized, the rest as tails of their own."""
         nk = flush_length(key_states.shape[2], self.k_residual_ratio, self.Kgroup_size, self.residual_length, True)
         nv = flush_length(value_states.shape[2], self.v_residual_ratio, self.Vgroup_size, self.residual_length, True)
+        if nk == 0 and nv == 0:
+            return None, key_states.contiguous(), None, None, None, value_states.contiguous(), None, None
         if nk > 0 and nv > 0 and self.Vgroup_size == 32 and self.v_bits != 3:
             # (the prompt is the old tail, nothing is appended to it)
             past = (None, key_states, None, None, None, value_states, None, None, 0)
