@@ -30,6 +30,18 @@ def test_the_plan_names_the_kernel_with_its_pieces():
     assert plan(30, 32, 4, 1024)["kernel"] == "gemv_rows_mfma<30,4,4>"
 
 
+def test_four_heads_fill_the_cus_in_whole_rounds():
+    """Blocks of eight waves are one to a CU, of four waves two.  None of these launches is a little more than one round of them."""
+    for rows in (72, 88, 104, 136, 160, 200, 240):
+        for K in (10016, 20000, 30016):
+            p = plan(2, 4 * rows, 4, K)
+            waves = rows * p["splits"] * p["block"][1]
+            assert waves <= 2048 or waves >= 3300, (rows, K, p)
+    assert (plan(2, 4 * 72, 4, 30016)["splits"], plan(2, 4 * 72, 4, 30016)["block"][1]) == (7, 4)
+    assert (plan(4, 4 * 240, 4, 10016)["splits"], plan(4, 4 * 240, 4, 10016)["block"][1]) == (1, 8)
+    assert (plan(2, 4 * 128, 4, 32640)["splits"], plan(2, 4 * 128, 4, 32640)["block"][1]) == (2, 8)  # (one round as it was)
+
+
 def operands(bits, B, nh, nkv, M, K, seed):
     gen = torch.Generator().manual_seed(seed)
     words = 12 if bits == 30 else 4 * bits
@@ -169,3 +181,18 @@ def test_long_rows_of_four_heads_round_no_more_than_those_of_one(dev):
                 for i, got in enumerate((four, one)):
                     off[i] += int(((got[b:b + 1] - want).abs() > (want.half().double() - want).abs()).sum())
     assert off[1] >= 900 and off[0] <= 1.1 * off[1], off
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 30])
+@pytest.mark.parametrize("B,K", [(20, 9100), (33, 9011)])
+def test_blocks_of_four_waves_of_four_heads(dev, bits, B, K):
+    """More rows than a round of blocks of eight waves holds: blocks of four, several along K, ragged ends."""
+    import KVmix
+
+    assert plan(bits, 32 * B, 4, K)["block"][1] == 4 and plan(bits, 32 * B, 4, K)["splits"] > 1
+    x, code, scale, zero = operands(bits, B, 32, 8, 1, K, K)
+    got = KVmix.quantized_gemm(32, *(t.to(dev) for t in (x, code, scale, zero)), 3 if bits == 30 else bits, *((1,) if bits == 30 else ())).double()
+    for b in range(B):
+        want, size = exact(bits, *(t[b:b + 1].to(dev) for t in (x, code, scale, zero)))
+        assert ((got[b:b + 1] - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -16 * size + 2.0 ** -25).all(), b
