@@ -2092,7 +2092,7 @@ __global__ void __launch_bounds__(64 * kColsWaves)
     // one (recomputed, stored twice with identical values): uniform control flow, no branches.
     // a.ksplit > 1: the block's waves share one tile, each with some of its chunks (and there is one tile per block).
     const int tpw = a.splits;
-    const bool shared = a.ksplit > 1;
+    const bool shared = NREP > 1 && a.ksplit > 1;  // (never with one head, whose code stays without it)
     const int tile0 = shared ? (int)bx : (int)bx * tpw * nw + wy;
     if (ngroups < TG || K < CH) return;  // (never launched so: a tile wider than the row, a chunk longer than K)
     if (tile0 * TG >= ngroups) return;  // (a whole block where its waves share the tile)
