@@ -3557,20 +3557,20 @@ struct RowsPlan {
     int64_t rows_per_split;
 };
 
-// gemv_rows_mfma, four heads, where the waves wanted are more than `target`, what the CUs hold: blocks of eight waves are one to
-// a CU, and 264 of them are two rounds, the second as long as the first.  Of blocks of eight and of four waves, with any
-// number of them along K, those that cost least in chunks that one wave walks after the other (3 us each with two waves per
+// gemv_rows_mfma, four heads, where the waves planned are more than `target`, what the CUs hold: blocks of eight waves are one to
+// a CU, and 264 of them are two rounds, the second as long as the first.  Of blocks of eight and of four waves, with up to
+// `most` of them along K (what a plan of blocks of four would take: the workspace stays as it is), those that cost least in chunks that one wave walks after the other (3 us each with two waves per
 // SIMD): a round is the chunks of a wave and about one more to start and end, four waves alone on a CU are four tenths faster, and
 // a second block along K brings the launch that adds the sums.  Measured, us, 2 bits, wanted -> chosen: 72 rows of 30016 (9
 // sequences of 8 kv heads) four blocks of eight waves 52.3 -> seven of four 35.9; 88 of 30016 65.4 -> 43.3; 104 of 30016 65.7 -> 50.6;
 // 136 of 10016 41.4 -> 29.6; 160 of 10016 42.1 -> 30.5 (38 with blocks of four waves and the kernel's three bf16 parts); 240 of 10016
-// 45.6 -> 37.5; 264 of 10016 64.7 -> 51.
-static void one_round_more_or_less(int64_t batch_rows, int64_t chunks, int64_t target, int64_t &waves, int64_t &splits)
+// 45.6 -> 37.5; 264 of 10016 64.7 -> 53.8.
+static void one_round_more_or_less(int64_t batch_rows, int64_t chunks, int64_t target, int64_t most, int64_t &waves, int64_t &splits)
 {
     int64_t least = INT64_MAX;
-    for (const int64_t w : {8, 4}) {
+    for (const int64_t w : {4, 8}) {
         const int64_t resident = target / w;
-        for (int64_t s = 1; s <= 32 && (s == 1 || s * w <= chunks); s++) {
+        for (int64_t s = 1; s <= most && (s == 1 || s * w <= chunks); s++) {
             const int64_t blocks = batch_rows * s, rounds = (blocks + resident - 1) / resident, last = blocks - (rounds - 1) * resident;
             const int64_t walked = ((chunks + s - 1) / s + w - 1) / w;
             const int64_t cost = 10 * rounds * (walked + 1) - (w == 4 && last <= resident / 2 ? 4 * walked : 0) + (s > 1 ? 15 : 0);
@@ -3620,7 +3620,8 @@ static RowsPlan plan_rows(int64_t batch_rows, int64_t K, int64_t N, int max_wave
     // one block's waves get at most kRowsSingleBlockChunks chunks each
     if (splits > 1 && chunks <= waves * kRowsSingleBlockChunks) splits = 1;
     if (splits > 64) splits = 64;
-    if (max_waves == kRowsMfmaHeadsWaves && batch_rows * splits * waves > target) one_round_more_or_less(batch_rows, chunks, target, waves, splits);
+    if (max_waves == kRowsMfmaHeadsWaves && batch_rows * splits * waves > target)
+        one_round_more_or_less(batch_rows, chunks, target, plan_rows(batch_rows, K, N, kRowsHeadsWaves).splits, waves, splits);
     int64_t rps = (K + splits - 1) / splits;
     rps = (rps + chunk - 1) / chunk * chunk;
     splits = (K + rps - 1) / rps;

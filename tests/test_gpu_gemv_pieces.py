@@ -37,6 +37,12 @@ def test_four_heads_fill_the_cus_in_whole_rounds():
             p = plan(2, 4 * rows, 4, K)
             waves = rows * p["splits"] * p["block"][1]
             assert waves <= 2048 or waves >= 3300, (rows, K, p)
+    for rows in range(8, 600, 8):  # (the workspace is what it would be for blocks of four waves)
+        for K in (1024, 5000, 10016, 30016):
+            most = _lib.load().kvmix_gemv_workspace_bytes(4 * rows, 1, K, 128)
+            p = plan(2, 4 * rows, 4, K)
+            assert p["splits"] == 1 or p["splits"] * 4 * rows * 128 * 4 <= most, (rows, K, p)
+    assert _lib.load().kvmix_gemv_workspace_bytes(4 * 264, 1, 10016, 128) <= 2 << 20
     assert (plan(2, 4 * 72, 4, 30016)["splits"], plan(2, 4 * 72, 4, 30016)["block"][1]) == (7, 4)
     assert (plan(4, 4 * 240, 4, 10016)["splits"], plan(4, 4 * 240, 4, 10016)["block"][1]) == (1, 8)
     assert (plan(2, 4 * 128, 4, 32640)["splits"], plan(2, 4 * 128, 4, 32640)["block"][1]) == (2, 8)  # (one round as it was)
