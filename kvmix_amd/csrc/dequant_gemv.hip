@@ -3559,12 +3559,12 @@ struct RowsPlan {
 
 // gemv_rows_mfma, four heads, where the waves planned are more than `target`, what the CUs hold: blocks of eight waves are one to
 // a CU, and 264 of them are two rounds, the second as long as the first.  Of blocks of eight and of four waves, with up to
-// `most` of them along K (what a plan of blocks of four would take: the workspace stays as it is), those that cost least in chunks that one wave walks after the other (3 us each with two waves per
-// SIMD): a round is the chunks of a wave and about one more to start and end, four waves alone on a CU are four tenths faster, and
-// a second block along K brings the launch that adds the sums.  Measured, us, 2 bits, wanted -> chosen: 72 rows of 30016 (9
-// sequences of 8 kv heads) four blocks of eight waves 52.3 -> seven of four 35.9; 88 of 30016 65.4 -> 43.3; 104 of 30016 65.7 -> 50.6;
-// 136 of 10016 41.4 -> 29.6; 160 of 10016 42.1 -> 30.5 (38 with blocks of four waves and the kernel's three bf16 parts); 240 of 10016
-// 45.6 -> 37.5; 264 of 10016 64.7 -> 53.8.
+// `most` of them along K (what a plan of blocks of four would take: the workspace stays as it is), those that cost least in
+// chunks that one wave walks after the other (3 us each with two waves per SIMD): a round is the chunks of a wave and about one
+// more to start and end, four waves alone on a CU are four tenths faster, and a second block along K brings the launch that adds
+// the sums.  Measured, us, 2 bits, wanted -> chosen: 72 rows of 30016 (9 sequences of 8 kv heads) four blocks of eight waves 52.3
+// -> seven of four 35.9; 88 of 30016 65.4 -> 43.3; 104 of 30016 65.7 -> 50.6; 136 of 10016 41.4 -> 29.6; 160 of 10016 42.1 -> 30.5
+// (38 with blocks of four waves and the kernel's three bf16 parts); 240 of 10016 45.6 -> 37.5; 264 of 10016 64.7 -> 53.8.
 static void one_round_more_or_less(int64_t batch_rows, int64_t chunks, int64_t target, int64_t most, int64_t &waves, int64_t &splits)
 {
     int64_t least = INT64_MAX;
