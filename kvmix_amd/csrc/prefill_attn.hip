@@ -42,7 +42,7 @@ struct PrefillArgs {
     int64_t m_bs, m_hs, m_rs;
     int flag_b, flag_h;        // mask slice of (batch b, head h): b * flag_b + h * flag_h
     const uint8_t *flags;      // [mask slices][key tiles][query parts]: what the tile of a part's 32 queries holds (kHas*)
-    const uint2 *rows;         // [mask slices][query parts][chunks]: bit per query, see kRow*
+    const uint2 *rows;         // [mask slices][query parts][chunks]: bit per query, with an entry not `absorbed` (x), of at least -30000 (y)
     const uint64_t *bits;      // [mask slices][query parts][key tiles][32 queries]: bit 16 j + i = key 4 i + j is masked
     int heads, heads_per_kv, q_len, kv_len, q_tiles, k_tiles, parts, chunks;  // parts: 32 queries each, whole blocks of them
     float scale;
